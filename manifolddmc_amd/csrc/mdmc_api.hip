@@ -67,6 +67,20 @@ mdmc_status fromException(mdmc_ctx* ctx, const std::exception& e) {
     return fail(ctx, MDMC_ERR_HIP, e.what());
 }
 
+// the adjoint's launches; dproc (the processed-grid gradient, outDims points) only with refinement
+void launchAdjoint(const AdjointState& a, const int32_t* map, const int32_t* cell, const float* dL_dpos, float* contrib, float* dproc, float* dL_dfield,
+                   int accumulate, hipStream_t s) {
+    const int64_t P = (int64_t)a.outDims[0] * a.outDims[1] * a.outDims[2], Pin = (int64_t)a.inDims[0] * a.inDims[1] * a.inDims[2];
+    if (a.refinement == 0) {
+        mdmc::launchAdjointVertex(a.g, a.iso, map, cell, a.V, dL_dpos, contrib, accumulate ? nullptr : dL_dfield, Pin, s);
+        mdmc::launchAdjointPoints(a.inDims, a.outDims, a.pad, map, cell, a.V, contrib, dL_dfield, accumulate, s);
+    } else {
+        mdmc::launchAdjointVertex(a.g, a.iso, map, cell, a.V, dL_dpos, contrib, dproc, P, s);
+        mdmc::launchAdjointPoints(a.outDims, a.outDims, 0, map, cell, a.V, contrib, dproc, 0, s);
+        mdmc::launchPrepareAdjoint(a.inDims, a.outDims, a.refinement, a.pad, dproc, dL_dfield, accumulate, s);
+    }
+}
+
 struct DeviceGuard {
     int prev = -1;
     explicit DeviceGuard(int dev) {
@@ -472,15 +486,7 @@ mdmc_status mdmc_backward_noalloc(mdmc_ctx* ctx, const float* dL_dpos, float* dL
     const int32_t* cell = p.arena.ptr<int32_t>("gp_vcell");
     // contributions at the start of the scratch, the processed-grid gradient after them (both
     // written in full by their kernels, so nothing from an earlier call needs clearing)
-    float* contrib = base;
-    mdmc::launchAdjointVertex(a.g, a.iso, map, cell, a.V, dL_dpos, contrib, s);
-    if (direct) {
-        mdmc::launchAdjointGather(a.g, map, contrib, dL_dfield, accumulate ? 1 : 0, s);
-    } else {
-        float* dproc = base + 8 * a.V;
-        mdmc::launchAdjointGather(a.g, map, contrib, dproc, 0, s);
-        mdmc::launchPrepareAdjoint(a.inDims, a.outDims, a.refinement, a.pad, dproc, dL_dfield, accumulate ? 1 : 0, s);
-    }
+    launchAdjoint(a, map, cell, dL_dpos, base, base + 8 * a.V, dL_dfield, accumulate ? 1 : 0, s);
     if (hipGetLastError() != hipSuccess) return fail(ctx, MDMC_ERR_HIP, "mdmc_backward_noalloc: kernel launch failed");
     return MDMC_OK;
 }
@@ -499,15 +505,9 @@ mdmc_status mdmc_backward(mdmc_ctx* ctx, const float* dL_dpos, float* dL_dfield,
         const int32_t* map = p.arena.ptr<int32_t>("adj_map");
         const int32_t* cell = p.arena.ptr<int32_t>("gp_vcell");
         float* contrib = p.arena.get<float>("adj_contrib", 8 * (size_t)std::max<int64_t>(a.V, 1));
-        mdmc::launchAdjointVertex(a.g, a.iso, map, cell, a.V, dL_dpos, contrib, s);
-        if (a.pad == 0 && a.refinement == 0) {
-            mdmc::launchAdjointGather(a.g, map, contrib, dL_dfield, accumulate ? 1 : 0, s);
-        } else {
-            const int64_t P = (int64_t)a.outDims[0] * a.outDims[1] * a.outDims[2];
-            float* dproc = p.arena.get<float>("adj_dproc", (size_t)P);
-            mdmc::launchAdjointGather(a.g, map, contrib, dproc, 0, s);
-            mdmc::launchPrepareAdjoint(a.inDims, a.outDims, a.refinement, a.pad, dproc, dL_dfield, accumulate ? 1 : 0, s);
-        }
+        const size_t P = (size_t)a.outDims[0] * a.outDims[1] * a.outDims[2];
+        float* dproc = a.refinement ? p.arena.get<float>("adj_dproc", P) : nullptr;
+        launchAdjoint(a, map, cell, dL_dpos, contrib, dproc, dL_dfield, accumulate ? 1 : 0, s);
         MDMC_HIP(hipGetLastError());
         return MDMC_OK;
     } catch (const std::exception& e) {
