@@ -218,6 +218,11 @@ mdmc_status mdmc_backward(mdmc_ctx* ctx, const float* dL_dpos, float* dL_dfield,
  * race, so serialise them.  Asynchronous on the context's stream. */
 mdmc_status mdmc_backward_noalloc(mdmc_ctx* ctx, const float* dL_dpos, float* dL_dfield, int32_t accumulate);
 
+/* The surface as an autograd graph holds it (no reference counterpart): positions float[3*nV] and
+ * the faces' vertex ids int64[4*nF] in walk order (Mesh.cu:446-506), device buffers; either may be
+ * NULL.  Asynchronous on the context's stream, like mdmc_backward. */
+mdmc_status mdmc_mesh_quads(const mdmc_ctx* ctx, float* positions, int64_t* quads);
+
 /* Triangle index buffer, two triangles per face (x,y,z),(z,w,x): HalfedgeMesh.cu:690-714.
  * indices uint32[6*nF], device or host. */
 mdmc_status mdmc_mesh_triangles(const mdmc_ctx* ctx, uint32_t* indices, int32_t dst_on_device);

@@ -106,7 +106,7 @@ EXPORTS = ["mdmc_create", "mdmc_destroy", "mdmc_last_error", "mdmc_set_stream", 
            "mdmc_extract_batch", "mdmc_batch_offsets", "mdmc_batch_stats", "mdmc_set_tile_shape", "mdmc_get_tile_shape",
            "mdmc_generate_surface", "mdmc_generate_edge_case", "mdmc_mesh_face_colors", "mdmc_mesh_triangulate_maxmin",
            "mdmc_backward_noalloc", "mdmc_set_graphs", "mdmc_get_graph_replays", "mdmc_processed_grid",
-           "mdmc_set_local_merges", "mdmc_set_sequential_merges"]
+           "mdmc_set_local_merges", "mdmc_set_sequential_merges", "mdmc_mesh_quads"]
 
 
 def lib():
@@ -140,6 +140,8 @@ def lib():
         L.mdmc_mesh_get_info.restype = i32
         L.mdmc_mesh_copy.argtypes = [vp] + [vp] * 7 + [i32]
         L.mdmc_mesh_copy.restype = i32
+        L.mdmc_mesh_quads.argtypes = [vp, vp, vp]
+        L.mdmc_mesh_quads.restype = i32
         L.mdmc_mesh_triangles.argtypes = [vp, vp, i32]
         L.mdmc_mesh_triangles.restype = i32
         L.mdmc_mesh_render_vertices.argtypes = [vp, vp, i32]
@@ -422,6 +424,11 @@ class DualMarchingCubes:
         p = lambda a: ctypes.c_void_p(a) if a else None
         self._check(lib().mdmc_mesh_copy(self._ctx, p(positions), p(normals), p(halfedges), p(face_halfedge), p(face_attr),
                                          p(vertex_flags), p(vertex_halfedge), 1))
+
+    def copy_quads(self, positions=0, quads=0):
+        """mdmc_mesh_quads into device buffers given by pointer (0 = skip): positions float32 [V, 3], the
+        faces' vertex ids int64 [F, 4].  Asynchronous on the context's stream."""
+        self._check(lib().mdmc_mesh_quads(self._ctx, ctypes.c_void_p(positions), ctypes.c_void_p(quads)))
 
     def mesh_torch(self):
         """The resident mesh copied into new torch tensors on the context's device (needs torch):

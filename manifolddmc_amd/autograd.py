@@ -31,17 +31,9 @@ class DMCFunction(torch.autograd.Function):
         dmc.extract_raw(field.data_ptr(), (nx, ny, nz), origin, delta, float(iso), flags, refinement, True)
         V, H, F = dmc.info()
         pos = torch.empty((V, 3), dtype=torch.float32, device=field.device)
-        he = torch.empty((H, 4), dtype=torch.int32, device=field.device)
-        fh = torch.empty((F,), dtype=torch.int32, device=field.device)
-        if V:
-            dmc.copy_device(positions=pos.data_ptr(), halfedges=he.data_ptr() if H else 0, face_halfedge=fh.data_ptr() if F else 0)
-        # quads from the halfedge cycles: first halfedge of each face, then three next steps
         quads = torch.empty((F, 4), dtype=torch.int64, device=field.device)
-        if F:
-            h = fh.long()
-            for i in range(4):
-                quads[:, i] = he[h, 0].long()
-                h = he[h, 2].long()
+        if V:
+            dmc.copy_quads(pos.data_ptr(), quads.data_ptr() if F else 0)
         ctx.dmc = dmc
         ctx.generation = dmc.generation
         ctx.shape = field.shape

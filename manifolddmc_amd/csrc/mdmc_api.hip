@@ -539,6 +539,21 @@ mdmc_status mdmc_mesh_copy(const mdmc_ctx* cctx, float* positions, float* normal
     }
 }
 
+mdmc_status mdmc_mesh_quads(const mdmc_ctx* cctx, float* positions, int64_t* quads) {
+    mdmc_ctx* ctx = const_cast<mdmc_ctx*>(cctx);
+    if (!ctx) return MDMC_ERR_INVALID_ARG;
+    if (!ctx->hasResult) return fail(ctx, MDMC_ERR_NO_RESULT, "no extraction result");
+    DeviceGuard dg(ctx->device);
+    try {
+        mdmc::Pipeline& p = ctx->p;
+        mdmc::launchQuadIds(p.arena.ptr<int4>("he"), p.arena.ptr<int32_t>("face_he"), p.F, p.arena.ptr<float>("pos"), p.V, positions, quads, p.stream);
+        MDMC_HIP(hipGetLastError());
+        return MDMC_OK;
+    } catch (const std::exception& e) {
+        return fromException(ctx, e);
+    }
+}
+
 mdmc_status mdmc_mesh_triangles(const mdmc_ctx* cctx, uint32_t* indices, int32_t dst_on_device) {
     mdmc_ctx* ctx = const_cast<mdmc_ctx*>(cctx);
     if (!ctx || !indices) return MDMC_ERR_INVALID_ARG;

@@ -129,6 +129,36 @@ __global__ void kTriangles(const int4* __restrict__ he, const int32_t* __restric
     o[3] = v[2]; o[4] = v[3]; o[5] = v[0];
 }
 
+// The faces' vertex ids as 64-bit indices (thread f < nq walks face f; its four records share a
+// 64-byte line, so the walk costs one miss), and the positions in the blocks after them.
+// Launch-bound at the sizes an optimisation loop uses: the ids through torch (first halfedge,
+// then three gathers of origin and next) were 24 kernels of 3-6 us each.
+__global__ void kQuadIds(const int4* __restrict__ he, const int32_t* __restrict__ face_he, int64_t nq, const float* __restrict__ src, int64_t n3,
+                         float* __restrict__ positions, int64_t* __restrict__ quads, int64_t qBlocks) {
+    if (blockIdx.x < qBlocks) {
+        const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+        if (f >= nq) return;
+        int h = face_he[f];
+        int64_t v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int4 e = he[h];
+            v[i] = e.x;
+            h = e.z;
+        }
+        longlong2* o = reinterpret_cast<longlong2*>(quads + 4 * f);
+        if ((((uintptr_t)quads) & 15) == 0) {
+            o[0] = make_longlong2(v[0], v[1]);
+            o[1] = make_longlong2(v[2], v[3]);
+        } else {
+            for (int i = 0; i < 4; ++i) quads[4 * f + i] = v[i];
+        }
+        return;
+    }
+    const int64_t i = ((int64_t)blockIdx.x - qBlocks) * blockDim.x + threadIdx.x;
+    if (i < n3) positions[i] = src[i];
+}
+
 // LazyEngine::Color::HSVtoRGB (LazyEngine/Renderer/Materials/Colors.h:15-56)
 __device__ __forceinline__ f3 hsvToRgb(float h, float sat, float val) {
     float f = h / 60.0f;
@@ -194,6 +224,11 @@ void launchPrepareGrids(const PrepareDesc* descDev, int G, int64_t blocks, int r
 
 void launchDmcTrianglesFromFaces(const int4* he, const int32_t* face_he, int64_t F, uint32_t* idx, hipStream_t s) {
     if (F > 0) kTriangles<<<gridFor(F), kBlock, 0, s>>>(he, face_he, F, idx);
+}
+
+void launchQuadIds(const int4* he, const int32_t* face_he, int64_t F, const float* src, int64_t V, float* positions, int64_t* quads, hipStream_t s) {
+    const int64_t qb = quads ? (F + kBlock - 1) / kBlock : 0, pb = positions ? (3 * V + kBlock - 1) / kBlock : 0;
+    if (qb + pb > 0) kQuadIds<<<(unsigned)(qb + pb), kBlock, 0, s>>>(he, face_he, F, src, 3 * V, positions, quads, qb);
 }
 
 void launchRenderVertices(const int4* he, int64_t H, const float* pos, const float* nrm, const uint32_t* vflags, float* out, hipStream_t s) {
