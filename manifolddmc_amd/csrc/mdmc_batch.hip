@@ -263,14 +263,13 @@ int32_t* Pipeline::stableSortByKey(const int32_t* key, int64_t n, int B, const s
     int32_t* flag = arena.get<int32_t>("sort_flag", (size_t)std::max<int64_t>(n, 1));
     int64_t* pre = arena.get<int64_t>("sort_pre", (size_t)n + 1);
     int64_t* zeros = arena.get<int64_t>("sort_zeros", 1);
-    void* scratch = arena.get<char>("sort_scan", scanScratchBytes(n + 1));
     if (n == 0) return a;
     kIota<<<gridFor(n), kBlock, 0, stream>>>(a, n);
     int bits = 0;
     while ((1 << bits) < B) ++bits;
     for (int bit = 0; bit < bits; ++bit) {
         kSplitFlags<<<gridFor(n), kBlock, 0, stream>>>(a, key, n, bit, flag);
-        scanExclusiveI32(flag, pre, n, zeros, scratch, stream, lookbackDiag());
+        scan(flag, pre, n, zeros);
         kSplitScatter<<<gridFor(n), kBlock, 0, stream>>>(a, flag, pre, n, zeros, b);
         std::swap(a, b);
     }

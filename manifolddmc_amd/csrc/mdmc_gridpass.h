@@ -59,6 +59,9 @@ struct GridPassArgs {
     // per active cell (concatenated cell index): vertex index inside its tile (14 bits) and the
     // contour of each edge a later cell's quads read (2 bits each for edges 1,2,4,5,6,7,9,10,11)
     uint32_t* cellMap;
+    // look-back words that classify clears for the scan of the tile counts
+    unsigned long long* lb;
+    int64_t lbWords;
     // exclusive prefix of tileV / tileQ: each tile's first vertex / quad
     const int64_t* tileVOff;
     const int64_t* tileQOff;

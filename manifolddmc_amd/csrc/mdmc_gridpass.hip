@@ -429,6 +429,7 @@ __global__ void __launch_bounds__(GP_THREADS) kClassify(GridPassArgs a, int chun
     __shared__ int64_t s_t;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wid = tid >> 6;
+    for (int64_t i = (int64_t)blockIdx.x * GP_THREADS + tid; i < a.lbWords; i += (int64_t)gridDim.x * GP_THREADS) a.lb[i] = 0;
     // the two small tables in LDS (read after the first barrier below)
     s_base[tid] = c_polyBase[tid];
     for (int i = tid; i < kPolyTabSize; i += GP_THREADS) s_tab[i] = c_polyCmap[i];

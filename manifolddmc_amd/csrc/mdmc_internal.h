@@ -17,18 +17,27 @@ struct GridDev {
     float dx, dy, dz;
 };
 
-// --- scans (mdmc_scan.hip): exclusive prefix of n int32 values into int64,
-// returns the total through *total_dev (device int64).  scratch is sized by scanScratchBytes.
-// The result is exact in every case; a tile whose look-back wait passed its spin limit
-// summed its prefix directly and adds 1 to *directOut (when given; device memory), a
-// diagnostic only.
-size_t scanScratchBytes(int64_t n);
-// total_dev may point into mapped pinned host memory
-void scanExclusiveI32(const int32_t* in, int64_t* out, int64_t n, int64_t* total_dev, void* scratch, hipStream_t s, int64_t* directOut = nullptr);
+// --- scans (mdmc_scan.hip): exclusive prefix of n int32 values into int64 offsets, the total
+// through *total (device or mapped pinned host memory; may be null); up to kScanJobs arrays in
+// one launch, each with scanTiles(n) look-back words of its own.  The words are either all zero
+// (epoch 0) or hold nothing of this epoch.  The result is exact in every case; a tile whose
+// look-back wait passed its spin limit summed its prefix directly and adds 1 to *directOut
+// (device memory), a diagnostic only.
+constexpr int kScanTile = 4096, kScanJobs = 3;
+// at least one tile: an empty array's total is written too
+__host__ __device__ inline int64_t scanTiles(int64_t n) { return n > 0 ? (n + kScanTile - 1) / kScanTile : 1; }
+struct ScanJob {
+    const int32_t* in;
+    int64_t* out;
+    int64_t n;
+    int64_t* total;
+    unsigned long long* words;
+};
+void scanExclusiveI32(const ScanJob* jobs, int count, uint32_t epoch, hipStream_t s, int64_t* directOut);
 // stream compaction in one pass: the i < n with (attr[i] & mask) != 0, ascending, into
-// idx (capacity n); the count through *total_dev; scratch sized by scanScratchBytes(n)
-void compactFlagged(const uint32_t* attr, int64_t n, uint32_t mask, int32_t* idx, int64_t* total_dev, void* scratch, hipStream_t s,
-                    int64_t* directOut = nullptr);
+// idx (capacity n); the count through *total
+void compactFlagged(const uint32_t* attr, int64_t n, uint32_t mask, int32_t* idx, int64_t* total, unsigned long long* words, uint32_t epoch,
+                    hipStream_t s, int64_t* directOut);
 
 inline unsigned gridFor(int64_t n, int block = kBlock) { return (unsigned)((n + block - 1) / block); }
 

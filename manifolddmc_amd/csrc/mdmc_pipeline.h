@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <initializer_list>
 #include <map>
 #include <string>
 #include <vector>
@@ -161,6 +162,18 @@ class Pipeline {
     int64_t* nmSlotParts();
     int64_t* nmFoundParts();
     int64_t scan32(const int32_t* in, int64_t n, const std::string& outName, int64_t** out);
+    // exclusive prefix sums in one launch (words of the jobs are set here); total may be null
+    void scan(std::initializer_list<ScanJob> jobs);
+    void scan(const int32_t* in, int64_t* out, int64_t n, int64_t* total = nullptr) { scan({ScanJob{in, out, n, total, nullptr}}); }
+    // look-back words for one launch over `words` tiles: the launches of a stream run one after
+    // the other, so all share one buffer, told apart by the epoch (cleared when the buffer is
+    // new and before the 16-bit epochs repeat)
+    struct Lookback {
+        unsigned long long* words;
+        uint32_t epoch;
+    };
+    Lookback lookback(int64_t words);
+    uint32_t lbEpoch_ = 0;
     int64_t compactNM(int32_t* nm);
     void zero(void* p, size_t bytes);
     void fillNeg(void* p, size_t bytes);

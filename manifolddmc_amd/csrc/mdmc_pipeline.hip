@@ -1493,7 +1493,7 @@ template <int R>
 __global__ void __launch_bounds__(kLbBlock) kCompactVertices(const int32_t* __restrict__ vtype, int64_t V, int dropType, const uint8_t* __restrict__ vdead,
                                                              const int32_t* __restrict__ pid, const int32_t* __restrict__ vslot, int32_t* __restrict__ npid,
                                                              int32_t* __restrict__ address, int32_t* __restrict__ oldV, int32_t* __restrict__ nvslot,
-                                                             int64_t numTiles, unsigned long long* __restrict__ status, int64_t* __restrict__ total,
+                                                             int64_t numTiles, unsigned long long* __restrict__ status, uint32_t epoch, int64_t* __restrict__ total,
                                                              int64_t* __restrict__ directOut) {
     __shared__ int s_cnt[R * (kLbBlock / 64)], s_pre[R * (kLbBlock / 64) + 1];
     __shared__ long long s_off;
@@ -1513,7 +1513,7 @@ __global__ void __launch_bounds__(kLbBlock) kCompactVertices(const int32_t* __re
     const int tileSum = lbBlockRanks<R>(m, s_cnt, s_pre);
     if (threadIdx.x < 64)
         lbTileOffset(
-            status, t, tileSum,
+            status, epoch, t, tileSum,
             [&](int l) {
                 int64_t c = 0;
                 for (int64_t e = l; e < base; e += 64) c += keepOf(e) ? 1 : 0;
@@ -1611,7 +1611,7 @@ __device__ __forceinline__ void compactQuad(int64_t q, bool kept, int64_t d, con
 // order (tile counts, block ranks, look-back) into qnew, -1 for removed ones
 template <int R>
 __global__ void __launch_bounds__(kLbBlock) kNumberQuads(const uint32_t* __restrict__ attr, int64_t Q, int32_t* __restrict__ qnew, int64_t numTiles,
-                                                         unsigned long long* __restrict__ status, int64_t* __restrict__ total,
+                                                         unsigned long long* __restrict__ status, uint32_t epoch, int64_t* __restrict__ total,
                                                          int64_t* __restrict__ directOut) {
     __shared__ int s_cnt[R * (kLbBlock / 64)], s_pre[R * (kLbBlock / 64) + 1];
     __shared__ long long s_off;
@@ -1632,7 +1632,7 @@ __global__ void __launch_bounds__(kLbBlock) kNumberQuads(const uint32_t* __restr
     const int tileSum = lbBlockRanks<R>(m, s_cnt, s_pre);
     if (threadIdx.x < 64)
         lbTileOffset(
-            status, t, tileSum,
+            status, epoch, t, tileSum,
             [&](int l) {
                 int64_t c = 0;
                 for (int64_t e = l; e < base; e += 64) c += keepOf(e) ? 1 : 0;
@@ -2691,23 +2691,48 @@ const uint8_t* Pipeline::canonFlags() { return canonTracked ? arena.ptr<uint8_t>
 
 const int32_t* Pipeline::vertexSlots() { return posSlotted ? arena.ptr<int32_t>("vslot") : nullptr; }
 
+Pipeline::Lookback Pipeline::lookback(int64_t words) {
+    const size_t before = arena.capacity<unsigned long long>("lb_words");
+    unsigned long long* w = arena.get<unsigned long long>("lb_words", (size_t)words);
+    const size_t cap = arena.capacity<unsigned long long>("lb_words");
+    if (cap != before || lbEpoch_ == 0xFFFFu) {
+        launchFill(w, 0x00, cap * sizeof(unsigned long long));
+        lbEpoch_ = 0;
+    }
+    return Lookback{w, ++lbEpoch_};
+}
+
+void Pipeline::scan(std::initializer_list<ScanJob> jobs) {
+    ScanJob j[kScanJobs];
+    int count = 0;
+    int64_t words = 0;
+    for (const ScanJob& x : jobs) words += scanTiles(x.n);
+    const Lookback lb = lookback(words);
+    words = 0;
+    for (const ScanJob& x : jobs) {
+        j[count] = x;
+        j[count++].words = lb.words + words;
+        words += scanTiles(x.n);
+    }
+    scanExclusiveI32(j, count, lb.epoch, stream, lookbackDiag());
+}
+
 int64_t Pipeline::scan32(const int32_t* in, int64_t n, const std::string& outName, int64_t** out) {
     *out = arena.get<int64_t>(outName, (size_t)n + 1);
-    void* scratch = arena.get<char>("scan_scratch", scanScratchBytes(n + 1));
     // total straight into pinned host memory
     int64_t* h = pinHost();
     int64_t* d = pinDev();
-    scanExclusiveI32(in, *out, n, d + 1, scratch, stream, lookbackDiag());
+    scan(in, *out, n, d + 1);
     MDMC_HIP(hipStreamSynchronize(stream));
     return h[1];
 }
 
 // the faces with the NM bit, ascending, into nm (capacity F); returns their number
 int64_t Pipeline::compactNM(int32_t* nm) {
-    void* scratch = arena.get<char>("scan_scratch", scanScratchBytes(F + 1));
     int64_t* h = pinHost();
     int64_t* d = pinDev();
-    compactFlagged(arena.ptr<uint32_t>("fattr"), F, (uint32_t)QA_NM, nm, d + 1, scratch, stream, lookbackDiag());
+    const Lookback lb = lookback(scanTiles(F));
+    compactFlagged(arena.ptr<uint32_t>("fattr"), F, (uint32_t)QA_NM, nm, d + 1, lb.words, lb.epoch, stream, lookbackDiag());
     // with the count, the invalid-record counter: a refresh's face walks add to it
     if (refreshUnchecked) MDMC_HIP(hipMemcpyAsync(h + 2, counters() + A_INVALID, sizeof(int64_t), hipMemcpyDeviceToHost, stream));
     MDMC_HIP(hipStreamSynchronize(stream));
@@ -2808,15 +2833,12 @@ void Pipeline::slabPass(std::vector<ProblemDev>& problems, int64_t C, int shape,
     int64_t* sqo = arena.get<int64_t>("gp_segqo", (size_t)segs + 1);
     a.segVOff = svo;
     a.segQOff = sqo;
-    void* scratchV = arena.get<char>("scan_scratch", scanScratchBytes(segs + 1));
-    void* scratchQ = arena.get<char>("scan_scratch2", scanScratchBytes(segs + 1));
     int64_t* h = pinHost();
     int64_t* pd = pinDev();
     h[1] = h[2] = 0;
     MDMC_HIP(hipEventRecord(kev[0], stream));
     launchSlabCount(shape, a, stream);
-    scanExclusiveI32(a.segV, svo, segs + 1, pd + 1, scratchV, stream, lookbackDiag());
-    scanExclusiveI32(a.segQ, sqo, segs + 1, pd + 2, scratchQ, stream, lookbackDiag());
+    scan({ScanJob{a.segV, svo, segs + 1, pd + 1, nullptr}, ScanJob{a.segQ, sqo, segs + 1, pd + 2, nullptr}});
     MDMC_HIP(hipEventRecord(kev[1], stream));
     MDMC_HIP(hipStreamSynchronize(stream));
     V = h[1];
@@ -2909,7 +2931,7 @@ void Pipeline::dmc(std::vector<ProblemDev>& problems, bool surfIter, bool record
 std::vector<int64_t> Pipeline::frontBuffers() {
     std::vector<int64_t> b;
     for (const char* n : {"counters", "grid", "prep_desc", "gp_probs", "gp_queue", "gp_rec", "gp_tv", "gp_tq", "gp_tna", "gp_map", "gp_tvo", "gp_tqo",
-                          "scan_scratch", "scan_scratch2"})
+                          "gp_lb"})
         b.push_back((int64_t)(intptr_t)arena.ptr<char>(n));
     b.push_back((int64_t)(intptr_t)pinDev());
     return b;
@@ -3028,15 +3050,18 @@ void Pipeline::gridPassFront(std::vector<ProblemDev>& problems, int64_t C, int s
     int64_t* tqo = arena.get<int64_t>("gp_tqo", (size_t)numTiles + 1);
     a.tileVOff = tvo;
     a.tileQOff = tqo;
-    void* scratchV = arena.get<char>("scan_scratch", scanScratchBytes(numTiles + 1));
-    void* scratchQ = arena.get<char>("scan_scratch2", scanScratchBytes(numTiles + 1));
+    // look-back words of the two scans of the tile counts, cleared by classify (a captured launch
+    // replays its epoch, so this part goes without)
+    const int64_t words = scanTiles(numTiles + 1);
+    a.lb = arena.get<unsigned long long>("gp_lb", 2 * (size_t)words);
+    a.lbWords = 2 * words;
     // totals straight into pinned host memory: [1] V, [2] Q
     int64_t* pd = pinDev();
     if (events) MDMC_HIP(hipEventRecord(kev[0], stream));
     launchGridClassify(shape, a, stream);
     if (numTiles > 0) {
-        scanExclusiveI32(a.tileV, tvo, numTiles + 1, pd + 1, scratchV, stream, lookbackDiag());
-        scanExclusiveI32(a.tileQ, tqo, numTiles + 1, pd + 2, scratchQ, stream, lookbackDiag());
+        const ScanJob jobs[2] = {{a.tileV, tvo, numTiles + 1, pd + 1, a.lb}, {a.tileQ, tqo, numTiles + 1, pd + 2, a.lb + words}};
+        scanExclusiveI32(jobs, 2, 0, stream, lookbackDiag());
     } else {
         zero(pd + 1, 2 * sizeof(int64_t));
     }
@@ -3083,8 +3108,7 @@ void Pipeline::buildBuckets(const int32_t* list, int64_t n) {
     int4* he = arena.ptr<int4>("he");
     int32_t* degM = arena.ptr<int32_t>("degM");
     int64_t* offM = arena.get<int64_t>("offM", (size_t)V + 1);
-    void* scratch = arena.get<char>("scan_scratch", scanScratchBytes(V + 1));
-    scanExclusiveI32(degM, offM, V + 1, arena.get<int64_t>("scan_total", 1), scratch, stream, lookbackDiag());
+    scan(degM, offM, V + 1);
     int2* A = arena.get<int2>("listA", (size_t)std::max<int64_t>(H, 1));
     int32_t* bsize = arena.ptr<int32_t>("bsize");
     int32_t* brank = arena.ptr<int32_t>("brank");
@@ -3133,8 +3157,7 @@ void Pipeline::halfedgeInitialize() {
     // corner vertices' contours: no counting atomics
     zero(cnt + V, sizeof(int32_t));
     int64_t* off = arena.get<int64_t>("out_off", (size_t)V + 1);
-    scanExclusiveI32(cnt, off, V + 1, arena.get<int64_t>("scan_total", 1), arena.get<char>("scan_scratch", scanScratchBytes(V + 1)), stream,
-                     lookbackDiag());
+    scan(cnt, off, V + 1);
     int32_t* out = arena.get<int32_t>("out_list", (size_t)std::max<int64_t>(H, 1));
     int2* ends = arena.get<int2>("out_ends", (size_t)std::max<int64_t>(H, 1));
     launchQuadLists(quads, qattr, Q, V, arena.ptr<int32_t>("gp_vcell"), arena.ptr<uint16_t>("gp_vct"), pid(), probsDev, off, out, ends, face_he, fattr,
@@ -3265,8 +3288,6 @@ void Pipeline::simplifyCompactAndRebuild(int dropType, bool p3333) {
     // both totals; the outputs are sized for the inputs (at most as many are kept)
     constexpr int RV = 16, RQ = 16;  // rounds per tile (tiles of 4096 elements)
     const int64_t tV = (V + RV * kLbBlock - 1) / (RV * kLbBlock), tQ = (Q + RQ * kLbBlock - 1) / (RQ * kLbBlock);
-    unsigned long long* sv = arena.get<unsigned long long>("compact_lb_v", (size_t)std::max<int64_t>(tV, 1));
-    unsigned long long* sq = arena.get<unsigned long long>("compact_lb_q", (size_t)std::max<int64_t>(tQ, 1));
     int32_t* address = arena.get<int32_t>("vaddress", (size_t)std::max<int64_t>(V, 1));  // written for every vertex below
     // the compacted arrays go to the second buffers, which then swap with the primary ones;
     // both are sized for the grid pass's output so that later extractions of the same
@@ -3286,19 +3307,19 @@ void Pipeline::simplifyCompactAndRebuild(int dropType, bool p3333) {
     int32_t* outdeg = chained ? arena.ptr<int32_t>("outdeg") : nullptr;
     {
         FillBatch fb(*this);
-        fb.add(sv, 0x00, (size_t)tV * sizeof(unsigned long long));
-        fb.add(sq, 0x00, (size_t)tQ * sizeof(unsigned long long));
         if (removedAt) fb.add(removedAt, 0x00, (size_t)V * sizeof(int32_t));
     }
     // totals straight into pinned host memory: [1] V, [2] Q
     int64_t* h = pinHost();
     int64_t* pd = pinDev();
     h[1] = h[2] = 0;
+    const Lookback lbV = lookback(std::max<int64_t>(tV, 1));
     if (V > 0)
         kCompactVertices<RV><<<(unsigned)tV, kLbBlock, 0, stream>>>(vtype, V, dropType, chained ? arena.ptr<uint8_t>("vdead") : nullptr, pid(), vertexSlots(),
-                                                                npid, address, oldV, nvslot, tV, sv, pd + 1, lookbackDiag());
+                                                                npid, address, oldV, nvslot, tV, lbV.words, lbV.epoch, pd + 1, lookbackDiag());
     if (Q > 0) {
-        kNumberQuads<RQ><<<(unsigned)tQ, kLbBlock, 0, stream>>>(attr, Q, qnew, tQ, sq, pd + 2, lookbackDiag());
+        const Lookback lbQ = lookback(tQ);
+        kNumberQuads<RQ><<<(unsigned)tQ, kLbBlock, 0, stream>>>(attr, Q, qnew, tQ, lbQ.words, lbQ.epoch, pd + 2, lookbackDiag());
         kCompactQuads<<<gridFor(Q), kBlock, 0, stream>>>(quads, attr, Q, vtarget, address, p3333 ? 1 : 0, nquads, nattr, oldQ, qnew, removedAt, outdeg,
                                                          V, counters());
     }
@@ -3324,8 +3345,7 @@ void Pipeline::simplifyCompactAndRebuild(int dropType, bool p3333) {
     zero(cnt + nV, sizeof(int32_t));
     if (nV > 0) kOutCount<<<gridFor(nV), kBlock, 0, stream>>>(oldV, nV, off, removedAt, srcHead, srcNext, outdeg, cnt);
     int64_t* off2 = arena.get<int64_t>("out_off2", (size_t)std::max<int64_t>(nV, dmcV) + 1);
-    scanExclusiveI32(cnt, off2, nV + 1, arena.get<int64_t>("scan_total", 1), arena.get<char>("scan_scratch", scanScratchBytes(nV + 1)), stream,
-                     lookbackDiag());
+    scan(cnt, off2, nV + 1);
     int32_t* out2 = arena.get<int32_t>("out_list2", 4 * capQ);
     if (nV > 0)
         kOutFill<<<gridFor(nV), kBlock, 0, stream>>>(oldV, nV, off, out, qnew, srcHead, srcNext, off2, out2, nH, counters());
@@ -3584,9 +3604,7 @@ void Pipeline::split(int step, int maxIters) {
             int64_t* hp = pinHost();
             int64_t* dp = pinDev();
             hp[1] = hp[2] = hp[3] = 0;
-            scanExclusiveI32(pv, av, vsize, dp + 1, arena.get<char>("cb_scan_v", scanScratchBytes(vsize + 1)), stream, lookbackDiag());
-            scanExclusiveI32(ph, ah, hsize, dp + 2, arena.get<char>("cb_scan_h", scanScratchBytes(hsize + 1)), stream, lookbackDiag());
-            scanExclusiveI32(pf, af, fsize, dp + 3, arena.get<char>("cb_scan_f", scanScratchBytes(fsize + 1)), stream, lookbackDiag());
+            scan({ScanJob{pv, av, vsize, dp + 1, nullptr}, ScanJob{ph, ah, hsize, dp + 2, nullptr}, ScanJob{pf, af, fsize, dp + 3, nullptr}});
             MDMC_HIP(hipStreamSynchronize(stream));
             const int64_t addV = hp[1], addH = hp[2], addF = hp[3];
             // vertices
@@ -3659,8 +3677,7 @@ void Pipeline::buildMergeList(const int2* rec, int64_t R, int count, int32_t* nu
     if (R > 0) kRecCount<<<gridFor(R), kBlock, 0, stream>>>(rec, R, count, cnt, counters());
     // offsets only: the total is not needed on the host
     int64_t* roff = arena.get<int64_t>(tag + "_off", (size_t)count + 2);
-    scanExclusiveI32(cnt, roff, count + 1, arena.get<int64_t>(tag + "_tot", 1), arena.get<char>(tag + "_scan", scanScratchBytes(count + 1)), stream,
-                     lookbackDiag());
+    scan(cnt, roff, count + 1);
     int32_t* cursor = arena.get<int32_t>(tag + "_cur", (size_t)count + 1);
     zero(cursor, ((size_t)count + 1) * sizeof(int32_t));
     int32_t* idx = arena.get<int32_t>(tag + "_idx", (size_t)R);
@@ -3706,8 +3723,7 @@ void Pipeline::detectNonManifoldVertices() {
     int32_t* deg = arena.get<int32_t>("deg", (size_t)V + 1);
     kSlowDegree<<<gridFor(V + 1), kBlock, 0, stream>>>(slow, outdeg, V, deg);
     int64_t* off = arena.get<int64_t>("off", (size_t)V + 1);
-    void* scratch = arena.get<char>("scan_scratch", scanScratchBytes(V + 1));
-    scanExclusiveI32(deg, off, V + 1, arena.get<int64_t>("scan_total", 1), scratch, stream, lookbackDiag());
+    scan(deg, off, V + 1);
     int32_t* list = arena.get<int32_t>("list", (size_t)H);
     const bool copyLists = nSlowOff == 0;  // every slow vertex keeps the build's list
     if (copyLists) kCopySlowLists<<<gridFor(V), kBlock, 0, stream>>>(slow, V, arena.ptr<int64_t>("out_off"), arena.ptr<int32_t>("out_list"), off, list);

@@ -13,9 +13,10 @@
 // slower), then publishes as usual, so a tile that waits on an unstarted one still ends
 // and frees its slot.
 //
-// Look-back words pack flag (2 bits) and value (62 bits), so relaxed device-scope
-// atomics suffice: a reader needs nothing beyond the word it reads.
+// Look-back words pack flag, the launch's epoch and value (mdmc_lookback.h), so relaxed
+// device-scope atomics suffice: a reader needs nothing beyond the word it reads.
 #include "mdmc_internal.h"
+#include "mdmc_lookback.h"
 
 namespace mdmc {
 
@@ -23,34 +24,25 @@ namespace {
 constexpr int kScanBlock = 256;
 constexpr int kScanItems = 16;
 constexpr int kTile = kScanBlock * kScanItems;
-constexpr int kSpinLimit = 1 << 22;
+static_assert(kTile == kScanTile, "tile size");
+static_assert(kScanBlock == kLbBlock, "block size of the look-back");
 
-constexpr uint64_t FLAG_AGG = 1ULL, FLAG_INC = 2ULL;
-constexpr uint64_t VAL_MASK = (1ULL << 62) - 1;
+// One launch scans up to kScanJobs arrays: blockIdx.y picks the job, blockIdx.x its tile (a job
+// with fewer tiles than the widest leaves the rest of its row idle).
+struct ScanJobs {
+    ScanJob job[kScanJobs];
+};
 
-__device__ __forceinline__ uint64_t loadRelaxed(const unsigned long long* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void storeRelaxed(unsigned long long* p, uint64_t v) {
-    __hip_atomic_store(p, (unsigned long long)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// scratch layout: [0], [1] unused, [2 ..] one look-back word per tile
-__global__ void kScanReset(unsigned long long* scratch, int64_t words) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < words) scratch[i] = 0;
-}
-
-__global__ void __launch_bounds__(kScanBlock) kScan(const int32_t* __restrict__ in, int64_t* __restrict__ out, int64_t n, int64_t numTiles,
-                                                    unsigned long long* __restrict__ scratch, int64_t* __restrict__ total,
-                                                    int64_t* __restrict__ directOut) {
+__global__ void __launch_bounds__(kScanBlock) kScan(ScanJobs jobs, uint32_t epoch, int64_t* __restrict__ directOut) {
     __shared__ __align__(16) int32_t s_in[kTile];
     __shared__ int64_t s_wave[kScanBlock / 64];
     __shared__ long long s_off;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const int64_t t = blockIdx.x;
+    const ScanJob& job = jobs.job[blockIdx.y];
+    const int64_t t = blockIdx.x, n = job.n, numTiles = scanTiles(n);
     if (t >= numTiles) return;
-    unsigned long long* status = scratch + 2;
+    const int32_t* __restrict__ in = job.in;
+    int64_t* __restrict__ out = job.out;
     const int64_t base = t * kTile;
 
     // 16 consecutive counts per thread: four 16-byte loads each when the tile is full and
@@ -96,58 +88,15 @@ __global__ void __launch_bounds__(kScanBlock) kScan(const int32_t* __restrict__ 
     }
     int64_t run = x - acc + add;  // exclusive prefix of this thread inside the tile
 
-    // look-back (wave 0)
-    if (tid < 64) {
-        if (t == 0) {
-            if (lane == 0) {
-                storeRelaxed(&status[0], (FLAG_INC << 62) | ((uint64_t)tileSum & VAL_MASK));
-                s_off = 0;
-            }
-        } else {
-            if (lane == 0) storeRelaxed(&status[t], (FLAG_AGG << 62) | ((uint64_t)tileSum & VAL_MASK));
-            int64_t accum = 0;
-            int64_t i = t - 1;
-            int spins = 0;
-            bool done = false, direct = false;
-            while (!done) {
-                const int64_t j = i - lane;
-                const uint64_t st = j >= 0 ? loadRelaxed(&status[j]) : (FLAG_INC << 62);
-                const uint64_t f = st >> 62;
-                const uint64_t incMask = __ballot(f == FLAG_INC);
-                const uint64_t zeroMask = __ballot(f == 0);
-                const int firstInc = incMask ? __ffsll((unsigned long long)incMask) - 1 : 64;
-                const uint64_t upto = firstInc >= 63 ? ~0ULL : ((1ULL << (firstInc + 1)) - 1ULL);
-                if (zeroMask & upto) {
-                    // the ballots make this branch and the counter uniform over the wave
-                    if (++spins > kSpinLimit) {
-                        direct = true;
-                        break;
-                    }
-                    __builtin_amdgcn_s_sleep(1);
-                    continue;
-                }
-                int64_t val = lane <= firstInc ? (int64_t)(st & VAL_MASK) : 0;
-#pragma unroll
-                for (int d = 32; d > 0; d >>= 1) val += __shfl_down(val, d, 64);
-                accum += __shfl(val, 0, 64);
-                if (firstInc < 64) done = true;
-                else i -= 64;
-            }
-            if (direct) {
-                // the exclusive prefix straight from the counts before this tile
+    if (tid < 64)
+        lbTileOffset(
+            job.words, epoch, t, tileSum,
+            [&](int l) {
                 int64_t sum = 0;
-                for (int64_t k = lane; k < base; k += 64) sum += in[k];
-#pragma unroll
-                for (int d = 32; d > 0; d >>= 1) sum += __shfl_down(sum, d, 64);
-                accum = __shfl(sum, 0, 64);
-                if (lane == 0 && directOut) atomicAdd((unsigned long long*)directOut, 1ULL);
-            }
-            if (lane == 0) {
-                storeRelaxed(&status[t], (FLAG_INC << 62) | ((uint64_t)(accum + tileSum) & VAL_MASK));
-                s_off = accum;
-            }
-        }
-    }
+                for (int64_t k = l; k < base; k += 64) sum += in[k];
+                return sum;
+            },
+            directOut, &s_off);
     __syncthreads();
     run += s_off;
 
@@ -176,7 +125,7 @@ __global__ void __launch_bounds__(kScanBlock) kScan(const int32_t* __restrict__ 
                 if (o + i < n) out[o + i] = s_out[i];
         }
     }
-    if (t == numTiles - 1 && tid == 0) *total = s_off + tileSum;
+    if (t == numTiles - 1 && tid == 0 && job.total) *job.total = s_off + tileSum;
 }
 // Stream compaction in the same single pass: the indices i < n with (attr[i] & mask) != 0, in
 // increasing order, into idx[0 .. total).  Each tile counts its selected elements (16 per
@@ -184,14 +133,13 @@ __global__ void __launch_bounds__(kScanBlock) kScan(const int32_t* __restrict__ 
 // look-back as kScan (and the same exact fallback: a direct count of the selected elements
 // before the tile) and writes its indices; nothing is written per unselected element.
 __global__ void __launch_bounds__(kScanBlock) kCompactFlagged(const uint32_t* __restrict__ attr, int64_t n, uint32_t mask, int32_t* __restrict__ idx,
-                                                              int64_t numTiles, unsigned long long* __restrict__ scratch,
+                                                              unsigned long long* __restrict__ words, uint32_t epoch,
                                                               int64_t* __restrict__ total, int64_t* __restrict__ directOut) {
     __shared__ int s_wave[kScanBlock / 64];
     __shared__ long long s_off;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const int64_t t = blockIdx.x;
+    const int64_t t = blockIdx.x, numTiles = scanTiles(n);
     if (t >= numTiles) return;
-    unsigned long long* status = scratch + 2;
     const int64_t base = t * kTile;
     const int64_t first = base + (int64_t)tid * kScanItems;  // this thread's 16 consecutive elements
 
@@ -228,57 +176,15 @@ __global__ void __launch_bounds__(kScanBlock) kCompactFlagged(const uint32_t* __
     }
     const int run = x - cnt + add;  // exclusive prefix of this thread inside the tile
 
-    if (tid < 64) {
-        if (t == 0) {
-            if (lane == 0) {
-                storeRelaxed(&status[0], (FLAG_INC << 62) | ((uint64_t)tileSum & VAL_MASK));
-                s_off = 0;
-            }
-        } else {
-            if (lane == 0) storeRelaxed(&status[t], (FLAG_AGG << 62) | ((uint64_t)tileSum & VAL_MASK));
-            int64_t accum = 0;
-            int64_t i = t - 1;
-            int spins = 0;
-            bool done = false, direct = false;
-            while (!done) {
-                const int64_t j = i - lane;
-                const uint64_t st = j >= 0 ? loadRelaxed(&status[j]) : (FLAG_INC << 62);
-                const uint64_t f = st >> 62;
-                const uint64_t incMask = __ballot(f == FLAG_INC);
-                const uint64_t zeroMask = __ballot(f == 0);
-                const int firstInc = incMask ? __ffsll((unsigned long long)incMask) - 1 : 64;
-                const uint64_t upto = firstInc >= 63 ? ~0ULL : ((1ULL << (firstInc + 1)) - 1ULL);
-                if (zeroMask & upto) {
-                    // the ballots make this branch and the counter uniform over the wave
-                    if (++spins > kSpinLimit) {
-                        direct = true;
-                        break;
-                    }
-                    __builtin_amdgcn_s_sleep(1);
-                    continue;
-                }
-                int64_t val = lane <= firstInc ? (int64_t)(st & VAL_MASK) : 0;
-#pragma unroll
-                for (int d = 32; d > 0; d >>= 1) val += __shfl_down(val, d, 64);
-                accum += __shfl(val, 0, 64);
-                if (firstInc < 64) done = true;
-                else i -= 64;
-            }
-            if (direct) {
-                // the selected elements before this tile, counted straight from the input
+    if (tid < 64)
+        lbTileOffset(
+            words, epoch, t, tileSum,
+            [&](int l) {
                 int64_t sum = 0;
-                for (int64_t k = lane; k < base; k += 64) sum += (attr[k] & mask) ? 1 : 0;
-#pragma unroll
-                for (int d = 32; d > 0; d >>= 1) sum += __shfl_down(sum, d, 64);
-                accum = __shfl(sum, 0, 64);
-                if (lane == 0 && directOut) atomicAdd((unsigned long long*)directOut, 1ULL);
-            }
-            if (lane == 0) {
-                storeRelaxed(&status[t], (FLAG_INC << 62) | ((uint64_t)(accum + tileSum) & VAL_MASK));
-                s_off = accum;
-            }
-        }
-    }
+                for (int64_t k = l; k < base; k += 64) sum += (attr[k] & mask) ? 1 : 0;
+                return sum;
+            },
+            directOut, &s_off);
     __syncthreads();
     int64_t o = s_off + run;
     for (uint32_t b = bits; b; b &= b - 1) idx[o++] = (int32_t)(first + __ffs(b) - 1);
@@ -286,33 +192,19 @@ __global__ void __launch_bounds__(kScanBlock) kCompactFlagged(const uint32_t* __
 }
 }  // namespace
 
-size_t scanScratchBytes(int64_t n) {
-    const int64_t tiles = (n + kTile - 1) / kTile;
-    return (size_t)(tiles + 2) * sizeof(unsigned long long) + 256;
+void scanExclusiveI32(const ScanJob* jobs, int count, uint32_t epoch, hipStream_t s, int64_t* directOut) {
+    ScanJobs j{};
+    int64_t tiles = 0;
+    for (int k = 0; k < count; ++k) {
+        j.job[k] = jobs[k];
+        tiles = tiles > scanTiles(jobs[k].n) ? tiles : scanTiles(jobs[k].n);
+    }
+    kScan<<<dim3((unsigned)tiles, (unsigned)count), kScanBlock, 0, s>>>(j, epoch, directOut);
 }
 
-void scanExclusiveI32(const int32_t* in, int64_t* out, int64_t n, int64_t* total, void* scratch, hipStream_t s, int64_t* directOut) {
-    unsigned long long* w = (unsigned long long*)scratch;
-    const int64_t tiles = n > 0 ? (n + kTile - 1) / kTile : 0;
-    const int64_t words = tiles + 2;
-    kScanReset<<<(unsigned)((words + 255) / 256), 256, 0, s>>>(w, words);
-    if (tiles == 0) {
-        kScanReset<<<1, 1, 0, s>>>((unsigned long long*)total, 1);
-        return;
-    }
-    kScan<<<(unsigned)tiles, kScanBlock, 0, s>>>(in, out, n, tiles, w, total, directOut);
-}
-
-void compactFlagged(const uint32_t* attr, int64_t n, uint32_t mask, int32_t* idx, int64_t* total, void* scratch, hipStream_t s, int64_t* directOut) {
-    unsigned long long* w = (unsigned long long*)scratch;
-    const int64_t tiles = n > 0 ? (n + kTile - 1) / kTile : 0;
-    const int64_t words = tiles + 2;
-    kScanReset<<<(unsigned)((words + 255) / 256), 256, 0, s>>>(w, words);
-    if (tiles == 0) {
-        kScanReset<<<1, 1, 0, s>>>((unsigned long long*)total, 1);
-        return;
-    }
-    kCompactFlagged<<<(unsigned)tiles, kScanBlock, 0, s>>>(attr, n, mask, idx, tiles, w, total, directOut);
+void compactFlagged(const uint32_t* attr, int64_t n, uint32_t mask, int32_t* idx, int64_t* total, unsigned long long* words, uint32_t epoch,
+                    hipStream_t s, int64_t* directOut) {
+    kCompactFlagged<<<(unsigned)scanTiles(n), kScanBlock, 0, s>>>(attr, n, mask, idx, words, epoch, total, directOut);
 }
 
 }  // namespace mdmc
