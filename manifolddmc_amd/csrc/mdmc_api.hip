@@ -236,7 +236,6 @@ mdmc_status runExtraction(mdmc_ctx* ctx, const mdmc_grid* grids, int G, const fl
     try {
         hipStream_t s = p.stream;
         MDMC_HIP(hipEventRecord(ctx->ev[0], s));
-        p.resetCounters();
         p.splitIterations = 0;
         p.extraAnomalies = 0;
         // ---- grids: upload if needed, then pad / refine (refineGrid)
@@ -244,7 +243,8 @@ mdmc_status runExtraction(mdmc_ctx* ctx, const mdmc_grid* grids, int G, const fl
         float* up = PinTot ? p.arena.get<float>("input", (size_t)PinTot) : nullptr;
         std::vector<mdmc::ProblemDev> problems;
         problems.reserve((size_t)B);
-        std::vector<mdmc::PrepareDesc> prep((size_t)G);
+        std::vector<mdmc::PrepareDesc>& prep = p.prep.desc;
+        prep.resize((size_t)G);
         int64_t prepBlocks = 0;
         mdmc::GridDev g0{};
         for (int gi = 0; gi < G; ++gi) {
@@ -286,7 +286,10 @@ mdmc_status runExtraction(mdmc_ctx* ctx, const mdmc_grid* grids, int G, const fl
             }
         }
         const bool surf = (flags & MDMC_SURF_ITER) != 0;
-        mdmc::PrepareDesc* pd = p.arena.get<mdmc::PrepareDesc>("prep_desc", (size_t)G);
+        p.prep.dev = G > 1 || B > 1 ? p.arena.get<mdmc::PrepareDesc>("prep_desc", (size_t)G) : nullptr;
+        p.prep.rows = prepBlocks;
+        p.prep.refinement = r;
+        p.prep.pad = pad;
         // A batch of grids already on the device, with a tile shape chosen: the shape-determined
         // front (padding, classification, tile-count scans) goes through a graph captured once
         // for these shapes and replayed (stage times then count it under the grid pass)
@@ -299,13 +302,12 @@ mdmc_status runExtraction(mdmc_ctx* ctx, const mdmc_grid* grids, int G, const fl
             for (int gi = 0; gi < G; ++gi)
                 for (int k = 0; k < 3; ++k) shapeSig.push_back(grids[gi].dims[k]);
         }
-        if (graphable && p.runFrontGraph(shapeSig, prep.data(), (size_t)G * sizeof(mdmc::PrepareDesc), pd, G, prepBlocks, r, pad, problems, C,
-                                         shapeNow, surf)) {
+        if (graphable && p.runFrontGraph(shapeSig, problems, C, shapeNow, surf)) {
             MDMC_HIP(hipEventRecord(ctx->ev[1], s));
-            p.gridPassBack(C, shapeNow, record);
+            p.gridPassBack(problems, C, shapeNow, surf, record);
         } else {
-            p.upload(pd, prep.data(), (size_t)G * sizeof(mdmc::PrepareDesc), 1);
-            mdmc::launchPrepareGrids(pd, G, prepBlocks, r, pad, p.prepSpecial(), s);
+            if (p.prep.dev) p.upload(p.prep.dev, prep.data(), (size_t)G * sizeof(mdmc::PrepareDesc), 1);
+            p.prepare(problems, false);
             MDMC_HIP(hipEventRecord(ctx->ev[1], s));
             // ---- DMC
             p.dmc(problems, surf, record);

@@ -4,6 +4,7 @@
 //   refineGrid                      UniformGrid.inl:279-319
 // The cell classification, dual vertices and quads are in mdmc_gridpass.hip.
 #include "mdmc_device.h"
+#include "mdmc_gridpass.h"
 #include "mdmc_internal.h"
 
 #include <algorithm>
@@ -22,12 +23,15 @@ __device__ __forceinline__ int clampi(int i, int lo, int hi) { return i < lo ? l
 // MODE 1 (no refinement, exact): the sample position is the point itself: x / 1 = x exactly,
 //   floor(x) = x and the weights are +0, the same values the general path computes, so the
 //   8 corner loads and the trilinear blend stay (a non-finite neighbour still reaches the
-//   result through 0 * s).  Runs only when *special is set, as a grid-stride loop.
+//   result through 0 * s).  Runs only when MODE 0 asked for it.
 // MODE 0 (no refinement, plain): when every input value v has |v| < 2^126 and is not -0, each
 //   difference of two of them is finite, so s0 + 0 * (s1 - s0) = s0 and every level of the
 //   zero-weight blend returns its first operand: the result is the first corner, bit for bit.
-//   This mode copies that corner and sets *special when it meets any other value (every input
-//   point is some output point's first corner, so none is missed); MODE 1 then redoes all.
+//   This mode copies that corner and raises the setup's special word when it meets any other
+//   value (every input point is some output point's first corner, so none is missed); the host
+//   sees it with the grid pass's totals and runs MODE 1 over all grids, then classifies again.
+//   (A second launch that looks at the flag on the GPU cost every extraction 3 us of launch time
+//   and 4 us there, and such values -- -0, infinities, |v| >= 2^126 -- are rare in fields.)
 __device__ __forceinline__ bool plainValue(float v) {
     const uint32_t b = __float_as_uint(v);
     return (b & 0x7FFFFFFFu) < 0x7E800000u && b != 0x80000000u;
@@ -35,15 +39,15 @@ __device__ __forceinline__ bool plainValue(float v) {
 
 // one output row; its points x = lane, lane + width, ... (a block, or one wave in MODE 0)
 template <int MODE>
-__device__ __forceinline__ void prepareRow(const PrepareDesc* __restrict__ d, int G, int refinement, int pad, int64_t row, int64_t* special,
-                                           int lane, int width) {
-    int lo = 0, hi = G;  // d[lo].base <= row
+__device__ __forceinline__ void prepareRow(const PrepareDesc& one, const PrepareDesc* __restrict__ d, int G, int refinement, int pad, int64_t row,
+                                           const PrepareSetup& setup, int lane, int width) {
+    int lo = 0, hi = d ? G : 1;  // d[lo].base <= row
     while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
         if (d[mid].base <= row) lo = mid;
         else hi = mid;
     }
-    const PrepareDesc& p = d[lo];
+    const PrepareDesc p = d ? d[lo] : one;
     const int onx = p.onx, ony = p.ony, onz = p.onz, inx = p.inx, iny = p.iny, inz = p.inz;
     const int r = (int)(row - p.base);  // < ony * onz < 2^31
     int y = r % ony, z = r / ony;
@@ -61,7 +65,10 @@ __device__ __forceinline__ void prepareRow(const PrepareDesc* __restrict__ d, in
             plain = plain && plainValue(v);
             out[x] = v;
         }
-        if (!plain) *special = 1;
+        if (!plain && (setup.token == 0 || *(volatile int64_t*)setup.gate != setup.token)) {
+            *(volatile int64_t*)setup.gate = setup.token;
+            *(volatile int64_t*)setup.special = 1;
+        }
         return;
     }
     const float rr = (float)(refinement + 1);
@@ -99,19 +106,19 @@ __device__ __forceinline__ void prepareRow(const PrepareDesc* __restrict__ d, in
 // block per row
 constexpr int kPlainRowsPerBlock = kBlock / 64;
 template <int MODE>
-__global__ void __launch_bounds__(kBlock) kPrepareGrids(const PrepareDesc* __restrict__ d, int G, int refinement, int pad, int64_t rows,
-                                                        int64_t* special) {
-    if (MODE == 1) {
-        if (*(volatile int64_t*)special == 0) return;
-        for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) prepareRow<1>(d, G, refinement, pad, row, special, threadIdx.x, kBlock);
-        return;
+__global__ void __launch_bounds__(kBlock) kPrepareGrids(PrepareDesc one, const PrepareDesc* __restrict__ d, int G, int refinement, int pad, int64_t rows,
+                                                        PrepareSetup setup) {
+    if (blockIdx.x == 0) {
+        for (int i = threadIdx.x; i < setup.nCtr; i += kBlock) setup.ctr[i] = 0;
+        for (int i = threadIdx.x; i < setup.nParts; i += kBlock) setup.parts[i] = 0;
+        if (setup.probs && threadIdx.x == 0) *setup.probs = setup.prob;
     }
     if (MODE == 0) {
         const int64_t row = (int64_t)blockIdx.x * kPlainRowsPerBlock + (threadIdx.x >> 6);
-        if (row < rows) prepareRow<0>(d, G, refinement, pad, row, special, threadIdx.x & 63, 64);
+        if (row < rows) prepareRow<0>(one, d, G, refinement, pad, row, setup, threadIdx.x & 63, 64);
         return;
     }
-    prepareRow<MODE>(d, G, refinement, pad, blockIdx.x, special, threadIdx.x, kBlock);
+    prepareRow<MODE>(one, d, G, refinement, pad, blockIdx.x, setup, threadIdx.x, kBlock);
 }
 
 __global__ void kTriangles(const int4* __restrict__ he, const int32_t* __restrict__ face_he, int64_t F, uint32_t* __restrict__ idx) {
@@ -211,15 +218,16 @@ __global__ void kRenderVertices(const int4* __restrict__ he, int64_t H, const fl
 
 int64_t prepareBlocks(const int od[3]) { return (int64_t)od[1] * od[2]; }
 
-void launchPrepareGrids(const PrepareDesc* descDev, int G, int64_t blocks, int refinement, int pad, int64_t* special, hipStream_t s) {
-    if (blocks <= 0) return;
-    if (refinement > 0) {
-        kPrepareGrids<2><<<(unsigned)blocks, kBlock, 0, s>>>(descDev, G, refinement, pad, blocks, special);
-        return;
-    }
-    // *special is zero on entry; the exact pass returns at once unless the copy set it
-    kPrepareGrids<0><<<(unsigned)((blocks + kPlainRowsPerBlock - 1) / kPlainRowsPerBlock), kBlock, 0, s>>>(descDev, G, refinement, pad, blocks, special);
-    kPrepareGrids<1><<<(unsigned)std::min<int64_t>(blocks, 2048), kBlock, 0, s>>>(descDev, G, refinement, pad, blocks, special);
+void launchPrepareGrids(const PrepareDesc& one, const PrepareDesc* descDev, int G, int64_t rows, int refinement, int pad, const PrepareSetup& setup,
+                        hipStream_t s) {
+    if (rows <= 0) return;
+    if (refinement > 0) kPrepareGrids<2><<<(unsigned)rows, kBlock, 0, s>>>(one, descDev, G, refinement, pad, rows, setup);
+    else kPrepareGrids<0><<<(unsigned)((rows + kPlainRowsPerBlock - 1) / kPlainRowsPerBlock), kBlock, 0, s>>>(one, descDev, G, refinement, pad, rows, setup);
+}
+
+void launchPrepareExact(const PrepareDesc& one, const PrepareDesc* descDev, int G, int64_t rows, int pad, hipStream_t s) {
+    PrepareSetup none{};
+    if (rows > 0) kPrepareGrids<1><<<(unsigned)rows, kBlock, 0, s>>>(one, descDev, G, 0, pad, rows, none);
 }
 
 void launchDmcTrianglesFromFaces(const int4* he, const int32_t* face_he, int64_t F, uint32_t* idx, hipStream_t s) {

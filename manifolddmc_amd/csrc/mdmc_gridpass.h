@@ -42,6 +42,24 @@ struct ProblemDev {
     int64_t blockBase, segBase;
 };
 
+// What the padding / refinement launch sets up for the rest of an extraction: the counters and
+// partial sums cleared, a single problem's descriptor stored (probs null: uploaded elsewhere).
+// A plain-copy launch (no refinement) that meets a value needing the exact blend raises
+// *special (mapped pinned host memory); gate (device memory) keeps that to about one store per
+// XCD: it holds the call's token once raised (token 0: no gate, for captured launches).
+struct PrepareSetup {
+    int64_t *ctr, *parts;
+    int nCtr, nParts;
+    ProblemDev* probs;
+    ProblemDev prob;
+    int64_t *special, *gate, token;
+};
+// descDev: the G grids' descriptors, or null with one (G = 1) by value
+void launchPrepareGrids(const PrepareDesc& one, const PrepareDesc* descDev, int G, int64_t rows, int refinement, int pad, const PrepareSetup& setup,
+                        hipStream_t s);
+// the exact blend of every grid, after a plain copy that raised *special (no refinement)
+void launchPrepareExact(const PrepareDesc& one, const PrepareDesc* descDev, int G, int64_t rows, int pad, hipStream_t s);
+
 struct GridPassArgs {
     const ProblemDev* probs;
     int nProblems;

@@ -64,8 +64,6 @@ struct PrepareDesc {
 };
 // blocks of the padding / refinement pass over one processed grid of od points: one per row
 int64_t prepareBlocks(const int od[3]);
-// special: a device word that is zero on entry (set when an input value needs the exact blend)
-void launchPrepareGrids(const PrepareDesc* descDev, int G, int64_t blocks, int refinement, int pad, int64_t* special, hipStream_t s);
 void launchDmcTrianglesFromFaces(const int4* he, const int32_t* face_he, int64_t F, uint32_t* idx, hipStream_t s);
 // positions copied from src to positions[3V] and the faces' vertex ids to quads[4F], in one launch
 // (either output may be null)

@@ -65,14 +65,25 @@ class Pipeline {
     bool posSlotted = false;
     const int32_t* vertexSlots();
 
-    void resetCounters();
+    // one extraction's padding / refinement: its grids' descriptors (host copy, and the device
+    // copy of more than one), and the launch that also clears the counters and stores a
+    // single problem (captured: for a graph)
+    struct Prepare {
+        std::vector<PrepareDesc> desc;
+        PrepareDesc* dev = nullptr;
+        int64_t rows = 0;
+        int refinement = 0, pad = 0;
+    } prep;
+    void prepare(const std::vector<ProblemDev>& problems, bool captured);
+    // waits for the front of the grid pass; where the plain copy met values that need the exact
+    // blend, redoes the padding and calls again() (the front over it)
+    template <class Again>
+    void finishPrepare(Again again);
     // the counters an extraction reports, in one read-back: anomalies, split iterations that
     // took the sequential merge pass, look-back tiles that summed their prefix directly
     void counterTotals(int64_t* anomalyCount, int64_t* mergeSeq, int64_t* lookbackDirect);
     // device word the single-pass scans and compactions count their direct-sum tiles in
     int64_t* lookbackDiag();
-    // the padding pass's flag word (one of the counters, zeroed by resetCounters)
-    int64_t* prepSpecial();
 
     // the grid pass over one or more (grid, iso) problems (their cellBase / tileBase and
     // cell counts are filled in); recordAdjoint keeps the cell -> vertex map ("adj_map") that
@@ -85,11 +96,10 @@ class Pipeline {
     int64_t dmcSetup(std::vector<ProblemDev>& problems, bool recordAdjoint);
     int64_t assignTiles(std::vector<ProblemDev>& problems, int shape);
     void gridPassFront(std::vector<ProblemDev>& problems, int64_t C, int shape, bool surfIter, void* stagedProbs, bool events);
-    void gridPassBack(int64_t C, int shape, bool recordAdjoint);
+    void gridPassBack(std::vector<ProblemDev>& problems, int64_t C, int shape, bool surfIter, bool recordAdjoint);
     int shapeClass(int64_t C, bool surfIter) const;
     int resolveShape(int64_t C, bool surfIter);
-    bool runFrontGraph(const std::vector<int64_t>& shapeSig, const void* prep, size_t prepBytes, void* prepDev, int G, int64_t prepBlocks,
-                       int refinement, int pad, std::vector<ProblemDev>& problems, int64_t C, int shape, bool surfIter);
+    bool runFrontGraph(const std::vector<int64_t>& shapeSig, std::vector<ProblemDev>& problems, int64_t C, int shape, bool surfIter);
     void noteEagerFront(const std::vector<int64_t>& shapeSig) {
         fgLastEager_ = shapeSig;
         const std::vector<int64_t> b = frontBuffers();
@@ -174,6 +184,7 @@ class Pipeline {
     };
     Lookback lookback(int64_t words);
     uint32_t lbEpoch_ = 0;
+    int64_t prepToken_ = 0;
     int64_t compactNM(int32_t* nm);
     void zero(void* p, size_t bytes);
     void fillNeg(void* p, size_t bytes);

@@ -37,7 +37,7 @@ constexpr int kMaxBucket = 16;
 constexpr int kFanGuard = 4096;
 
 // ---------------------------------------------------------------- counters
-enum : int { A_ANOMALY = 0, A_CONFLICT = 1, A_INVALID = 2, A_DIRTY = 3, A_PREP_SPECIAL = 4, A_FALLBACK = 5, A_MERGE_SEQ = 6, A_LB_DIRECT = 7, A_NCOUNTERS = 8 };
+enum : int { A_ANOMALY = 0, A_CONFLICT = 1, A_INVALID = 2, A_DIRTY = 3, A_FALLBACK = 5, A_MERGE_SEQ = 6, A_LB_DIRECT = 7, A_NCOUNTERS = 8 };
 // the slotted non-manifold halfedges the split's working copy marks (markHalfedgesAsNonManifold,
 // ManifoldSplitter.cu:527-555, reads the four slots of every full vertex-pair bucket): every
 // halfedge of a bucket of 4, and of a larger bucket the ones at ranks 1, 2, 3 and size - 1
@@ -2778,9 +2778,39 @@ void Pipeline::FillBatch::flush() {
     blocks = 0;
 }
 
-void Pipeline::resetCounters() {
-    zero(counters(), A_NCOUNTERS * sizeof(int64_t));
+// pinned word of the padding pass's "needs the exact blend"
+constexpr int kPinSpecial = 3;
+
+void Pipeline::prepare(const std::vector<ProblemDev>& problems, bool captured) {
     refreshUnchecked = false;
+    PrepareSetup su{};
+    su.ctr = counters();
+    su.nCtr = A_NCOUNTERS;
+    su.parts = nmSlotParts();
+    su.nParts = kPartSlots * kPartStride;
+    if (problems.size() == 1) {
+        probsDev = arena.get<ProblemDev>("gp_probs", 1);
+        su.probs = probsDev;
+        su.prob = problems[0];
+    }
+    const bool fresh = arena.capacity<int64_t>("prep_gate") == 0;
+    su.gate = arena.get<int64_t>("prep_gate", 1);
+    if (fresh) zero(su.gate, sizeof(int64_t));
+    su.special = pinDev() + kPinSpecial;
+    su.token = captured ? 0 : ++prepToken_;
+    pinHost()[kPinSpecial] = 0;
+    launchPrepareGrids(prep.desc[0], prep.dev, (int)prep.desc.size(), prep.rows, prep.refinement, prep.pad, su, stream);
+}
+
+template <class Again>
+void Pipeline::finishPrepare(Again again) {
+    MDMC_HIP(hipStreamSynchronize(stream));
+    int64_t* h = pinHost();
+    if (!h[kPinSpecial]) return;
+    h[kPinSpecial] = 0;
+    launchPrepareExact(prep.desc[0], prep.dev, (int)prep.desc.size(), prep.rows, prep.pad, stream);
+    again();
+    MDMC_HIP(hipStreamSynchronize(stream));
 }
 
 int64_t* Pipeline::lookbackDiag() { return counters() + A_LB_DIRECT; }
@@ -2794,7 +2824,6 @@ void Pipeline::counterTotals(int64_t* anomalyCount, int64_t* mergeSeq, int64_t* 
     *lookbackDirect = h[A_LB_DIRECT];
 }
 
-int64_t* Pipeline::prepSpecial() { return counters() + A_PREP_SPECIAL; }
 
 // ---- grid pass
 // Row slabs: bands of at most SLAB_XMAX cells per row, R rows per block, and chunks of slices
@@ -2903,7 +2932,9 @@ int Pipeline::resolveShape(int64_t C, bool surfIter) {
 
 void Pipeline::dmc(std::vector<ProblemDev>& problems, bool surfIter, bool recordAdjoint) {
     const int64_t C = dmcSetup(problems, recordAdjoint);
-    if (resolveShape(C, surfIter) == GP_SHAPE_AUTO) {
+    const bool tune = resolveShape(C, surfIter) == GP_SHAPE_AUTO;
+    if (tune || gridPassIsSlab(lastShape)) finishPrepare([] {});
+    if (tune) {
         // autotuner: on the first extraction of a workload class, time every shape on this
         // very input and keep the fastest for the class.  The XCD-chunked shapes (1-3, 7, 8)
         // move less data out of L2 (about half for the tiles, measured at 512^3); a
@@ -2930,7 +2961,7 @@ void Pipeline::dmc(std::vector<ProblemDev>& problems, bool surfIter, bool record
 // addresses of every device buffer the front of a tile-shape grid pass touches
 std::vector<int64_t> Pipeline::frontBuffers() {
     std::vector<int64_t> b;
-    for (const char* n : {"counters", "grid", "prep_desc", "gp_probs", "gp_queue", "gp_rec", "gp_tv", "gp_tq", "gp_tna", "gp_map", "gp_tvo", "gp_tqo",
+    for (const char* n : {"counters", "nm_slot_parts", "prep_gate", "grid", "prep_desc", "gp_probs", "gp_queue", "gp_rec", "gp_tv", "gp_tq", "gp_tna", "gp_map", "gp_tvo", "gp_tqo",
                           "gp_lb"})
         b.push_back((int64_t)(intptr_t)arena.ptr<char>(n));
     b.push_back((int64_t)(intptr_t)pinDev());
@@ -2946,8 +2977,8 @@ void Pipeline::releaseGraphs() {
     fg_.stageCap = 0;
 }
 
-bool Pipeline::runFrontGraph(const std::vector<int64_t>& shapeSig, const void* prep, size_t prepBytes, void* prepDev, int G, int64_t prepBlocks,
-                             int refinement, int pad, std::vector<ProblemDev>& problems, int64_t C, int shape, bool surfIter) {
+bool Pipeline::runFrontGraph(const std::vector<int64_t>& shapeSig, std::vector<ProblemDev>& problems, int64_t C, int shape, bool surfIter) {
+    const size_t prepBytes = prep.desc.size() * sizeof(PrepareDesc);
     std::vector<int64_t> sig = shapeSig;
     const std::vector<int64_t> bufs = frontBuffers();
     sig.insert(sig.end(), bufs.begin(), bufs.end());
@@ -2956,9 +2987,11 @@ bool Pipeline::runFrontGraph(const std::vector<int64_t>& shapeSig, const void* p
     if (fg_.exec && fg_.sig == sig) {
         // replay: the descriptors of this call into the graph's staging, then the graph
         assignTiles(problems, shape);
-        std::memcpy(fg_.stage, prep, prepBytes);
+        std::memcpy(fg_.stage, prep.desc.data(), prepBytes);
         std::memcpy((char*)fg_.stage + probOff, problems.data(), pbytes);
         probsDev = arena.ptr<ProblemDev>("gp_probs");
+        refreshUnchecked = false;
+        pinHost()[kPinSpecial] = 0;
         ga_ = fgArgs_;
         MDMC_HIP(hipEventRecord(kev[0], stream));
         MDMC_HIP(hipGraphLaunch(fg_.exec, stream));
@@ -2971,12 +3004,12 @@ bool Pipeline::runFrontGraph(const std::vector<int64_t>& shapeSig, const void* p
     releaseGraphs();
     fg_.stageCap = probOff + pbytes;
     MDMC_HIP(hipHostMalloc(&fg_.stage, fg_.stageCap, hipHostMallocDefault));
-    std::memcpy(fg_.stage, prep, prepBytes);
+    std::memcpy(fg_.stage, prep.desc.data(), prepBytes);
     hipGraph_t graph = nullptr;
     MDMC_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeRelaxed));
     try {
-        MDMC_HIP(hipMemcpyAsync(prepDev, fg_.stage, prepBytes, hipMemcpyHostToDevice, stream));
-        launchPrepareGrids((const PrepareDesc*)prepDev, G, prepBlocks, refinement, pad, prepSpecial(), stream);
+        MDMC_HIP(hipMemcpyAsync(prep.dev, fg_.stage, prepBytes, hipMemcpyHostToDevice, stream));
+        prepare(problems, true);
         gridPassFront(problems, C, shape, surfIter, (char*)fg_.stage + probOff, false);
     } catch (...) {
         (void)hipStreamEndCapture(stream, &graph);
@@ -3006,7 +3039,7 @@ void Pipeline::gridPass(std::vector<ProblemDev>& problems, int64_t C, int shape,
         return;
     }
     gridPassFront(problems, C, shape, surfIter, nullptr, true);
-    gridPassBack(C, shape, recordAdjoint);
+    gridPassBack(problems, C, shape, surfIter, recordAdjoint);
 }
 
 int64_t Pipeline::assignTiles(std::vector<ProblemDev>& problems, int shape) {
@@ -3028,7 +3061,9 @@ void Pipeline::gridPassFront(std::vector<ProblemDev>& problems, int64_t C, int s
     const int64_t numTiles = assignTiles(problems, shape);
     probsDev = arena.get<ProblemDev>("gp_probs", problems.size());
     const size_t pbytes = problems.size() * sizeof(ProblemDev);
-    if (stagedProbs) {
+    if (problems.size() == 1) {
+        // stored by prepare()
+    } else if (stagedProbs) {
         std::memcpy(stagedProbs, problems.data(), pbytes);
         MDMC_HIP(hipMemcpyAsync(probsDev, stagedProbs, pbytes, hipMemcpyHostToDevice, stream));
     } else {
@@ -3069,10 +3104,10 @@ void Pipeline::gridPassFront(std::vector<ProblemDev>& problems, int64_t C, int s
 }
 
 // the rest: read the totals back, size the outputs, emit quads and dual vertices
-void Pipeline::gridPassBack(int64_t C, int shape, bool recordAdjoint) {
+void Pipeline::gridPassBack(std::vector<ProblemDev>& problems, int64_t C, int shape, bool surfIter, bool recordAdjoint) {
     GridPassArgs& a = ga_;
     int64_t* h = pinHost();
-    MDMC_HIP(hipStreamSynchronize(stream));
+    finishPrepare([&] { gridPassFront(problems, C, shape, surfIter, nullptr, true); });
     V = h[1];
     Q = h[2];
     if (V >= (int64_t)INT32_MAX / 2 || 4 * Q >= (int64_t)INT32_MAX) throw HipError("mesh exceeds the int32 id range", -3);
