@@ -33,7 +33,6 @@ struct mdmc_ctx {
     mdmc::Pipeline p;
     std::string err;
     bool hasResult = false;
-    hipEvent_t ev[9] = {};
     AdjointState adj;
     int nProblems = 0;  // problems of the resident result
     int flags = 0;
@@ -133,11 +132,6 @@ mdmc_status mdmc_create(mdmc_ctx** out, int32_t device) {
         delete ctx;
         return MDMC_ERR_HIP;
     }
-    for (auto& e : ctx->ev)
-        if (hipEventCreate(&e) != hipSuccess) {
-            delete ctx;
-            return MDMC_ERR_HIP;
-        }
     ctx->p.stream = ctx->own;
     *out = ctx;
     return MDMC_OK;
@@ -149,8 +143,6 @@ void mdmc_destroy(mdmc_ctx* ctx) {
         DeviceGuard g(ctx->device);
         if (ctx->p.stream) (void)hipStreamSynchronize(ctx->p.stream);
         ctx->p.arena.release();
-        for (auto& e : ctx->ev)
-            if (e) (void)hipEventDestroy(e);
         if (ctx->own) (void)hipStreamDestroy(ctx->own);
     }
     delete ctx;
@@ -235,7 +227,6 @@ mdmc_status runExtraction(mdmc_ctx* ctx, const mdmc_grid* grids, int G, const fl
     const int B = G * I;
     try {
         hipStream_t s = p.stream;
-        MDMC_HIP(hipEventRecord(ctx->ev[0], s));
         p.splitIterations = 0;
         p.extraAnomalies = 0;
         // ---- grids: upload if needed, then pad / refine (refineGrid)
@@ -303,37 +294,30 @@ mdmc_status runExtraction(mdmc_ctx* ctx, const mdmc_grid* grids, int G, const fl
                 for (int k = 0; k < 3; ++k) shapeSig.push_back(grids[gi].dims[k]);
         }
         if (graphable && p.runFrontGraph(shapeSig, problems, C, shapeNow, surf)) {
-            MDMC_HIP(hipEventRecord(ctx->ev[1], s));
             p.gridPassBack(problems, C, shapeNow, surf, record);
         } else {
             if (p.prep.dev) p.upload(p.prep.dev, prep.data(), (size_t)G * sizeof(mdmc::PrepareDesc), 1);
             p.prepare(problems, false);
-            MDMC_HIP(hipEventRecord(ctx->ev[1], s));
             // ---- DMC
             p.dmc(problems, surf, record);
             if (graphable) p.noteEagerFront(shapeSig);
         }
         if (B > 1) p.problemDmcCounts(B);
-        MDMC_HIP(hipEventRecord(ctx->ev[2], s));
         int64_t st9[9] = {0};
         if (p.V > 0) {
             p.simplifyQueue = ((flags & MDMC_P3X3Y_COLOR) ? 1 : 0) + ((flags & MDMC_P3X3Y_OLD) ? 1 : 0) + ((flags & MDMC_P3333) ? 1 : 0);
             p.halfedgeInitialize();
-            MDMC_HIP(hipEventRecord(ctx->ev[3], s));
             if (flags & MDMC_P3X3Y_COLOR) p.simplify3X3Y(true);
             if (flags & MDMC_P3X3Y_OLD) p.simplify3X3Y(false);
             if (flags & MDMC_P3333) p.simplify3333();
-            MDMC_HIP(hipEventRecord(ctx->ev[4], s));
             p.fixManifoldTwins();
-            MDMC_HIP(hipEventRecord(ctx->ev[5], s));
             if (flags & MDMC_SPLIT_NM) p.split(opt->split_step, opt->max_split_iters > 0 ? opt->max_split_iters : 64);
-            MDMC_HIP(hipEventRecord(ctx->ev[6], s));
             if (flags & MDMC_DETECT_NM_VERTS) p.detectNonManifoldVertices();
-            MDMC_HIP(hipEventRecord(ctx->ev[7], s));
             if (B == 1) {
                 p.computeStats(st9);
             } else {
                 p.regroupBatch(B);
+                p.finishBatch();
                 for (int b = 0; b < B; ++b)
                     for (int k = 0; k < 9; ++k) st9[k] += p.batchStats[9 * (size_t)b + k];
             }
@@ -346,10 +330,8 @@ mdmc_status runExtraction(mdmc_ctx* ctx, const mdmc_grid* grids, int G, const fl
                 p.batchFOff.assign((size_t)B + 1, 0);
                 p.batchStats.assign(9 * (size_t)B, 0);
             }
-            for (int i = 3; i < 8; ++i) MDMC_HIP(hipEventRecord(ctx->ev[i], s));
+            p.computeStats(st9);
         }
-        MDMC_HIP(hipEventRecord(ctx->ev[8], s));
-        MDMC_HIP(hipEventSynchronize(ctx->ev[8]));
         ctx->hasResult = true;
         ctx->nProblems = B;
         ctx->flags = flags;
@@ -385,16 +367,11 @@ mdmc_status runExtraction(mdmc_ctx* ctx, const mdmc_grid* grids, int G, const fl
             p.counterTotals(&anomalyCount, &stats->split_sequential_merges, &stats->lookback_fallbacks);
             stats->anomalies = anomalyCount + p.extraAnomalies;
             stats->cells = cells;
-            float ms = 0.f;
-            double* outs[8] = {&stats->ms_total, &stats->ms_grid, &stats->ms_dmc, &stats->ms_halfedge,
-                               &stats->ms_simplify, &stats->ms_fix_twins, &stats->ms_split, &stats->ms_detect};
-            MDMC_HIP(hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[8]));
-            *outs[0] = ms;
-            for (int i = 1; i < 8; ++i) {
-                MDMC_HIP(hipEventElapsedTime(&ms, ctx->ev[i - 1], ctx->ev[i]));
-                *outs[i] = ms;
-            }
-            p.kernelTimes(&stats->ms_grid_pass_kernel);
+            double ms[9];
+            p.stageTimes(ms);
+            double* outs[9] = {&stats->ms_total, &stats->ms_grid, &stats->ms_dmc, &stats->ms_halfedge, &stats->ms_simplify,
+                               &stats->ms_fix_twins, &stats->ms_split, &stats->ms_detect, &stats->ms_grid_pass_kernel};
+            for (int i = 0; i < 9; ++i) *outs[i] = ms[i];
         }
         return MDMC_OK;
     } catch (const std::exception& e) {

@@ -335,7 +335,11 @@ void Pipeline::placeByProblem(const int32_t* key, int64_t n0, int64_t n, int B, 
 }
 
 void Pipeline::regroupBatch(int B) {
-    zero(arena.get<int>("batch_bad", 1), sizeof(int));
+    {
+        FillBatch fb(*this);
+        fb.stampAt(stamp(ST_STATS));
+        fb.add(arena.get<int>("batch_bad", 1), 0x00, sizeof(int));
+    }
     int32_t* vp = pid();
     int4* he = arena.ptr<int4>("he");
     int32_t* face_he = arena.ptr<int32_t>("face_he");

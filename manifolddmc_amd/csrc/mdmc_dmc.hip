@@ -112,6 +112,8 @@ __global__ void __launch_bounds__(kBlock) kPrepareGrids(PrepareDesc one, const P
         for (int i = threadIdx.x; i < setup.nCtr; i += kBlock) setup.ctr[i] = 0;
         for (int i = threadIdx.x; i < setup.nParts; i += kBlock) setup.parts[i] = 0;
         if (setup.probs && threadIdx.x == 0) *setup.probs = setup.prob;
+        __syncthreads();
+        stampClock(setup.stamp);  // one of the counters cleared above
     }
     if (MODE == 0) {
         const int64_t row = (int64_t)blockIdx.x * kPlainRowsPerBlock + (threadIdx.x >> 6);

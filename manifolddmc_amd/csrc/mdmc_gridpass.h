@@ -53,6 +53,7 @@ struct PrepareSetup {
     ProblemDev* probs;
     ProblemDev prob;
     int64_t *special, *gate, token;
+    int64_t* stamp;
 };
 // descDev: the G grids' descriptors, or null with one (G = 1) by value
 void launchPrepareGrids(const PrepareDesc& one, const PrepareDesc* descDev, int G, int64_t rows, int refinement, int pad, const PrepareSetup& setup,
@@ -77,6 +78,8 @@ struct GridPassArgs {
     // per active cell (concatenated cell index): vertex index inside its tile (14 bits) and the
     // contour of each edge a later cell's quads read (2 bits each for edges 1,2,4,5,6,7,9,10,11)
     uint32_t* cellMap;
+    // stage clocks: classification's first run in this extraction and its last, emit
+    int64_t *stampFirst, *stampRun, *stampEmit;
     // look-back words that classify clears for the scan of the tile counts
     unsigned long long* lb;
     int64_t lbWords;

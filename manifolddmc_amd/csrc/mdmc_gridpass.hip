@@ -412,6 +412,13 @@ __device__ __forceinline__ void tileCellXYZ(const TileBase& b, int l, const Smal
     z = b.z0 + (int)zz;
 }
 
+__device__ __forceinline__ void stampClassify(const GridPassArgs& a) {
+    if (blockIdx.x != 0) return;
+    stampClock(a.stampRun);
+    if (threadIdx.x == 0 && a.stampFirst && __hip_atomic_load(a.stampFirst, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) stampClock(a.stampFirst);
+    for (int i = threadIdx.x; i < (int)a.lbWords; i += blockDim.x) a.lb[i] = 0;
+}
+
 // ---- classify: active cells of one tile, their records, counts and map entries
 template <int CPT, bool QUEUE>
 __global__ void __launch_bounds__(GP_THREADS) kClassify(GridPassArgs a, int chunked) {
@@ -429,7 +436,7 @@ __global__ void __launch_bounds__(GP_THREADS) kClassify(GridPassArgs a, int chun
     __shared__ int64_t s_t;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wid = tid >> 6;
-    for (int64_t i = (int64_t)blockIdx.x * GP_THREADS + tid; i < a.lbWords; i += (int64_t)gridDim.x * GP_THREADS) a.lb[i] = 0;
+    stampClassify(a);
     // the two small tables in LDS (read after the first barrier below)
     s_base[tid] = c_polyBase[tid];
     for (int i = tid; i < kPolyTabSize; i += GP_THREADS) s_tab[i] = c_polyCmap[i];
@@ -562,6 +569,7 @@ __global__ void __launch_bounds__(GP_THREADS) kEmit(GridPassArgs a, int chunked)
     __shared__ int s_wave[GP_WAVES];
 
     __shared__ int64_t s_t;
+    stampClock(a.stampEmit);
     const int tid = threadIdx.x;
     for (int i = tid; i < kPolyTabSize; i += GP_THREADS) s_tab[i] = c_polyCmap[i];
     for (int iter = 0;; ++iter) {
@@ -717,6 +725,8 @@ __device__ __forceinline__ int64_t segIndex(const ProblemDev& P, int z, int y, i
 // vertex work items (cell, contour word) of the block's cells.
 template <int R, bool EMIT>
 __global__ void __launch_bounds__(SLAB_COLS) kSlab(GridPassArgs a, int chunked) {
+    if (EMIT) stampClock(a.stampEmit);
+    else stampClassify(a);
     constexpr int NR = R + 1;             // cell rows: the halo row and the R own rows
     constexpr int PR = R + 2;             // point rows y0 - 1 .. y0 + R
     constexpr int NC = NR * SLAB_COLS;    // cell slots per slice: row * SLAB_COLS + column

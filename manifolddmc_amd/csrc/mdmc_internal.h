@@ -33,11 +33,25 @@ struct ScanJob {
     int64_t* total;
     unsigned long long* words;
 };
-void scanExclusiveI32(const ScanJob* jobs, int count, uint32_t epoch, hipStream_t s, int64_t* directOut);
+// stampStart / stampEnd (may be null): clock at the launch's start and the first job's end
+void scanExclusiveI32(const ScanJob* jobs, int count, uint32_t epoch, hipStream_t s, int64_t* directOut, int64_t* stampStart = nullptr,
+                      int64_t* stampEnd = nullptr);
 // stream compaction in one pass: the i < n with (attr[i] & mask) != 0, ascending, into
 // idx (capacity n); the count through *total
 void compactFlagged(const uint32_t* attr, int64_t n, uint32_t mask, int32_t* idx, int64_t* total, unsigned long long* words, uint32_t epoch,
-                    hipStream_t s, int64_t* directOut);
+                    hipStream_t s, int64_t* directOut, int64_t* stamp);
+
+// --- stage times: the first block of a stage's first kernel stores the GPU's constant-rate clock
+// (null: no stamp).  Timing events instead cost about 5 us of idle GPU at every boundary.
+__device__ __forceinline__ void stampClock(int64_t* stamp) {
+    // the block first: the others then never wait for the pointer's load (kEmit at 512^3: 5%)
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0 && stamp)
+        __hip_atomic_store(stamp, (int64_t)wall_clock64(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// slots: the start of each stage in order (padding, classification, halfedge initialize,
+// simplifications, records + twin repair, split, detection, statistics), the end, then the grid
+// pass's second part, the end of its first, the start of its last run
+enum : int { ST_PAD = 0, ST_DMC, ST_INIT, ST_SIMPLIFY, ST_TWINS, ST_SPLIT, ST_DETECT, ST_STATS, ST_END, ST_EMIT, ST_TOTALS, ST_CLASSIFY, ST_COUNT };
 
 inline unsigned gridFor(int64_t n, int block = kBlock) { return (unsigned)((n + block - 1) / block); }
 

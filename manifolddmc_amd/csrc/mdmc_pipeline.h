@@ -24,6 +24,7 @@ struct FillSet {
     unsigned start[kFillSetMax];
     uint8_t byte[kFillSetMax];
     int count = 0;
+    int64_t* stamp = nullptr;
 };
 
 class Pipeline {
@@ -79,9 +80,16 @@ class Pipeline {
     // blend, redoes the padding and calls again() (the front over it)
     template <class Again>
     void finishPrepare(Again again);
-    // the counters an extraction reports, in one read-back: anomalies, split iterations that
-    // took the sequential merge pass, look-back tiles that summed their prefix directly
+    // the end of an extraction: with the statistics kernel's last block (one problem), or after a
+    // batch's regroup, the counters, statistics and stage clocks go to pinned memory in one
+    // read-back; the getters below read that copy
+    void computeStats(int64_t out[9]);
+    void finishBatch();
     void counterTotals(int64_t* anomalyCount, int64_t* mergeSeq, int64_t* lookbackDirect);
+    // stage times in ms, from the clock stamps of the stages' first kernels: whole call, then the
+    // seven stages of mdmc_stats in order, then the grid pass alone
+    void stageTimes(double ms[9]);
+    int64_t* stamp(int slot);
     // device word the single-pass scans and compactions count their direct-sum tiles in
     int64_t* lookbackDiag();
 
@@ -95,7 +103,7 @@ class Pipeline {
     // with the same shapes and buffers (false: not replayable yet, run it eagerly), then the rest
     int64_t dmcSetup(std::vector<ProblemDev>& problems, bool recordAdjoint);
     int64_t assignTiles(std::vector<ProblemDev>& problems, int shape);
-    void gridPassFront(std::vector<ProblemDev>& problems, int64_t C, int shape, bool surfIter, void* stagedProbs, bool events);
+    void gridPassFront(std::vector<ProblemDev>& problems, int64_t C, int shape, bool surfIter, void* stagedProbs);
     void gridPassBack(std::vector<ProblemDev>& problems, int64_t C, int shape, bool surfIter, bool recordAdjoint);
     int shapeClass(int64_t C, bool surfIter) const;
     int resolveShape(int64_t C, bool surfIter);
@@ -133,7 +141,6 @@ class Pipeline {
     void fixManifoldTwins();
     void split(int step, int maxIters);
     void detectNonManifoldVertices();
-    void computeStats(int64_t out[9]);
 
     void copyOut(float* positions, float* normals, int32_t* halfedges, int32_t* face_halfedge, uint16_t* face_attr, uint8_t* vertex_flags,
                  int32_t* vertex_halfedge, bool dstDevice);
@@ -151,10 +158,14 @@ class Pipeline {
     // host -> device copy of a small host array through pinned staging (region 0 or 1, so
     // that two uploads of one stage do not share a buffer); returns after queueing the copy
     void upload(void* dst, const void* src, size_t bytes, int region);
-    // duration of the last grid pass (classify + scan, then emit), from events on the
+    // while tuning, the duration of a grid pass (classify + scan, then emit) from events on the
     // launch stream; the host read-back of the sizes between them is not counted
     void kernelTimes(double* msGridPass);
     hipEvent_t kev[4] = {nullptr, nullptr, nullptr, nullptr};
+    bool tuning_ = false;
+    void tuneEvent(int k) {
+        if (tuning_) MDMC_HIP(hipEventRecord(kev[k], stream));
+    }
     // grid-pass tile shape: GP_SHAPE_AUTO (autotuned per workload class) or a fixed shape;
     // lastShape is the one the last extraction used, tuneMs the last tuning's timings
     int tileShape = GP_SHAPE_AUTO;
@@ -173,7 +184,7 @@ class Pipeline {
     int64_t* nmFoundParts();
     int64_t scan32(const int32_t* in, int64_t n, const std::string& outName, int64_t** out);
     // exclusive prefix sums in one launch (words of the jobs are set here); total may be null
-    void scan(std::initializer_list<ScanJob> jobs);
+    void scan(std::initializer_list<ScanJob> jobs, int64_t* stampStart = nullptr, int64_t* stampEnd = nullptr);
     void scan(const int32_t* in, int64_t* out, int64_t n, int64_t* total = nullptr) { scan({ScanJob{in, out, n, total, nullptr}}); }
     // look-back words for one launch over `words` tiles: the launches of a stream run one after
     // the other, so all share one buffer, told apart by the epoch (cleared when the buffer is
@@ -185,7 +196,8 @@ class Pipeline {
     Lookback lookback(int64_t words);
     uint32_t lbEpoch_ = 0;
     int64_t prepToken_ = 0;
-    int64_t compactNM(int32_t* nm);
+    int clockKHz_ = 0;
+    int64_t compactNM(int32_t* nm, bool first);
     void zero(void* p, size_t bytes);
     void fillNeg(void* p, size_t bytes);
     void launchFill(void* p, uint8_t byte, size_t bytes);
@@ -196,6 +208,7 @@ class Pipeline {
         ~FillBatch() { flush(); }
         void add(void* p, uint8_t byte, size_t bytes);
         void flush();
+        void stampAt(int64_t* stamp) { fs.stamp = stamp; }
 
        private:
         Pipeline& pl;

@@ -37,7 +37,8 @@ constexpr int kMaxBucket = 16;
 constexpr int kFanGuard = 4096;
 
 // ---------------------------------------------------------------- counters
-enum : int { A_ANOMALY = 0, A_CONFLICT = 1, A_INVALID = 2, A_DIRTY = 3, A_FALLBACK = 5, A_MERGE_SEQ = 6, A_LB_DIRECT = 7, A_NCOUNTERS = 8 };
+enum : int { A_ANOMALY = 0, A_CONFLICT = 1, A_INVALID = 2, A_DIRTY = 3, A_FALLBACK = 5, A_MERGE_SEQ = 6, A_LB_DIRECT = 7,
+             A_STAMP = 8, A_STATS = A_STAMP + ST_COUNT, A_TICKET = A_STATS + 9, A_NCOUNTERS };
 // the slotted non-manifold halfedges the split's working copy marks (markHalfedgesAsNonManifold,
 // ManifoldSplitter.cu:527-555, reads the four slots of every full vertex-pair bucket): every
 // halfedge of a bucket of 4, and of a larger bucket the ones at ranks 1, 2, 3 and size - 1
@@ -96,6 +97,7 @@ __global__ void kFillBytes(uint8_t* __restrict__ p, uint8_t byte, size_t head, s
 // several fills in one launch: block b works on the range j with start[j] <= b < start[j + 1],
 // as kFillBytes does on one range
 __global__ void kFillMany(FillSet fs) {
+    stampClock(fs.stamp);
     int j = 0;
     while (j + 1 < fs.count && (unsigned)blockIdx.x >= fs.start[j + 1]) ++j;
     const size_t t = (size_t)(blockIdx.x - fs.start[j]) * blockDim.x + threadIdx.x;
@@ -550,7 +552,8 @@ __global__ void kBucketsAll(const int4* __restrict__ quads, int64_t H, const int
 // the halfedge records of the quads, from the ids and the twins, and the bucket sizes / ranks
 __global__ void __launch_bounds__(kBlock) kMaterialize(const int4* __restrict__ quads, int64_t H, const int32_t* __restrict__ twin,
                                                        const uint32_t* __restrict__ bpack, int4* __restrict__ he, int32_t* __restrict__ bsize,
-                                                       int32_t* __restrict__ brank, int64_t* nmParts) {
+                                                       int32_t* __restrict__ brank, int64_t* nmParts, int64_t* stamp) {
+    stampClock(stamp);
     const int64_t hh = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     int slotted = 0;
     if (hh < H) {
@@ -1542,7 +1545,8 @@ __global__ void __launch_bounds__(kLbBlock) kCompactVertices(const int32_t* __re
 
 // positions and normals of the current vertices, gathered from their slots
 __global__ void kGatherVertices(const float* __restrict__ pos, const float* __restrict__ nrm, const int32_t* __restrict__ vslot, int64_t V,
-                                float* __restrict__ npos, float* __restrict__ nnrm) {
+                                float* __restrict__ npos, float* __restrict__ nnrm, int64_t* stamp) {
+    stampClock(stamp);
     const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= V) return;
     const int64_t sl = vslot[v];
@@ -2480,8 +2484,10 @@ __global__ void __launch_bounds__(kBlock) kDetectFans(const int4* __restrict__ h
 // counts over the vertex-pair buckets (HalfedgeMesh.cu:1164-1239, ManifoldCreator.cu:545-549)
 __global__ void __launch_bounds__(kBlock) kStats(const int4* __restrict__ he, int64_t H, const int32_t* __restrict__ face_he, int64_t F,
                                                  const int32_t* __restrict__ bsize, const int32_t* __restrict__ brank, const uint32_t* __restrict__ vflags,
-                                                 int64_t V, const uint8_t* __restrict__ canon, unsigned long long* __restrict__ out) {
+                                                 int64_t V, const uint8_t* __restrict__ canon, int64_t* __restrict__ ctr, int64_t* __restrict__ pin) {
+    stampClock(ctr + A_STAMP + ST_STATS);
     __shared__ unsigned int acc[9];
+    __shared__ bool s_last;
     if (threadIdx.x < 9) acc[threadIdx.x] = 0;
     __syncthreads();
     unsigned int loc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
@@ -2532,8 +2538,24 @@ __global__ void __launch_bounds__(kBlock) kStats(const int4* __restrict__ he, in
         if ((threadIdx.x & 63) == 0 && v) atomicAdd(&acc[k], v);
     }
     __syncthreads();
-    if (threadIdx.x < 9 && acc[threadIdx.x]) atomicAdd(&out[threadIdx.x], (unsigned long long)acc[threadIdx.x]);
+    if (threadIdx.x < 9 && acc[threadIdx.x]) atomicAdd((unsigned long long*)&ctr[A_STATS + threadIdx.x], (unsigned long long)acc[threadIdx.x]);
+    // the last block to finish hands the counters over: no copy, no second wait.  The block's
+    // sums were added by its first wave, which waits for its own atomics before it takes its
+    // ticket; the sums are read back with atomic loads, so no block needs a device-scope fence
+    // (each would write its XCD's L2 back: +0.1 ms at 128^3)
+    if (threadIdx.x < 64) {
+        __builtin_amdgcn_s_waitcnt(0);
+        if (threadIdx.x == 0) s_last = atomicAdd((unsigned long long*)&ctr[A_TICKET], 1ULL) == gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!s_last) return;
+    if (threadIdx.x < A_NCOUNTERS && threadIdx.x != A_STAMP + ST_END)
+        pin[threadIdx.x] = __hip_atomic_load(&ctr[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == 0) pin[A_STAMP + ST_END] = wall_clock64();
 }
+
+// the clock alone, where no kernel begins or ends a stage
+__global__ void kStamp(int64_t* stamp) { *stamp = wall_clock64(); }
 
 // The resident mesh into the caller's device buffers, every array in one launch: block b works
 // on the array j with start[j] <= b < start[j + 1], kCopyPer * kBlock of its items (16 bytes of
@@ -2702,7 +2724,7 @@ Pipeline::Lookback Pipeline::lookback(int64_t words) {
     return Lookback{w, ++lbEpoch_};
 }
 
-void Pipeline::scan(std::initializer_list<ScanJob> jobs) {
+void Pipeline::scan(std::initializer_list<ScanJob> jobs, int64_t* stampStart, int64_t* stampEnd) {
     ScanJob j[kScanJobs];
     int count = 0;
     int64_t words = 0;
@@ -2714,7 +2736,7 @@ void Pipeline::scan(std::initializer_list<ScanJob> jobs) {
         j[count++].words = lb.words + words;
         words += scanTiles(x.n);
     }
-    scanExclusiveI32(j, count, lb.epoch, stream, lookbackDiag());
+    scanExclusiveI32(j, count, lb.epoch, stream, lookbackDiag(), stampStart, stampEnd);
 }
 
 int64_t Pipeline::scan32(const int32_t* in, int64_t n, const std::string& outName, int64_t** out) {
@@ -2728,11 +2750,12 @@ int64_t Pipeline::scan32(const int32_t* in, int64_t n, const std::string& outNam
 }
 
 // the faces with the NM bit, ascending, into nm (capacity F); returns their number
-int64_t Pipeline::compactNM(int32_t* nm) {
+int64_t Pipeline::compactNM(int32_t* nm, bool first) {
     int64_t* h = pinHost();
     int64_t* d = pinDev();
     const Lookback lb = lookback(scanTiles(F));
-    compactFlagged(arena.ptr<uint32_t>("fattr"), F, (uint32_t)QA_NM, nm, d + 1, lb.words, lb.epoch, stream, lookbackDiag());
+    compactFlagged(arena.ptr<uint32_t>("fattr"), F, (uint32_t)QA_NM, nm, d + 1, lb.words, lb.epoch, stream, lookbackDiag(),
+                   first ? stamp(ST_SPLIT) : nullptr);
     // with the count, the invalid-record counter: a refresh's face walks add to it
     if (refreshUnchecked) MDMC_HIP(hipMemcpyAsync(h + 2, counters() + A_INVALID, sizeof(int64_t), hipMemcpyDeviceToHost, stream));
     MDMC_HIP(hipStreamSynchronize(stream));
@@ -2774,12 +2797,14 @@ void Pipeline::FillBatch::add(void* p, uint8_t byte, size_t bytes) {
 void Pipeline::FillBatch::flush() {
     if (fs.count == 0) return;
     kFillMany<<<blocks, kBlock, 0, pl.stream>>>(fs);
+    fs.stamp = nullptr;
     fs.count = 0;
     blocks = 0;
 }
 
-// pinned word of the padding pass's "needs the exact blend"
-constexpr int kPinSpecial = 3;
+// pinned words: the padding pass's "needs the exact blend", the copy of the counters at the end
+constexpr int kPinSpecial = 3, kPinFinal = 16;
+static_assert(kPinFinal + A_NCOUNTERS <= Pipeline::kPinSlots, "pinned words");
 
 void Pipeline::prepare(const std::vector<ProblemDev>& problems, bool captured) {
     refreshUnchecked = false;
@@ -2796,6 +2821,7 @@ void Pipeline::prepare(const std::vector<ProblemDev>& problems, bool captured) {
     const bool fresh = arena.capacity<int64_t>("prep_gate") == 0;
     su.gate = arena.get<int64_t>("prep_gate", 1);
     if (fresh) zero(su.gate, sizeof(int64_t));
+    su.stamp = stamp(ST_PAD);
     su.special = pinDev() + kPinSpecial;
     su.token = captured ? 0 : ++prepToken_;
     pinHost()[kPinSpecial] = 0;
@@ -2815,15 +2841,32 @@ void Pipeline::finishPrepare(Again again) {
 
 int64_t* Pipeline::lookbackDiag() { return counters() + A_LB_DIRECT; }
 
+int64_t* Pipeline::stamp(int slot) { return counters() + A_STAMP + slot; }
+
 void Pipeline::counterTotals(int64_t* anomalyCount, int64_t* mergeSeq, int64_t* lookbackDirect) {
-    int64_t* h = pinHost();
-    MDMC_HIP(hipMemcpyAsync(h, counters(), A_NCOUNTERS * sizeof(int64_t), hipMemcpyDeviceToHost, stream));
-    MDMC_HIP(hipStreamSynchronize(stream));
+    const int64_t* h = pinHost() + kPinFinal;
     *anomalyCount = h[A_ANOMALY];
     *mergeSeq = h[A_MERGE_SEQ];
     *lookbackDirect = h[A_LB_DIRECT];
 }
 
+void Pipeline::stageTimes(double ms[9]) {
+    if (!clockKHz_) {
+        int dev = 0, khz = 0;
+        MDMC_HIP(hipGetDevice(&dev));
+        MDMC_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
+        clockKHz_ = khz > 0 ? khz : 100000;
+    }
+    // a stage that launched nothing began when the next one did
+    int64_t t[ST_COUNT];
+    std::memcpy(t, pinHost() + kPinFinal + A_STAMP, sizeof t);
+    for (int i = ST_END - 1; i >= 0; --i)
+        if (t[i] == 0) t[i] = t[i + 1];
+    const double k = 1.0 / clockKHz_;
+    ms[0] = (double)(t[ST_END] - t[ST_PAD]) * k;
+    for (int i = 0; i < 7; ++i) ms[1 + i] = (double)(t[i + 1] - t[i]) * k;
+    ms[8] = t[ST_CLASSIFY] ? (double)(t[ST_TOTALS] - t[ST_CLASSIFY] + (t[ST_EMIT] ? t[ST_INIT] - t[ST_EMIT] : 0)) * k : 0.0;
+}
 
 // ---- grid pass
 // Row slabs: bands of at most SLAB_XMAX cells per row, R rows per block, and chunks of slices
@@ -2855,6 +2898,9 @@ void Pipeline::slabPass(std::vector<ProblemDev>& problems, int64_t C, int shape,
     a.nProblems = nProblems;
     a.surfIter = surfIter ? 1 : 0;
     a.numBlocks = blocks;
+    a.stampFirst = stamp(ST_DMC);
+    a.stampRun = stamp(ST_CLASSIFY);
+    a.stampEmit = stamp(ST_EMIT);
     a.numSegs = segs;
     a.segV = arena.get<int32_t>("gp_segv", (size_t)segs + 1);
     a.segQ = arena.get<int32_t>("gp_segq", (size_t)segs + 1);
@@ -2865,10 +2911,10 @@ void Pipeline::slabPass(std::vector<ProblemDev>& problems, int64_t C, int shape,
     int64_t* h = pinHost();
     int64_t* pd = pinDev();
     h[1] = h[2] = 0;
-    MDMC_HIP(hipEventRecord(kev[0], stream));
+    tuneEvent(0);
     launchSlabCount(shape, a, stream);
-    scan({ScanJob{a.segV, svo, segs + 1, pd + 1, nullptr}, ScanJob{a.segQ, sqo, segs + 1, pd + 2, nullptr}});
-    MDMC_HIP(hipEventRecord(kev[1], stream));
+    scan({ScanJob{a.segV, svo, segs + 1, pd + 1, nullptr}, ScanJob{a.segQ, sqo, segs + 1, pd + 2, nullptr}}, nullptr, stamp(ST_TOTALS));
+    tuneEvent(1);
     MDMC_HIP(hipStreamSynchronize(stream));
     V = h[1];
     Q = h[2];
@@ -2885,15 +2931,16 @@ void Pipeline::slabPass(std::vector<ProblemDev>& problems, int64_t C, int shape,
     a.outdeg = arena.get<int32_t>("out_cnt", (size_t)V + 1);  // the halfedge initialize's list lengths
     a.V = V;
     a.vpid = nProblems > 1 ? arena.get<int32_t>("pid", (size_t)std::max<int64_t>(V, 1)) : nullptr;
-    MDMC_HIP(hipEventRecord(kev[2], stream));
+    tuneEvent(2);
     launchSlabEmit(shape, a, stream);
-    MDMC_HIP(hipEventRecord(kev[3], stream));
+    tuneEvent(3);
     dmcV = V;
     dmcQ = Q;
 }
 int64_t Pipeline::dmcSetup(std::vector<ProblemDev>& problems, bool recordAdjoint) {
     vertHeV = vertHeQ = 0;
     batchVertHe = false;
+    tuning_ = false;
     nProblems = (int)problems.size();
     if (recordAdjoint && nProblems != 1) throw HipError("adjoint recording needs a single problem", -4);
     int64_t C = 0;
@@ -2907,8 +2954,6 @@ int64_t Pipeline::dmcSetup(std::vector<ProblemDev>& problems, bool recordAdjoint
         // the grid pass splits tile cell offsets with a float-reciprocal division (exact below 2^24)
         if (pr.CX >= (1 << 23) || pr.CY >= (1 << 23)) throw HipError("a grid has 2^23 cells or more along x or y", -3);
     }
-    if (!kev[0])
-        for (auto& e : kev) MDMC_HIP(hipEventCreate(&e));
     return C;
 }
 
@@ -2940,6 +2985,9 @@ void Pipeline::dmc(std::vector<ProblemDev>& problems, bool surfIter, bool record
         // move less data out of L2 (about half for the tiles, measured at 512^3); a
         // launch-order or work-queue shape (4-6, 9) must beat them by 3% to be chosen.
         double best = 1e30;
+        if (!kev[0])
+            for (auto& e : kev) MDMC_HIP(hipEventCreate(&e));
+        tuning_ = true;
         for (int sh = GP_SHAPE_FIRST; sh <= GP_SHAPE_LAST; ++sh) {
             gridPass(problems, C, sh, surfIter, recordAdjoint);
             MDMC_HIP(hipEventSynchronize(kev[3]));
@@ -2952,6 +3000,7 @@ void Pipeline::dmc(std::vector<ProblemDev>& problems, bool surfIter, bool record
                 lastShape = sh;
             }
         }
+        tuning_ = false;
         tuned[shapeClass(C, surfIter)] = lastShape;
         if (lastShape == GP_SHAPE_LAST) return;  // the last candidate's output is in place
     }
@@ -2993,9 +3042,7 @@ bool Pipeline::runFrontGraph(const std::vector<int64_t>& shapeSig, std::vector<P
         refreshUnchecked = false;
         pinHost()[kPinSpecial] = 0;
         ga_ = fgArgs_;
-        MDMC_HIP(hipEventRecord(kev[0], stream));
         MDMC_HIP(hipGraphLaunch(fg_.exec, stream));
-        MDMC_HIP(hipEventRecord(kev[1], stream));
         ++graphReplays;
         return true;
     }
@@ -3010,7 +3057,7 @@ bool Pipeline::runFrontGraph(const std::vector<int64_t>& shapeSig, std::vector<P
     try {
         MDMC_HIP(hipMemcpyAsync(prep.dev, fg_.stage, prepBytes, hipMemcpyHostToDevice, stream));
         prepare(problems, true);
-        gridPassFront(problems, C, shape, surfIter, (char*)fg_.stage + probOff, false);
+        gridPassFront(problems, C, shape, surfIter, (char*)fg_.stage + probOff);
     } catch (...) {
         (void)hipStreamEndCapture(stream, &graph);
         if (graph) (void)hipGraphDestroy(graph);
@@ -3025,9 +3072,7 @@ bool Pipeline::runFrontGraph(const std::vector<int64_t>& shapeSig, std::vector<P
     fg_.exec = exec;
     fg_.sig = sig;
     fgArgs_ = ga_;
-    MDMC_HIP(hipEventRecord(kev[0], stream));
     MDMC_HIP(hipGraphLaunch(fg_.exec, stream));
-    MDMC_HIP(hipEventRecord(kev[1], stream));
     ++graphReplays;
     return true;
 }
@@ -3038,7 +3083,7 @@ void Pipeline::gridPass(std::vector<ProblemDev>& problems, int64_t C, int shape,
         slabPass(problems, C, shape, surfIter, recordAdjoint);
         return;
     }
-    gridPassFront(problems, C, shape, surfIter, nullptr, true);
+    gridPassFront(problems, C, shape, surfIter, nullptr);
     gridPassBack(problems, C, shape, surfIter, recordAdjoint);
 }
 
@@ -3055,8 +3100,8 @@ int64_t Pipeline::assignTiles(std::vector<ProblemDev>& problems, int shape) {
 // The part of a tile-shape grid pass that the shapes alone determine: the problems' upload,
 // classification and the tile-count scans, with no host synchronisation.  stagedProbs: copy
 // the problems from that pinned buffer (a graph capture; the caller fills it before every
-// replay) instead of through upload().  events: time the part with kev[0] / kev[1].
-void Pipeline::gridPassFront(std::vector<ProblemDev>& problems, int64_t C, int shape, bool surfIter, void* stagedProbs, bool events) {
+// replay) instead of through upload().
+void Pipeline::gridPassFront(std::vector<ProblemDev>& problems, int64_t C, int shape, bool surfIter, void* stagedProbs) {
     const int T = gridPassTile(shape);
     const int64_t numTiles = assignTiles(problems, shape);
     probsDev = arena.get<ProblemDev>("gp_probs", problems.size());
@@ -3075,6 +3120,9 @@ void Pipeline::gridPassFront(std::vector<ProblemDev>& problems, int64_t C, int s
     a.nProblems = nProblems;
     a.surfIter = surfIter ? 1 : 0;
     a.numTiles = numTiles;
+    a.stampFirst = stamp(ST_DMC);
+    a.stampRun = stamp(ST_CLASSIFY);
+    a.stampEmit = stamp(ST_EMIT);
     a.queue = arena.get<int64_t>("gp_queue", 2);
     a.rec = arena.get<uint32_t>("gp_rec", (size_t)std::max<int64_t>(numTiles * T, 1));
     a.tileV = arena.get<int32_t>("gp_tv", (size_t)numTiles + 1);
@@ -3092,22 +3140,22 @@ void Pipeline::gridPassFront(std::vector<ProblemDev>& problems, int64_t C, int s
     a.lbWords = 2 * words;
     // totals straight into pinned host memory: [1] V, [2] Q
     int64_t* pd = pinDev();
-    if (events) MDMC_HIP(hipEventRecord(kev[0], stream));
+    tuneEvent(0);
     launchGridClassify(shape, a, stream);
     if (numTiles > 0) {
         const ScanJob jobs[2] = {{a.tileV, tvo, numTiles + 1, pd + 1, a.lb}, {a.tileQ, tqo, numTiles + 1, pd + 2, a.lb + words}};
-        scanExclusiveI32(jobs, 2, 0, stream, lookbackDiag());
+        scanExclusiveI32(jobs, 2, 0, stream, lookbackDiag(), nullptr, stamp(ST_TOTALS));
     } else {
         zero(pd + 1, 2 * sizeof(int64_t));
     }
-    if (events) MDMC_HIP(hipEventRecord(kev[1], stream));
+    tuneEvent(1);
 }
 
 // the rest: read the totals back, size the outputs, emit quads and dual vertices
 void Pipeline::gridPassBack(std::vector<ProblemDev>& problems, int64_t C, int shape, bool surfIter, bool recordAdjoint) {
     GridPassArgs& a = ga_;
     int64_t* h = pinHost();
-    finishPrepare([&] { gridPassFront(problems, C, shape, surfIter, nullptr, true); });
+    finishPrepare([&] { gridPassFront(problems, C, shape, surfIter, nullptr); });
     V = h[1];
     Q = h[2];
     if (V >= (int64_t)INT32_MAX / 2 || 4 * Q >= (int64_t)INT32_MAX) throw HipError("mesh exceeds the int32 id range", -3);
@@ -3123,9 +3171,9 @@ void Pipeline::gridPassBack(std::vector<ProblemDev>& problems, int64_t C, int sh
     a.outdeg = arena.get<int32_t>("out_cnt", (size_t)V + 1);  // the halfedge initialize's list lengths
     a.V = V;
     a.vpid = nProblems > 1 ? arena.get<int32_t>("pid", (size_t)std::max<int64_t>(V, 1)) : nullptr;
-    MDMC_HIP(hipEventRecord(kev[2], stream));
+    tuneEvent(2);
     launchGridEmit(shape, a, stream);
-    MDMC_HIP(hipEventRecord(kev[3], stream));
+    tuneEvent(3);
     dmcV = V;
     dmcQ = Q;
 }
@@ -3192,7 +3240,7 @@ void Pipeline::halfedgeInitialize() {
     // corner vertices' contours: no counting atomics
     zero(cnt + V, sizeof(int32_t));
     int64_t* off = arena.get<int64_t>("out_off", (size_t)V + 1);
-    scan(cnt, off, V + 1);
+    scan({ScanJob{cnt, off, V + 1, nullptr, nullptr}}, stamp(ST_INIT));
     int32_t* out = arena.get<int32_t>("out_list", (size_t)std::max<int64_t>(H, 1));
     int2* ends = arena.get<int2>("out_ends", (size_t)std::max<int64_t>(H, 1));
     launchQuadLists(quads, qattr, Q, V, arena.ptr<int32_t>("gp_vcell"), arena.ptr<uint16_t>("gp_vct"), pid(), probsDev, off, out, ends, face_he, fattr,
@@ -3419,6 +3467,7 @@ void Pipeline::simplifyCompactAndRebuild(int dropType, bool p3333) {
 }
 
 void Pipeline::simplifyInit(int32_t** valence, int32_t** count, bool needCount) {
+    const bool firstOfChain = deferredSteps == 0 && !posSlotted;
     if (simplifyQueue > 0) --simplifyQueue;
     *valence = arena.get<int32_t>("valence", (size_t)V);
     *count = arena.get<int32_t>("vcount", (size_t)V);
@@ -3427,6 +3476,7 @@ void Pipeline::simplifyInit(int32_t** valence, int32_t** count, bool needCount) 
     {
         // (the pattern counts only serve the old P3X3Y rule)
         FillBatch fb(*this);
+        fb.stampAt(firstOfChain ? stamp(ST_SIMPLIFY) : nullptr);
         if (needCount) fb.add(*count, 0x00, (size_t)V * sizeof(int32_t));
         fb.add(vtype, 0x00, (size_t)V * sizeof(int32_t));
         fb.add(vtarget, 0xFF, (size_t)V * sizeof(int32_t));
@@ -3468,12 +3518,13 @@ void Pipeline::simplify3333() {
 
 // the full halfedge records, once the simplifications (which read ids and twins only) are done
 void Pipeline::materializeHalfedges() {
+    const bool gathered = posSlotted && V > 0;
     if (posSlotted) {
         // positions and normals by vertex again, from the slots the simplifications kept them in
         const size_t cap = (size_t)std::max(V, dmcV);
         float* npos = arena.get<float>("pos2", 3 * cap);
         float* nnrm = arena.get<float>("nrm2", 3 * cap);
-        if (V > 0) kGatherVertices<<<gridFor(V), kBlock, 0, stream>>>(arena.ptr<float>("pos"), arena.ptr<float>("nrm"), vertexSlots(), V, npos, nnrm);
+        if (V > 0) kGatherVertices<<<gridFor(V), kBlock, 0, stream>>>(arena.ptr<float>("pos"), arena.ptr<float>("nrm"), vertexSlots(), V, npos, nnrm, stamp(ST_TWINS));
         arena.swap("pos", "pos2");
         arena.swap("nrm", "nrm2");
         posSlotted = false;
@@ -3482,10 +3533,10 @@ void Pipeline::materializeHalfedges() {
     int4* he = arena.get<int4>("he", (size_t)std::max<int64_t>(H, 1));
     int32_t* bsize = arena.get<int32_t>("bsize", (size_t)std::max<int64_t>(H, 1));
     int32_t* brank = arena.get<int32_t>("brank", (size_t)std::max<int64_t>(H, 1));
-    zero(nmSlotParts(), kPartSlots * kPartStride * sizeof(int64_t));  // recounted from the bucket sizes written here
+    // (the partial sums are clear since the extraction's start)
     if (H > 0)
         kMaterialize<<<gridFor(H), kBlock, 0, stream>>>(arena.ptr<int4>("quads"), H, arena.ptr<int32_t>("twin"), arena.ptr<uint32_t>("bpack"), he, bsize,
-                                                        brank, nmSlotParts());
+                                                        brank, nmSlotParts(), gathered ? nullptr : stamp(ST_TWINS));
     heMaterialized = true;
 }
 
@@ -3510,7 +3561,7 @@ void Pipeline::split(int step, int maxIters) {
         const int64_t iterH = H;
         // countNonManifoldFaces: the NM faces' ids, ascending, in one compaction pass
         int32_t* nm = arena.get<int32_t>("nmlist", (size_t)std::max<int64_t>(F, 1));
-        const int64_t n64 = compactNM(nm);
+        const int64_t n64 = compactNM(nm, iter == 0);
         if (n64 == 0) break;
         // still non-manifold after the allowed iterations (the reference loops until clean)
         if (iter >= maxIters) {
@@ -3728,11 +3779,15 @@ void Pipeline::detectNonManifoldVertices() {
     int32_t* outdeg = arena.get<int32_t>("outdeg", (size_t)V);
     int32_t* rep = arena.get<int32_t>("outrep", (size_t)V);
     uint8_t* slow = arena.get<uint8_t>("fan_slow", (size_t)V);
-    zero(outdeg, (size_t)V * sizeof(int32_t));
     // the slow-vertex count is accumulated in device memory (atomics on mapped host memory
     // cross the bus one by one) and read back once
     int64_t* nslow = arena.get<int64_t>("fan_nslow", 2);
-    zero(nslow, 2 * sizeof(int64_t));
+    {
+        FillBatch fb(*this);
+        fb.stampAt(stamp(ST_DETECT));
+        fb.add(outdeg, 0x00, (size_t)V * sizeof(int32_t));
+        fb.add(nslow, 0x00, 2 * sizeof(int64_t));
+    }
     const bool fromLists = listsV >= 0 && listsV <= V;
     const uint8_t* touched = (fromLists && splitTouched) ? arena.ptr<uint8_t>("split_touched") : nullptr;
     if (fromLists) {
@@ -3768,13 +3823,17 @@ void Pipeline::detectNonManifoldVertices() {
 }
 
 void Pipeline::computeStats(int64_t out[9]) {
-    unsigned long long* d = arena.get<unsigned long long>("stats", 9);
-    zero(d, 9 * sizeof(unsigned long long));
-    const int64_t n = std::max(H, std::max(F, V));
-    if (n > 0 && H > 0)
-        kStats<<<(unsigned)std::min<int64_t>(gridFor(n), 4096), kBlock, 0, stream>>>(arena.ptr<int4>("he"), H, arena.ptr<int32_t>("face_he"), F, arena.ptr<int32_t>("bsize"),
-                                                  arena.ptr<int32_t>("brank"), arena.ptr<uint32_t>("vflags"), V, canonFlags(), d);
-    MDMC_HIP(hipMemcpyAsync(out, d, 9 * sizeof(int64_t), hipMemcpyDeviceToHost, stream));
+    const int64_t n = std::max<int64_t>(std::max(H, std::max(F, V)), 1);
+    kStats<<<(unsigned)std::min<int64_t>(gridFor(n), 4096), kBlock, 0, stream>>>(arena.ptr<int4>("he"), H, arena.ptr<int32_t>("face_he"), F, arena.ptr<int32_t>("bsize"),
+                                              arena.ptr<int32_t>("brank"), arena.ptr<uint32_t>("vflags"), V, canonFlags(), counters(), pinDev() + kPinFinal);
+    MDMC_HIP(hipStreamSynchronize(stream));
+    MDMC_HIP(hipGetLastError());
+    std::memcpy(out, pinHost() + kPinFinal + A_STATS, 9 * sizeof(int64_t));
+}
+
+void Pipeline::finishBatch() {
+    kStamp<<<1, 1, 0, stream>>>(stamp(ST_END));
+    MDMC_HIP(hipMemcpyAsync(pinHost() + kPinFinal, counters(), A_NCOUNTERS * sizeof(int64_t), hipMemcpyDeviceToHost, stream));
     MDMC_HIP(hipStreamSynchronize(stream));
 }
 

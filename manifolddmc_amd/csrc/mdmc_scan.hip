@@ -31,6 +31,7 @@ static_assert(kScanBlock == kLbBlock, "block size of the look-back");
 // with fewer tiles than the widest leaves the rest of its row idle).
 struct ScanJobs {
     ScanJob job[kScanJobs];
+    int64_t *stampStart, *stampEnd;
 };
 
 __global__ void __launch_bounds__(kScanBlock) kScan(ScanJobs jobs, uint32_t epoch, int64_t* __restrict__ directOut) {
@@ -38,6 +39,7 @@ __global__ void __launch_bounds__(kScanBlock) kScan(ScanJobs jobs, uint32_t epoc
     __shared__ int64_t s_wave[kScanBlock / 64];
     __shared__ long long s_off;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    stampClock(jobs.stampStart);
     const ScanJob& job = jobs.job[blockIdx.y];
     const int64_t t = blockIdx.x, n = job.n, numTiles = scanTiles(n);
     if (t >= numTiles) return;
@@ -125,7 +127,10 @@ __global__ void __launch_bounds__(kScanBlock) kScan(ScanJobs jobs, uint32_t epoc
                 if (o + i < n) out[o + i] = s_out[i];
         }
     }
-    if (t == numTiles - 1 && tid == 0 && job.total) *job.total = s_off + tileSum;
+    if (t == numTiles - 1 && tid == 0) {
+        if (job.total) *job.total = s_off + tileSum;
+        if (jobs.stampEnd && blockIdx.y == 0) *jobs.stampEnd = wall_clock64();
+    }
 }
 // Stream compaction in the same single pass: the indices i < n with (attr[i] & mask) != 0, in
 // increasing order, into idx[0 .. total).  Each tile counts its selected elements (16 per
@@ -134,7 +139,8 @@ __global__ void __launch_bounds__(kScanBlock) kScan(ScanJobs jobs, uint32_t epoc
 // before the tile) and writes its indices; nothing is written per unselected element.
 __global__ void __launch_bounds__(kScanBlock) kCompactFlagged(const uint32_t* __restrict__ attr, int64_t n, uint32_t mask, int32_t* __restrict__ idx,
                                                               unsigned long long* __restrict__ words, uint32_t epoch,
-                                                              int64_t* __restrict__ total, int64_t* __restrict__ directOut) {
+                                                              int64_t* __restrict__ total, int64_t* __restrict__ directOut, int64_t* stamp) {
+    stampClock(stamp);
     __shared__ int s_wave[kScanBlock / 64];
     __shared__ long long s_off;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
@@ -192,8 +198,10 @@ __global__ void __launch_bounds__(kScanBlock) kCompactFlagged(const uint32_t* __
 }
 }  // namespace
 
-void scanExclusiveI32(const ScanJob* jobs, int count, uint32_t epoch, hipStream_t s, int64_t* directOut) {
+void scanExclusiveI32(const ScanJob* jobs, int count, uint32_t epoch, hipStream_t s, int64_t* directOut, int64_t* stampStart, int64_t* stampEnd) {
     ScanJobs j{};
+    j.stampStart = stampStart;
+    j.stampEnd = stampEnd;
     int64_t tiles = 0;
     for (int k = 0; k < count; ++k) {
         j.job[k] = jobs[k];
@@ -203,8 +211,8 @@ void scanExclusiveI32(const ScanJob* jobs, int count, uint32_t epoch, hipStream_
 }
 
 void compactFlagged(const uint32_t* attr, int64_t n, uint32_t mask, int32_t* idx, int64_t* total, unsigned long long* words, uint32_t epoch,
-                    hipStream_t s, int64_t* directOut) {
-    kCompactFlagged<<<(unsigned)scanTiles(n), kScanBlock, 0, s>>>(attr, n, mask, idx, words, epoch, total, directOut);
+                    hipStream_t s, int64_t* directOut, int64_t* stamp) {
+    kCompactFlagged<<<(unsigned)scanTiles(n), kScanBlock, 0, s>>>(attr, n, mask, idx, words, epoch, total, directOut, stamp);
 }
 
 }  // namespace mdmc
