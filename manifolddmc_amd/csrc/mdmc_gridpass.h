@@ -95,8 +95,11 @@ struct GridPassArgs {
     int32_t* vcell;
     uint16_t* vct;
     int64_t V;
-    // per vertex its out-degree in the halfedge mesh (interior edges of its contour), when not null
-    int32_t* outdeg;
+    // the halfedge initialize's per-vertex arrays, which the vertex kernel starts: the out-degree in
+    // the halfedge mesh (interior edges of its contour; [V + 1], last entry 0), the valence the
+    // same (when a simplification follows, else null), cleared flags
+    int32_t *outdeg, *valence;
+    uint32_t* vflags;
     // recorded for the adjoint when not null: per cell (first vertex << 2 | contours - 1) or -1
     // (single-problem extractions only)
     int32_t* adjMap;
@@ -122,9 +125,10 @@ void launchSlabCount(int shape, const GridPassArgs& a, hipStream_t s);
 void launchSlabEmit(int shape, const GridPassArgs& a, hipStream_t s);
 // the halfedge initialize's outgoing lists from the grid pass's quads: entry off[v] + rank (the
 // rank from v's contour) of halfedge 4q + i from corner v = i holds 4q + i (out) and corners
-// i + 1 and i - 1 (ends); also the face -> halfedge array and the face attributes
+// i + 1 and i - 1 (ends); also the face -> halfedge array and the face attributes.  Inconsistent
+// quads are counted in *invalid (device) and raise *invalidPin (mapped pinned host memory)
 void launchQuadLists(const int4* quads, const uint32_t* qattr, int64_t Q, int64_t V, const int32_t* vcell, const uint16_t* vct, const int32_t* vpid,
                      const ProblemDev* probs, const int64_t* off, int32_t* out, int2* ends, int32_t* face_he, uint32_t* fattr, int64_t* invalid,
-                     hipStream_t s);
+                     int64_t* invalidPin, hipStream_t s);
 
 }  // namespace mdmc

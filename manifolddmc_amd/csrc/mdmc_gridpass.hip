@@ -997,7 +997,11 @@ __global__ void __launch_bounds__(GP_THREADS) kVertices(GridPassArgs a, int chun
         const uint64_t cw = contourWord(c_polyTab[ct & 0x3FF], ct >> 10);
         p = edgeMean(s, iso, cw);
         // out-degree of the vertex in the halfedge mesh: one quad per interior edge of its contour
-        if (a.outdeg) a.outdeg[v] = __popc(interiorEdgeMask(x, y, z, P.CX, P.CY, g.nz - 1) & c_contourEdges[4 * (ct & 0x3FF) + (ct >> 10)]);
+        const int deg = __popc(interiorEdgeMask(x, y, z, P.CX, P.CY, g.nz - 1) & c_contourEdges[4 * (ct & 0x3FF) + (ct >> 10)]);
+        a.outdeg[v] = deg;
+        if (a.valence) a.valence[v] = deg;
+        a.vflags[v] = 0;
+        if (v == a.V - 1) a.outdeg[a.V] = 0;
         if (a.surfIter) {
             moverInit(m, s, p);
             for (int k = 0; k < kMoveSteps && !m.done; ++k) moverStep(m, s, iso);
@@ -1074,7 +1078,8 @@ __global__ void __launch_bounds__(GP_THREADS) kVertices(GridPassArgs a, int chun
 __global__ void kQuadLists(const int4* __restrict__ quads, const uint32_t* __restrict__ qattr, int64_t Q, int64_t V,
                            const int32_t* __restrict__ vcell, const uint16_t* __restrict__ vct, const int32_t* __restrict__ vpid,
                            const ProblemDev* __restrict__ probs, const int64_t* __restrict__ off, int32_t* __restrict__ out,
-                           int2* __restrict__ ends, int32_t* __restrict__ face_he, uint32_t* __restrict__ fattr, int64_t* invalid) {
+                           int2* __restrict__ ends, int32_t* __restrict__ face_he, uint32_t* __restrict__ fattr, int64_t* invalid,
+                           int64_t* invalidPin) {
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= Q) return;
     const int4 v4 = quads[q];
@@ -1087,6 +1092,7 @@ __global__ void kQuadLists(const int4* __restrict__ quads, const uint32_t* __res
     for (int i = 0; i < 4; ++i) bad = bad || v[i] < 0 || v[i] >= V;
     if (bad) {
         atomicAdd((unsigned long long*)invalid, 1ULL);
+        *(volatile int64_t*)invalidPin = 1;
         return;
     }
     const ProblemDev& P = probs[vpid ? vpid[v[0]] : 0];
@@ -1126,7 +1132,10 @@ __global__ void kQuadLists(const int4* __restrict__ quads, const uint32_t* __res
         out[pos] = (int)(4 * q + i);
         ends[pos] = make_int2(v[(i + 1) & 3], v[(i + 3) & 3]);
     }
-    if (nbad) atomicAdd((unsigned long long*)invalid, (unsigned long long)nbad);
+    if (nbad) {
+        atomicAdd((unsigned long long*)invalid, (unsigned long long)nbad);
+        *(volatile int64_t*)invalidPin = 1;
+    }
 }
 
 }  // namespace
@@ -1246,8 +1255,8 @@ void launchSlabEmit(int shape, const GridPassArgs& a, hipStream_t s) {
 
 void launchQuadLists(const int4* quads, const uint32_t* qattr, int64_t Q, int64_t V, const int32_t* vcell, const uint16_t* vct, const int32_t* vpid,
                      const ProblemDev* probs, const int64_t* off, int32_t* out, int2* ends, int32_t* face_he, uint32_t* fattr, int64_t* invalid,
-                     hipStream_t s) {
-    if (Q > 0) kQuadLists<<<(unsigned)((Q + 255) / 256), 256, 0, s>>>(quads, qattr, Q, V, vcell, vct, vpid, probs, off, out, ends, face_he, fattr, invalid);
+                     int64_t* invalidPin, hipStream_t s) {
+    if (Q > 0) kQuadLists<<<(unsigned)((Q + 255) / 256), 256, 0, s>>>(quads, qattr, Q, V, vcell, vct, vpid, probs, off, out, ends, face_he, fattr, invalid, invalidPin);
 }
 
 void launchGridEmit(int shape, const GridPassArgs& a, hipStream_t s) {

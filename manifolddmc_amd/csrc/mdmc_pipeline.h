@@ -242,6 +242,10 @@ class Pipeline {
     // a refresh ran whose face-walk check (the invalid-record counter) is not read back yet
     bool refreshUnchecked = false;
     void checkValid(const char* what);
+    // after a wait: whether the initialize's quads were consistent (its count raises a pinned word)
+    void checkInit();
+    bool initUnchecked = false;
+    void emitArgs(GridPassArgs& a, int64_t C, bool recordAdjoint);
     void simplifyInit(int32_t** valence, int32_t** count, bool needCount);
     void simplifyCompactAndRebuild(int dropType, bool p3333);
     void simplifyDeferredStep(int dropType, bool p3333);

@@ -549,6 +549,39 @@ __global__ void kBucketsAll(const int4* __restrict__ quads, int64_t H, const int
     storeHalfedge(h, a, b, bucketFromOutEnds(h, a, b, H, off, out, ends, ctr), twin, bpack, vflags, fattr, qattr, valence);
 }
 
+// The same with the records, sizes and ranks written at once, when no simplification (which
+// reads ids and twins only) follows: one launch and 24 bytes per halfedge less to move than
+// kBucketsAll and kMaterialize.  Bound by the list gathers, as kBucketsAll is.  The quads are
+// checked (kQuadLists) but the host has not looked yet: if any was inconsistent, every record is
+// a boundary halfedge of vertex 0, which the kernels launched before the host's next wait can
+// follow.
+__global__ void __launch_bounds__(kBlock) kBuildHalfedges(const int4* __restrict__ quads, int64_t H, const int64_t* __restrict__ off,
+                                                          const int32_t* __restrict__ out, const int2* __restrict__ ends, int4* __restrict__ he,
+                                                          int32_t* __restrict__ bsize, int32_t* __restrict__ brank, uint32_t* __restrict__ vflags,
+                                                          uint32_t* __restrict__ fattr, int64_t* nmParts, int64_t* ctr) {
+    const int64_t hh = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const bool bad = ctr[A_INVALID] != 0;
+    int slotted = 0;
+    if (hh < H) {
+        const int h = (int)hh, f = h >> 2;
+        int a = 0;
+        BucketOf bk{2, 1, -1};
+        if (!bad) {
+            const int4 q = quads[f];
+            a = quadCorner(q, h & 3);
+            bk = bucketFromOutEnds(h, a, quadCorner(q, (h + 1) & 3), H, off, out, ends, ctr);
+        }
+        he[h] = make_int4(a, f, quadNext(h, 1), bk.twin);
+        bsize[h] = min(bk.n, 0xFFFF);
+        brank[h] = min(bk.rank, 0xFFFF);
+        slotted = slottedNM(min(bk.n, 0xFFFF), min(bk.rank, 0xFFFF)) ? 1 : 0;
+        const uint32_t vf = bad ? 0u : bucketVertexFlag(bk.n);
+        if (vf) atomicOr(&vflags[a], vf);
+        if (bk.n == 4) atomicOr(&fattr[f], (uint32_t)QA_NM);
+    }
+    blockAdd(nmParts, slotted);
+}
+
 // the halfedge records of the quads, from the ids and the twins, and the bucket sizes / ranks
 __global__ void __launch_bounds__(kBlock) kMaterialize(const int4* __restrict__ quads, int64_t H, const int32_t* __restrict__ twin,
                                                        const uint32_t* __restrict__ bpack, int4* __restrict__ he, int32_t* __restrict__ bsize,
@@ -2759,6 +2792,7 @@ int64_t Pipeline::compactNM(int32_t* nm, bool first) {
     // with the count, the invalid-record counter: a refresh's face walks add to it
     if (refreshUnchecked) MDMC_HIP(hipMemcpyAsync(h + 2, counters() + A_INVALID, sizeof(int64_t), hipMemcpyDeviceToHost, stream));
     MDMC_HIP(hipStreamSynchronize(stream));
+    checkInit();
     if (refreshUnchecked) {
         refreshUnchecked = false;
         if (h[2]) throw HipError("inconsistent mesh after splitting (" + std::to_string(h[2]) + " bad ids)", -4);
@@ -2802,8 +2836,9 @@ void Pipeline::FillBatch::flush() {
     blocks = 0;
 }
 
-// pinned words: the padding pass's "needs the exact blend", the copy of the counters at the end
-constexpr int kPinSpecial = 3, kPinFinal = 16;
+// pinned words: the padding pass's "needs the exact blend", the initialize's "inconsistent
+// quads", the copy of the counters at the end
+constexpr int kPinSpecial = 3, kPinInvalid = 4, kPinFinal = 16;
 static_assert(kPinFinal + A_NCOUNTERS <= Pipeline::kPinSlots, "pinned words");
 
 void Pipeline::prepare(const std::vector<ProblemDev>& problems, bool captured) {
@@ -2825,6 +2860,8 @@ void Pipeline::prepare(const std::vector<ProblemDev>& problems, bool captured) {
     su.special = pinDev() + kPinSpecial;
     su.token = captured ? 0 : ++prepToken_;
     pinHost()[kPinSpecial] = 0;
+    pinHost()[kPinInvalid] = 0;
+    initUnchecked = false;
     launchPrepareGrids(prep.desc[0], prep.dev, (int)prep.desc.size(), prep.rows, prep.refinement, prep.pad, su, stream);
 }
 
@@ -2869,6 +2906,25 @@ void Pipeline::stageTimes(double ms[9]) {
 }
 
 // ---- grid pass
+// the outputs of the emit part, sized exactly
+void Pipeline::emitArgs(GridPassArgs& a, int64_t C, bool recordAdjoint) {
+    if (V >= (int64_t)INT32_MAX / 2 || 4 * Q >= (int64_t)INT32_MAX) throw HipError("mesh exceeds the int32 id range", -3);
+    if (recordAdjoint && (V >= ((int64_t)1 << 29) || C >= (int64_t)INT32_MAX))
+        throw HipError("adjoint recording needs fewer than 2^29 vertices and 2^31 cells", -3);
+    a.pos = arena.get<float>("pos", 3 * (size_t)std::max<int64_t>(V, 1));
+    a.nrm = arena.get<float>("nrm", 3 * (size_t)std::max<int64_t>(V, 1));
+    a.quads = arena.get<int4>("quads", (size_t)std::max<int64_t>(Q, 1));
+    a.qattr = arena.get<uint32_t>("qattr", (size_t)std::max<int64_t>(Q, 1));
+    a.adjMap = recordAdjoint ? arena.get<int32_t>("adj_map", (size_t)std::max<int64_t>(C, 1)) : nullptr;
+    a.vcell = arena.get<int32_t>("gp_vcell", (size_t)std::max<int64_t>(V, 1));
+    a.vct = arena.get<uint16_t>("gp_vct", (size_t)std::max<int64_t>(V, 1));
+    a.outdeg = arena.get<int32_t>("out_cnt", (size_t)V + 1);  // the halfedge initialize's list lengths
+    a.vflags = arena.get<uint32_t>("vflags", (size_t)std::max<int64_t>(V, 1));
+    a.valence = simplifyQueue > 0 ? arena.get<int32_t>("valence", (size_t)std::max<int64_t>(V, 1)) : nullptr;
+    a.V = V;
+    a.vpid = nProblems > 1 ? arena.get<int32_t>("pid", (size_t)std::max<int64_t>(V, 1)) : nullptr;
+}
+
 // Row slabs: bands of at most SLAB_XMAX cells per row, R rows per block, and chunks of slices
 // sized so that the launch has about 4096 blocks (a problem gets its share by its cell count;
 // at least 8 slices per chunk, each chunk re-reads one slice before it for its quads).
@@ -2918,19 +2974,7 @@ void Pipeline::slabPass(std::vector<ProblemDev>& problems, int64_t C, int shape,
     MDMC_HIP(hipStreamSynchronize(stream));
     V = h[1];
     Q = h[2];
-    if (V >= (int64_t)INT32_MAX / 2 || 4 * Q >= (int64_t)INT32_MAX) throw HipError("mesh exceeds the int32 id range", -3);
-    if (recordAdjoint && (V >= ((int64_t)1 << 29) || C >= (int64_t)INT32_MAX))
-        throw HipError("adjoint recording needs fewer than 2^29 vertices and 2^31 cells", -3);
-    a.pos = arena.get<float>("pos", 3 * (size_t)std::max<int64_t>(V, 1));
-    a.nrm = arena.get<float>("nrm", 3 * (size_t)std::max<int64_t>(V, 1));
-    a.quads = arena.get<int4>("quads", (size_t)std::max<int64_t>(Q, 1));
-    a.qattr = arena.get<uint32_t>("qattr", (size_t)std::max<int64_t>(Q, 1));
-    a.adjMap = recordAdjoint ? arena.get<int32_t>("adj_map", (size_t)std::max<int64_t>(C, 1)) : nullptr;
-    a.vcell = arena.get<int32_t>("gp_vcell", (size_t)std::max<int64_t>(V, 1));
-    a.vct = arena.get<uint16_t>("gp_vct", (size_t)std::max<int64_t>(V, 1));
-    a.outdeg = arena.get<int32_t>("out_cnt", (size_t)V + 1);  // the halfedge initialize's list lengths
-    a.V = V;
-    a.vpid = nProblems > 1 ? arena.get<int32_t>("pid", (size_t)std::max<int64_t>(V, 1)) : nullptr;
+    emitArgs(a, C, recordAdjoint);
     tuneEvent(2);
     launchSlabEmit(shape, a, stream);
     tuneEvent(3);
@@ -3040,7 +3084,9 @@ bool Pipeline::runFrontGraph(const std::vector<int64_t>& shapeSig, std::vector<P
         std::memcpy((char*)fg_.stage + probOff, problems.data(), pbytes);
         probsDev = arena.ptr<ProblemDev>("gp_probs");
         refreshUnchecked = false;
+        initUnchecked = false;
         pinHost()[kPinSpecial] = 0;
+        pinHost()[kPinInvalid] = 0;
         ga_ = fgArgs_;
         MDMC_HIP(hipGraphLaunch(fg_.exec, stream));
         ++graphReplays;
@@ -3158,19 +3204,7 @@ void Pipeline::gridPassBack(std::vector<ProblemDev>& problems, int64_t C, int sh
     finishPrepare([&] { gridPassFront(problems, C, shape, surfIter, nullptr); });
     V = h[1];
     Q = h[2];
-    if (V >= (int64_t)INT32_MAX / 2 || 4 * Q >= (int64_t)INT32_MAX) throw HipError("mesh exceeds the int32 id range", -3);
-    if (recordAdjoint && (V >= ((int64_t)1 << 29) || C >= (int64_t)INT32_MAX))
-        throw HipError("adjoint recording needs fewer than 2^29 vertices and 2^31 cells", -3);
-    a.pos = arena.get<float>("pos", 3 * (size_t)std::max<int64_t>(V, 1));
-    a.nrm = arena.get<float>("nrm", 3 * (size_t)std::max<int64_t>(V, 1));
-    a.quads = arena.get<int4>("quads", (size_t)std::max<int64_t>(Q, 1));
-    a.qattr = arena.get<uint32_t>("qattr", (size_t)std::max<int64_t>(Q, 1));
-    a.adjMap = recordAdjoint ? arena.get<int32_t>("adj_map", (size_t)std::max<int64_t>(C, 1)) : nullptr;
-    a.vcell = arena.get<int32_t>("gp_vcell", (size_t)std::max<int64_t>(V, 1));
-    a.vct = arena.get<uint16_t>("gp_vct", (size_t)std::max<int64_t>(V, 1));
-    a.outdeg = arena.get<int32_t>("out_cnt", (size_t)V + 1);  // the halfedge initialize's list lengths
-    a.V = V;
-    a.vpid = nProblems > 1 ? arena.get<int32_t>("pid", (size_t)std::max<int64_t>(V, 1)) : nullptr;
+    emitArgs(a, C, recordAdjoint);
     tuneEvent(2);
     launchGridEmit(shape, a, stream);
     tuneEvent(3);
@@ -3225,12 +3259,11 @@ int32_t* Pipeline::bucketPassValence(const int64_t* off, int64_t nV) {
 void Pipeline::halfedgeInitialize() {
     H = 4 * Q;
     F = Q;
-    int32_t* twin = arena.get<int32_t>("twin", (size_t)std::max<int64_t>(H, 1));
     int32_t* face_he = arena.get<int32_t>("face_he", (size_t)F);
     uint32_t* fattr = arena.get<uint32_t>("fattr", (size_t)F);
-    uint32_t* vflags = arena.get<uint32_t>("vflags", (size_t)V);
-    int32_t* cnt = arena.get<int32_t>("out_cnt", (size_t)V + 1);
-    uint32_t* bpack = arena.get<uint32_t>("bpack", (size_t)std::max<int64_t>(H, 1));
+    // (cleared flags, list lengths and valence come from the grid pass's vertex kernel)
+    uint32_t* vflags = arena.ptr<uint32_t>("vflags");
+    const int32_t* cnt = arena.ptr<int32_t>("out_cnt");
     const int4* quads = arena.ptr<int4>("quads");
     uint32_t* qattr = arena.ptr<uint32_t>("qattr");
     // the vertex -> halfedge array is derived from these quads when it is copied out
@@ -3238,23 +3271,43 @@ void Pipeline::halfedgeInitialize() {
     vertHeQ = Q;
     // the list lengths (out-degrees) come from the grid pass's vertex kernel, the ranks from the
     // corner vertices' contours: no counting atomics
-    zero(cnt + V, sizeof(int32_t));
     int64_t* off = arena.get<int64_t>("out_off", (size_t)V + 1);
     scan({ScanJob{cnt, off, V + 1, nullptr, nullptr}}, stamp(ST_INIT));
     int32_t* out = arena.get<int32_t>("out_list", (size_t)std::max<int64_t>(H, 1));
     int2* ends = arena.get<int2>("out_ends", (size_t)std::max<int64_t>(H, 1));
     launchQuadLists(quads, qattr, Q, V, arena.ptr<int32_t>("gp_vcell"), arena.ptr<uint16_t>("gp_vct"), pid(), probsDev, off, out, ends, face_he, fattr,
-                    counters() + A_INVALID, stream);
-    checkValid("quad vertex ids");
-    zero(vflags, (size_t)V * sizeof(uint32_t));
-    int32_t* valence = bucketPassValence(off, V);
-    if (H > 0) kBucketsAll<<<gridFor(H), kBlock, 0, stream>>>(quads, H, off, out, ends, twin, bpack, vflags, fattr, qattr, valence, counters());
-    heMaterialized = false;
+                    counters() + A_INVALID, pinDev() + kPinInvalid, stream);
+    initUnchecked = true;
+    valenceReady = simplifyQueue > 0;
+    if (simplifyQueue > 0) {
+        MDMC_HIP(hipStreamSynchronize(stream));
+        checkInit();
+        int32_t* twin = arena.get<int32_t>("twin", (size_t)std::max<int64_t>(H, 1));
+        uint32_t* bpack = arena.get<uint32_t>("bpack", (size_t)std::max<int64_t>(H, 1));
+        if (H > 0)
+            kBucketsAll<<<gridFor(H), kBlock, 0, stream>>>(quads, H, off, out, ends, twin, bpack, vflags, fattr, qattr, arena.ptr<int32_t>("valence"),
+                                                           counters());
+        heMaterialized = false;
+    } else {
+        // no simplification reads ids and twins only: the records at once
+        int4* he = arena.get<int4>("he", (size_t)std::max<int64_t>(H, 1));
+        int32_t* bsize = arena.get<int32_t>("bsize", (size_t)std::max<int64_t>(H, 1));
+        int32_t* brank = arena.get<int32_t>("brank", (size_t)std::max<int64_t>(H, 1));
+        if (H > 0)
+            kBuildHalfedges<<<gridFor(H), kBlock, 0, stream>>>(quads, H, off, out, ends, he, bsize, brank, vflags, fattr, nmSlotParts(), counters());
+        heMaterialized = true;
+    }
     posSlotted = false;  // the grid pass wrote positions by vertex
     deferredSteps = 0;
     listsV = V;
     splitTouched = false;
     canonTracked = false;
+}
+
+void Pipeline::checkInit() {
+    if (!initUnchecked) return;
+    initUnchecked = false;
+    if (pinHost()[kPinInvalid]) checkValid("quad vertex ids");
 }
 
 void Pipeline::checkValid(const char* what) {
@@ -3773,6 +3826,10 @@ void Pipeline::buildMergeList(const int2* rec, int64_t R, int count, int32_t* nu
 
 void Pipeline::detectNonManifoldVertices() {
     if (H == 0 || V == 0) return;
+    if (initUnchecked) {  // the walks follow the lists
+        MDMC_HIP(hipStreamSynchronize(stream));
+        checkInit();
+    }
     int4* he = arena.ptr<int4>("he");
     uint32_t* vflags = arena.ptr<uint32_t>("vflags");
     // fast path: vertices with one closed fan
@@ -3828,6 +3885,7 @@ void Pipeline::computeStats(int64_t out[9]) {
                                               arena.ptr<int32_t>("brank"), arena.ptr<uint32_t>("vflags"), V, canonFlags(), counters(), pinDev() + kPinFinal);
     MDMC_HIP(hipStreamSynchronize(stream));
     MDMC_HIP(hipGetLastError());
+    checkInit();
     std::memcpy(out, pinHost() + kPinFinal + A_STATS, 9 * sizeof(int64_t));
 }
 
