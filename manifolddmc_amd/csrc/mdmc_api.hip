@@ -311,11 +311,12 @@ mdmc_status runExtraction(mdmc_ctx* ctx, const mdmc_grid* grids, int G, const fl
             if (flags & MDMC_P3X3Y_OLD) p.simplify3X3Y(false);
             if (flags & MDMC_P3333) p.simplify3333();
             p.fixManifoldTwins();
-            if (flags & MDMC_SPLIT_NM) p.split(opt->split_step, opt->max_split_iters > 0 ? opt->max_split_iters : 64);
-            if (flags & MDMC_DETECT_NM_VERTS) p.detectNonManifoldVertices();
+            const int maxIters = opt->max_split_iters > 0 ? opt->max_split_iters : 64;
             if (B == 1) {
-                p.computeStats(st9);
+                p.finishSingle((flags & MDMC_SPLIT_NM) != 0, opt->split_step, maxIters, (flags & MDMC_DETECT_NM_VERTS) != 0, st9);
             } else {
+                if (flags & MDMC_SPLIT_NM) p.split(opt->split_step, maxIters);
+                if (flags & MDMC_DETECT_NM_VERTS) p.detectNonManifoldVertices();
                 p.regroupBatch(B);
                 p.finishBatch();
                 for (int b = 0; b < B; ++b)
@@ -330,7 +331,7 @@ mdmc_status runExtraction(mdmc_ctx* ctx, const mdmc_grid* grids, int G, const fl
                 p.batchFOff.assign((size_t)B + 1, 0);
                 p.batchStats.assign(9 * (size_t)B, 0);
             }
-            p.computeStats(st9);
+            p.finishEmpty();
         }
         ctx->hasResult = true;
         ctx->nProblems = B;

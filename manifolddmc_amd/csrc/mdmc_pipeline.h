@@ -83,8 +83,9 @@ class Pipeline {
     // the end of an extraction: with the statistics kernel's last block (one problem), or after a
     // batch's regroup, the counters, statistics and stage clocks go to pinned memory in one
     // read-back; the getters below read that copy
-    void computeStats(int64_t out[9]);
+    void finishSingle(bool doSplit, int step, int maxIters, bool doDetect, int64_t st9[9]);
     void finishBatch();
+    void finishEmpty();
     void counterTotals(int64_t* anomalyCount, int64_t* mergeSeq, int64_t* lookbackDirect);
     // stage times in ms, from the clock stamps of the stages' first kernels: whole call, then the
     // seven stages of mdmc_stats in order, then the grid pass alone
@@ -197,7 +198,15 @@ class Pipeline {
     uint32_t lbEpoch_ = 0;
     int64_t prepToken_ = 0;
     int clockKHz_ = 0;
-    int64_t compactNM(int32_t* nm, bool first);
+    int32_t* listNM(bool first);
+    int64_t checkNM(const int64_t* h);
+    const int64_t* readCounters();
+    void splitStep(int step, int64_t n64, const int32_t* nm);
+    void launchDetect(int guarded);
+    void detectSlow(int64_t nSlow, int64_t nSlowOff);
+    void launchStats(int guarded);
+    const int64_t* waitStats();
+    int64_t touchedV = 0;  // vertices the splitter's touched flags cover
     void zero(void* p, size_t bytes);
     void fillNeg(void* p, size_t bytes);
     void launchFill(void* p, uint8_t byte, size_t bytes);

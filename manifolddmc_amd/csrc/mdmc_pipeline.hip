@@ -38,7 +38,7 @@ constexpr int kFanGuard = 4096;
 
 // ---------------------------------------------------------------- counters
 enum : int { A_ANOMALY = 0, A_CONFLICT = 1, A_INVALID = 2, A_DIRTY = 3, A_FALLBACK = 5, A_MERGE_SEQ = 6, A_LB_DIRECT = 7,
-             A_STAMP = 8, A_STATS = A_STAMP + ST_COUNT, A_TICKET = A_STATS + 9, A_NCOUNTERS };
+             A_NM = 8, A_NSLOW = 9, A_NSLOW_OFF = 10, A_STAMP = 11, A_STATS = A_STAMP + ST_COUNT, A_TICKET = A_STATS + 9, A_NCOUNTERS };
 // the slotted non-manifold halfedges the split's working copy marks (markHalfedgesAsNonManifold,
 // ManifoldSplitter.cu:527-555, reads the four slots of every full vertex-pair bucket): every
 // halfedge of a bucket of 4, and of a larger bucket the ones at ranks 1, 2, 3 and size - 1
@@ -65,6 +65,15 @@ __device__ __forceinline__ int64_t sumParts(const int64_t* parts, int lane) {
 #pragma unroll
     for (int d = 32; d > 0; d >>= 1) v += __shfl_down(v, d, 64);
     return v;
+}
+
+// The kernels that end an extraction are launched behind the list of the non-manifold faces
+// without waiting for its length (kAwaitSplit): they return at once where faces are left to
+// split, or a check failed, and the host then splits and launches them again.  The statistics
+// also wait (kAwaitFans) where the fan detection left vertices to its slow pass.
+enum : int { kAwaitSplit = 1, kAwaitFans = 2 };
+__device__ __forceinline__ bool notYet(const int64_t* ctr, int guarded) {
+    return ((guarded & kAwaitSplit) && (ctr[A_NM] != 0 || ctr[A_INVALID] != 0)) || ((guarded & kAwaitFans) && ctr[A_NSLOW] != 0);
 }
 
 __device__ __forceinline__ void anomaly(int64_t* ctr) { atomicAdd((unsigned long long*)&ctr[A_ANOMALY], 1ULL); }
@@ -119,6 +128,11 @@ __device__ __forceinline__ int64_t firstOfFour() { return 4 * ((int64_t)blockIdx
 __device__ __forceinline__ bool vec4(int64_t i0, int64_t n, const void* a, const void* b) {
     return i0 + 3 < n && ((((uintptr_t)a) | ((uintptr_t)b)) & 15) == 0;
 }
+
+// pinned words: the padding pass's "needs the exact blend", the initialize's "inconsistent
+// quads", the copy of the counters at the end
+constexpr int kPinSpecial = 3, kPinInvalid = 4, kPinFinal = 16;
+static_assert(kPinFinal + A_NCOUNTERS <= Pipeline::kPinSlots, "pinned words");
 
 // ---------------------------------------------------------------- halfedge construction
 // bucket order after refreshHashTable: (face, position along the face from its first halfedge)
@@ -1139,10 +1153,12 @@ __global__ void __launch_bounds__(kBlock) kAffectedFlags(const uint8_t* __restri
 
 // list lengths of the fan detection's slow vertices: their out-degree (the halfedges
 // kOutDegree / the outgoing lists counted per origin), 0 for the others
-__global__ void kSlowDegree(const uint8_t* __restrict__ slow, const int32_t* __restrict__ outdeg, int64_t V, int32_t* __restrict__ deg) {
+// (outdeg null: the build's list lengths)
+__global__ void kSlowDegree(const uint8_t* __restrict__ slow, const int32_t* __restrict__ outdeg, const int64_t* __restrict__ listOff, int64_t V,
+                            int32_t* __restrict__ deg) {
     const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (v > V) return;
-    deg[v] = (v < V && slow[v]) ? outdeg[v] : 0;
+    deg[v] = (v < V && slow[v]) ? (outdeg ? outdeg[v] : (int32_t)(listOff[v + 1] - listOff[v])) : 0;
 }
 
 // outgoing-halfedge lists (by origin) for the fan detection, of the vertices in `only`
@@ -1191,7 +1207,9 @@ __global__ void kOutDegree(const int4* __restrict__ he, int64_t H, int64_t V, in
 // counts every touched vertex from all records.  Vertices from listsV on are counted there.
 __global__ void __launch_bounds__(kBlock) kOutFromLists(const int64_t* __restrict__ off, const int32_t* __restrict__ out, int64_t listsV,
                                                         const uint8_t* __restrict__ touched, const uint8_t* __restrict__ canon, int64_t V,
-                                                        int32_t* __restrict__ outdeg, int32_t* __restrict__ rep) {
+                                                        int32_t* __restrict__ outdeg, int32_t* __restrict__ rep, int64_t* ctr, int guarded) {
+    if (notYet(ctr, guarded)) return;
+    stampClock(ctr + A_STAMP + ST_DETECT);
     __shared__ int s_list[kSparsePer * kBlock];
     __shared__ int s_n;
     const int total = gatherSparse(
@@ -1227,7 +1245,9 @@ __global__ void __launch_bounds__(kBlock) kOutFromLists(const int64_t* __restric
 // its origin's out-degree, and the first one of a vertex with no other outgoing halfedge
 // becomes its walk start
 __global__ void kOutDegreeMoved(const int4* __restrict__ he, int64_t H, int64_t V, int64_t listsV, const uint8_t* __restrict__ touched,
-                                const uint8_t* __restrict__ canon, int32_t* __restrict__ outdeg, int32_t* __restrict__ rep, int64_t* ctr) {
+                                const uint8_t* __restrict__ canon, int32_t* __restrict__ outdeg, int32_t* __restrict__ rep, int64_t* ctr,
+                                int guarded) {
+    if (notYet(ctr, guarded)) return;
     const int64_t h = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (h >= H || canon[h]) return;
     const int o = heO(he, (int)h);
@@ -1264,17 +1284,29 @@ __global__ void kOutDegreeTouched(const int4* __restrict__ he, int64_t H, int64_
 // halfedges, the vertex has one fan.  Every fan walk of fanWalk from any of them then covers
 // both chains: faces are quads, and at a vertex with no bucket of 3 among its edges
 // (VF_WEIRD unset) every twin involved is mutual, so each walk direction undoes the other.
-__global__ void kFanFast(const int4* __restrict__ he, int64_t H, int64_t V, const int32_t* __restrict__ outdeg, const int32_t* __restrict__ rep,
-                         uint32_t* __restrict__ vflags, uint8_t* __restrict__ slow, const uint8_t* __restrict__ touched, int64_t listsV,
-                         const uint8_t* __restrict__ canon, int64_t* __restrict__ nslow) {
+// LISTS: nothing was split, so out-degree and start come from the build's lists (off, out) here;
+// else outdeg and rep hold them.
+template <bool LISTS>
+__global__ void kFanFast(const int4* __restrict__ he, int64_t H, int64_t V, const int64_t* __restrict__ off, const int32_t* __restrict__ out,
+                         const int32_t* __restrict__ outdeg, const int32_t* __restrict__ rep, uint32_t* __restrict__ vflags, uint8_t* __restrict__ slow,
+                         const uint8_t* __restrict__ touched, int64_t listsV, const uint8_t* __restrict__ canon, int64_t* __restrict__ ctr, int guarded) {
+    if (notYet(ctr, guarded)) return;
+    if (LISTS) stampClock(ctr + A_STAMP + ST_DETECT);
     const int64_t vv = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (vv >= V) return;
     const int v = (int)vv;
-    const int d = outdeg[v];
+    int64_t o = 0;
+    int d;
+    if (LISTS) {
+        o = off[v];
+        d = (int)(off[v + 1] - o);
+    } else {
+        d = outdeg[v];
+    }
     bool single = d == 0;  // no outgoing halfedge: no fan, flag cleared
     const bool mayMove = canon && (!touched || v >= listsV || touched[v]);
     if (d > 0) {
-        const int start = rep[v];
+        const int start = LISTS ? out[o] : rep[v];
         int cur = start;
         int4 e = he[start];  // the record of cur: one load gives the next step's origin check and twin
         int open = 0;        // the outgoing halfedges the clockwise walk visited before it stopped
@@ -1329,8 +1361,8 @@ __global__ void kFanFast(const int4* __restrict__ he, int64_t H, int64_t V, cons
     const uint64_t m = __ballot(!single);
     const uint64_t mt = __ballot(!single && (v >= listsV || (touched && touched[v])));
     const int leader = (int)(threadIdx.x & 63) == __ffsll((unsigned long long)(m ? m : 1ULL)) - 1;
-    if (m && leader) atomicAdd((unsigned long long*)nslow, (unsigned long long)__popcll(m));
-    if (mt && leader) atomicAdd((unsigned long long*)(nslow + 1), (unsigned long long)__popcll(mt));
+    if (m && leader) atomicAdd((unsigned long long*)&ctr[A_NSLOW], (unsigned long long)__popcll(m));
+    if (mt && leader) atomicAdd((unsigned long long*)&ctr[A_NSLOW_OFF], (unsigned long long)__popcll(mt));
 }
 
 // ---------------------------------------------------------------- simplifications
@@ -2517,7 +2549,12 @@ __global__ void __launch_bounds__(kBlock) kDetectFans(const int4* __restrict__ h
 // counts over the vertex-pair buckets (HalfedgeMesh.cu:1164-1239, ManifoldCreator.cu:545-549)
 __global__ void __launch_bounds__(kBlock) kStats(const int4* __restrict__ he, int64_t H, const int32_t* __restrict__ face_he, int64_t F,
                                                  const int32_t* __restrict__ bsize, const int32_t* __restrict__ brank, const uint32_t* __restrict__ vflags,
-                                                 int64_t V, const uint8_t* __restrict__ canon, int64_t* __restrict__ ctr, int64_t* __restrict__ pin) {
+                                                 int64_t V, const uint8_t* __restrict__ canon, int64_t* __restrict__ ctr, int64_t* __restrict__ pin,
+                                                 int guarded) {
+    if (notYet(ctr, guarded)) {
+        if (blockIdx.x == 0 && threadIdx.x < A_NCOUNTERS) pin[threadIdx.x] = ctr[threadIdx.x];
+        return;
+    }
     stampClock(ctr + A_STAMP + ST_STATS);
     __shared__ unsigned int acc[9];
     __shared__ bool s_last;
@@ -2782,24 +2819,32 @@ int64_t Pipeline::scan32(const int32_t* in, int64_t n, const std::string& outNam
     return h[1];
 }
 
-// the faces with the NM bit, ascending, into nm (capacity F); returns their number
-int64_t Pipeline::compactNM(int32_t* nm, bool first) {
-    int64_t* h = pinHost();
-    int64_t* d = pinDev();
+// lists the faces with the NM bit, ascending (countNonManifoldFaces); their number goes to the
+// counter A_NM
+int32_t* Pipeline::listNM(bool first) {
+    int32_t* nm = arena.get<int32_t>("nmlist", (size_t)std::max<int64_t>(F, 1));
     const Lookback lb = lookback(scanTiles(F));
-    compactFlagged(arena.ptr<uint32_t>("fattr"), F, (uint32_t)QA_NM, nm, d + 1, lb.words, lb.epoch, stream, lookbackDiag(),
+    compactFlagged(arena.ptr<uint32_t>("fattr"), F, (uint32_t)QA_NM, nm, counters() + A_NM, lb.words, lb.epoch, stream, lookbackDiag(),
                    first ? stamp(ST_SPLIT) : nullptr);
-    // with the count, the invalid-record counter: a refresh's face walks add to it
-    if (refreshUnchecked) MDMC_HIP(hipMemcpyAsync(h + 2, counters() + A_INVALID, sizeof(int64_t), hipMemcpyDeviceToHost, stream));
-    MDMC_HIP(hipStreamSynchronize(stream));
-    checkInit();
-    if (refreshUnchecked) {
-        refreshUnchecked = false;
-        if (h[2]) throw HipError("inconsistent mesh after splitting (" + std::to_string(h[2]) + " bad ids)", -4);
-    }
-    const int64_t n = h[1];
+    return nm;
+}
+
+// the checks and the number of listed faces, from the counters in h
+int64_t Pipeline::checkNM(const int64_t* h) {
+    if (h[A_INVALID])
+        throw HipError(std::string("inconsistent mesh after ") + (refreshUnchecked ? "splitting" : "quad vertex ids") + " (" +
+                           std::to_string(h[A_INVALID]) + " bad ids)", -4);
+    initUnchecked = refreshUnchecked = false;
+    const int64_t n = h[A_NM];
     if (n < 0 || n > F) throw HipError("inconsistent NM-face count (" + std::to_string(n) + ")", -4);
     return n;
+}
+
+const int64_t* Pipeline::readCounters() {
+    int64_t* h = pinHost() + kPinFinal;
+    MDMC_HIP(hipMemcpyAsync(h, counters(), A_NCOUNTERS * sizeof(int64_t), hipMemcpyDeviceToHost, stream));
+    MDMC_HIP(hipStreamSynchronize(stream));
+    return h;
 }
 
 // fills with one launch (the runtime's memset launches a body and a tail kernel)
@@ -2835,11 +2880,6 @@ void Pipeline::FillBatch::flush() {
     fs.count = 0;
     blocks = 0;
 }
-
-// pinned words: the padding pass's "needs the exact blend", the initialize's "inconsistent
-// quads", the copy of the counters at the end
-constexpr int kPinSpecial = 3, kPinInvalid = 4, kPinFinal = 16;
-static_assert(kPinFinal + A_NCOUNTERS <= Pipeline::kPinSlots, "pinned words");
 
 void Pipeline::prepare(const std::vector<ProblemDev>& problems, bool captured) {
     refreshUnchecked = false;
@@ -3601,29 +3641,80 @@ void Pipeline::fixManifoldTwins() {
                                                  counters());
 }
 
-// ---- ManifoldSplitter::run
-void Pipeline::split(int step, int maxIters) {
-    const bool copyDataBack = true;
+// ---- ManifoldSplitter::run, one problem and all that follows: the last stages are launched
+// behind the face list without waiting for its length (see notYet), so a mesh with nothing to
+// split waits once, at its end, instead of after the list, the fan detection and the statistics
+// (about 12 us of idle GPU each); where faces are split, the launches that returned at once
+// cost about 10 us an iteration.
+void Pipeline::finishSingle(bool doSplit, int step, int maxIters, bool doDetect, int64_t st9[9]) {
     int iter = 0;
-    // every vertex any step touches (for the NM-vertex detection's use of the outgoing lists)
-    int64_t touchedV = V;
-    uint8_t* touched = arena.get<uint8_t>("split_touched", (size_t)std::max<int64_t>(V, 1));
-    zero(touched, (size_t)V);
-    splitTouched = true;
+    bool again = doSplit;
     while (true) {
-        const int64_t iterH = H;
-        // countNonManifoldFaces: the NM faces' ids, ascending, in one compaction pass
-        int32_t* nm = arena.get<int32_t>("nmlist", (size_t)std::max<int64_t>(F, 1));
-        const int64_t n64 = compactNM(nm, iter == 0);
-        if (n64 == 0) break;
-        // still non-manifold after the allowed iterations (the reference loops until clean)
+        const int32_t* nm = again ? listNM(iter == 0) : nullptr;
+        const int guarded = again || iter == 0 ? kAwaitSplit : 0;
+        if (doDetect) launchDetect(guarded);
+        launchStats(guarded | kAwaitFans);
+        const int64_t* h = waitStats();
+        const int64_t n = guarded ? checkNM(h) : 0;
+        if (n == 0) break;
+        if (iter >= maxIters) {
+            // still non-manifold after the allowed iterations (the reference loops until clean)
+            extraAnomalies += 1;
+            if (doDetect) launchDetect(0);
+            launchStats(kAwaitFans);
+            waitStats();
+            break;
+        }
+        splitStep(step, n, nm);
+        ++iter;
+        splitIterations = iter;
+        again = step >= 6;
+    }
+    const int64_t* h = pinHost() + kPinFinal;
+    if (doDetect && h[A_NSLOW] != 0) {
+        detectSlow(h[A_NSLOW], h[A_NSLOW_OFF]);
+        launchStats(0);
+        h = waitStats();
+    }
+    if (h[A_INVALID]) checkNM(h);
+    refreshUnchecked = false;
+    std::memcpy(st9, h + A_STATS, 9 * sizeof(int64_t));
+}
+
+// the splitter alone (a batch, whose regroup follows)
+void Pipeline::split(int step, int maxIters) {
+    int iter = 0;
+    while (true) {
+        const int32_t* nm = listNM(iter == 0);
+        const int64_t n = checkNM(readCounters());
+        if (n == 0) break;
         if (iter >= maxIters) {
             extraAnomalies += 1;
             break;
         }
-        if (20 * n64 >= (int64_t)INT32_MAX / 2) throw HipError("working copy exceeds the int32 id range", -3);
-        const int n = (int)n64;
+        splitStep(step, n, nm);
+        splitIterations = ++iter;
+        if (step < 6) break;
+    }
+    if (refreshUnchecked) {
+        refreshUnchecked = false;
+        checkValid("splitting");
+    }
+}
 
+// one iteration over the n listed faces
+void Pipeline::splitStep(int step, int64_t n64, const int32_t* nm) {
+    if (20 * n64 >= (int64_t)INT32_MAX / 2) throw HipError("working copy exceeds the int32 id range", -3);
+    const int n = (int)n64;
+    const int64_t iterH = H;
+    // every vertex any step touches (for the NM-vertex detection's use of the outgoing lists)
+    if (!splitTouched) {
+        touchedV = V;
+        zero(arena.get<uint8_t>("split_touched", (size_t)std::max<int64_t>(V, 1)), (size_t)V);
+        splitTouched = true;
+    }
+    uint8_t* touched = arena.ptr<uint8_t>("split_touched");
+    {
         WC w;
         w.n = n;
         const int nv = 8 * n, nh = 20 * n, nf = 5 * n;
@@ -3728,7 +3819,7 @@ void Pipeline::split(int step, int maxIters) {
         }
         if (step >= 5) kMoveToSurface<<<gridFor(vsize), kBlock, 0, stream>>>(w, vsize, probsDev);
 
-        if (copyDataBack || step >= 6) {
+        {
             // the new vertices, halfedges and faces of the working copy: three prefix sums
             // and one read-back of their totals ([1..3])
             int32_t* pv = arena.get<int32_t>("cb_pred_v", (size_t)std::max(vsize, 1));
@@ -3799,14 +3890,6 @@ void Pipeline::split(int step, int maxIters) {
         }
         if (vsize > 0) kMarkWcVertices<<<gridFor(vsize), kBlock, 0, stream>>>(w, vsize, dirtyV, touched);
         refreshHashTable(dirtyV, iterH);
-        ++iter;
-        splitIterations = iter;
-        if (!(step >= 6) || !copyDataBack) break;
-    }
-    if (iter == 0) splitTouched = false;  // nothing changed: the lists describe every vertex
-    if (refreshUnchecked) {
-        refreshUnchecked = false;
-        checkValid("splitting");
     }
 }
 
@@ -3824,51 +3907,58 @@ void Pipeline::buildMergeList(const int2* rec, int64_t R, int count, int32_t* nu
     if (count > 0) kRecApply<<<gridFor(count), kBlock, 0, stream>>>(rec, count, roff, idx, cnt, num, ex, ey);
 }
 
-void Pipeline::detectNonManifoldVertices() {
+void Pipeline::launchDetect(int guarded) {
     if (H == 0 || V == 0) return;
-    if (initUnchecked) {  // the walks follow the lists
-        MDMC_HIP(hipStreamSynchronize(stream));
-        checkInit();
-    }
-    int4* he = arena.ptr<int4>("he");
+    const int4* he = arena.ptr<int4>("he");
     uint32_t* vflags = arena.ptr<uint32_t>("vflags");
-    // fast path: vertices with one closed fan
-    int32_t* outdeg = arena.get<int32_t>("outdeg", (size_t)V);
-    int32_t* rep = arena.get<int32_t>("outrep", (size_t)V);
     uint8_t* slow = arena.get<uint8_t>("fan_slow", (size_t)V);
-    // the slow-vertex count is accumulated in device memory (atomics on mapped host memory
-    // cross the bus one by one) and read back once
-    int64_t* nslow = arena.get<int64_t>("fan_nslow", 2);
-    {
-        FillBatch fb(*this);
-        fb.stampAt(stamp(ST_DETECT));
-        fb.add(outdeg, 0x00, (size_t)V * sizeof(int32_t));
-        fb.add(nslow, 0x00, 2 * sizeof(int64_t));
-    }
+    const int64_t *off = arena.ptr<int64_t>("out_off");
+    const int32_t* out = arena.ptr<int32_t>("out_list");
     const bool fromLists = listsV >= 0 && listsV <= V;
     const uint8_t* touched = (fromLists && splitTouched) ? arena.ptr<uint8_t>("split_touched") : nullptr;
+    const uint8_t* canon = canonFlags();  // kept since the splitter's first write-back
+    if (fromLists && listsV == V && !touched && !canon) {
+        kFanFast<true><<<gridFor(V), kBlock, 0, stream>>>(he, H, V, off, out, nullptr, nullptr, vflags, slow, nullptr, V, nullptr, counters(), guarded);
+        return;
+    }
+    int32_t* outdeg = arena.get<int32_t>("outdeg", (size_t)V);
+    int32_t* rep = arena.get<int32_t>("outrep", (size_t)V);
     if (fromLists) {
-        const uint8_t* canon = canonFlags();  // kept since the splitter's first write-back
-        if (V > 0)
-            kOutFromLists<<<sparseBlocks(V), kBlock, 0, stream>>>(arena.ptr<int64_t>("out_off"), arena.ptr<int32_t>("out_list"), listsV, touched, canon,
-                                                                  V, outdeg, rep);
+        // (writes every vertex's out-degree)
+        kOutFromLists<<<sparseBlocks(V), kBlock, 0, stream>>>(off, out, listsV, touched, canon, V, outdeg, rep, counters(), guarded);
         if (canon) {
-            if (H > 0) kOutDegreeMoved<<<gridFor(H), kBlock, 0, stream>>>(he, H, V, listsV, touched, canon, outdeg, rep, counters());
+            kOutDegreeMoved<<<gridFor(H), kBlock, 0, stream>>>(he, H, V, listsV, touched, canon, outdeg, rep, counters(), guarded);
         } else if (touched || V > listsV) {
             kOutDegreeTouched<<<gridFor(H), kBlock, 0, stream>>>(he, H, V, listsV, touched, outdeg, rep, counters());
         }
     } else {
+        zero(outdeg, (size_t)V * sizeof(int32_t));
         kOutDegree<<<gridFor(H), kBlock, 0, stream>>>(he, H, V, outdeg, rep, counters());
     }
-    kFanFast<<<gridFor(V), kBlock, 0, stream>>>(he, H, V, outdeg, rep, vflags, slow, touched, fromLists ? listsV : 0, canonFlags(), nslow);
-    int64_t* hc = pinHost();
-    MDMC_HIP(hipMemcpyAsync(hc, nslow, 2 * sizeof(int64_t), hipMemcpyDeviceToHost, stream));
-    MDMC_HIP(hipStreamSynchronize(stream));
-    const int64_t nSlow = hc[0], nSlowOff = hc[1];
-    if (nSlow == 0) return;  // every vertex has one closed fan, or none
-    // the others over their outgoing lists
+    kFanFast<false><<<gridFor(V), kBlock, 0, stream>>>(he, H, V, off, out, outdeg, rep, vflags, slow, touched, fromLists ? listsV : 0, canon, counters(),
+                                                       guarded);
+}
+
+void Pipeline::detectNonManifoldVertices() {
+    if (initUnchecked) {  // the walks follow the lists
+        MDMC_HIP(hipStreamSynchronize(stream));
+        checkInit();
+    }
+    launchDetect(0);
+    const int64_t* h = readCounters();
+    if (h[A_NSLOW]) detectSlow(h[A_NSLOW], h[A_NSLOW_OFF]);
+}
+
+// the vertices launchDetect left, over their outgoing lists (nSlowOff of them with lists that
+// are not the build's)
+void Pipeline::detectSlow(int64_t nSlow, int64_t nSlowOff) {
+    const int4* he = arena.ptr<int4>("he");
+    uint32_t* vflags = arena.ptr<uint32_t>("vflags");
+    const uint8_t* slow = arena.ptr<uint8_t>("fan_slow");
+    const bool fast = listsV == V && !splitTouched && !canonFlags();
+    int32_t* outdeg = arena.get<int32_t>("outdeg", (size_t)V);
     int32_t* deg = arena.get<int32_t>("deg", (size_t)V + 1);
-    kSlowDegree<<<gridFor(V + 1), kBlock, 0, stream>>>(slow, outdeg, V, deg);
+    kSlowDegree<<<gridFor(V + 1), kBlock, 0, stream>>>(slow, fast ? nullptr : outdeg, fast ? arena.ptr<int64_t>("out_off") : nullptr, V, deg);
     int64_t* off = arena.get<int64_t>("off", (size_t)V + 1);
     scan(deg, off, V + 1);
     int32_t* list = arena.get<int32_t>("list", (size_t)H);
@@ -3879,20 +3969,28 @@ void Pipeline::detectNonManifoldVertices() {
     kDetectFans<<<gridFor(V), kBlock, 0, stream>>>(he, V, slow, off, list, copyLists ? nullptr : deg, vflags, key, counters());
 }
 
-void Pipeline::computeStats(int64_t out[9]) {
+void Pipeline::launchStats(int guarded) {
     const int64_t n = std::max<int64_t>(std::max(H, std::max(F, V)), 1);
     kStats<<<(unsigned)std::min<int64_t>(gridFor(n), 4096), kBlock, 0, stream>>>(arena.ptr<int4>("he"), H, arena.ptr<int32_t>("face_he"), F, arena.ptr<int32_t>("bsize"),
-                                              arena.ptr<int32_t>("brank"), arena.ptr<uint32_t>("vflags"), V, canonFlags(), counters(), pinDev() + kPinFinal);
-    MDMC_HIP(hipStreamSynchronize(stream));
+                                              arena.ptr<int32_t>("brank"), arena.ptr<uint32_t>("vflags"), V, canonFlags(), counters(), pinDev() + kPinFinal, guarded);
     MDMC_HIP(hipGetLastError());
-    checkInit();
-    std::memcpy(out, pinHost() + kPinFinal + A_STATS, 9 * sizeof(int64_t));
+}
+
+// waits for the statistics; the counters they handed over
+const int64_t* Pipeline::waitStats() {
+    MDMC_HIP(hipStreamSynchronize(stream));
+    return pinHost() + kPinFinal;
+}
+
+void Pipeline::finishEmpty() {
+    launchStats(0);
+    waitStats();
 }
 
 void Pipeline::finishBatch() {
     kStamp<<<1, 1, 0, stream>>>(stamp(ST_END));
-    MDMC_HIP(hipMemcpyAsync(pinHost() + kPinFinal, counters(), A_NCOUNTERS * sizeof(int64_t), hipMemcpyDeviceToHost, stream));
-    MDMC_HIP(hipStreamSynchronize(stream));
+    const int64_t* h = readCounters();
+    if (h[A_INVALID]) checkNM(h);
 }
 
 void Pipeline::copyOut(float* positions, float* normals, int32_t* halfedges, int32_t* face_halfedge, uint16_t* face_attr, uint8_t* vertex_flags,
