@@ -114,6 +114,7 @@ __global__ void __launch_bounds__(kBlock) kPrepareGrids(PrepareDesc one, const P
         if (setup.probs && threadIdx.x == 0) *setup.probs = setup.prob;
         __syncthreads();
         stampClock(setup.stamp);  // one of the counters cleared above
+        if (setup.pin && threadIdx.x == 0) setup.ctr[setup.pinAt] = (int64_t)(intptr_t)setup.pin;
     }
     if (MODE == 0) {
         const int64_t row = (int64_t)blockIdx.x * kPlainRowsPerBlock + (threadIdx.x >> 6);

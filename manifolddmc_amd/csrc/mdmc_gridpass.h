@@ -54,6 +54,9 @@ struct PrepareSetup {
     ProblemDev prob;
     int64_t *special, *gate, token;
     int64_t* stamp;
+    // ctr[pinAt] = the address of the pinned word that failed checks raise (see the counters)
+    int64_t* pin;
+    int pinAt;
 };
 // descDev: the G grids' descriptors, or null with one (G = 1) by value
 void launchPrepareGrids(const PrepareDesc& one, const PrepareDesc* descDev, int G, int64_t rows, int refinement, int pad, const PrepareSetup& setup,

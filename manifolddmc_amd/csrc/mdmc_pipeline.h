@@ -57,14 +57,11 @@ class Pipeline {
     // id / 4): tracked once a split step writes records back; before that every one has
     bool canonTracked = false;
     const uint8_t* canonFlags();
-    // the halfedge records (he) are written from the quads and the twins after the
-    // simplifications, which read only those
-    bool heMaterialized = false;
-    void materializeHalfedges();
     // while the simplifications run, vertex v's position and normal stay at slot vslot[v] of
-    // pos / nrm (not moved by each compaction); materializeHalfedges gathers them back
+    // pos / nrm (not moved by each compaction); gatherVertices puts them back
     bool posSlotted = false;
     const int32_t* vertexSlots();
+    void gatherVertices();
 
     // one extraction's padding / refinement: its grids' descriptors (host copy, and the device
     // copy of more than one), and the launch that also clears the counters and stores a
@@ -246,7 +243,6 @@ class Pipeline {
     std::vector<int64_t> fgLastEager_;
     std::vector<int64_t> frontBuffers();
     void buildBuckets(const int32_t* list, int64_t n);
-    int32_t* bucketPassValence(const int64_t* off, int64_t nV);
     void refreshHashTable(const uint8_t* dirtyV, int64_t oldH);
     // a refresh ran whose face-walk check (the invalid-record counter) is not read back yet
     bool refreshUnchecked = false;

@@ -38,7 +38,7 @@ constexpr int kFanGuard = 4096;
 
 // ---------------------------------------------------------------- counters
 enum : int { A_ANOMALY = 0, A_CONFLICT = 1, A_INVALID = 2, A_DIRTY = 3, A_FALLBACK = 5, A_MERGE_SEQ = 6, A_LB_DIRECT = 7,
-             A_NM = 8, A_NSLOW = 9, A_NSLOW_OFF = 10, A_STAMP = 11, A_STATS = A_STAMP + ST_COUNT, A_TICKET = A_STATS + 9, A_NCOUNTERS };
+             A_NM = 8, A_NSLOW = 9, A_NSLOW_OFF = 10, A_PIN = 11, A_STAMP = 12, A_STATS = A_STAMP + ST_COUNT, A_TICKET = A_STATS + 9, A_NCOUNTERS };
 // the slotted non-manifold halfedges the split's working copy marks (markHalfedgesAsNonManifold,
 // ManifoldSplitter.cu:527-555, reads the four slots of every full vertex-pair bucket): every
 // halfedge of a bucket of 4, and of a larger bucket the ones at ranks 1, 2, 3 and size - 1
@@ -60,6 +60,13 @@ __device__ __forceinline__ void blockAdd(int64_t* parts, int c) {
         if (t) atomicAdd((unsigned long long*)&parts[(blockIdx.x % kPartSlots) * kPartStride], (unsigned long long)t);
     }
 }
+// the same from one wave, where few waves have anything to add (no barrier: the block's other
+// waves may be done); called by the lanes that are still running
+__device__ __forceinline__ void waveAdd(int64_t* parts, bool c) {
+    const uint64_t m = __ballot(c);
+    if (m && (int)(threadIdx.x & 63) == __ffsll((unsigned long long)m) - 1)
+        atomicAdd((unsigned long long*)&parts[(blockIdx.x % kPartSlots) * kPartStride], (unsigned long long)__popcll(m));
+}
 __device__ __forceinline__ int64_t sumParts(const int64_t* parts, int lane) {
     int64_t v = parts[lane * kPartStride];
 #pragma unroll
@@ -74,6 +81,13 @@ __device__ __forceinline__ int64_t sumParts(const int64_t* parts, int lane) {
 enum : int { kAwaitSplit = 1, kAwaitFans = 2 };
 __device__ __forceinline__ bool notYet(const int64_t* ctr, int guarded) {
     return ((guarded & kAwaitSplit) && (ctr[A_NM] != 0 || ctr[A_INVALID] != 0)) || ((guarded & kAwaitFans) && ctr[A_NSLOW] != 0);
+}
+
+// a failed check: counted, and reported through the pinned word whose address the counters hold,
+// so that a host that waits anyway sees it without a copy
+__device__ __forceinline__ void invalid(int64_t* ctr, int n = 1) {
+    atomicAdd((unsigned long long*)&ctr[A_INVALID], (unsigned long long)n);
+    *(volatile int64_t*)(intptr_t)ctr[A_PIN] = 1;
 }
 
 __device__ __forceinline__ void anomaly(int64_t* ctr) { atomicAdd((unsigned long long*)&ctr[A_ANOMALY], 1ULL); }
@@ -160,7 +174,7 @@ __global__ void kFaceClear(const int32_t* __restrict__ face_he, int64_t F, int64
             fattr[f] &= keep;
         }
     }
-    if (bad) atomicAdd((unsigned long long*)&ctr[A_INVALID], (unsigned long long)bad);
+    if (bad) invalid(ctr, bad);
 }
 
 // ---- buckets: the halfedges joining one vertex pair.  They are listed under the
@@ -230,7 +244,7 @@ __global__ void __launch_bounds__(kBlock) kDirtyRecords(const int4* __restrict__
     __syncthreads();
     const int64_t base = s_base;
     for (int i = threadIdx.x; i < n; i += kBlock) dlist[base + i] = s_list[i];
-    if (nbad) atomicAdd((unsigned long long*)&ctr[A_INVALID], (unsigned long long)nbad);
+    if (nbad) invalid(ctr, nbad);
 }
 
 // one thread per listed halfedge h (its ids checked by kDirtyRecords): its list vertex
@@ -260,7 +274,7 @@ __global__ void kDirtyKeys(const int4* __restrict__ he, int64_t H, const int32_t
         k = heN(he, k);
         ++pos;
     }
-    if (k != h) atomicAdd((unsigned long long*)&ctr[A_INVALID], 1ULL);
+    if (k != h) invalid(ctr);
     const int m = min(e.x, b);
     lm[t] = m;
     lent[t] = make_int2(pairEntry(e.x, b), k == h ? 4 * e.y + pos : 0x7FFFFFFF);
@@ -512,7 +526,7 @@ __device__ int gatherBucketOut(int h, const int4* __restrict__ quads, int64_t H,
 // attributes), an incoming boundary halfedge's share of the destination's valence.  Until the
 // simplifications are done a halfedge is its id (origin = corner i of quad f, face f, next
 // 4f + (i + 1) % 4) and its twin; the full records are written once after them
-// (kMaterialize).
+// (kRemapRebuild, or kBuildHalfedges where none runs).
 __device__ __forceinline__ void storeHalfedge(int h, int a, int b, const BucketOf& bk, int32_t* __restrict__ twin, uint32_t* __restrict__ bpack,
                                               uint32_t* __restrict__ vflags, uint32_t* __restrict__ fattr,
                                               uint32_t* __restrict__ qattr, int32_t* __restrict__ valence) {
@@ -528,27 +542,18 @@ __device__ __forceinline__ void storeHalfedge(int h, int a, int b, const BucketO
     }
 }
 
-// valence = outgoing halfedges (the list length); incoming boundary halfedges are added by
-// the bucket pass
-__global__ void kValenceFromOff(const int64_t* __restrict__ off, int64_t V, int32_t* __restrict__ valence) {
-    const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= V) return;
-    valence[v] = (int32_t)(off[v + 1] - off[v]);
-}
-
-__global__ void kFaceInit(const uint32_t* __restrict__ qattr, int64_t Q, int32_t* __restrict__ face_he, uint32_t* __restrict__ fattr) {
-    const int64_t q0 = firstOfFour();
-    if (q0 >= Q) return;
-    if (vec4(q0, Q, qattr, face_he) && vec4(q0, Q, fattr, fattr)) {
-        const int b = (int)(4 * q0);
-        reinterpret_cast<int4*>(face_he)[q0 >> 2] = make_int4(b, b + 4, b + 8, b + 12);
-        reinterpret_cast<uint4*>(fattr)[q0 >> 2] = reinterpret_cast<const uint4*>(qattr)[q0 >> 2];
-    } else {
-        for (int64_t q = q0; q < q0 + 4 && q < Q; ++q) {
-            face_he[q] = (int32_t)(4 * q);
-            fattr[q] = qattr[q];
-        }
-    }
+// the same as a finished record with its bucket size and rank (nothing reads ids and twins
+// only any more); returns whether the split's working copy would mark it (slottedNM)
+__device__ __forceinline__ bool storeRecord(int h, int a, const BucketOf& bk, int4* __restrict__ he, int32_t* __restrict__ bsize,
+                                           int32_t* __restrict__ brank, uint32_t* __restrict__ vflags, uint32_t* __restrict__ fattr) {
+    const int n = min(bk.n, 0xFFFF), r = min(bk.rank, 0xFFFF);
+    he[h] = make_int4(a, h >> 2, quadNext(h, 1), bk.twin);
+    bsize[h] = n;
+    brank[h] = r;
+    const uint32_t vf = bucketVertexFlag(n);
+    if (vf) atomicOr(&vflags[a], vf);
+    if (n == 4) atomicOr(&fattr[h >> 2], (uint32_t)QA_NM);
+    return slottedNM(n, r);
 }
 
 // every halfedge from its bucket
@@ -565,7 +570,7 @@ __global__ void kBucketsAll(const int4* __restrict__ quads, int64_t H, const int
 
 // The same with the records, sizes and ranks written at once, when no simplification (which
 // reads ids and twins only) follows: one launch and 24 bytes per halfedge less to move than
-// kBucketsAll and kMaterialize.  Bound by the list gathers, as kBucketsAll is.  The quads are
+// kBucketsAll and a pass that turns its words into records.  Bound by the list gathers, as kBucketsAll is.  The quads are
 // checked (kQuadLists) but the host has not looked yet: if any was inconsistent, every record is
 // a boundary halfedge of vertex 0, which the kernels launched before the host's next wait can
 // follow.
@@ -575,44 +580,19 @@ __global__ void __launch_bounds__(kBlock) kBuildHalfedges(const int4* __restrict
                                                           uint32_t* __restrict__ fattr, int64_t* nmParts, int64_t* ctr) {
     const int64_t hh = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const bool bad = ctr[A_INVALID] != 0;
-    int slotted = 0;
+    bool slotted = false;
     if (hh < H) {
-        const int h = (int)hh, f = h >> 2;
+        const int h = (int)hh;
         int a = 0;
         BucketOf bk{2, 1, -1};
         if (!bad) {
-            const int4 q = quads[f];
+            const int4 q = quads[h >> 2];
             a = quadCorner(q, h & 3);
             bk = bucketFromOutEnds(h, a, quadCorner(q, (h + 1) & 3), H, off, out, ends, ctr);
         }
-        he[h] = make_int4(a, f, quadNext(h, 1), bk.twin);
-        bsize[h] = min(bk.n, 0xFFFF);
-        brank[h] = min(bk.rank, 0xFFFF);
-        slotted = slottedNM(min(bk.n, 0xFFFF), min(bk.rank, 0xFFFF)) ? 1 : 0;
-        const uint32_t vf = bad ? 0u : bucketVertexFlag(bk.n);
-        if (vf) atomicOr(&vflags[a], vf);
-        if (bk.n == 4) atomicOr(&fattr[f], (uint32_t)QA_NM);
+        slotted = storeRecord(h, a, bk, he, bsize, brank, vflags, fattr);
     }
-    blockAdd(nmParts, slotted);
-}
-
-// the halfedge records of the quads, from the ids and the twins, and the bucket sizes / ranks
-__global__ void __launch_bounds__(kBlock) kMaterialize(const int4* __restrict__ quads, int64_t H, const int32_t* __restrict__ twin,
-                                                       const uint32_t* __restrict__ bpack, int4* __restrict__ he, int32_t* __restrict__ bsize,
-                                                       int32_t* __restrict__ brank, int64_t* nmParts, int64_t* stamp) {
-    stampClock(stamp);
-    const int64_t hh = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int slotted = 0;
-    if (hh < H) {
-        const int h = (int)hh;
-        he[h] = make_int4(quadCorner(quads[h >> 2], h & 3), h >> 2, quadNext(h, 1), twin[h]);
-        const uint32_t b = bpack[h];
-        const int n = (int)(b & 0xFFFFu), r = (int)(b >> 16);
-        bsize[h] = n;
-        brank[h] = r;
-        slotted = slottedNM(n, r) ? 1 : 0;
-    }
-    blockAdd(nmParts, slotted);
+    waveAdd(nmParts, slotted);
 }
 
 // ---- rebuild after a simplification's compaction.  New vertex v' = address[v]; a dropped
@@ -748,18 +728,22 @@ __global__ void kOutFill(const int32_t* __restrict__ oldV, int64_t Vn, const int
 
 // a halfedge with two untouched endpoints takes size, rank and renumbered twin from its old
 // halfedge; the block's other halfedges are gathered in LDS and recomputed from their
-// buckets by the block's first lanes, so that the long path runs on full waves
+// buckets by the block's first lanes, so that the long path runs on full waves.  The chain ends
+// here, so the finished records are written: 902 us at the 512^3 gyroid, against 783 us for
+// twins and bucket words and 315 us for a pass that turned them into records.  No barrier
+// follows the second part: waves without recomputed halfedges end early and make room (a
+// block-wide sum or an ordered store behind it: 1215-1264 us).
 __global__ void __launch_bounds__(kBlock) kRemapRebuild(const int4* __restrict__ quads2, int64_t H2, const uint8_t* __restrict__ touched,
                                                         const int32_t* __restrict__ oldQ, const int32_t* __restrict__ twinOld, int64_t Hold,
                                                         const uint32_t* __restrict__ bpackOld,
                                                         const int32_t* __restrict__ qnew, const int64_t* __restrict__ off2,
-                                                        const int32_t* __restrict__ out2, int32_t* __restrict__ twin, uint32_t* __restrict__ bpack,
-                                                        uint32_t* __restrict__ vflags, uint32_t* __restrict__ fattr,
-                                                        uint32_t* __restrict__ qattr, int32_t* __restrict__ valence, int64_t* ctr) {
+                                                        const int32_t* __restrict__ out2, int4* __restrict__ he, int32_t* __restrict__ bsize,
+                                                        int32_t* __restrict__ brank, uint32_t* __restrict__ vflags, uint32_t* __restrict__ fattr,
+                                                        int64_t* nmParts, int64_t* ctr) {
     __shared__ int s_list[kBlock];
     __shared__ int s_wave[kBlock / 64];
     const int64_t hh = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    bool later = false;
+    bool later = false, slotted = false;
     if (hh < H2) {
         const int h = (int)hh;
         // the old halfedge's twin and packed bucket are loaded alongside the touched flags
@@ -780,12 +764,13 @@ __global__ void __launch_bounds__(kBlock) kRemapRebuild(const int4* __restrict__
                 if (fo < 0) anomaly(ctr);
                 else t = 4 * fo + (tt & 3);
             }
-            storeHalfedge(h, a, b, BucketOf{(int)(bo & 0xFFFFu), (int)(bo >> 16), t}, twin, bpack, vflags, fattr, qattr, valence);
+            slotted = storeRecord(h, a, BucketOf{(int)(bo & 0xFFFFu), (int)(bo >> 16), t}, he, bsize, brank, vflags, fattr);
         }
     }
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const uint64_t m = __ballot(later);
     if (lane == 0) s_wave[wid] = __popcll(m);
+    waveAdd(nmParts, slotted);
     __syncthreads();
     int base = 0, total = 0;
     for (int w = 0; w < kBlock / 64; ++w) {
@@ -798,7 +783,7 @@ __global__ void __launch_bounds__(kBlock) kRemapRebuild(const int4* __restrict__
         const int h = s_list[threadIdx.x];
         const int4 q = quads2[h >> 2];
         const int a = quadCorner(q, h & 3), b = quadCorner(q, (h + 1) & 3);
-        storeHalfedge(h, a, b, bucketFromOut(h, a, b, quads2, H2, off2, out2, ctr), twin, bpack, vflags, fattr, qattr, valence);
+        waveAdd(nmParts, storeRecord(h, a, bucketFromOut(h, a, b, quads2, H2, off2, out2, ctr), he, bsize, brank, vflags, fattr));
     }
 }
 
@@ -957,7 +942,7 @@ __device__ __forceinline__ void dropVertex(int u, const int32_t* __restrict__ vt
                                            int32_t* __restrict__ outdeg, const int2* __restrict__ zslot, int64_t* ctr) {
     const int t = vtarget[u];
     if (t < 0 || t >= V || vtype[t] == dropType) {
-        atomicAdd((unsigned long long*)&ctr[A_INVALID], 1ULL);
+        invalid(ctr);
         return;
     }
     int* qc = reinterpret_cast<int*>(quads);
@@ -1552,24 +1537,50 @@ __global__ void kMark3333(const int4* __restrict__ quads, const int32_t* __restr
     }
 }
 
-// The chain's vertex compaction in one pass: a vertex is kept unless it is dropped by this
-// step (vtype == dropType) or died in an earlier step of the chain; kept vertices are numbered
-// in order (tile counts, block ranks, look-back), every vertex gets its new address (-1 when
-// dropped) and the kept ones their old id, slot and problem.  Positions and normals are not
-// moved: the new vertex keeps the slot of its old vertex.
+// The chain's compaction numbers vertices and quads in one launch: blocks [0, tV) take tiles of
+// vertices, the following tQ tiles of quads; kept elements are numbered in order (tile counts,
+// block ranks, look-back over the own kind's tiles).
+// A vertex is kept unless it is dropped by this step (vtype == dropType) or died in an earlier
+// step of the chain; every vertex gets its new address (-1 when dropped) and the kept ones
+// their old id, slot and problem.  Positions and normals are not moved: the new vertex
+// keeps the slot of its old vertex.  A quad is kept without remove or dead bit (qnew, -1
+// otherwise).  The arrays the following kernels start from (touched, flags, the list lengths' end;
+// the chain heads and removal counts of a chain of one) are cleared along the way.
+struct NumberArgs {
+    const int32_t* vtype;
+    int64_t V;
+    int dropType;
+    const uint8_t* vdead;
+    const int32_t *pid, *vslot;
+    int32_t *npid, *address, *oldV, *nvslot;
+    uint8_t* touched;
+    uint32_t* vflags;
+    int32_t *cnt, *srcHead, *removedAt;
+    int64_t tV;
+    unsigned long long* wordsV;
+    uint32_t epochV;
+    const uint32_t* attr;
+    int64_t Q;
+    int32_t* qnew;
+    int64_t tQ;
+    unsigned long long* wordsQ;
+    uint32_t epochQ;
+    int64_t *totalV, *totalQ, *directOut;
+};
 template <int R>
-__global__ void __launch_bounds__(kLbBlock) kCompactVertices(const int32_t* __restrict__ vtype, int64_t V, int dropType, const uint8_t* __restrict__ vdead,
-                                                             const int32_t* __restrict__ pid, const int32_t* __restrict__ vslot, int32_t* __restrict__ npid,
-                                                             int32_t* __restrict__ address, int32_t* __restrict__ oldV, int32_t* __restrict__ nvslot,
-                                                             int64_t numTiles, unsigned long long* __restrict__ status, uint32_t epoch, int64_t* __restrict__ total,
-                                                             int64_t* __restrict__ directOut) {
+__global__ void __launch_bounds__(kLbBlock) kNumber(NumberArgs a) {
     __shared__ int s_cnt[R * (kLbBlock / 64)], s_pre[R * (kLbBlock / 64) + 1];
     __shared__ long long s_off;
-    const int64_t t = blockIdx.x;
-    if (t >= numTiles) return;
+    const bool quad = (int64_t)blockIdx.x >= a.tV;
+    const int64_t t = quad ? (int64_t)blockIdx.x - a.tV : (int64_t)blockIdx.x, n = quad ? a.Q : a.V;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const int64_t base = t * (int64_t)(R * kLbBlock);
-    auto keepOf = [&](int64_t e) { return e < V && vtype[e] != dropType && !(vdead && vdead[e]); };
+    constexpr uint32_t gone = QA_REMOVE | QA_DEAD;
+    auto keepOf = [&](int64_t e) {
+        if (e >= n) return false;
+        if (quad) return !(a.attr[e] & gone);
+        return a.vtype[e] != a.dropType && !(a.vdead && a.vdead[e]);
+    };
     uint64_t m[R];
     uint32_t kb = 0;
 #pragma unroll
@@ -1581,31 +1592,40 @@ __global__ void __launch_bounds__(kLbBlock) kCompactVertices(const int32_t* __re
     const int tileSum = lbBlockRanks<R>(m, s_cnt, s_pre);
     if (threadIdx.x < 64)
         lbTileOffset(
-            status, epoch, t, tileSum,
+            quad ? a.wordsQ : a.wordsV, quad ? a.epochQ : a.epochV, t, tileSum,
             [&](int l) {
                 int64_t c = 0;
                 for (int64_t e = l; e < base; e += 64) c += keepOf(e) ? 1 : 0;
                 return c;
             },
-            directOut, &s_off);
+            a.directOut, &s_off);
     __syncthreads();
     const int64_t off = s_off;
     const uint64_t below = (1ULL << lane) - 1ULL;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        const int64_t v = base + r * kLbBlock + threadIdx.x;
-        if (v >= V) continue;
-        if (!((kb >> r) & 1u)) {
-            address[v] = -1;
+        const int64_t e = base + r * kLbBlock + threadIdx.x;
+        if (e >= n) continue;
+        const bool keep = (kb >> r) & 1u;
+        const int64_t o = off + s_pre[r * (kLbBlock / 64) + wid] + __popcll(m[r] & below);
+        if (quad) {
+            a.qnew[e] = keep ? (int32_t)o : -1;
             continue;
         }
-        const int64_t o = off + s_pre[r * (kLbBlock / 64) + wid] + __popcll(m[r] & below);
-        address[v] = (int32_t)o;
-        oldV[o] = (int32_t)v;
-        nvslot[o] = vslot ? vslot[v] : (int32_t)v;
-        if (pid) npid[o] = pid[v];
+        a.address[e] = keep ? (int32_t)o : -1;
+        if (a.srcHead) a.srcHead[e] = -1;
+        if (a.removedAt) a.removedAt[e] = 0;
+        if (!keep) continue;
+        a.oldV[o] = (int32_t)e;
+        a.nvslot[o] = a.vslot ? a.vslot[e] : (int32_t)e;
+        a.touched[o] = 0;
+        a.vflags[o] = 0;
+        if (a.pid) a.npid[o] = a.pid[e];
     }
-    if (t == numTiles - 1 && threadIdx.x == 0) *total = off + tileSum;
+    if (t == (quad ? a.tQ : a.tV) - 1 && threadIdx.x == 0) {
+        *(quad ? a.totalQ : a.totalV) = off + tileSum;
+        if (!quad) a.cnt[off + tileSum] = 0;
+    }
 }
 
 // positions and normals of the current vertices, gathered from their slots
@@ -1625,8 +1645,8 @@ __global__ void kGatherVertices(const float* __restrict__ pos, const float* __re
 // quad q, kept (new id d) or removed (a quad is removed when it has the remove or the dead bit)
 __device__ __forceinline__ void compactQuad(int64_t q, bool kept, int64_t d, const int4* __restrict__ quads, const uint32_t* __restrict__ attr,
                                             const int32_t* __restrict__ vtarget, const int32_t* __restrict__ address, int p3333,
-                                            int4* __restrict__ nquads, uint32_t* __restrict__ nattr, int32_t* __restrict__ oldQ,
-                                            int32_t* __restrict__ removedAt, int32_t* __restrict__ outdeg, int64_t V, int64_t* ctr) {
+                                            int4* __restrict__ nquads, uint32_t* __restrict__ nattr, uint32_t* __restrict__ nfattr,
+                                            int32_t* __restrict__ face_he, int32_t* __restrict__ oldQ, int32_t* __restrict__ removedAt, int32_t* __restrict__ outdeg, int64_t V, int64_t* ctr) {
     if (!kept) {
         // the outgoing halfedges this quad takes from its corners' lists (when the lists are
         // by current corner; a quad dead since an earlier step of the chain takes none)
@@ -1667,67 +1687,26 @@ __device__ __forceinline__ void compactQuad(int64_t q, bool kept, int64_t d, con
         }
         bad = bad || o[i] < 0;  // a dropped vertex or a missing target: the quad is invalid
     }
-    if (bad) atomicAdd((unsigned long long*)&ctr[A_INVALID], 1ULL);
+    if (bad) invalid(ctr);
     nquads[d] = make_int4(o[0], o[1], o[2], o[3]);
     uint32_t na = QA_COLOR;
     if (a & QA_NM) na |= QA_NM;
     if (a & QA_BOUNDARY) na |= QA_BOUNDARY;
     nattr[d] = na;
+    nfattr[d] = na;
+    face_he[d] = (int32_t)(4 * d);
     oldQ[d] = (int32_t)q;
-}
-
-// the quad compaction's numbering in one pass: kept quads (no remove or dead bit) numbered in
-// order (tile counts, block ranks, look-back) into qnew, -1 for removed ones
-template <int R>
-__global__ void __launch_bounds__(kLbBlock) kNumberQuads(const uint32_t* __restrict__ attr, int64_t Q, int32_t* __restrict__ qnew, int64_t numTiles,
-                                                         unsigned long long* __restrict__ status, uint32_t epoch, int64_t* __restrict__ total,
-                                                         int64_t* __restrict__ directOut) {
-    __shared__ int s_cnt[R * (kLbBlock / 64)], s_pre[R * (kLbBlock / 64) + 1];
-    __shared__ long long s_off;
-    const int64_t t = blockIdx.x;
-    if (t >= numTiles) return;
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const int64_t base = t * (int64_t)(R * kLbBlock);
-    constexpr uint32_t gone = QA_REMOVE | QA_DEAD;
-    auto keepOf = [&](int64_t e) { return e < Q && !(attr[e] & gone); };
-    uint64_t m[R];
-    uint32_t kb = 0;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const bool k = keepOf(base + r * kLbBlock + threadIdx.x);
-        m[r] = __ballot(k);
-        kb |= (k ? 1u : 0u) << r;
-    }
-    const int tileSum = lbBlockRanks<R>(m, s_cnt, s_pre);
-    if (threadIdx.x < 64)
-        lbTileOffset(
-            status, epoch, t, tileSum,
-            [&](int l) {
-                int64_t c = 0;
-                for (int64_t e = l; e < base; e += 64) c += keepOf(e) ? 1 : 0;
-                return c;
-            },
-            directOut, &s_off);
-    __syncthreads();
-    const int64_t off = s_off;
-    const uint64_t below = (1ULL << lane) - 1ULL;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const int64_t q = base + r * kLbBlock + threadIdx.x;
-        if (q < Q) qnew[q] = ((kb >> r) & 1u) ? (int32_t)(off + s_pre[r * (kLbBlock / 64) + wid] + __popcll(m[r] & below)) : -1;
-    }
-    if (t == numTiles - 1 && threadIdx.x == 0) *total = off + tileSum;
 }
 
 // removeQuadrilateralsP3X3Y / removeQuadsP3333 from the numbering, one thread per quad
 __global__ void kCompactQuads(const int4* __restrict__ quads, const uint32_t* __restrict__ attr, int64_t Q, const int32_t* __restrict__ vtarget,
                               const int32_t* __restrict__ address, int p3333, int4* __restrict__ nquads, uint32_t* __restrict__ nattr,
-                              int32_t* __restrict__ oldQ, const int32_t* __restrict__ qnew, int32_t* __restrict__ removedAt,
+                              uint32_t* __restrict__ nfattr, int32_t* __restrict__ face_he, int32_t* __restrict__ oldQ, const int32_t* __restrict__ qnew, int32_t* __restrict__ removedAt,
                               int32_t* __restrict__ outdeg, int64_t V, int64_t* ctr) {
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= Q) return;
     const int32_t d = qnew[q];
-    compactQuad(q, d >= 0, d, quads, attr, vtarget, address, p3333, nquads, nattr, oldQ, removedAt, outdeg, V, ctr);
+    compactQuad(q, d >= 0, d, quads, attr, vtarget, address, p3333, nquads, nattr, nfattr, face_he, oldQ, removedAt, outdeg, V, ctr);
 }
 
 // ---------------------------------------------------------------- fixManifoldTwins
@@ -1865,7 +1844,8 @@ constexpr int kFixPer = 16;
 __global__ void __launch_bounds__(kBlock) kFixTwins(int4* __restrict__ he, int64_t H, const int4* __restrict__ quads, const int64_t* __restrict__ off,
                                                     const int32_t* __restrict__ out, const int32_t* __restrict__ bsize, const int32_t* __restrict__ brank,
                                                     const float* __restrict__ pos, const ProblemDev* __restrict__ probs, const int32_t* __restrict__ pid,
-                                                    int64_t* ctr) {
+                                                    int64_t* ctr, int64_t* stamp) {
+    stampClock(stamp);
     __shared__ int s_list[kFixPer * kBlock];
     __shared__ int s_n;
     const int lane = threadIdx.x & 63;
@@ -2897,6 +2877,8 @@ void Pipeline::prepare(const std::vector<ProblemDev>& problems, bool captured) {
     su.gate = arena.get<int64_t>("prep_gate", 1);
     if (fresh) zero(su.gate, sizeof(int64_t));
     su.stamp = stamp(ST_PAD);
+    su.pin = pinDev() + kPinInvalid;
+    su.pinAt = A_PIN;
     su.special = pinDev() + kPinSpecial;
     su.token = captured ? 0 : ++prepToken_;
     pinHost()[kPinSpecial] = 0;
@@ -3283,17 +3265,6 @@ void Pipeline::buildBuckets(const int32_t* list, int64_t n) {
     if (H > 0) kFlagsFromBuckets<<<gridFor((H + 3) / 4), kBlock, 0, stream>>>(he, H, bsize, brank, vflags, fattr, nmSlotParts());
 }
 
-// the valence the next simplification starts from, when one follows: the outgoing list
-// lengths here, incoming boundary halfedges added by the bucket pass
-int32_t* Pipeline::bucketPassValence(const int64_t* off, int64_t nV) {
-    valenceReady = false;
-    if (simplifyQueue <= 0) return nullptr;
-    int32_t* valence = arena.get<int32_t>("valence", (size_t)std::max<int64_t>(nV, 1));
-    if (nV > 0) kValenceFromOff<<<gridFor(nV), kBlock, 0, stream>>>(off, nV, valence);
-    valenceReady = true;
-    return valence;
-}
-
 // HalfedgeMesh::initialize from the grid pass's output: outgoing lists (lengths and ranks from
 // the vertices' contours), then every halfedge from its bucket
 void Pipeline::halfedgeInitialize() {
@@ -3327,7 +3298,6 @@ void Pipeline::halfedgeInitialize() {
         if (H > 0)
             kBucketsAll<<<gridFor(H), kBlock, 0, stream>>>(quads, H, off, out, ends, twin, bpack, vflags, fattr, qattr, arena.ptr<int32_t>("valence"),
                                                            counters());
-        heMaterialized = false;
     } else {
         // no simplification reads ids and twins only: the records at once
         int4* he = arena.get<int4>("he", (size_t)std::max<int64_t>(H, 1));
@@ -3335,7 +3305,6 @@ void Pipeline::halfedgeInitialize() {
         int32_t* brank = arena.get<int32_t>("brank", (size_t)std::max<int64_t>(H, 1));
         if (H > 0)
             kBuildHalfedges<<<gridFor(H), kBlock, 0, stream>>>(quads, H, off, out, ends, he, bsize, brank, vflags, fattr, nmSlotParts(), counters());
-        heMaterialized = true;
     }
     posSlotted = false;  // the grid pass wrote positions by vertex
     deferredSteps = 0;
@@ -3444,7 +3413,6 @@ void Pipeline::simplifyDeferredStep(int dropType, bool p3333) {
     if (V > 0) kValenceFromBdin<<<gridFor(V), kBlock, 0, stream>>>(outdeg, bdin, V, valence);
     valenceReady = true;
     ++deferredSteps;
-    heMaterialized = false;
     splitTouched = false;
     canonTracked = false;
 }
@@ -3462,8 +3430,8 @@ void Pipeline::simplifyCompactAndRebuild(int dropType, bool p3333) {
     const uint32_t* attr = p3333 ? arena.ptr<uint32_t>("fattr") : arena.ptr<uint32_t>("qattr");
     // vertex and quad compaction, each one pass (look-back over tiles), with one read-back of
     // both totals; the outputs are sized for the inputs (at most as many are kept)
-    constexpr int RV = 16, RQ = 16;  // rounds per tile (tiles of 4096 elements)
-    const int64_t tV = (V + RV * kLbBlock - 1) / (RV * kLbBlock), tQ = (Q + RQ * kLbBlock - 1) / (RQ * kLbBlock);
+    constexpr int R = 16;  // rounds per tile (tiles of 4096 elements)
+    const int64_t tV = (V + R * kLbBlock - 1) / (R * kLbBlock), tQ = (Q + R * kLbBlock - 1) / (R * kLbBlock);
     int32_t* address = arena.get<int32_t>("vaddress", (size_t)std::max<int64_t>(V, 1));  // written for every vertex below
     // the compacted arrays go to the second buffers, which then swap with the primary ones;
     // both are sized for the grid pass's output so that later extractions of the same
@@ -3481,44 +3449,64 @@ void Pipeline::simplifyCompactAndRebuild(int dropType, bool p3333) {
     // corner; after deferred steps the lists are the initialize's and kOutCount checks entries
     int32_t* removedAt = chained ? nullptr : arena.get<int32_t>("removed_at", (size_t)std::max<int64_t>(V, 1));
     int32_t* outdeg = chained ? arena.ptr<int32_t>("outdeg") : nullptr;
-    {
-        FillBatch fb(*this);
-        if (removedAt) fb.add(removedAt, 0x00, (size_t)V * sizeof(int32_t));
-    }
+    // source chains by old vertex id (kept from the deferred steps of the chain)
+    int32_t* srcHead = arena.get<int32_t>("src_head", (size_t)std::max<int64_t>(V, 1));
+    int32_t* srcNext = arena.get<int32_t>("src_next", (size_t)std::max<int64_t>(V, 1));
+    uint8_t* touched = arena.get<uint8_t>("touched", (size_t)std::max<int64_t>(V, 1));
+    uint32_t* vflags = arena.ptr<uint32_t>("vflags");
+    int32_t* cnt = arena.get<int32_t>("out_cnt", (size_t)V + 1);
+    int32_t* face_he = arena.ptr<int32_t>("face_he");
+    uint32_t* nfattr = arena.get<uint32_t>("fattr2", capQ);
     // totals straight into pinned host memory: [1] V, [2] Q
     int64_t* h = pinHost();
     int64_t* pd = pinDev();
     h[1] = h[2] = 0;
-    const Lookback lbV = lookback(std::max<int64_t>(tV, 1));
-    if (V > 0)
-        kCompactVertices<RV><<<(unsigned)tV, kLbBlock, 0, stream>>>(vtype, V, dropType, chained ? arena.ptr<uint8_t>("vdead") : nullptr, pid(), vertexSlots(),
-                                                                npid, address, oldV, nvslot, tV, lbV.words, lbV.epoch, pd + 1, lookbackDiag());
-    if (Q > 0) {
-        const Lookback lbQ = lookback(tQ);
-        kNumberQuads<RQ><<<(unsigned)tQ, kLbBlock, 0, stream>>>(attr, Q, qnew, tQ, lbQ.words, lbQ.epoch, pd + 2, lookbackDiag());
-        kCompactQuads<<<gridFor(Q), kBlock, 0, stream>>>(quads, attr, Q, vtarget, address, p3333 ? 1 : 0, nquads, nattr, oldQ, qnew, removedAt, outdeg,
-                                                         V, counters());
+    {
+        NumberArgs na{};
+        na.vtype = vtype;
+        na.V = V;
+        na.dropType = dropType;
+        na.vdead = chained ? arena.ptr<uint8_t>("vdead") : nullptr;
+        na.pid = pid();
+        na.vslot = vertexSlots();
+        na.npid = npid;
+        na.address = address;
+        na.oldV = oldV;
+        na.nvslot = nvslot;
+        na.touched = touched;
+        na.vflags = vflags;
+        na.cnt = cnt;
+        na.srcHead = chained ? nullptr : srcHead;
+        na.removedAt = removedAt;
+        na.tV = tV;
+        na.attr = attr;
+        na.Q = Q;
+        na.qnew = qnew;
+        na.tQ = tQ;
+        const Lookback lb = lookback(std::max<int64_t>(tV + tQ, 1));
+        na.wordsV = lb.words;
+        na.wordsQ = lb.words + tV;
+        na.epochV = na.epochQ = lb.epoch;
+        na.totalV = pd + 1;
+        na.totalQ = pd + 2;
+        na.directOut = lookbackDiag();
+        if (tV + tQ > 0) kNumber<R><<<(unsigned)(tV + tQ), kLbBlock, 0, stream>>>(na);
     }
+    if (Q > 0)
+        kCompactQuads<<<gridFor(Q), kBlock, 0, stream>>>(quads, attr, Q, vtarget, address, p3333 ? 1 : 0, nquads, nattr, nfattr, face_he, oldQ, qnew,
+                                                         removedAt, outdeg, V, counters());
     MDMC_HIP(hipStreamSynchronize(stream));
     const int64_t nV = h[1], nQ = h[2];
     if (nV < 0 || nV > V || nQ < 0 || nQ > Q) throw HipError("inconsistent compaction counts", -4);
-    checkValid("quad vertex ids");
+    if (h[kPinInvalid]) checkValid("quad vertex ids");
 
     // HalfedgeMesh::initialize of the compacted quads, from the previous build: the new
     // outgoing lists are the old ones of each new vertex's own and relabelled vertices,
     // renumbered; halfedges with untouched endpoints keep their bucket results
     const int64_t nH = 4 * nQ;
-    uint8_t* touched = arena.get<uint8_t>("touched", (size_t)std::max<int64_t>(nV, 1));
-    // source chains by old vertex id (kept from the deferred steps of the chain)
-    int32_t* srcHead = arena.get<int32_t>("src_head", (size_t)std::max<int64_t>(V, 1));
-    int32_t* srcNext = arena.get<int32_t>("src_next", (size_t)std::max<int64_t>(V, 1));
-    zero(touched, (size_t)nV);
-    if (!chained) fillNeg(srcHead, (size_t)V * sizeof(int32_t));
     if (V > 0) kSources<<<sparseBlocks(V), kBlock, 0, stream>>>(vtype, vtarget, address, V, dropType, touched, srcHead, srcNext, outdeg);
     const int64_t* off = arena.ptr<int64_t>("out_off");
     const int32_t* out = arena.ptr<int32_t>("out_list");
-    int32_t* cnt = arena.get<int32_t>("out_cnt", (size_t)nV + 1);
-    zero(cnt + nV, sizeof(int32_t));
     if (nV > 0) kOutCount<<<gridFor(nV), kBlock, 0, stream>>>(oldV, nV, off, removedAt, srcHead, srcNext, outdeg, cnt);
     int64_t* off2 = arena.get<int64_t>("out_off2", (size_t)std::max<int64_t>(nV, dmcV) + 1);
     scan(cnt, off2, nV + 1);
@@ -3526,25 +3514,19 @@ void Pipeline::simplifyCompactAndRebuild(int dropType, bool p3333) {
     if (nV > 0)
         kOutFill<<<gridFor(nV), kBlock, 0, stream>>>(oldV, nV, off, out, qnew, srcHead, srcNext, off2, out2, nH, counters());
 
-    int32_t* twin2 = arena.get<int32_t>("twin2", 4 * capQ);
-    uint32_t* bpack2 = arena.get<uint32_t>("bpack2", 4 * capQ);
-    int32_t* face_he = arena.get<int32_t>("face_he", (size_t)std::max<int64_t>(nQ, 1));
-    uint32_t* fattr = arena.get<uint32_t>("fattr", (size_t)std::max<int64_t>(nQ, 1));
-    uint32_t* vflags = arena.get<uint32_t>("vflags", (size_t)std::max<int64_t>(nV, 1));
-    if (nQ > 0) kFaceInit<<<gridFor((nQ + 3) / 4), kBlock, 0, stream>>>(nattr, nQ, face_he, fattr);
-    zero(vflags, (size_t)nV * sizeof(uint32_t));
-    int32_t* valence = bucketPassValence(off2, nV);
+    int4* he = arena.get<int4>("he", (size_t)std::max<int64_t>(nH, 1));
+    int32_t* bsize = arena.get<int32_t>("bsize", (size_t)std::max<int64_t>(nH, 1));
+    int32_t* brank = arena.get<int32_t>("brank", (size_t)std::max<int64_t>(nH, 1));
+    // (the partial sums of slotted halfedges are clear since the extraction's start)
     if (nH > 0)
         kRemapRebuild<<<gridFor(nH), kBlock, 0, stream>>>(nquads, nH, touched, oldQ, arena.ptr<int32_t>("twin"), H, arena.ptr<uint32_t>("bpack"),
-                                                         qnew, off2, out2, twin2, bpack2, vflags, fattr, nattr,
-                                                         valence, counters());
+                                                         qnew, off2, out2, he, bsize, brank, vflags, nfattr, nmSlotParts(), counters());
     arena.swap("vslot", "vslot2");
     posSlotted = true;
     arena.swap("quads", "quads2");
     arena.swap("qattr", "qattr2");
+    arena.swap("fattr", "fattr2");
     if (npid) arena.swap("pid", "pid2");
-    arena.swap("twin", "twin2");
-    arena.swap("bpack", "bpack2");
     arena.swap("out_off", "out_off2");
     arena.swap("out_list", "out_list2");
     V = nV;
@@ -3553,7 +3535,7 @@ void Pipeline::simplifyCompactAndRebuild(int dropType, bool p3333) {
     F = nQ;
     vertHeV = V;
     vertHeQ = Q;
-    heMaterialized = false;
+    valenceReady = false;
     listsV = V;
     splitTouched = false;
     canonTracked = false;
@@ -3609,36 +3591,25 @@ void Pipeline::simplify3333() {
     simplifyCompactAndRebuild(1, true);
 }
 
-// the full halfedge records, once the simplifications (which read ids and twins only) are done
-void Pipeline::materializeHalfedges() {
-    const bool gathered = posSlotted && V > 0;
-    if (posSlotted) {
-        // positions and normals by vertex again, from the slots the simplifications kept them in
-        const size_t cap = (size_t)std::max(V, dmcV);
-        float* npos = arena.get<float>("pos2", 3 * cap);
-        float* nnrm = arena.get<float>("nrm2", 3 * cap);
-        if (V > 0) kGatherVertices<<<gridFor(V), kBlock, 0, stream>>>(arena.ptr<float>("pos"), arena.ptr<float>("nrm"), vertexSlots(), V, npos, nnrm, stamp(ST_TWINS));
-        arena.swap("pos", "pos2");
-        arena.swap("nrm", "nrm2");
-        posSlotted = false;
-    }
-    if (heMaterialized) return;
-    int4* he = arena.get<int4>("he", (size_t)std::max<int64_t>(H, 1));
-    int32_t* bsize = arena.get<int32_t>("bsize", (size_t)std::max<int64_t>(H, 1));
-    int32_t* brank = arena.get<int32_t>("brank", (size_t)std::max<int64_t>(H, 1));
-    // (the partial sums are clear since the extraction's start)
-    if (H > 0)
-        kMaterialize<<<gridFor(H), kBlock, 0, stream>>>(arena.ptr<int4>("quads"), H, arena.ptr<int32_t>("twin"), arena.ptr<uint32_t>("bpack"), he, bsize,
-                                                        brank, nmSlotParts(), gathered ? nullptr : stamp(ST_TWINS));
-    heMaterialized = true;
+// positions and normals by vertex again, from the slots the simplifications kept them in
+void Pipeline::gatherVertices() {
+    if (!posSlotted) return;
+    const size_t cap = (size_t)std::max(V, dmcV);
+    float* npos = arena.get<float>("pos2", 3 * cap);
+    float* nnrm = arena.get<float>("nrm2", 3 * cap);
+    if (V > 0) kGatherVertices<<<gridFor(V), kBlock, 0, stream>>>(arena.ptr<float>("pos"), arena.ptr<float>("nrm"), vertexSlots(), V, npos, nnrm, stamp(ST_TWINS));
+    arena.swap("pos", "pos2");
+    arena.swap("nrm", "nrm2");
+    posSlotted = false;
 }
 
 void Pipeline::fixManifoldTwins() {
-    materializeHalfedges();
+    int64_t* st = posSlotted ? nullptr : stamp(ST_TWINS);
+    gatherVertices();
     if (H == 0) return;
     kFixTwins<<<(unsigned)((H + kFixPer * kBlock - 1) / (kFixPer * kBlock)), kBlock, 0, stream>>>(arena.ptr<int4>("he"), H, arena.ptr<int4>("quads"), arena.ptr<int64_t>("out_off"), arena.ptr<int32_t>("out_list"),
                                                  arena.ptr<int32_t>("bsize"), arena.ptr<int32_t>("brank"), arena.ptr<float>("pos"), probsDev, pid(),
-                                                 counters());
+                                                 counters(), st);
 }
 
 // ---- ManifoldSplitter::run, one problem and all that follows: the last stages are launched
