@@ -229,7 +229,7 @@ mdmc_status runExtraction(mdmc_ctx* ctx, const mdmc_grid* grids, int G, const fl
         hipStream_t s = p.stream;
         p.splitIterations = 0;
         p.extraAnomalies = 0;
-        p.simplifyQueue = ((flags & MDMC_P3X3Y_COLOR) ? 1 : 0) + ((flags & MDMC_P3X3Y_OLD) ? 1 : 0) + ((flags & MDMC_P3333) ? 1 : 0);
+        p.setChain((flags & MDMC_P3X3Y_COLOR) != 0, (flags & MDMC_P3X3Y_OLD) != 0, (flags & MDMC_P3333) != 0);
         // ---- grids: upload if needed, then pad / refine (refineGrid)
         float* gp = p.arena.get<float>("grid", (size_t)Ptot);
         float* up = PinTot ? p.arena.get<float>("input", (size_t)PinTot) : nullptr;
@@ -307,9 +307,7 @@ mdmc_status runExtraction(mdmc_ctx* ctx, const mdmc_grid* grids, int G, const fl
         int64_t st9[9] = {0};
         if (p.V > 0) {
             p.halfedgeInitialize();
-            if (flags & MDMC_P3X3Y_COLOR) p.simplify3X3Y(true);
-            if (flags & MDMC_P3X3Y_OLD) p.simplify3X3Y(false);
-            if (flags & MDMC_P3333) p.simplify3333();
+            p.simplify();
             p.fixManifoldTwins();
             const int maxIters = opt->max_split_iters > 0 ? opt->max_split_iters : 64;
             if (B == 1) {

@@ -64,6 +64,15 @@ void launchPrepareGrids(const PrepareDesc& one, const PrepareDesc* descDev, int 
 // the exact blend of every grid, after a plain copy that raised *special (no refinement)
 void launchPrepareExact(const PrepareDesc& one, const PrepareDesc* descDev, int G, int64_t rows, int pad, hipStream_t s);
 
+// What a chain of simplifications starts from, per vertex: no type and target, the valence (the
+// out-degree until the bucket pass adds boundary halfedges); count (pattern counts of the old
+// P3X3Y rule) and, when more than one step follows, the deferred steps' arrays; null: not needed
+struct ChainInit {
+    int32_t *vtype, *vtarget, *valence, *count;
+    int32_t *head, *outdeg, *bdin;
+    uint8_t *vdead, *touched;
+};
+
 struct GridPassArgs {
     const ProblemDev* probs;
     int nProblems;
@@ -99,10 +108,11 @@ struct GridPassArgs {
     uint16_t* vct;
     int64_t V;
     // the halfedge initialize's per-vertex arrays, which the vertex kernel starts: the out-degree in
-    // the halfedge mesh (interior edges of its contour; [V + 1], last entry 0), the valence the
-    // same (when a simplification follows, else null), cleared flags
-    int32_t *outdeg, *valence;
+    // the halfedge mesh (interior edges of its contour; [V + 1], last entry 0), cleared flags
+    int32_t* outdeg;
     uint32_t* vflags;
+    // and those of a chain of simplifications, when one follows (else null)
+    ChainInit chain;
     // recorded for the adjoint when not null: per cell (first vertex << 2 | contours - 1) or -1
     // (single-problem extractions only)
     int32_t* adjMap;

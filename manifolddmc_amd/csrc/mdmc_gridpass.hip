@@ -999,7 +999,19 @@ __global__ void __launch_bounds__(GP_THREADS) kVertices(GridPassArgs a, int chun
         // out-degree of the vertex in the halfedge mesh: one quad per interior edge of its contour
         const int deg = __popc(interiorEdgeMask(x, y, z, P.CX, P.CY, g.nz - 1) & c_contourEdges[4 * (ct & 0x3FF) + (ct >> 10)]);
         a.outdeg[v] = deg;
-        if (a.valence) a.valence[v] = deg;
+        if (a.chain.vtype) {
+            a.chain.vtype[v] = 0;
+            a.chain.vtarget[v] = -1;
+            a.chain.valence[v] = deg;
+            if (a.chain.count) a.chain.count[v] = 0;
+            if (a.chain.head) {
+                a.chain.head[v] = -1;
+                a.chain.outdeg[v] = deg;
+                a.chain.bdin[v] = 0;
+                a.chain.vdead[v] = 0;
+                a.chain.touched[v] = 0;
+            }
+        }
         a.vflags[v] = 0;
         if (v == a.V - 1) a.outdeg[a.V] = 0;
         if (a.surfIter) {

@@ -43,12 +43,11 @@ class Pipeline {
     int64_t splitIterations = 0;
     int64_t extraAnomalies = 0;
 
-    // simplifications still to run: while positive, the halfedge initialize computes the
-    // vertex valence they start from
-    int simplifyQueue = 0;
-    bool valenceReady = false;
-    // simplifications run since the initialize without compaction (the last of a chain compacts)
-    int deferredSteps = 0;
+    // the simplifications of this extraction, in order (set before the grid pass, whose vertex
+    // kernel starts their arrays)
+    enum : int { S_COLOUR, S_OLD, S_3333 };
+    std::vector<int> chain;
+    void setChain(bool colour, bool old, bool p3333);
     // vertices the outgoing lists of the last halfedge build describe (-1: none), and
     // whether a split since then keeps the per-vertex "touched" flags
     int64_t listsV = -1;
@@ -57,12 +56,6 @@ class Pipeline {
     // id / 4): tracked once a split step writes records back; before that every one has
     bool canonTracked = false;
     const uint8_t* canonFlags();
-    // while the simplifications run, vertex v's position and normal stay at slot vslot[v] of
-    // pos / nrm (not moved by each compaction); gatherVertices puts them back
-    bool posSlotted = false;
-    const int32_t* vertexSlots();
-    void gatherVertices();
-
     // one extraction's padding / refinement: its grids' descriptors (host copy, and the device
     // copy of more than one), and the launch that also clears the counters and stores a
     // single problem (captured: for a graph)
@@ -134,8 +127,7 @@ class Pipeline {
     std::vector<int64_t> batchStats;                   // [9B], as computeStats
     bool batchVertHe = false;
     void halfedgeInitialize();
-    void simplify3X3Y(bool colour);
-    void simplify3333();
+    void simplify();
     void fixManifoldTwins();
     void split(int step, int maxIters);
     void detectNonManifoldVertices();
@@ -251,9 +243,10 @@ class Pipeline {
     void checkInit();
     bool initUnchecked = false;
     void emitArgs(GridPassArgs& a, int64_t C, bool recordAdjoint);
-    void simplifyInit(int32_t** valence, int32_t** count, bool needCount);
-    void simplifyCompactAndRebuild(int dropType, bool p3333);
-    void simplifyDeferredStep(int dropType, bool p3333);
+    void launchChain(int from, bool ended);
+    void launchCompaction();
+    void rebuildRegion();
+    void finishChain();
     void buildMergeList(const int2* rec, int64_t R, int count, int32_t* num, int32_t* ex, int32_t* ey, const std::string& tag);
     int32_t* stableSortByKey(const int32_t* key, int64_t n, int B, const std::string& tag);
     void countSorted(const int32_t* key, const int32_t* perm, int64_t n, int B, unsigned long long* count, int stride, int slot);

@@ -37,7 +37,7 @@ constexpr int kMaxBucket = 16;
 constexpr int kFanGuard = 4096;
 
 // ---------------------------------------------------------------- counters
-enum : int { A_ANOMALY = 0, A_CONFLICT = 1, A_INVALID = 2, A_DIRTY = 3, A_FALLBACK = 5, A_MERGE_SEQ = 6, A_LB_DIRECT = 7,
+enum : int { A_ANOMALY = 0, A_CONFLICT = 1, A_INVALID = 2, A_DIRTY = 3, A_FALLBACK = 4 /* two steps */, A_MERGE_SEQ = 6, A_LB_DIRECT = 7,
              A_NM = 8, A_NSLOW = 9, A_NSLOW_OFF = 10, A_PIN = 11, A_STAMP = 12, A_STATS = A_STAMP + ST_COUNT, A_TICKET = A_STATS + 9, A_NCOUNTERS };
 // the slotted non-manifold halfedges the split's working copy marks (markHalfedgesAsNonManifold,
 // ManifoldSplitter.cu:527-555, reads the four slots of every full vertex-pair bucket): every
@@ -88,6 +88,14 @@ __device__ __forceinline__ bool notYet(const int64_t* ctr, int guarded) {
 __device__ __forceinline__ void invalid(int64_t* ctr, int n = 1) {
     atomicAdd((unsigned long long*)&ctr[A_INVALID], (unsigned long long)n);
     *(volatile int64_t*)(intptr_t)ctr[A_PIN] = 1;
+}
+
+// A chain of simplifications is launched whole, without waiting for the checks before it or for
+// its steps' outcomes: its kernels return at once where the initialize's check failed or one of
+// the `before` steps before left merges that need the region rebuild (kLocalMerge); the host
+// sees both at the chain's end, runs the rebuild and launches the rest again.
+__device__ __forceinline__ bool chainHeld(const int64_t* ctr, int before) {
+    return ctr[A_INVALID] != 0 || (before > 0 && ctr[A_FALLBACK] != 0) || (before > 1 && ctr[A_FALLBACK + 1] != 0);
 }
 
 __device__ __forceinline__ void anomaly(int64_t* ctr) { atomicAdd((unsigned long long*)&ctr[A_ANOMALY], 1ULL); }
@@ -144,8 +152,8 @@ __device__ __forceinline__ bool vec4(int64_t i0, int64_t n, const void* a, const
 }
 
 // pinned words: the padding pass's "needs the exact blend", the initialize's "inconsistent
-// quads", the copy of the counters at the end
-constexpr int kPinSpecial = 3, kPinInvalid = 4, kPinFinal = 16;
+// quads", a deferred simplification's "region rebuild needed", the copy of the counters at the end
+constexpr int kPinSpecial = 3, kPinInvalid = 4, kPinFallback = 5 /* two steps */, kPinFinal = 16;
 static_assert(kPinFinal + A_NCOUNTERS <= Pipeline::kPinSlots, "pinned words");
 
 // ---------------------------------------------------------------- halfedge construction
@@ -529,11 +537,14 @@ __device__ int gatherBucketOut(int h, const int4* __restrict__ quads, int64_t H,
 // (kRemapRebuild, or kBuildHalfedges where none runs).
 __device__ __forceinline__ void storeHalfedge(int h, int a, int b, const BucketOf& bk, int32_t* __restrict__ twin, uint32_t* __restrict__ bpack,
                                               uint32_t* __restrict__ vflags, uint32_t* __restrict__ fattr,
-                                              uint32_t* __restrict__ qattr, int32_t* __restrict__ valence) {
+                                              uint32_t* __restrict__ qattr, int32_t* __restrict__ valence, int32_t* __restrict__ bdin) {
     const int f = h >> 2;
     twin[h] = bk.twin;
     bpack[h] = packBucket(bk.n, bk.rank);
-    if (valence && bk.twin == -1) atomicAdd(&valence[b], 1);
+    if (bk.twin == -1) {
+        atomicAdd(&valence[b], 1);
+        if (bdin) atomicAdd(&bdin[b], 1);
+    }
     const uint32_t vf = bucketVertexFlag(bk.n);
     if (vf) atomicOr(&vflags[a], vf);
     if (bk.n == 4) {
@@ -559,13 +570,14 @@ __device__ __forceinline__ bool storeRecord(int h, int a, const BucketOf& bk, in
 // every halfedge from its bucket
 __global__ void kBucketsAll(const int4* __restrict__ quads, int64_t H, const int64_t* __restrict__ off, const int32_t* __restrict__ out,
                             const int2* __restrict__ ends, int32_t* __restrict__ twin, uint32_t* __restrict__ bpack, uint32_t* __restrict__ vflags,
-                            uint32_t* __restrict__ fattr, uint32_t* __restrict__ qattr, int32_t* __restrict__ valence, int64_t* ctr) {
+                            uint32_t* __restrict__ fattr, uint32_t* __restrict__ qattr, int32_t* __restrict__ valence, int32_t* __restrict__ bdin,
+                            int64_t* ctr) {
     const int64_t hh = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (hh >= H) return;
+    if (hh >= H || chainHeld(ctr, 0)) return;
     const int h = (int)hh;
     const int4 q = quads[h >> 2];
     const int a = quadCorner(q, h & 3), b = quadCorner(q, (h + 1) & 3);
-    storeHalfedge(h, a, b, bucketFromOutEnds(h, a, b, H, off, out, ends, ctr), twin, bpack, vflags, fattr, qattr, valence);
+    storeHalfedge(h, a, b, bucketFromOutEnds(h, a, b, H, off, out, ends, ctr), twin, bpack, vflags, fattr, qattr, valence, bdin);
 }
 
 // The same with the records, sizes and ranks written at once, when no simplification (which
@@ -802,17 +814,6 @@ __device__ __forceinline__ bool pattern2(const int v[4]) { return v[0] >= 5 && v
 // the step-by-step compactions give (stable compactions compose, and bucket ranks and the
 // twin rules only compare ids, whose order every compaction keeps).
 
-// out-degree of every vertex from the initialize's lists, and its incoming boundary halfedges
-// (the rest of its valence)
-__global__ void kOutdegInit(const int64_t* __restrict__ off, int64_t V, const int32_t* __restrict__ valence, int32_t* __restrict__ outdeg,
-                            int32_t* __restrict__ bdin) {
-    const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= V) return;
-    const int32_t d = (int32_t)(off[v + 1] - off[v]);
-    outdeg[v] = d;
-    bdin[v] = valence[v] - d;
-}
-
 // P3X3Y merge (x, a1, z, a3) -> x whose neighbourhood is a plain patch: the four edges of the
 // removed quad Q are pairs, x and z each have a closed fan of three quads (Q, N_X, N_B and Q,
 // N_A, N_Z) with third neighbours d and c, and after every merge of the step is applied (a
@@ -823,7 +824,7 @@ __global__ void kOutdegInit(const int64_t* __restrict__ off, int64_t V, const in
 // neither meeting another), and no flag or boundary count moves, so the four twins and bucket
 // words are written here.  (Q's neighbours are not removed: two merges never share a quad,
 // and no other merge writes or reads the halfedges read or written here.)  Any other merge
-// marks its target touched for the region rebuild below and is counted in ctr[A_FALLBACK].  The block's
+// marks its target touched for the region rebuild below and is counted in ctr[A_FALLBACK + step].  The block's
 // merges are gathered in LDS first: each is a chain of dependent loads.
 // The same launch applies removeQuadrilateralsP3X3Y in place: every kept quad gets the
 // compaction's attributes (colour unset, NM and boundary kept: no REMOVE or DEAD bit before or
@@ -835,7 +836,8 @@ __global__ void __launch_bounds__(kBlock) kLocalMerge(int4* __restrict__ quads, 
                                                       const int32_t* __restrict__ valence, const int32_t* __restrict__ vtype,
                                                       const int32_t* __restrict__ vtarget, int32_t* __restrict__ twin, uint32_t* __restrict__ bpack,
                                                       int32_t* __restrict__ outdeg, int2* __restrict__ zslot, int64_t V, uint8_t* __restrict__ touched,
-                                                      int allowLocal, int64_t* ctr) {
+                                                      int allowLocal, int step, int64_t* ctr) {
+    if (chainHeld(ctr, step)) return;
     __shared__ int s_list[kSparsePer * kBlock];
     __shared__ int s_n;
     const int total = gatherSparse(
@@ -917,15 +919,24 @@ __global__ void __launch_bounds__(kBlock) kLocalMerge(int4* __restrict__ quads, 
         qattr[q] = QA_DEAD;
         fattr[q] = QA_DEAD;
     }
-    if (nfallback) atomicAdd((unsigned long long*)&ctr[A_FALLBACK], (unsigned long long)nfallback);
+    if (nfallback) {
+        atomicAdd((unsigned long long*)&ctr[A_FALLBACK + step], (unsigned long long)nfallback);
+        ((volatile int64_t*)(intptr_t)ctr[A_PIN])[kPinFallback - kPinInvalid + step] = 1;
+    }
 }
 
-// valence = out-degree + incoming boundary halfedges (a step with only local merges: no flag
-// or boundary count changed)
-__global__ void kValenceFromBdin(const int32_t* __restrict__ outdeg, const int32_t* __restrict__ bdin, int64_t V, int32_t* __restrict__ valence) {
+// the end of a deferred step: valence = out-degree + incoming boundary halfedges, and the next
+// step's start (types, targets, touched flags, the old rule's counts when that is next)
+__global__ void kStepEnd(const int32_t* __restrict__ outdeg, const int32_t* __restrict__ bdin, int64_t V, int32_t* __restrict__ valence,
+                         int32_t* __restrict__ vtype, int32_t* __restrict__ vtarget, uint8_t* __restrict__ touched, int32_t* __restrict__ count, int step,
+                         const int64_t* ctr) {
     const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= V) return;
+    if (v >= V || chainHeld(ctr, step + 1)) return;
     valence[v] = outdeg[v] + bdin[v];
+    vtype[v] = 0;
+    vtarget[v] = -1;
+    touched[v] = 0;
+    if (count) count[v] = 0;
 }
 
 // a dropped vertex u (P3X3Y: vtype == dropType) dies: the corners its live outgoing
@@ -973,7 +984,8 @@ __global__ void __launch_bounds__(kBlock) kDropVertices(const int32_t* __restric
                                                         int dropType, int4* __restrict__ quads, int64_t H, const int64_t* __restrict__ off,
                                                         const int32_t* __restrict__ out, uint8_t* __restrict__ vdead, int32_t* __restrict__ head,
                                                         int32_t* __restrict__ next, int32_t* __restrict__ outdeg, const int2* __restrict__ zslot,
-                                                        int64_t* ctr) {
+                                                        int step, int64_t* ctr) {
+    if (chainHeld(ctr, step)) return;
     __shared__ int s_list[kSparsePer * kBlock];
     __shared__ int s_n;
     const int total = gatherSparse(V, [&](int64_t i) { return vtype[i] == dropType; }, s_list, &s_n);
@@ -1351,18 +1363,11 @@ __global__ void kFanFast(const int4* __restrict__ he, int64_t H, int64_t V, cons
 }
 
 // ---------------------------------------------------------------- simplifications
-__global__ void kValence(const int4* __restrict__ quads, const int32_t* __restrict__ twin, int64_t H, int32_t* __restrict__ valence) {
-    const int64_t h = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= H) return;
-    const int4 q = quads[h >> 2];
-    atomicAdd(&valence[quadCorner(q, (int)(h & 3))], 1);
-    if (twin[h] == -1) atomicAdd(&valence[quadCorner(q, (int)((h + 1) & 3))], 1);
-}
-
-
-__global__ void kMark3x3y(const int4* __restrict__ quads, uint32_t* __restrict__ qattr, int64_t Q, const int32_t* __restrict__ valence) {
+__global__ void kMark3x3y(const int4* __restrict__ quads, uint32_t* __restrict__ qattr, int64_t Q, const int32_t* __restrict__ valence, int step,
+                          const int64_t* ctr, int64_t* stamp) {
+    stampClock(stamp);
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= Q) return;
+    if (q >= Q || chainHeld(ctr, step)) return;
     uint32_t a = qattr[q];
     if ((a & QA_NM) || (a & QA_BOUNDARY) || (a & QA_DEAD)) return;
     a &= 0x3F;
@@ -1373,9 +1378,10 @@ __global__ void kMark3x3y(const int4* __restrict__ quads, uint32_t* __restrict__
 }
 
 __global__ void kCount3x3yOld(const int4* __restrict__ quads, uint32_t* __restrict__ qattr, int64_t Q, const int32_t* __restrict__ valence,
-                              int32_t* __restrict__ count) {
+                              int32_t* __restrict__ count, int step, const int64_t* ctr, int64_t* stamp) {
+    stampClock(stamp);
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= Q) return;
+    if (q >= Q || chainHeld(ctr, step)) return;
     const uint32_t a0 = qattr[q];
     if (a0 & QA_DEAD) return;
     uint32_t a = a0 & 0x3F;
@@ -1393,13 +1399,12 @@ __global__ void kCount3x3yOld(const int4* __restrict__ quads, uint32_t* __restri
     qattr[q] = a;
 }
 
-// HalfedgeMesh.cu:368-388.  Positions and normals stay where the grid pass wrote them while
-// the simplifications run: vertex v's are at slot vslot[v] (v itself when vslot is null).
-// (markTarget: the target gets vtype kTargetType, for the deferred steps' local twin update)
+// HalfedgeMesh.cu:368-388 (markTarget: the target gets vtype kTargetType, for the deferred steps'
+// local twin update)
 constexpr int kTargetType = 4;
-__device__ __forceinline__ void handleMerge(float* pos, float* nrm, const int32_t* vslot, int32_t* vtype, int32_t* vtarget, int x, int y, int z, int w,
+__device__ __forceinline__ void handleMerge(float* pos, float* nrm, int32_t* vtype, int32_t* vtarget, int x, int y, int z, int w,
                                             int markTarget) {
-    const int64_t sx = vslot ? vslot[x] : x, sy = vslot ? vslot[y] : y, sw = vslot ? vslot[w] : w;
+    const int64_t sx = x, sy = y, sw = w;
     f3 p = mk3(pos[3 * sy], pos[3 * sy + 1], pos[3 * sy + 2]);
     const f3 pw = mk3(pos[3 * sw], pos[3 * sw + 1], pos[3 * sw + 2]);
     p = p + scl(0.5f, pw - p);
@@ -1435,8 +1440,9 @@ __device__ __forceinline__ bool neighborFaces(const int32_t* __restrict__ twin, 
 // mergeVerticesP3X3YColor (colour = 1) and mergeVerticesP3X3Y (colour = 0), HalfedgeMesh.cu:391-498
 __global__ void __launch_bounds__(kBlock) kMerge3x3y(const int4* __restrict__ quads, uint32_t* __restrict__ qattr, int64_t Q, const int32_t* __restrict__ twin,
                            const int32_t* __restrict__ valence, const int32_t* __restrict__ count,
-                           float* __restrict__ pos, float* __restrict__ nrm, const int32_t* __restrict__ vslot, int32_t* __restrict__ vtype, int32_t* __restrict__ vtarget, int colour,
-                           int markTarget) {
+                           float* __restrict__ pos, float* __restrict__ nrm, int32_t* __restrict__ vtype, int32_t* __restrict__ vtarget, int colour,
+                           int markTarget, int step, const int64_t* ctr) {
+    if (chainHeld(ctr, step)) return;
     // the block's pattern quads gathered in LDS and handled on consecutive lanes (each is a
     // chain of dependent loads; a few per wave would spread it over every wave)
     __shared__ int s_list[kBlock];
@@ -1476,28 +1482,23 @@ __global__ void __launch_bounds__(kBlock) kMerge3x3y(const int4* __restrict__ qu
             if ((na[i] & QA_PATTERN) && ((na[i] & QA_COLOR) <= c)) return;
     }
     if (pattern1(val) && (colour || (count[v.x] == 1 && count[v.z] == 1))) {
-        handleMerge(pos, nrm, vslot, vtype, vtarget, v.x, v.y, v.z, v.w, markTarget);
+        handleMerge(pos, nrm, vtype, vtarget, v.x, v.y, v.z, v.w, markTarget);
         atomicOr(&qattr[q], (uint32_t)QA_REMOVE);
     } else if (pattern2(val) && (colour || (count[v.y] == 1 && count[v.w] == 1))) {
-        handleMerge(pos, nrm, vslot, vtype, vtarget, v.y, v.x, v.w, v.z, markTarget);
+        handleMerge(pos, nrm, vtype, vtarget, v.y, v.x, v.w, v.z, markTarget);
         atomicOr(&qattr[q], (uint32_t)QA_REMOVE);
     }
 }
 
-// markElementsP3333 first half: every eligible face clears its pattern bits before any face marks
-__global__ void kClear3333(uint32_t* __restrict__ fattr, int64_t F) {
-    const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= F) return;
-    const uint32_t a = fattr[f];
-    if ((a & QA_NM) || (a & QA_BOUNDARY) || (a & QA_DEAD)) return;
-    fattr[f] = a & 0x3F;
-}
-
-// markElementsP3333 second half, HalfedgeMesh.cu:547-628
+// markElementsP3333, HalfedgeMesh.cu:547-628.  Its first half, in which every eligible face clears
+// its pattern bits before any face marks, has nothing to clear here: an initialize and a
+// deferred P3X3Y step leave eligible faces with their colour alone.
 __global__ void kMark3333(const int4* __restrict__ quads, const int32_t* __restrict__ twin, uint32_t* __restrict__ fattr, int64_t F,
-                          const int32_t* __restrict__ valence, int32_t* __restrict__ vtype, int32_t* __restrict__ vtarget) {
+                          const int32_t* __restrict__ valence, int32_t* __restrict__ vtype, int32_t* __restrict__ vtarget, int step, const int64_t* ctr,
+                          int64_t* stamp) {
+    stampClock(stamp);
     const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= F) return;
+    if (f >= F || chainHeld(ctr, step)) return;
     const uint32_t a0 = fattr[f];
     if ((a0 & QA_NM) || (a0 & QA_BOUNDARY) || (a0 & QA_DEAD)) return;
     const int4 qv = quads[f];
@@ -1542,8 +1543,7 @@ __global__ void kMark3333(const int4* __restrict__ quads, const int32_t* __restr
 // block ranks, look-back over the own kind's tiles).
 // A vertex is kept unless it is dropped by this step (vtype == dropType) or died in an earlier
 // step of the chain; every vertex gets its new address (-1 when dropped) and the kept ones
-// their old id, slot and problem.  Positions and normals are not moved: the new vertex
-// keeps the slot of its old vertex.  A quad is kept without remove or dead bit (qnew, -1
+// their old id, position, normal and problem.  A quad is kept without remove or dead bit (qnew, -1
 // otherwise).  The arrays the following kernels start from (touched, flags, the list lengths' end;
 // the chain heads and removal counts of a chain of one) are cleared along the way.
 struct NumberArgs {
@@ -1551,8 +1551,10 @@ struct NumberArgs {
     int64_t V;
     int dropType;
     const uint8_t* vdead;
-    const int32_t *pid, *vslot;
-    int32_t *npid, *address, *oldV, *nvslot;
+    const int32_t* pid;
+    const float *pos, *nrm;
+    int32_t *npid, *address, *oldV;
+    float *npos, *nnrm;
     uint8_t* touched;
     uint32_t* vflags;
     int32_t *cnt, *srcHead, *removedAt;
@@ -1566,9 +1568,12 @@ struct NumberArgs {
     unsigned long long* wordsQ;
     uint32_t epochQ;
     int64_t *totalV, *totalQ, *directOut;
+    int step;
+    const int64_t* ctr;
 };
 template <int R>
 __global__ void __launch_bounds__(kLbBlock) kNumber(NumberArgs a) {
+    if (chainHeld(a.ctr, a.step)) return;
     __shared__ int s_cnt[R * (kLbBlock / 64)], s_pre[R * (kLbBlock / 64) + 1];
     __shared__ long long s_off;
     const bool quad = (int64_t)blockIdx.x >= a.tV;
@@ -1617,7 +1622,10 @@ __global__ void __launch_bounds__(kLbBlock) kNumber(NumberArgs a) {
         if (a.removedAt) a.removedAt[e] = 0;
         if (!keep) continue;
         a.oldV[o] = (int32_t)e;
-        a.nvslot[o] = a.vslot ? a.vslot[e] : (int32_t)e;
+        for (int k = 0; k < 3; ++k) {
+            a.npos[3 * o + k] = a.pos[3 * e + k];
+            a.nnrm[3 * o + k] = a.nrm[3 * e + k];
+        }
         a.touched[o] = 0;
         a.vflags[o] = 0;
         if (a.pid) a.npid[o] = a.pid[e];
@@ -1625,19 +1633,6 @@ __global__ void __launch_bounds__(kLbBlock) kNumber(NumberArgs a) {
     if (t == (quad ? a.tQ : a.tV) - 1 && threadIdx.x == 0) {
         *(quad ? a.totalQ : a.totalV) = off + tileSum;
         if (!quad) a.cnt[off + tileSum] = 0;
-    }
-}
-
-// positions and normals of the current vertices, gathered from their slots
-__global__ void kGatherVertices(const float* __restrict__ pos, const float* __restrict__ nrm, const int32_t* __restrict__ vslot, int64_t V,
-                                float* __restrict__ npos, float* __restrict__ nnrm, int64_t* stamp) {
-    stampClock(stamp);
-    const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= V) return;
-    const int64_t sl = vslot[v];
-    for (int k = 0; k < 3; ++k) {
-        npos[3 * v + k] = pos[3 * sl + k];
-        nnrm[3 * v + k] = nrm[3 * sl + k];
     }
 }
 
@@ -1702,9 +1697,9 @@ __device__ __forceinline__ void compactQuad(int64_t q, bool kept, int64_t d, con
 __global__ void kCompactQuads(const int4* __restrict__ quads, const uint32_t* __restrict__ attr, int64_t Q, const int32_t* __restrict__ vtarget,
                               const int32_t* __restrict__ address, int p3333, int4* __restrict__ nquads, uint32_t* __restrict__ nattr,
                               uint32_t* __restrict__ nfattr, int32_t* __restrict__ face_he, int32_t* __restrict__ oldQ, const int32_t* __restrict__ qnew, int32_t* __restrict__ removedAt,
-                              int32_t* __restrict__ outdeg, int64_t V, int64_t* ctr) {
+                              int32_t* __restrict__ outdeg, int64_t V, int step, int64_t* ctr) {
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= Q) return;
+    if (q >= Q || chainHeld(ctr, step)) return;
     const int32_t d = qnew[q];
     compactQuad(q, d >= 0, d, quads, attr, vtarget, address, p3333, nquads, nattr, nfattr, face_he, oldQ, removedAt, outdeg, V, ctr);
 }
@@ -2762,8 +2757,6 @@ int64_t* Pipeline::nmFoundParts() {
 
 const uint8_t* Pipeline::canonFlags() { return canonTracked ? arena.ptr<uint8_t>("he_canon") : nullptr; }
 
-const int32_t* Pipeline::vertexSlots() { return posSlotted ? arena.ptr<int32_t>("vslot") : nullptr; }
-
 Pipeline::Lookback Pipeline::lookback(int64_t words) {
     const size_t before = arena.capacity<unsigned long long>("lb_words");
     unsigned long long* w = arena.get<unsigned long long>("lb_words", (size_t)words);
@@ -2943,7 +2936,20 @@ void Pipeline::emitArgs(GridPassArgs& a, int64_t C, bool recordAdjoint) {
     a.vct = arena.get<uint16_t>("gp_vct", (size_t)std::max<int64_t>(V, 1));
     a.outdeg = arena.get<int32_t>("out_cnt", (size_t)V + 1);  // the halfedge initialize's list lengths
     a.vflags = arena.get<uint32_t>("vflags", (size_t)std::max<int64_t>(V, 1));
-    a.valence = simplifyQueue > 0 ? arena.get<int32_t>("valence", (size_t)std::max<int64_t>(V, 1)) : nullptr;
+    if (!chain.empty()) {
+        const size_t nv = (size_t)std::max<int64_t>(V, 1);
+        a.chain.vtype = arena.get<int32_t>("vtype", nv);
+        a.chain.vtarget = arena.get<int32_t>("vtarget", nv);
+        a.chain.valence = arena.get<int32_t>("valence", nv);
+        if (std::count(chain.begin(), chain.end(), (int)S_OLD)) a.chain.count = arena.get<int32_t>("vcount", nv);
+        if (chain.size() > 1) {
+            a.chain.head = arena.get<int32_t>("src_head", nv);
+            a.chain.outdeg = arena.get<int32_t>("outdeg", nv);
+            a.chain.bdin = arena.get<int32_t>("bdin", nv);
+            a.chain.vdead = arena.get<uint8_t>("vdead", nv);
+            a.chain.touched = arena.get<uint8_t>("touched", nv);
+        }
+    }
     a.V = V;
     a.vpid = nProblems > 1 ? arena.get<int32_t>("pid", (size_t)std::max<int64_t>(V, 1)) : nullptr;
 }
@@ -3255,7 +3261,6 @@ void Pipeline::buildBuckets(const int32_t* list, int64_t n) {
     uint32_t* vflags = arena.ptr<uint32_t>("vflags");
     uint32_t* fattr = arena.ptr<uint32_t>("fattr");
     zero(vflags, (size_t)V * sizeof(uint32_t));
-    valenceReady = false;
     if (n > 0) {
         const int32_t* lm = arena.ptr<int32_t>("bl_m");
         const int2* lent = arena.ptr<int2>("bl_entry");
@@ -3290,15 +3295,12 @@ void Pipeline::halfedgeInitialize() {
     launchQuadLists(quads, qattr, Q, V, arena.ptr<int32_t>("gp_vcell"), arena.ptr<uint16_t>("gp_vct"), pid(), probsDev, off, out, ends, face_he, fattr,
                     counters() + A_INVALID, pinDev() + kPinInvalid, stream);
     initUnchecked = true;
-    valenceReady = simplifyQueue > 0;
-    if (simplifyQueue > 0) {
-        MDMC_HIP(hipStreamSynchronize(stream));
-        checkInit();
+    if (!chain.empty()) {
         int32_t* twin = arena.get<int32_t>("twin", (size_t)std::max<int64_t>(H, 1));
         uint32_t* bpack = arena.get<uint32_t>("bpack", (size_t)std::max<int64_t>(H, 1));
         if (H > 0)
             kBucketsAll<<<gridFor(H), kBlock, 0, stream>>>(quads, H, off, out, ends, twin, bpack, vflags, fattr, qattr, arena.ptr<int32_t>("valence"),
-                                                           counters());
+                                                           chain.size() > 1 ? arena.ptr<int32_t>("bdin") : nullptr, counters());
     } else {
         // no simplification reads ids and twins only: the records at once
         int4* he = arena.get<int4>("he", (size_t)std::max<int64_t>(H, 1));
@@ -3307,8 +3309,6 @@ void Pipeline::halfedgeInitialize() {
         if (H > 0)
             kBuildHalfedges<<<gridFor(H), kBlock, 0, stream>>>(quads, H, off, out, ends, he, bsize, brank, vflags, fattr, nmSlotParts(), counters());
     }
-    posSlotted = false;  // the grid pass wrote positions by vertex
-    deferredSteps = 0;
     listsV = V;
     splitTouched = false;
     canonTracked = false;
@@ -3361,71 +3361,113 @@ void Pipeline::refreshHashTable(const uint8_t* dirtyV, int64_t oldH) {
 }
 
 // ---- simplifications
-// a simplification followed by another one of the chain: removals and relabelling in place,
-// no compaction (the ids stay the initialize's; the chain's last step compacts)
-void Pipeline::simplifyDeferredStep(int dropType, bool p3333) {
-    int32_t* vtype = arena.ptr<int32_t>("vtype");
-    int32_t* vtarget = arena.ptr<int32_t>("vtarget");
-    uint32_t* qattr = arena.ptr<uint32_t>("qattr");
-    uint32_t* fattr = arena.ptr<uint32_t>("fattr");
-    int4* quads = arena.ptr<int4>("quads");
-    const int64_t* off = arena.ptr<int64_t>("out_off");
-    const int32_t* out = arena.ptr<int32_t>("out_list");
-    const size_t nv = (size_t)std::max<int64_t>(V, 1);
-    int32_t* outdeg = arena.get<int32_t>("outdeg", nv);
-    uint8_t* vdead = arena.get<uint8_t>("vdead", nv);
-    int32_t* head = arena.get<int32_t>("src_head", nv);
-    int32_t* next = arena.get<int32_t>("src_next", nv);
-    int32_t* bdin = arena.get<int32_t>("bdin", nv);
-    int32_t* valence = arena.get<int32_t>("valence", nv);
-    int32_t* twin = arena.ptr<int32_t>("twin");
-    uint32_t* bpack = arena.ptr<uint32_t>("bpack");
-    uint8_t* touched = arena.get<uint8_t>("touched", nv);
-    // (P3333 ends a chain, so a deferred step is a P3X3Y one: it drops single vertices)
-    if (p3333) throw HipError("deferred P3333 step", -4);
-    {
-        FillBatch fb(*this);
-        if (deferredSteps == 0) {
-            fb.add(vdead, 0x00, (size_t)V);
-            fb.add(head, 0xFF, (size_t)V * sizeof(int32_t));
-        }
-        fb.add(touched, 0x00, (size_t)V);
-        fb.add(counters() + A_FALLBACK, 0x00, sizeof(int64_t));
-    }
-    if (deferredSteps == 0 && V > 0) kOutdegInit<<<gridFor(V), kBlock, 0, stream>>>(off, V, valence, outdeg, bdin);
-    int2* zslot = arena.get<int2>("zslot", nv);
-    if (Q > 0)
-        kLocalMerge<<<sparseBlocks(Q), kBlock, 0, stream>>>(quads, qattr, fattr, Q, valence, vtype, vtarget, twin, bpack, outdeg, zslot, V, touched,
-                                                       localMerges ? 1 : 0, counters());
-    if (V > 0)
-        kDropVertices<<<sparseBlocks(V), kBlock, 0, stream>>>(vtype, vtarget, V, dropType, quads, H, off, out, vdead, head, next, outdeg, zslot, counters());
-    // the merges the local update could not take: their region's buckets, flags and boundary
-    // counts recomputed
-    if (readI64(counters() + A_FALLBACK) > 0) {
-        uint8_t* hdirty = arena.get<uint8_t>("hdirty", (size_t)std::max<int64_t>(H, 1));
-        uint8_t* aff = arena.get<uint8_t>("vaffected", nv);
-        zero(hdirty, (size_t)H);
-        zero(aff, (size_t)V);
-        uint32_t* vflags = arena.ptr<uint32_t>("vflags");
-        if (V > 0) kMarkDirtyRegion<<<gridFor(V), kBlock, 0, stream>>>(touched, V, quads, H, off, out, head, next, hdirty, aff);
-        if (H > 0) kRebuildDirty<<<gridFor(H), kBlock, 0, stream>>>(quads, H, hdirty, off, out, head, next, twin, bpack, fattr, qattr, counters());
-        if (V > 0) kAffectedFlags<<<gridFor(V), kBlock, 0, stream>>>(aff, V, quads, H, off, out, head, next, twin, bpack, vflags, bdin);
-    }
-    if (V > 0) kValenceFromBdin<<<gridFor(V), kBlock, 0, stream>>>(outdeg, bdin, V, valence);
-    valenceReady = true;
-    ++deferredSteps;
-    splitTouched = false;
-    canonTracked = false;
+void Pipeline::setChain(bool colour, bool old, bool p3333) {
+    chain.clear();
+    if (colour) chain.push_back(S_COLOUR);
+    if (old) chain.push_back(S_OLD);
+    if (p3333) chain.push_back(S_3333);
 }
 
-void Pipeline::simplifyCompactAndRebuild(int dropType, bool p3333) {
-    if (simplifyQueue > 0) {  // another simplification follows
-        simplifyDeferredStep(dropType, p3333);
-        return;
+// The chain: every step but the last removes and relabels in place (the ids stay the
+// initialize's), the last compacts.  All of it is launched at once (see chainHeld) and waited for
+// once, at the compaction's totals; a step whose merges need the region rebuild (none on smooth
+// or noisy fields of the benchmarks) costs one more round from there on.  Waiting after the
+// initialize's check and after every step instead: 337 us for the 64^3 blobs, 258 us now.
+void Pipeline::simplify() {
+    if (V == 0 || Q == 0 || chain.empty()) return;
+    int64_t* h = pinHost();
+    h[kPinFallback] = h[kPinFallback + 1] = 0;
+    int from = 0;
+    bool ended = false;  // step `from` has only its end left
+    while (true) {
+        launchChain(from, ended);
+        MDMC_HIP(hipStreamSynchronize(stream));
+        initUnchecked = false;
+        if (h[kPinInvalid]) checkValid("quad vertex ids");
+        int s = 0;
+        while (s < 2 && !h[kPinFallback + s]) ++s;
+        if (s == 2) break;
+        if (s + 1 >= (int)chain.size()) throw HipError("inconsistent simplification step", -4);
+        h[kPinFallback + s] = 0;
+        rebuildRegion();
+        zero(counters() + A_FALLBACK + s, sizeof(int64_t));
+        from = s;
+        ended = true;
     }
+    finishChain();
+}
+
+void Pipeline::launchChain(int from, bool ended) {
+    const int4* cquads = arena.ptr<int4>("quads");
+    int4* quads = arena.ptr<int4>("quads");
+    uint32_t* qattr = arena.ptr<uint32_t>("qattr");
+    uint32_t* fattr = arena.ptr<uint32_t>("fattr");
+    int32_t* twin = arena.ptr<int32_t>("twin");
+    int32_t* valence = arena.ptr<int32_t>("valence");
+    int32_t* count = arena.ptr<int32_t>("vcount");
+    int32_t* vtype = arena.ptr<int32_t>("vtype");
+    int32_t* vtarget = arena.ptr<int32_t>("vtarget");
+    const size_t nv = (size_t)V;
+    for (int k = from; k < (int)chain.size(); ++k) {
+        const bool last = k + 1 == (int)chain.size();
+        if (!(ended && k == from)) {
+            int64_t* st = k == 0 ? stamp(ST_SIMPLIFY) : nullptr;
+            if (chain[k] == S_3333) {
+                kMark3333<<<gridFor(F), kBlock, 0, stream>>>(cquads, twin, fattr, F, valence, vtype, vtarget, k, counters(), st);
+            } else {
+                const bool colour = chain[k] == S_COLOUR;
+                if (colour) kMark3x3y<<<gridFor(Q), kBlock, 0, stream>>>(cquads, qattr, Q, valence, k, counters(), st);
+                else kCount3x3yOld<<<gridFor(Q), kBlock, 0, stream>>>(cquads, qattr, Q, valence, count, k, counters(), st);
+                kMerge3x3y<<<gridFor(Q), kBlock, 0, stream>>>(cquads, qattr, Q, twin, valence, count, arena.ptr<float>("pos"), arena.ptr<float>("nrm"), vtype,
+                                                              vtarget, colour ? 1 : 0, last ? 0 : 1, k, counters());
+            }
+            if (!last) {
+                // (P3333 ends a chain, so a deferred step is a P3X3Y one: it drops single vertices)
+                int32_t* outdeg = arena.ptr<int32_t>("outdeg");
+                int2* zslot = arena.get<int2>("zslot", nv);
+                kLocalMerge<<<sparseBlocks(Q), kBlock, 0, stream>>>(quads, qattr, fattr, Q, valence, vtype, vtarget, twin, arena.ptr<uint32_t>("bpack"), outdeg,
+                                                               zslot, V, arena.ptr<uint8_t>("touched"), localMerges ? 1 : 0, k, counters());
+                kDropVertices<<<sparseBlocks(V), kBlock, 0, stream>>>(vtype, vtarget, V, 3, quads, H, arena.ptr<int64_t>("out_off"), arena.ptr<int32_t>("out_list"),
+                                                                 arena.ptr<uint8_t>("vdead"), arena.ptr<int32_t>("src_head"),
+                                                                 arena.get<int32_t>("src_next", nv), outdeg, zslot, k, counters());
+            }
+        }
+        if (!last)
+            kStepEnd<<<gridFor(V), kBlock, 0, stream>>>(arena.ptr<int32_t>("outdeg"), arena.ptr<int32_t>("bdin"), V, valence, vtype, vtarget,
+                                                        arena.ptr<uint8_t>("touched"), chain[k + 1] == S_OLD ? count : nullptr, k, counters());
+    }
+    launchCompaction();
+}
+
+// the merges the local update could not take: their region's buckets, flags and boundary
+// counts recomputed
+void Pipeline::rebuildRegion() {
+    uint8_t* hdirty = arena.get<uint8_t>("hdirty", (size_t)H);
+    uint8_t* aff = arena.get<uint8_t>("vaffected", (size_t)V);
+    {
+        FillBatch fb(*this);
+        fb.add(hdirty, 0x00, (size_t)H);
+        fb.add(aff, 0x00, (size_t)V);
+    }
+    const int4* quads = arena.ptr<int4>("quads");
+    const int64_t* off = arena.ptr<int64_t>("out_off");
+    const int32_t* out = arena.ptr<int32_t>("out_list");
+    const int32_t* head = arena.ptr<int32_t>("src_head");
+    const int32_t* next = arena.ptr<int32_t>("src_next");
+    int32_t* twin = arena.ptr<int32_t>("twin");
+    uint32_t* bpack = arena.ptr<uint32_t>("bpack");
+    kMarkDirtyRegion<<<gridFor(V), kBlock, 0, stream>>>(arena.ptr<uint8_t>("touched"), V, quads, H, off, out, head, next, hdirty, aff);
+    kRebuildDirty<<<gridFor(H), kBlock, 0, stream>>>(quads, H, hdirty, off, out, head, next, twin, bpack, arena.ptr<uint32_t>("fattr"),
+                                                     arena.ptr<uint32_t>("qattr"), counters());
+    kAffectedFlags<<<gridFor(V), kBlock, 0, stream>>>(aff, V, quads, H, off, out, head, next, twin, bpack, arena.ptr<uint32_t>("vflags"),
+                                                      arena.ptr<int32_t>("bdin"));
+}
+
+void Pipeline::launchCompaction() {
+    const int step = (int)chain.size() - 1;
+    const bool p3333 = chain[step] == S_3333, chained = step > 0;
+    const int dropType = p3333 ? 1 : 3;
     // the chain's last step: this step's removals and the dead elements of the earlier ones
-    const bool chained = deferredSteps > 0;
-    deferredSteps = 0;
     int32_t* vtype = arena.ptr<int32_t>("vtype");
     int32_t* vtarget = arena.ptr<int32_t>("vtarget");
     const uint32_t* attr = p3333 ? arena.ptr<uint32_t>("fattr") : arena.ptr<uint32_t>("qattr");
@@ -3440,7 +3482,8 @@ void Pipeline::simplifyCompactAndRebuild(int dropType, bool p3333) {
     const size_t capV = (size_t)std::max(V, dmcV), capQ = (size_t)std::max(Q, dmcQ);
     int32_t* npid = pid() ? arena.get<int32_t>("pid2", capV) : nullptr;
     int32_t* oldV = arena.get<int32_t>("oldV", (size_t)std::max<int64_t>(V, 1));
-    int32_t* nvslot = arena.get<int32_t>("vslot2", capV);
+    float* npos = arena.get<float>("pos2", 3 * capV);
+    float* nnrm = arena.get<float>("nrm2", 3 * capV);
     int4* quads = arena.ptr<int4>("quads");
     int4* nquads = arena.get<int4>("quads2", capQ);
     uint32_t* nattr = arena.get<uint32_t>("qattr2", capQ);
@@ -3469,11 +3512,13 @@ void Pipeline::simplifyCompactAndRebuild(int dropType, bool p3333) {
         na.dropType = dropType;
         na.vdead = chained ? arena.ptr<uint8_t>("vdead") : nullptr;
         na.pid = pid();
-        na.vslot = vertexSlots();
+        na.pos = arena.ptr<float>("pos");
+        na.nrm = arena.ptr<float>("nrm");
+        na.npos = npos;
+        na.nnrm = nnrm;
         na.npid = npid;
         na.address = address;
         na.oldV = oldV;
-        na.nvslot = nvslot;
         na.touched = touched;
         na.vflags = vflags;
         na.cnt = cnt;
@@ -3491,16 +3536,39 @@ void Pipeline::simplifyCompactAndRebuild(int dropType, bool p3333) {
         na.totalV = pd + 1;
         na.totalQ = pd + 2;
         na.directOut = lookbackDiag();
+        na.step = step;
+        na.ctr = counters();
         if (tV + tQ > 0) kNumber<R><<<(unsigned)(tV + tQ), kLbBlock, 0, stream>>>(na);
     }
     if (Q > 0)
         kCompactQuads<<<gridFor(Q), kBlock, 0, stream>>>(quads, attr, Q, vtarget, address, p3333 ? 1 : 0, nquads, nattr, nfattr, face_he, oldQ, qnew,
-                                                         removedAt, outdeg, V, counters());
-    MDMC_HIP(hipStreamSynchronize(stream));
+                                                         removedAt, outdeg, V, step, counters());
+}
+
+// the compacted mesh's lists and records, once its sizes are known
+void Pipeline::finishChain() {
+    const int step = (int)chain.size() - 1;
+    const bool p3333 = chain[step] == S_3333, chained = step > 0;
+    const int dropType = p3333 ? 1 : 3;
+    const int64_t* h = pinHost();
     const int64_t nV = h[1], nQ = h[2];
     if (nV < 0 || nV > V || nQ < 0 || nQ > Q) throw HipError("inconsistent compaction counts", -4);
-    if (h[kPinInvalid]) checkValid("quad vertex ids");
-
+    const size_t capQ = (size_t)std::max(Q, dmcQ);
+    const int32_t* vtype = arena.ptr<int32_t>("vtype");
+    const int32_t* vtarget = arena.ptr<int32_t>("vtarget");
+    const int32_t* address = arena.ptr<int32_t>("vaddress");
+    const int32_t* oldV = arena.ptr<int32_t>("oldV");
+    const int4* nquads = arena.ptr<int4>("quads2");
+    const int32_t* oldQ = arena.ptr<int32_t>("oldQ");
+    const int32_t* qnew = arena.ptr<int32_t>("qnew");
+    int32_t* removedAt = chained ? nullptr : arena.ptr<int32_t>("removed_at");
+    int32_t* outdeg = chained ? arena.ptr<int32_t>("outdeg") : nullptr;
+    int32_t* srcHead = arena.ptr<int32_t>("src_head");
+    int32_t* srcNext = arena.ptr<int32_t>("src_next");
+    uint8_t* touched = arena.ptr<uint8_t>("touched");
+    uint32_t* vflags = arena.ptr<uint32_t>("vflags");
+    int32_t* cnt = arena.ptr<int32_t>("out_cnt");
+    uint32_t* nfattr = arena.ptr<uint32_t>("fattr2");
     // HalfedgeMesh::initialize of the compacted quads, from the previous build: the new
     // outgoing lists are the old ones of each new vertex's own and relabelled vertices,
     // renumbered; halfedges with untouched endpoints keep their bucket results
@@ -3522,12 +3590,12 @@ void Pipeline::simplifyCompactAndRebuild(int dropType, bool p3333) {
     if (nH > 0)
         kRemapRebuild<<<gridFor(nH), kBlock, 0, stream>>>(nquads, nH, touched, oldQ, arena.ptr<int32_t>("twin"), H, arena.ptr<uint32_t>("bpack"),
                                                          qnew, off2, out2, he, bsize, brank, vflags, nfattr, nmSlotParts(), counters());
-    arena.swap("vslot", "vslot2");
-    posSlotted = true;
+    arena.swap("pos", "pos2");
+    arena.swap("nrm", "nrm2");
     arena.swap("quads", "quads2");
     arena.swap("qattr", "qattr2");
     arena.swap("fattr", "fattr2");
-    if (npid) arena.swap("pid", "pid2");
+    if (pid()) arena.swap("pid", "pid2");
     arena.swap("out_off", "out_off2");
     arena.swap("out_list", "out_list2");
     V = nV;
@@ -3536,81 +3604,16 @@ void Pipeline::simplifyCompactAndRebuild(int dropType, bool p3333) {
     F = nQ;
     vertHeV = V;
     vertHeQ = Q;
-    valenceReady = false;
     listsV = V;
     splitTouched = false;
     canonTracked = false;
 }
 
-void Pipeline::simplifyInit(int32_t** valence, int32_t** count, bool needCount) {
-    const bool firstOfChain = deferredSteps == 0 && !posSlotted;
-    if (simplifyQueue > 0) --simplifyQueue;
-    *valence = arena.get<int32_t>("valence", (size_t)V);
-    *count = arena.get<int32_t>("vcount", (size_t)V);
-    int32_t* vtype = arena.get<int32_t>("vtype", (size_t)V);
-    int32_t* vtarget = arena.get<int32_t>("vtarget", (size_t)V);
-    {
-        // (the pattern counts only serve the old P3X3Y rule)
-        FillBatch fb(*this);
-        fb.stampAt(firstOfChain ? stamp(ST_SIMPLIFY) : nullptr);
-        if (needCount) fb.add(*count, 0x00, (size_t)V * sizeof(int32_t));
-        fb.add(vtype, 0x00, (size_t)V * sizeof(int32_t));
-        fb.add(vtarget, 0xFF, (size_t)V * sizeof(int32_t));
-    }
-    if (!valenceReady) {  // not computed by the last bucket pass
-        zero(*valence, (size_t)V * sizeof(int32_t));
-        if (H > 0) kValence<<<gridFor(H), kBlock, 0, stream>>>(arena.ptr<int4>("quads"), arena.ptr<int32_t>("twin"), H, *valence);
-    }
-    valenceReady = false;
-}
-
-void Pipeline::simplify3X3Y(bool colour) {
-    if (V == 0) return;
-    int32_t *valence, *count;
-    simplifyInit(&valence, &count, !colour);
-    int4* quads = arena.ptr<int4>("quads");
-    uint32_t* qattr = arena.ptr<uint32_t>("qattr");
-    if (Q > 0) {
-        if (colour) kMark3x3y<<<gridFor(Q), kBlock, 0, stream>>>(quads, qattr, Q, valence);
-        else kCount3x3yOld<<<gridFor(Q), kBlock, 0, stream>>>(quads, qattr, Q, valence, count);
-        kMerge3x3y<<<gridFor(Q), kBlock, 0, stream>>>(quads, qattr, Q, arena.ptr<int32_t>("twin"), valence, count,
-                                                      arena.ptr<float>("pos"), arena.ptr<float>("nrm"), vertexSlots(), arena.ptr<int32_t>("vtype"),
-                                                      arena.ptr<int32_t>("vtarget"), colour ? 1 : 0, simplifyQueue > 0 ? 1 : 0);
-    }
-    simplifyCompactAndRebuild(3, false);
-}
-
-void Pipeline::simplify3333() {
-    if (V == 0) return;
-    int32_t *valence, *count;
-    simplifyInit(&valence, &count, false);
-    if (F > 0) {
-        kClear3333<<<gridFor(F), kBlock, 0, stream>>>(arena.ptr<uint32_t>("fattr"), F);
-        kMark3333<<<gridFor(F), kBlock, 0, stream>>>(arena.ptr<int4>("quads"), arena.ptr<int32_t>("twin"), arena.ptr<uint32_t>("fattr"), F, valence,
-                                                     arena.ptr<int32_t>("vtype"), arena.ptr<int32_t>("vtarget"));
-    }
-    simplifyCompactAndRebuild(1, true);
-}
-
-// positions and normals by vertex again, from the slots the simplifications kept them in
-void Pipeline::gatherVertices() {
-    if (!posSlotted) return;
-    const size_t cap = (size_t)std::max(V, dmcV);
-    float* npos = arena.get<float>("pos2", 3 * cap);
-    float* nnrm = arena.get<float>("nrm2", 3 * cap);
-    if (V > 0) kGatherVertices<<<gridFor(V), kBlock, 0, stream>>>(arena.ptr<float>("pos"), arena.ptr<float>("nrm"), vertexSlots(), V, npos, nnrm, stamp(ST_TWINS));
-    arena.swap("pos", "pos2");
-    arena.swap("nrm", "nrm2");
-    posSlotted = false;
-}
-
 void Pipeline::fixManifoldTwins() {
-    int64_t* st = posSlotted ? nullptr : stamp(ST_TWINS);
-    gatherVertices();
     if (H == 0) return;
     kFixTwins<<<(unsigned)((H + kFixPer * kBlock - 1) / (kFixPer * kBlock)), kBlock, 0, stream>>>(arena.ptr<int4>("he"), H, arena.ptr<int4>("quads"), arena.ptr<int64_t>("out_off"), arena.ptr<int32_t>("out_list"),
                                                  arena.ptr<int32_t>("bsize"), arena.ptr<int32_t>("brank"), arena.ptr<float>("pos"), probsDev, pid(),
-                                                 counters(), st);
+                                                 counters(), stamp(ST_TWINS));
 }
 
 // ---- ManifoldSplitter::run, one problem and all that follows: the last stages are launched
