@@ -303,7 +303,6 @@ mdmc_status runExtraction(mdmc_ctx* ctx, const mdmc_grid* grids, int G, const fl
             p.dmc(problems, surf, record);
             if (graphable) p.noteEagerFront(shapeSig);
         }
-        if (B > 1) p.problemDmcCounts(B);
         int64_t st9[9] = {0};
         if (p.V > 0) {
             p.halfedgeInitialize();
@@ -316,7 +315,6 @@ mdmc_status runExtraction(mdmc_ctx* ctx, const mdmc_grid* grids, int G, const fl
                 if (flags & MDMC_SPLIT_NM) p.split(opt->split_step, maxIters);
                 if (flags & MDMC_DETECT_NM_VERTS) p.detectNonManifoldVertices();
                 p.regroupBatch(B);
-                p.finishBatch();
                 for (int b = 0; b < B; ++b)
                     for (int k = 0; k < 9; ++k) st9[k] += p.batchStats[9 * (size_t)b + k];
             }
@@ -328,6 +326,7 @@ mdmc_status runExtraction(mdmc_ctx* ctx, const mdmc_grid* grids, int G, const fl
                 p.batchHOff.assign((size_t)B + 1, 0);
                 p.batchFOff.assign((size_t)B + 1, 0);
                 p.batchStats.assign(9 * (size_t)B, 0);
+                p.batchDmc.assign(2 * (size_t)B, 0);
             }
             p.finishEmpty();
         }

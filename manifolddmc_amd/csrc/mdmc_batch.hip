@@ -10,10 +10,14 @@
 // order a single extraction of that problem produces.
 //
 // Until the splitter runs, every array is ordered by problem (the grid pass emits the
-// problems in order and every compaction is stable).  The splitter only appends, so
-// each array is a sorted prefix of n0 elements plus a tail; the tail is sorted stably
-// by problem (least-significant-bit-first binary splits: per bit a prefix sum of the
-// "bit is 0" flags and a scatter) and each problem's tail goes after its prefix part.
+// problems in order and every compaction is stable), so each problem's first vertex and quad
+// follow from the grid pass's tile offsets and the compaction's numbering: a few loads per
+// problem, no pass over the elements.  The splitter only appends, so each array is a sorted
+// prefix plus a tail.  A split iteration appends its elements in the order of the faces it
+// split, so the tail is a few runs that are each in problem order; run starts are found where
+// a key falls, and each tail element's place follows from the runs' counts.  (A tail of more than
+// kMaxRuns runs is sorted instead: least-significant-bit-first binary splits, per bit a
+// prefix sum of the "bit is 0" flags and a scatter.)
 #include <algorithm>
 #include <vector>
 
@@ -27,20 +31,12 @@ namespace {
 
 __device__ __forceinline__ int heO(const int4* he, int h) { return ((const int*)he)[4 * (int64_t)h]; }
 
+// the clock alone, where no kernel begins or ends a stage
+__global__ void kStamp(int64_t* stamp) { *stamp = wall_clock64(); }
+
 __global__ void kIota(int32_t* __restrict__ p, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = (int32_t)i;
-}
-
-// problem of each halfedge (its origin's) and of each face (its first halfedge's origin's)
-__global__ void kHalfedgeKeys(const int4* __restrict__ he, int64_t H, const int32_t* __restrict__ pid, int32_t* __restrict__ key) {
-    const int64_t h = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (h < H) key[h] = pid[heO(he, (int)h)];
-}
-__global__ void kFaceKeys2(const int4* __restrict__ he, const int32_t* __restrict__ face_he, int64_t F, const int32_t* __restrict__ pid,
-                           int32_t* __restrict__ key) {
-    const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (f < F) key[f] = pid[heO(he, face_he[f])];
 }
 
 __global__ void kSplitFlags(const int32_t* __restrict__ perm, const int32_t* __restrict__ key, int64_t n, int bit, int32_t* __restrict__ zero) {
@@ -55,202 +51,336 @@ __global__ void kSplitScatter(const int32_t* __restrict__ perm, const int32_t* _
     out[zero[i] ? p : *zeros + (i - p)] = perm[i];
 }
 
-// final position of every element: prefix element i of problem b -> out[b] + i - pre[b];
-// tail element at sorted tail position j -> out[b] + preCount[b] + j - tail[b]
-// (offsets: [0, B] prefix starts, [B+1, 2B+1] tail starts, [2B+2, 3B+2] output starts)
-__global__ void kPlace(const int32_t* __restrict__ key, int64_t n0, int64_t n, const int32_t* __restrict__ tailPerm, const int64_t* __restrict__ offs,
-                       int B, int32_t* __restrict__ perm, int32_t* __restrict__ inv) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int64_t* pre = offs;
-    const int64_t* tail = offs + (B + 1);
-    const int64_t* out = offs + 2 * (B + 1);
-    int64_t old, dst;
-    if (i < n0) {
-        old = i;
-        const int b = key[i];
-        dst = out[b] + (i - pre[b]);
-    } else {
-        const int64_t j = i - n0;
-        old = n0 + tailPerm[j];
-        const int b = key[old];
-        dst = out[b] + (pre[b + 1] - pre[b]) + (j - tail[b]);
+// ---- where every element goes
+constexpr int kMaxRuns = 32;
+enum : int { RG_V = 0, RG_H = 1, RG_F = 2 };
+
+// per problem b in [0, B]: its first vertex and quad as the grid pass numbered them (vOff / qOff at
+// its first tile or row segment), and after the simplifications' compaction (the first kept one
+// from there on: address / qnew, -1 for removed elements; null: nothing was compacted)
+struct StartArgs {
+    const ProblemDev* probs;
+    int B, slab;
+    const int64_t *vOff, *qOff;
+    int64_t last;
+    const int32_t *address, *qnew;
+    int64_t dmcV, dmcQ, V, Q;
+    int64_t *dmcStartV, *dmcStartQ, *startV, *startQ;
+};
+__global__ void kProblemStarts(StartArgs a) {
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b > a.B) return;
+    const int64_t i = b == a.B ? a.last : (a.slab ? a.probs[b].segBase : a.probs[b].tileBase);
+    int64_t v = a.vOff[i], q = a.qOff[i];
+    a.dmcStartV[b] = v;
+    a.dmcStartQ[b] = q;
+    if (a.address) {
+        while (v < a.dmcV && a.address[v] < 0) ++v;
+        v = v < a.dmcV ? a.address[v] : a.V;
+        while (q < a.dmcQ && a.qnew[q] < 0) ++q;
+        q = q < a.dmcQ ? a.qnew[q] : a.Q;
     }
-    perm[dst] = (int32_t)old;
-    inv[old] = (int32_t)dst;
+    a.startV[b] = v;
+    a.startQ[b] = q;
 }
 
-// Per-key counts of keys that arrive sorted (key(i) = key[perm ? perm[i] : i], values in
-// [0, B)): thread i in [0, n] writes first[k] = i for every k in (key(i-1), key(i)], with
-// key(-1) = -1 and key(n) = B, so first[k] is the first index whose key is >= k and the
-// count of key k is first[k + 1] - first[k].  No atomics; a key out of order or out of
-// range raises *bad.
-__global__ void kKeyStarts(const int32_t* __restrict__ key, const int32_t* __restrict__ perm, int64_t n, int B, int64_t* __restrict__ first,
-                           int* __restrict__ bad) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i > n) return;
-    const int k = i < n ? key[perm ? perm[i] : i] : B;
-    const int kp = i > 0 ? key[perm ? perm[i - 1] : i - 1] : -1;
-    if (k < kp || k > B || (i < n && (k == B || k < 0))) {
+// the three arrays of the mesh, their prefixes [0, n0) and their ends
+struct RegroupArgs {
+    const int4* he;
+    const int32_t* face_he;
+    const int32_t* pid;
+    int B;
+    int64_t n0[3], n[3];
+    int32_t* tailKey[3];  // [n - n0]: the tail elements' problems
+    int32_t* tailDst[3];  // [n - n0]: their new ids
+    int32_t *runCount, *runList;  // [3], [3 * kMaxRuns]: tail indices where a run starts (unordered)
+    const int64_t *startV, *startQ;
+    int64_t* shift;  // [3 * B]: new id - old id of a problem's prefix elements
+};
+__device__ __forceinline__ int64_t prefixStart(const RegroupArgs& r, int arr, int b) {
+    return arr == RG_V ? r.startV[b] : (arr == RG_H ? 4 * r.startQ[b] : r.startQ[b]);
+}
+// one thread per tail element, over the three tails in turn
+__device__ __forceinline__ bool tailElement(const RegroupArgs& r, int64_t t, int& arr, int64_t& j) {
+    arr = 0;
+    while (arr < 3 && t >= r.n[arr] - r.n0[arr]) t -= r.n[arr] - r.n0[arr], ++arr;
+    j = t;
+    return arr < 3;
+}
+__device__ __forceinline__ int tailProblem(const RegroupArgs& r, int arr, int64_t i) {
+    if (arr == RG_V) return r.pid[i];
+    return r.pid[heO(r.he, arr == RG_H ? (int)i : r.face_he[i])];
+}
+__global__ void kTailKeys(RegroupArgs r) {
+    int arr;
+    int64_t j;
+    if (!tailElement(r, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, arr, j)) return;
+    const int k = tailProblem(r, arr, r.n0[arr] + j);
+    r.tailKey[arr][j] = k;
+    if (j > 0 && k < tailProblem(r, arr, r.n0[arr] + j - 1)) {
+        const int c = atomicAdd(&r.runCount[arr], 1);
+        if (c < kMaxRuns) r.runList[arr * kMaxRuns + c] = (int32_t)j;
+    }
+}
+// the runs of the three tails: run s of array a covers tail elements [start[a][s], start[a][s + 1])
+struct Runs {
+    int count[3];
+    int32_t start[3][kMaxRuns + 1];
+    const int32_t* order[3];  // a sorted tail's permutation (one run), else null
+};
+__device__ __forceinline__ int runOf(const Runs& u, int arr, int64_t j) {
+    int s = 0;
+    while (s + 1 < u.count[arr] && j >= u.start[arr][s + 1]) ++s;
+    return s;
+}
+// first[arr][s][b] = the first tail position of run s whose key is b or more (b in [0, B]): the
+// element before every boundary writes it, so no count and no atomics
+__device__ __forceinline__ int64_t firstAt(int arr, int s, int b, int B) { return ((int64_t)arr * kMaxRuns + s) * (B + 1) + b; }
+__global__ void kRunStarts(RegroupArgs r, Runs u, int32_t* __restrict__ first, int* __restrict__ bad) {
+    int arr;
+    int64_t j;
+    if (!tailElement(r, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, arr, j)) return;
+    const int s = runOf(u, arr, j), B = r.B;
+    const int32_t* key = r.tailKey[arr];
+    const int32_t* o = u.order[arr];
+    const int k = key[o ? o[j] : j];
+    const int kp = j > u.start[arr][s] ? key[o ? o[j - 1] : j - 1] : -1;
+    if (k < kp || k < 0 || k >= B) {
         atomicOr(bad, 1);
         return;
     }
-    for (int kk = kp + 1; kk <= k; ++kk) first[kk] = i;
+    for (int kk = kp + 1; kk <= k; ++kk) first[firstAt(arr, s, kk, B)] = (int32_t)j;
+    if (j + 1 == u.start[arr][s + 1])
+        for (int kk = k + 1; kk <= B; ++kk) first[firstAt(arr, s, kk, B)] = (int32_t)(j + 1);
 }
-__global__ void kCountsFromStarts(const int64_t* __restrict__ first, int B, unsigned long long* __restrict__ count, int stride, int slot) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < B) count[(int64_t)k * stride + slot] = (unsigned long long)(first[k + 1] - first[k]);
-}
-
-__global__ void kPermuteVertices(const int32_t* __restrict__ perm, int64_t V, const float* __restrict__ pos, const float* __restrict__ nrm,
-                                 const uint32_t* __restrict__ vflags, const int32_t* __restrict__ pid, float* __restrict__ npos,
-                                 float* __restrict__ nnrm, uint32_t* __restrict__ nvflags, int32_t* __restrict__ npid) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= V) return;
-    const int64_t o = perm[i];
-    for (int k = 0; k < 3; ++k) {
-        npos[3 * i + k] = pos[3 * o + k];
-        nnrm[3 * i + k] = nrm[3 * o + k];
+// one block: the problems' new offsets (off[arr][b], [B + 1] each), the shift of their prefixes and,
+// in place of first, the new id of a tail element less its tail position
+__global__ void __launch_bounds__(1024) kOffsets(RegroupArgs r, Runs u, int32_t* __restrict__ first, int64_t* __restrict__ off) {
+    __shared__ int64_t s_wave[16];
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, B = r.B;
+    for (int arr = 0; arr < 3; ++arr) {
+        int64_t carry = 0;
+        const int runs = r.n[arr] > r.n0[arr] ? u.count[arr] : 0;
+        for (int b0 = 0; b0 < B; b0 += 1024) {
+            const int b = b0 + tid;
+            int64_t c = 0, pre = 0;
+            if (b < B) {
+                pre = prefixStart(r, arr, b + 1) - prefixStart(r, arr, b);
+                c = pre;
+                for (int s = 0; s < runs; ++s) c += first[firstAt(arr, s, b + 1, B)] - first[firstAt(arr, s, b, B)];
+            }
+            int64_t x = c;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const int64_t y = __shfl_up(x, d, 64);
+                if (lane >= d) x += y;
+            }
+            if (lane == 63) s_wave[wid] = x;
+            __syncthreads();
+            int64_t add = 0, total = 0;
+            for (int w = 0; w < 16; ++w) {
+                if (w < wid) add += s_wave[w];
+                total += s_wave[w];
+            }
+            const int64_t o = carry + add + x - c;
+            // (every count of this chunk is read: first may be rewritten, b + 1's by its own thread
+            // only after this barrier, the next chunk's b not before its own reads)
+            int64_t tail = o + pre;
+            int64_t place[kMaxRuns];
+            for (int s = 0; s < runs; ++s) {
+                if (b < B) {
+                    const int64_t f = first[firstAt(arr, s, b, B)], g = first[firstAt(arr, s, b + 1, B)];
+                    place[s] = tail - f;
+                    tail += g - f;
+                }
+            }
+            __syncthreads();
+            if (b < B) {
+                off[(int64_t)arr * (B + 1) + b] = o;
+                r.shift[(int64_t)arr * B + b] = o - prefixStart(r, arr, b);
+                for (int s = 0; s < runs; ++s) first[firstAt(arr, s, b, B)] = (int32_t)place[s];
+            }
+            carry += total;
+        }
+        if (tid == 0) off[(int64_t)arr * (B + 1) + B] = carry;
+        __syncthreads();
     }
-    nvflags[i] = vflags[o];
-    npid[i] = pid[o];
 }
-
-__global__ void kPermuteHalfedges(const int32_t* __restrict__ perm, int64_t H, const int4* __restrict__ he, const int32_t* __restrict__ bsize,
-                                  const int32_t* __restrict__ brank, const int32_t* __restrict__ vNew, const int32_t* __restrict__ hNew,
-                                  const int32_t* __restrict__ fNew, int4* __restrict__ nhe, int32_t* __restrict__ nbsize,
-                                  int32_t* __restrict__ nbrank) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= H) return;
-    const int o = perm[i];
-    const int4 e = he[o];
-    nhe[i] = make_int4(vNew[e.x], fNew[e.y], hNew[e.z], e.w >= 0 ? hNew[e.w] : e.w);
-    nbsize[i] = bsize[o];
-    nbrank[i] = brank[o];
+__global__ void kTailPlaces(RegroupArgs r, Runs u, const int32_t* __restrict__ place) {
+    int arr;
+    int64_t j;
+    if (!tailElement(r, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, arr, j)) return;
+    const int s = runOf(u, arr, j);
+    const int64_t e = u.order[arr] ? u.order[arr][j] : j;
+    r.tailDst[arr][e] = (int32_t)(place[firstAt(arr, s, r.tailKey[arr][e], r.B)] + j);
 }
-
-__global__ void kPermuteFaces(const int32_t* __restrict__ perm, int64_t F, const int32_t* __restrict__ face_he, const uint32_t* __restrict__ fattr,
-                              const int32_t* __restrict__ hNew, int32_t* __restrict__ nface_he, uint32_t* __restrict__ nfattr) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= F) return;
-    const int o = perm[i];
-    nface_he[i] = hNew[face_he[o]];
-    nfattr[i] = fattr[o];
+// the new id of element x of array arr, which belongs to problem b
+__device__ __forceinline__ int newId(const RegroupArgs& r, int arr, int b, int x) {
+    return x < r.n0[arr] ? (int)(x + r.shift[(int64_t)arr * r.B + b]) : r.tailDst[arr][x - r.n0[arr]];
 }
-
-// the vertex -> halfedge array of each problem as its own extraction leaves it: highest
-// initialize-time halfedge 4q+i starting at the vertex, q counted inside the problem;
-// -1 where none; 0 for vertices the splitter added
-__global__ void kVertexHalfedgeInitBatch(int32_t* __restrict__ vh, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) vh[i] = -1;
-}
-__global__ void kVertexHalfedgeMax(const int4* __restrict__ quads, int64_t Q, int32_t* __restrict__ vh) {
-    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= Q) return;
-    const int4 v = quads[q];
-    const int b = (int)(4 * q);
-    atomicMax(&vh[v.x], b + 0);
-    atomicMax(&vh[v.y], b + 1);
-    atomicMax(&vh[v.z], b + 2);
-    atomicMax(&vh[v.w], b + 3);
-}
-__global__ void kVertexHalfedgeLocal(const int32_t* __restrict__ vhInit, int64_t Vinit, const int32_t* __restrict__ vNew, const int32_t* __restrict__ pidNew,
-                                     const int64_t* __restrict__ qBase, int64_t V, int32_t* __restrict__ out) {
-    const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= V) return;
-    if (v >= Vinit) {
-        out[vNew[v]] = 0;
-        return;
+// the problem of prefix halfedge or face: the last b with startQ[b] <= q; the lanes of a wave
+// mostly share one, found once for the wave's first lane
+__device__ __forceinline__ int problemOfQuad(const int64_t* __restrict__ startQ, int B, int64_t q) {
+    int lo = 0, hi = B;
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (startQ[mid] <= q) lo = mid;
+        else hi = mid;
     }
-    const int h = vhInit[v];
-    const int64_t nv = vNew[v];
-    out[nv] = h < 0 ? -1 : (int32_t)(h - 4 * qBase[pidNew[nv]]);
+    return lo;
 }
 
 // bucket / face / vertex counters of HalfedgeMesh.cu:1164-1239 per problem.  Elements are
 // sorted by problem, so a wave usually holds one problem: it then adds its sums once.
 // Per-problem statistics of one element kind over its regrouped range [0, n), where every
-// problem's elements are contiguous and problems ascend: each block reduces a chunk of
-// kStatChunk elements in LDS, one row per problem the chunk touches (up to kStatRows; the
+// problem's elements are contiguous and problems ascend: each block reduces a chunk
+// of elements in LDS, one row per problem the chunk touches (up to kStatRows; the
 // elements of further ones add to global memory directly), and adds every non-zero row
 // entry once.  KIND 0: halfedges (slots 0-2: NM-4 / NM-3 / all edges, counted at the
 // bucket's first member), 1: faces (slots 3-7: quads with k NM edges), 2: vertices (slot 8:
 // non-manifold vertices).  out[9 * problem + slot].
-constexpr int kStatChunk = 4096, kStatRows = 32;
+constexpr int kStatRows = 32;
+// elements per block: up to 4096 (fewer global additions), down to one per thread while that
+// gives fewer than 1024 blocks (110 k vertices: 56 us in 27 blocks, 6 us in 432)
+inline int64_t statChunk(int64_t n) { return std::min<int64_t>(4096, std::max<int64_t>(kBlock, n / 1024 / kBlock * kBlock)); }
 
-__device__ __forceinline__ void statAdd(unsigned* acc, unsigned long long* out, bool live, int p, int pbase, int slot, int accSlot, unsigned v) {
+__device__ __forceinline__ void statAdd(unsigned* acc, unsigned long long* out, bool live, int p, int pbase, int slot, int accSlot, bool v) {
     // one LDS atomic per wave when all its live lanes share the problem
-    const int p0 = __shfl(p, 0, 64);
-    const uint64_t alive = __ballot(live);
-    const uint64_t same = __ballot(live && p == p0);
-    if (alive == 0) return;
-    if (same == alive) {
-        unsigned sum = live ? v : 0u;
-#pragma unroll
-        for (int d = 32; d > 0; d >>= 1) sum += __shfl_down(sum, d, 64);
-        const int pk = __shfl(p, __ffsll((unsigned long long)alive) - 1, 64);
-        if ((threadIdx.x & 63) == 0 && sum) {
+    const uint64_t alive = __ballot(live), on = __ballot(live && v);
+    if (on == 0) return;
+    const int pk = __shfl(p, __ffsll((unsigned long long)alive) - 1, 64);
+    if (__ballot(live && p == pk) == alive) {
+        if ((threadIdx.x & 63) == 0) {
             const int r = pk - pbase;
+            const unsigned sum = (unsigned)__popcll(on);
             if (r >= 0 && r < kStatRows) atomicAdd(&acc[r * 5 + accSlot], sum);
             else atomicAdd(&out[(int64_t)pk * 9 + slot], (unsigned long long)sum);
         }
     } else if (live && v) {
         const int r = p - pbase;
-        if (r >= 0 && r < kStatRows) atomicAdd(&acc[r * 5 + accSlot], v);
-        else atomicAdd(&out[(int64_t)p * 9 + slot], (unsigned long long)v);
+        if (r >= 0 && r < kStatRows) atomicAdd(&acc[r * 5 + accSlot], 1u);
+        else atomicAdd(&out[(int64_t)p * 9 + slot], 1ULL);
     }
 }
 
-template <int KIND>
-__global__ void kStatsBatch(const int4* __restrict__ he, const int32_t* __restrict__ face_he, const int32_t* __restrict__ bsize,
-                            const int32_t* __restrict__ brank, const uint32_t* __restrict__ vflags, const int32_t* __restrict__ pid, int64_t n,
-                            unsigned long long* __restrict__ out) {
-    constexpr int nslots = KIND == 0 ? 3 : (KIND == 1 ? 5 : 1);
-    constexpr int base = KIND == 0 ? 0 : (KIND == 1 ? 3 : 8);
+// The regroup's pass over one kind of element, a block per chunk of them: moves every element
+// to its place with its ids renumbered (MOVE; without a tail every place is the old one and
+// nothing is moved) and takes the problems' statistics on the way.  Vertices also get their
+// vertex -> halfedge value as the problem's own extraction leaves it: the highest
+// initialize-time halfedge 4q+i starting at the vertex (the maximum of its outgoing list), q
+// counted inside the problem; -1 where none; 0 for vertices the splitter added.
+//
+// Bound by HBM: the permutations, their inverses and a copy back of every array, keys for every
+// element and an atomicMax per halfedge came to 3.1 ms of the 64-grid batch's 9.4 ms (5.4 M
+// vertices); 1.0 ms now.
+struct MoveArgs {
+    RegroupArgs r;
+    const float *pos, *nrm;
+    const uint32_t *vflags, *fattr;
+    const int32_t *bsize, *brank;
+    const uint8_t* canon;
+    const int64_t* listOff;  // the outgoing lists of the last initialize's vertices (the prefix)
+    const int32_t* list;
+    float *npos, *nnrm;
+    uint32_t *nvflags, *nfattr;
+    int32_t *npid, *nbsize, *nbrank, *nface_he, *vh;
+    int4* nhe;
+    unsigned long long* out;
+    int* bad;
+};
+template <int KIND, bool MOVE>
+__global__ void __launch_bounds__(kBlock) kRegroup(MoveArgs a, int64_t chunk) {
+    constexpr int nslots = KIND == RG_H ? 3 : (KIND == RG_F ? 5 : 1);
+    constexpr int base = KIND == RG_H ? 0 : (KIND == RG_F ? 3 : 8);
+    const RegroupArgs& r = a.r;
     __shared__ unsigned acc[kStatRows * 5];
-    const int64_t c0 = (int64_t)blockIdx.x * kStatChunk;
-    const int64_t c1 = c0 + kStatChunk < n ? c0 + kStatChunk : n;
-    for (int t = threadIdx.x; t < kStatRows * 5; t += blockDim.x) acc[t] = 0;
+    const int64_t n = r.n[KIND], n0 = r.n0[KIND];
+    const int64_t c0 = (int64_t)blockIdx.x * chunk;
+    const int64_t c1 = c0 + chunk < n ? c0 + chunk : n;
+    for (int t = threadIdx.x; t < kStatRows * 5; t += kBlock) acc[t] = 0;
     auto problemOf = [&](int64_t i) -> int {
-        if (KIND == 0) return pid[heO(he, (int)i)];
-        if (KIND == 1) return pid[heO(he, face_he[i])];
-        return pid[i];
+        if (KIND == RG_V) return r.pid[i];
+        if (i >= n0) return r.tailKey[KIND][i - n0];
+        return problemOfQuad(r.startQ, r.B, KIND == RG_H ? i >> 2 : i);
     };
     const int pbase = problemOf(c0);
+    // most blocks lie in one problem's prefix: no search per element
+    const bool one = KIND != RG_V && c1 <= n0 && problemOf(c1 - 1) == pbase;
     __syncthreads();
     // uniform trip count so that every lane takes part in the wave reductions
-    for (int64_t i0 = c0; i0 < c1; i0 += blockDim.x) {
+    for (int64_t i0 = c0; i0 < c1; i0 += kBlock) {
         const int64_t i = i0 + threadIdx.x;
-        const bool inRange = i < c1;
-        if (KIND == 0) {
-            const bool live = inRange && brank[i] == 0;
-            const int p = live ? problemOf(i) : 0;
-            const int nb = live ? bsize[i] : 0;
-            statAdd(acc, out, live, p, pbase, 0, 0, nb == 4);
-            statAdd(acc, out, live, p, pbase, 1, 1, nb == 3);
-            statAdd(acc, out, live, p, pbase, 2, 2, nb > 0);
-        } else if (KIND == 1) {
-            int p = 0, k = 0;
-            if (inRange) {
-                int h = face_he[i];
-                p = pid[heO(he, h)];
-                for (int j = 0; j < 4; ++j) {
-                    if (bsize[h] > 2) ++k;
-                    h = ((const int*)he)[4 * (int64_t)h + 2];
+        const bool live = i < c1;
+        const int p = !live ? 0 : (one ? pbase : problemOf(i));
+        const int64_t d = !live ? 0 : (MOVE ? newId(r, KIND, p, (int)i) : i);
+        if (KIND == RG_H) {
+            int nb = 0, rk = 1;
+            if (live) {
+                nb = a.bsize[i];
+                rk = a.brank[i];
+                if (MOVE) {
+                    const int4 e = r.he[i];
+                    a.nhe[d] = make_int4(newId(r, RG_V, p, e.x), newId(r, RG_F, p, e.y), newId(r, RG_H, p, e.z), e.w >= 0 ? newId(r, RG_H, p, e.w) : e.w);
+                    a.nbsize[d] = nb;
+                    a.nbrank[d] = rk;
                 }
             }
-            for (int kk = 0; kk < 5; ++kk) statAdd(acc, out, inRange, p, pbase, 3 + kk, kk, k == kk);
+            const bool count = live && rk == 0;
+            statAdd(acc, a.out, count, p, pbase, 0, 0, nb == 4);
+            statAdd(acc, a.out, count, p, pbase, 1, 1, nb == 3);
+            statAdd(acc, a.out, count, p, pbase, 2, 2, nb > 0);
+        } else if (KIND == RG_F) {
+            int k = 0;
+            if (live) {
+                const int h0 = a.r.face_he[i];
+                // a face whose four records keep the build's layout: one load of their sizes
+                const int q4 = h0 & ~3;
+                if (q4 + 3 < r.n[RG_H] && (!a.canon || *reinterpret_cast<const uint32_t*>(a.canon + q4) == 0x01010101u)) {
+                    const int4 s = reinterpret_cast<const int4*>(a.bsize)[q4 >> 2];
+                    k = (s.x > 2) + (s.y > 2) + (s.z > 2) + (s.w > 2);
+                } else {
+                    int h = h0;
+                    for (int j = 0; j < 4; ++j) {
+                        if (a.bsize[h] > 2) ++k;
+                        h = ((const int*)r.he)[4 * (int64_t)h + 2];
+                    }
+                }
+                if (MOVE) {
+                    a.nface_he[d] = newId(r, RG_H, p, h0);
+                    a.nfattr[d] = a.fattr[i];
+                }
+            }
+            for (int kk = 0; kk < 5; ++kk) statAdd(acc, a.out, live, p, pbase, 3 + kk, kk, k == kk);
         } else {
-            const int p = inRange ? pid[i] : 0;
-            statAdd(acc, out, inRange, p, pbase, 8, 0, inRange && (vflags[i] & VF_FANS) ? 1u : 0u);
+            uint32_t fl = 0;
+            if (live) {
+                fl = a.vflags[i];
+                int best = 0;
+                if (i < n0) {
+                    if (p < 0 || p >= r.B || i < r.startV[p] || i >= r.startV[p + 1]) atomicOr(a.bad, 1);
+                    best = -1;
+                    const int64_t e = a.listOff[i + 1];
+                    for (int64_t q = a.listOff[i]; q < e; ++q) best = max(best, a.list[q]);
+                    if (best >= 0) best -= (int)(4 * r.startQ[p]);
+                }
+                a.vh[d] = best;
+                if (MOVE) {
+                    for (int k = 0; k < 3; ++k) {
+                        a.npos[3 * d + k] = a.pos[3 * i + k];
+                        a.nnrm[3 * d + k] = a.nrm[3 * i + k];
+                    }
+                    a.nvflags[d] = fl;
+                    a.npid[d] = p;
+                }
+            }
+            statAdd(acc, a.out, live, p, pbase, 8, 0, (fl & VF_FANS) != 0);
         }
     }
     __syncthreads();
-    for (int t = threadIdx.x; t < kStatRows * nslots; t += blockDim.x) {
-        const int r = t / nslots, s = t % nslots;
-        const unsigned v = acc[r * 5 + s];
-        if (v) atomicAdd(&out[(int64_t)(pbase + r) * 9 + base + s], (unsigned long long)v);
+    for (int t = threadIdx.x; t < kStatRows * nslots; t += kBlock) {
+        const int row = t / nslots, sl = t % nslots;
+        const unsigned v = acc[row * 5 + sl];
+        if (v) atomicAdd(&a.out[(int64_t)(pbase + row) * 9 + base + sl], (unsigned long long)v);
     }
 }
 
@@ -276,147 +406,152 @@ int32_t* Pipeline::stableSortByKey(const int32_t* key, int64_t n, int B, const s
     return a;
 }
 
-// counts of keys that arrive sorted, into count[k * stride + slot] (k in [0, B))
-void Pipeline::countSorted(const int32_t* key, const int32_t* perm, int64_t n, int B, unsigned long long* count, int stride, int slot) {
-    int64_t* first = arena.get<int64_t>("key_first", (size_t)B + 1);
-    int* bad = arena.get<int>("batch_bad", 1);
-    kKeyStarts<<<gridFor(n + 1), kBlock, 0, stream>>>(key, perm, n, B, first, bad);
-    kCountsFromStarts<<<gridFor(B), kBlock, 0, stream>>>(first, B, count, stride, slot);
-}
-
-void Pipeline::checkBatchKeys() {
-    int bad = 0;
-    MDMC_HIP(hipMemcpyAsync(&bad, arena.get<int>("batch_bad", 1), sizeof(int), hipMemcpyDeviceToHost, stream));
-    MDMC_HIP(hipStreamSynchronize(stream));
-    if (bad) throw HipError("batched form: elements out of problem order", -4);
-}
-
-void Pipeline::problemDmcCounts(int B) {
-    zero(arena.get<int>("batch_bad", 1), sizeof(int));
-    batchDmc.assign(2 * (size_t)B, 0);
-    unsigned long long* cnt = arena.get<unsigned long long>("batch_dmc", 2 * (size_t)B);
-    zero(cnt, 2 * (size_t)B * sizeof(unsigned long long));
-    if (V > 0) countSorted(pid(), nullptr, V, B, cnt, 2, 0);
-    if (Q > 0) {
-        int32_t* qk = arena.get<int32_t>("batch_qkey", (size_t)Q);
-        // a quad's problem is its first vertex's: reuse the halfedge-key kernel on the quads (x = first vertex)
-        kHalfedgeKeys<<<gridFor(Q), kBlock, 0, stream>>>(arena.ptr<int4>("quads"), Q, pid(), qk);
-        countSorted(qk, nullptr, Q, B, cnt, 2, 1);
-    }
-    MDMC_HIP(hipMemcpyAsync(batchDmc.data(), cnt, 2 * (size_t)B * sizeof(int64_t), hipMemcpyDeviceToHost, stream));
-    checkBatchKeys();
-}
-
-// permutation (new -> old) and its inverse for one array of n elements whose first n0
-// are ordered by key; per-key counts go to cnt[4 * b + slot]
-void Pipeline::placeByProblem(const int32_t* key, int64_t n0, int64_t n, int B, const std::string& tag, int32_t** perm, int32_t** inv,
-                              std::vector<int64_t>& off) {
-    *perm = arena.get<int32_t>(tag + "_perm", (size_t)std::max<int64_t>(n, 1));
-    *inv = arena.get<int32_t>(tag + "_inv", (size_t)std::max<int64_t>(n, 1));
-    const int64_t nt = n - n0;
-    const int32_t* tp = stableSortByKey(key + n0, nt, B, tag + "_tail");
-    unsigned long long* cnt = arena.get<unsigned long long>(tag + "_cnt", 2 * (size_t)B);
-    zero(cnt, 2 * (size_t)B * sizeof(unsigned long long));
-    if (n0 > 0) countSorted(key, nullptr, n0, B, cnt, 2, 0);
-    if (nt > 0) countSorted(key + n0, tp, nt, B, cnt, 2, 1);
-    std::vector<unsigned long long> c(2 * (size_t)B);
-    MDMC_HIP(hipMemcpyAsync(c.data(), cnt, c.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, stream));
-    MDMC_HIP(hipStreamSynchronize(stream));
-    std::vector<int64_t> offs(3 * ((size_t)B + 1), 0);
-    for (int b = 0; b < B; ++b) {
-        offs[b + 1] = offs[b] + (int64_t)c[2 * b];
-        offs[(B + 1) + b + 1] = offs[(B + 1) + b] + (int64_t)c[2 * b + 1];
-        offs[2 * (B + 1) + b + 1] = offs[2 * (B + 1) + b] + (int64_t)(c[2 * b] + c[2 * b + 1]);
-    }
-    off.assign(offs.begin() + 2 * (B + 1), offs.end());
-    int64_t* od = arena.get<int64_t>(tag + "_offs", offs.size());
-    upload(od, offs.data(), offs.size() * sizeof(int64_t), 0);
-    if (n > 0) kPlace<<<gridFor(n), kBlock, 0, stream>>>(key, n0, n, tp, od, B, *perm, *inv);
-}
-
 void Pipeline::regroupBatch(int B) {
+    // results the host reads: dmcStart V / Q, offsets V / H / F ([B + 1] each), statistics [9B], bad
+    const size_t nb = (size_t)B, words = 5 * (nb + 1) + 9 * nb + 1;
+    int64_t* res = arena.get<int64_t>("batch_result", words);
+    int64_t* off = res + 2 * (nb + 1);
+    unsigned long long* st = (unsigned long long*)(res + 5 * (nb + 1));
+    int* bad = (int*)(res + 5 * (nb + 1) + 9 * nb);
+    int32_t* runCount = arena.get<int32_t>("rg_runs", 3 * (kMaxRuns + 1));
     {
         FillBatch fb(*this);
         fb.stampAt(stamp(ST_STATS));
-        fb.add(arena.get<int>("batch_bad", 1), 0x00, sizeof(int));
+        fb.add(st, 0x00, (9 * nb + 1) * sizeof(int64_t));
+        fb.add(runCount, 0x00, 3 * sizeof(int32_t));
     }
-    int32_t* vp = pid();
-    int4* he = arena.ptr<int4>("he");
-    int32_t* face_he = arena.ptr<int32_t>("face_he");
-    // quads per problem at the last initialize (for the vertex -> halfedge values)
-    unsigned long long* qc = arena.get<unsigned long long>("batch_qcnt", (size_t)B);
-    zero(qc, (size_t)B * sizeof(unsigned long long));
-    if (vertHeQ > 0) {
-        int32_t* qk = arena.get<int32_t>("batch_qkey", (size_t)vertHeQ);
-        kHalfedgeKeys<<<gridFor(vertHeQ), kBlock, 0, stream>>>(arena.ptr<int4>("quads"), vertHeQ, vp, qk);
-        countSorted(qk, nullptr, vertHeQ, B, qc, 1, 0);
+    StartArgs sa{};
+    sa.probs = probsDev;
+    sa.B = B;
+    sa.slab = gridPassIsSlab(lastShape) ? 1 : 0;
+    sa.vOff = gpVOff_;
+    sa.qOff = gpQOff_;
+    sa.last = gpLast_;
+    const bool compacted = !chain.empty() && dmcQ > 0;
+    sa.address = compacted ? arena.ptr<int32_t>("vaddress") : nullptr;
+    sa.qnew = compacted ? arena.ptr<int32_t>("qnew") : nullptr;
+    sa.dmcV = dmcV;
+    sa.dmcQ = dmcQ;
+    sa.V = vertHeV;
+    sa.Q = vertHeQ;
+    sa.dmcStartV = res;
+    sa.dmcStartQ = res + (nb + 1);
+    sa.startV = arena.get<int64_t>("rg_start", 2 * (nb + 1));
+    sa.startQ = sa.startV + (nb + 1);
+    kProblemStarts<<<gridFor(B + 1), kBlock, 0, stream>>>(sa);
+
+    MoveArgs m{};
+    RegroupArgs& r = m.r;
+    r.he = arena.ptr<int4>("he");
+    r.face_he = arena.ptr<int32_t>("face_he");
+    r.pid = pid();
+    r.B = B;
+    r.n0[RG_V] = std::min(vertHeV, V);
+    r.n0[RG_H] = std::min(4 * vertHeQ, H);
+    r.n0[RG_F] = std::min(vertHeQ, F);
+    r.n[RG_V] = V;
+    r.n[RG_H] = H;
+    r.n[RG_F] = F;
+    r.startV = sa.startV;
+    r.startQ = sa.startQ;
+    r.shift = arena.get<int64_t>("rg_shift", 3 * nb);
+    r.runCount = runCount;
+    r.runList = runCount + 3;
+    Runs u{};
+    int32_t* first = nullptr;
+    int64_t tail = 0;
+    for (int k = 0; k < 3; ++k) tail += r.n[k] - r.n0[k];
+    if (tail > 0) {
+        static const char* keyName[3] = {"rg_key_v", "rg_key_h", "rg_key_f"};
+        static const char* dstName[3] = {"rg_dst_v", "rg_dst_h", "rg_dst_f"};
+        for (int k = 0; k < 3; ++k) {
+            r.tailKey[k] = arena.get<int32_t>(keyName[k], (size_t)(r.n[k] - r.n0[k]));
+            r.tailDst[k] = arena.get<int32_t>(dstName[k], (size_t)(r.n[k] - r.n0[k]));
+        }
+        kTailKeys<<<gridFor(tail), kBlock, 0, stream>>>(r);
+        int32_t* hr = (int32_t*)pinBatch(3 * (kMaxRuns + 1) * sizeof(int32_t));
+        MDMC_HIP(hipMemcpyAsync(hr, runCount, 3 * (kMaxRuns + 1) * sizeof(int32_t), hipMemcpyDeviceToHost, stream));
+        MDMC_HIP(hipStreamSynchronize(stream));
+        for (int k = 0; k < 3; ++k) {
+            const int32_t n = (int32_t)(r.n[k] - r.n0[k]);
+            u.count[k] = 1;
+            if (hr[k] < kMaxRuns) {
+                u.count[k] = hr[k] + 1;
+                int32_t* l = hr + 3 + k * kMaxRuns;
+                std::sort(l, l + hr[k]);
+                for (int s = 0; s < hr[k]; ++s) u.start[k][s + 1] = l[s];
+            } else {
+                static const char* tag[3] = {"rg_sort_v", "rg_sort_h", "rg_sort_f"};
+                u.order[k] = stableSortByKey(r.tailKey[k], n, B, tag[k]);
+            }
+            u.start[k][u.count[k]] = n;
+        }
+        first = arena.get<int32_t>("rg_first", (size_t)3 * kMaxRuns * (nb + 1));
+        kRunStarts<<<gridFor(tail), kBlock, 0, stream>>>(r, u, first, bad);
     }
-    int32_t* vhInit = arena.get<int32_t>("batch_vh_init", (size_t)std::max<int64_t>(vertHeV, 1));
-    if (vertHeV > 0) kVertexHalfedgeInitBatch<<<gridFor(vertHeV), kBlock, 0, stream>>>(vhInit, vertHeV);
-    if (vertHeQ > 0) kVertexHalfedgeMax<<<gridFor(vertHeQ), kBlock, 0, stream>>>(arena.ptr<int4>("quads"), vertHeQ, vhInit);
-    std::vector<unsigned long long> qcount((size_t)B);
-    MDMC_HIP(hipMemcpyAsync(qcount.data(), qc, (size_t)B * sizeof(unsigned long long), hipMemcpyDeviceToHost, stream));
-    // keys; the elements that existed at the last initialize come first, in problem order
-    int32_t* hk = arena.get<int32_t>("batch_hkey", (size_t)std::max<int64_t>(H, 1));
-    int32_t* fk = arena.get<int32_t>("batch_fkey", (size_t)std::max<int64_t>(F, 1));
-    if (H > 0) kHalfedgeKeys<<<gridFor(H), kBlock, 0, stream>>>(he, H, vp, hk);
-    if (F > 0) kFaceKeys2<<<gridFor(F), kBlock, 0, stream>>>(he, face_he, F, vp, fk);
-    int32_t *pv, *ph, *pf, *vNew, *hNew, *fNew;
-    placeByProblem(vp, std::min(vertHeV, V), V, B, "sv", &pv, &vNew, batchVOff);
-    placeByProblem(hk, std::min(4 * vertHeQ, H), H, B, "sh", &ph, &hNew, batchHOff);
-    placeByProblem(fk, std::min(vertHeQ, F), F, B, "sf", &pf, &fNew, batchFOff);
-    std::vector<int64_t> qBase((size_t)B + 1, 0);
-    for (int b = 0; b < B; ++b) qBase[b + 1] = qBase[b] + (int64_t)qcount[b];
-    int64_t* qBaseDev = arena.get<int64_t>("batch_qbase", (size_t)B + 1);
-    upload(qBaseDev, qBase.data(), qBase.size() * sizeof(int64_t), 1);
-    float* npos = arena.get<float>("pos2", 3 * (size_t)std::max<int64_t>(V, 1));
-    float* nnrm = arena.get<float>("nrm2", 3 * (size_t)std::max<int64_t>(V, 1));
-    uint32_t* nvf = arena.get<uint32_t>("vflags2", (size_t)std::max<int64_t>(V, 1));
-    int32_t* npid = arena.get<int32_t>("pid2", (size_t)std::max<int64_t>(V, 1));
-    int4* nhe = arena.get<int4>("he2", (size_t)std::max<int64_t>(H, 1));
-    int32_t* nbs = arena.get<int32_t>("bsize2", (size_t)std::max<int64_t>(H, 1));
-    int32_t* nbr = arena.get<int32_t>("brank2", (size_t)std::max<int64_t>(H, 1));
-    int32_t* nfh = arena.get<int32_t>("face_he2", (size_t)std::max<int64_t>(F, 1));
-    uint32_t* nfa = arena.get<uint32_t>("fattr2", (size_t)std::max<int64_t>(F, 1));
-    if (V > 0)
-        kPermuteVertices<<<gridFor(V), kBlock, 0, stream>>>(pv, V, arena.ptr<float>("pos"), arena.ptr<float>("nrm"), arena.ptr<uint32_t>("vflags"), vp, npos,
-                                                            nnrm, nvf, npid);
-    if (H > 0)
-        kPermuteHalfedges<<<gridFor(H), kBlock, 0, stream>>>(ph, H, he, arena.ptr<int32_t>("bsize"), arena.ptr<int32_t>("brank"), vNew, hNew, fNew, nhe,
-                                                             nbs, nbr);
-    if (F > 0) kPermuteFaces<<<gridFor(F), kBlock, 0, stream>>>(pf, F, face_he, arena.ptr<uint32_t>("fattr"), hNew, nfh, nfa);
-    int32_t* vh = arena.get<int32_t>("batch_vert_he", (size_t)std::max<int64_t>(V, 1));
-    if (V > 0) kVertexHalfedgeLocal<<<gridFor(V), kBlock, 0, stream>>>(vhInit, vertHeV, vNew, npid, qBaseDev, V, vh);
-    auto back = [&](const char* name, const void* src, size_t bytes) {
-        if (bytes) MDMC_HIP(hipMemcpyAsync(arena.ptr<char>(name), src, bytes, hipMemcpyDeviceToDevice, stream));
-    };
-    back("pos", npos, 3 * (size_t)V * sizeof(float));
-    back("nrm", nnrm, 3 * (size_t)V * sizeof(float));
-    back("vflags", nvf, (size_t)V * sizeof(uint32_t));
-    back("pid", npid, (size_t)V * sizeof(int32_t));
-    back("he", nhe, (size_t)H * sizeof(int4));
-    back("bsize", nbs, (size_t)H * sizeof(int32_t));
-    back("brank", nbr, (size_t)H * sizeof(int32_t));
-    back("face_he", nfh, (size_t)F * sizeof(int32_t));
-    back("fattr", nfa, (size_t)F * sizeof(uint32_t));
+    kOffsets<<<1, 1024, 0, stream>>>(r, u, first, off);
+    if (tail > 0) kTailPlaces<<<gridFor(tail), kBlock, 0, stream>>>(r, u, first);
+    m.pos = arena.ptr<float>("pos");
+    m.nrm = arena.ptr<float>("nrm");
+    m.vflags = arena.ptr<uint32_t>("vflags");
+    m.fattr = arena.ptr<uint32_t>("fattr");
+    m.bsize = arena.ptr<int32_t>("bsize");
+    m.brank = arena.ptr<int32_t>("brank");
+    m.canon = canonFlags();
+    m.listOff = arena.ptr<int64_t>("out_off");
+    m.list = arena.ptr<int32_t>("out_list");
+    m.out = st;
+    m.bad = bad;
+    const size_t nv = (size_t)std::max<int64_t>(V, 1), nh = (size_t)std::max<int64_t>(H, 1), nf = (size_t)std::max<int64_t>(F, 1);
+    m.vh = arena.get<int32_t>("batch_vert_he", nv);
+    auto chunks = [](int64_t n) { return (unsigned)((n + statChunk(n) - 1) / statChunk(n)); };
+    if (tail > 0) {
+        m.npos = arena.get<float>("pos2", 3 * nv);
+        m.nnrm = arena.get<float>("nrm2", 3 * nv);
+        m.nvflags = arena.get<uint32_t>("vflags2", nv);
+        m.npid = arena.get<int32_t>("pid2", nv);
+        m.nhe = arena.get<int4>("he2", nh);
+        m.nbsize = arena.get<int32_t>("bsize2", nh);
+        m.nbrank = arena.get<int32_t>("brank2", nh);
+        m.nface_he = arena.get<int32_t>("face_he2", nf);
+        m.nfattr = arena.get<uint32_t>("fattr2", nf);
+        if (H > 0) kRegroup<RG_H, true><<<chunks(H), kBlock, 0, stream>>>(m, statChunk(H));
+        if (F > 0) kRegroup<RG_F, true><<<chunks(F), kBlock, 0, stream>>>(m, statChunk(F));
+        if (V > 0) kRegroup<RG_V, true><<<chunks(V), kBlock, 0, stream>>>(m, statChunk(V));
+        for (const char* name : {"pos", "nrm", "vflags", "pid", "he", "bsize", "brank", "face_he", "fattr"}) arena.swap(name, std::string(name) + "2");
+    } else {
+        if (H > 0) kRegroup<RG_H, false><<<chunks(H), kBlock, 0, stream>>>(m, statChunk(H));
+        if (F > 0) kRegroup<RG_F, false><<<chunks(F), kBlock, 0, stream>>>(m, statChunk(F));
+        if (V > 0) kRegroup<RG_V, false><<<chunks(V), kBlock, 0, stream>>>(m, statChunk(V));
+    }
     batchVertHe = true;
-    // per-problem statistics
-    unsigned long long* st = arena.get<unsigned long long>("batch_stats", 9 * (size_t)B);
-    zero(st, 9 * (size_t)B * sizeof(unsigned long long));
-    {
-        const int4* h4 = arena.ptr<int4>("he");
-        const int32_t* fh = arena.ptr<int32_t>("face_he");
-        const int32_t* bs = arena.ptr<int32_t>("bsize");
-        const int32_t* br = arena.ptr<int32_t>("brank");
-        const uint32_t* vf = arena.ptr<uint32_t>("vflags");
-        auto chunks = [](int64_t n) { return (unsigned)((n + kStatChunk - 1) / kStatChunk); };
-        if (H > 0) kStatsBatch<0><<<chunks(H), kBlock, 0, stream>>>(h4, fh, bs, br, vf, pid(), H, st);
-        if (F > 0) kStatsBatch<1><<<chunks(F), kBlock, 0, stream>>>(h4, fh, bs, br, vf, pid(), F, st);
-        if (V > 0) kStatsBatch<2><<<chunks(V), kBlock, 0, stream>>>(h4, fh, bs, br, vf, pid(), V, st);
+    kStamp<<<1, 1, 0, stream>>>(stamp(ST_END));
+    const int64_t* h = (const int64_t*)pinBatch(words * sizeof(int64_t));
+    MDMC_HIP(hipMemcpyAsync((void*)h, res, words * sizeof(int64_t), hipMemcpyDeviceToHost, stream));
+    const int64_t* ctr = readCounters();
+    if (initUnchecked || refreshUnchecked) checkNM(ctr);
+    if (*(const int*)(h + 5 * (nb + 1) + 9 * nb)) throw HipError("batched form: elements out of problem order", -4);
+    batchDmc.resize(2 * nb);
+    for (size_t b = 0; b < nb; ++b) {
+        batchDmc[2 * b] = h[b + 1] - h[b];
+        batchDmc[2 * b + 1] = h[(nb + 1) + b + 1] - h[(nb + 1) + b];
     }
-    batchStats.assign(9 * (size_t)B, 0);
-    MDMC_HIP(hipMemcpyAsync(batchStats.data(), st, batchStats.size() * sizeof(int64_t), hipMemcpyDeviceToHost, stream));
-    checkBatchKeys();
+    batchVOff.assign(h + 2 * (nb + 1), h + 3 * (nb + 1));
+    batchHOff.assign(h + 3 * (nb + 1), h + 4 * (nb + 1));
+    batchFOff.assign(h + 4 * (nb + 1), h + 5 * (nb + 1));
+    batchStats.assign(h + 5 * (nb + 1), h + 5 * (nb + 1) + 9 * nb);
+}
+
+// pinned host memory for a batch's results
+void* Pipeline::pinBatch(size_t bytes) {
+    if (pinBatchCap_ < bytes) {
+        if (pinBatch_) MDMC_HIP(hipHostFree(pinBatch_));
+        pinBatch_ = nullptr;
+        pinBatchCap_ = 0;
+        MDMC_HIP(hipHostMalloc(&pinBatch_, bytes + bytes / 2, hipHostMallocDefault));
+        pinBatchCap_ = bytes + bytes / 2;
+    }
+    return pinBatch_;
 }
 
 }  // namespace mdmc

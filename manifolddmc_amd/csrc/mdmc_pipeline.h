@@ -74,7 +74,6 @@ class Pipeline {
     // batch's regroup, the counters, statistics and stage clocks go to pinned memory in one
     // read-back; the getters below read that copy
     void finishSingle(bool doSplit, int step, int maxIters, bool doDetect, int64_t st9[9]);
-    void finishBatch();
     void finishEmpty();
     void counterTotals(int64_t* anomalyCount, int64_t* mergeSeq, int64_t* lookbackDirect);
     // stage times in ms, from the clock stamps of the stages' first kernels: whole call, then the
@@ -117,10 +116,9 @@ class Pipeline {
     // per vertex its problem (several problems), else nullptr
     int32_t* pid();
 
-    // batched form (mdmc_batch.hip): per-problem DMC vertex / quad counts right after the
-    // grid pass, then the final regroup into contiguous per-problem ranges with offsets,
-    // per-problem vertex -> halfedge values and statistics
-    void problemDmcCounts(int B);
+    // batched form (mdmc_batch.hip): the final regroup into contiguous per-problem ranges with
+    // offsets, per-problem vertex -> halfedge values, DMC counts and statistics; ends the
+    // extraction (one read-back of all of it and the counters)
     void regroupBatch(int B);
     std::vector<int64_t> batchDmc;                     // [2B]: vertices, quads
     std::vector<int64_t> batchVOff, batchHOff, batchFOff;  // [B + 1]
@@ -249,10 +247,12 @@ class Pipeline {
     void finishChain();
     void buildMergeList(const int2* rec, int64_t R, int count, int32_t* num, int32_t* ex, int32_t* ey, const std::string& tag);
     int32_t* stableSortByKey(const int32_t* key, int64_t n, int B, const std::string& tag);
-    void countSorted(const int32_t* key, const int32_t* perm, int64_t n, int B, unsigned long long* count, int stride, int slot);
-    void checkBatchKeys();
-    void placeByProblem(const int32_t* key, int64_t n0, int64_t n, int B, const std::string& tag, int32_t** perm, int32_t** inv,
-                        std::vector<int64_t>& off);
+    void* pinBatch(size_t bytes);
+    void* pinBatch_ = nullptr;
+    size_t pinBatchCap_ = 0;
+    // the last grid pass's vertex / quad offsets by tile or row segment, and their last index
+    const int64_t *gpVOff_ = nullptr, *gpQOff_ = nullptr;
+    int64_t gpLast_ = 0;
 };
 
 }  // namespace mdmc

@@ -2600,8 +2600,6 @@ __global__ void __launch_bounds__(kBlock) kStats(const int4* __restrict__ he, in
     if (threadIdx.x == 0) pin[A_STAMP + ST_END] = wall_clock64();
 }
 
-// the clock alone, where no kernel begins or ends a stage
-__global__ void kStamp(int64_t* stamp) { *stamp = wall_clock64(); }
 
 // The resident mesh into the caller's device buffers, every array in one launch: block b works
 // on the array j with start[j] <= b < start[j + 1], kCopyPer * kBlock of its items (16 bytes of
@@ -2689,6 +2687,7 @@ Pipeline::~Pipeline() {
     for (auto& e : kev)
         if (e) (void)hipEventDestroy(e);
     if (pinH_) (void)hipHostFree(pinH_);
+    if (pinBatch_) (void)hipHostFree(pinBatch_);
     for (auto& e : upEv_)
         if (e) (void)hipEventSynchronize(e), (void)hipEventDestroy(e);
     for (void* u : up_)
@@ -3004,6 +3003,9 @@ void Pipeline::slabPass(std::vector<ProblemDev>& problems, int64_t C, int shape,
     V = h[1];
     Q = h[2];
     emitArgs(a, C, recordAdjoint);
+    gpVOff_ = svo;
+    gpQOff_ = sqo;
+    gpLast_ = segs;
     tuneEvent(2);
     launchSlabEmit(shape, a, stream);
     tuneEvent(3);
@@ -3234,6 +3236,9 @@ void Pipeline::gridPassBack(std::vector<ProblemDev>& problems, int64_t C, int sh
     V = h[1];
     Q = h[2];
     emitArgs(a, C, recordAdjoint);
+    gpVOff_ = a.tileVOff;
+    gpQOff_ = a.tileQOff;
+    gpLast_ = a.numTiles;
     tuneEvent(2);
     launchGridEmit(shape, a, stream);
     tuneEvent(3);
@@ -3965,12 +3970,6 @@ const int64_t* Pipeline::waitStats() {
 void Pipeline::finishEmpty() {
     launchStats(0);
     waitStats();
-}
-
-void Pipeline::finishBatch() {
-    kStamp<<<1, 1, 0, stream>>>(stamp(ST_END));
-    const int64_t* h = readCounters();
-    if (h[A_INVALID]) checkNM(h);
 }
 
 void Pipeline::copyOut(float* positions, float* normals, int32_t* halfedges, int32_t* face_halfedge, uint16_t* face_attr, uint8_t* vertex_flags,
