@@ -685,13 +685,21 @@ __global__ void __launch_bounds__(kBlock) kSources(const int32_t* __restrict__ v
 // vertices on that vertex's chain, counted (every list by current corner: list lengths less the
 // halfedges of removed quads, removedAt; after deferred steps: the out-degree kept through the
 // chain's removals and drops), then written with their new ids (the bucket pass checks every
-// entry it reads against the quad's corner)
+// entry it reads against the quad's corner).  The counting pass also moves the vertex's
+// position and normal (each new vertex gathers its old one's: 173 us at the 512^3 gyroid with the
+// count; scattered by old vertex instead 252 us alone, inside kNumber's rounds 255 us)
 __global__ void kOutCount(const int32_t* __restrict__ oldV, int64_t Vn, const int64_t* __restrict__ off, const int32_t* __restrict__ removedAt,
                           const int32_t* __restrict__ srcHead, const int32_t* __restrict__ srcNext, const int32_t* __restrict__ outdeg,
-                          int32_t* __restrict__ cnt) {
+                          int32_t* __restrict__ cnt, const float* __restrict__ pos, const float* __restrict__ nrm, float* __restrict__ npos,
+                          float* __restrict__ nnrm) {
     const int64_t vn = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (vn >= Vn) return;
     int u = oldV[vn];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        npos[3 * vn + k] = pos[3 * (int64_t)u + k];
+        nnrm[3 * vn + k] = nrm[3 * (int64_t)u + k];
+    }
     if (outdeg) {
         cnt[vn] = outdeg[u];
         return;
@@ -1543,7 +1551,7 @@ __global__ void kMark3333(const int4* __restrict__ quads, const int32_t* __restr
 // block ranks, look-back over the own kind's tiles).
 // A vertex is kept unless it is dropped by this step (vtype == dropType) or died in an earlier
 // step of the chain; every vertex gets its new address (-1 when dropped) and the kept ones
-// their old id, position, normal and problem.  A quad is kept without remove or dead bit (qnew, -1
+// their old id and problem.  A quad is kept without remove or dead bit (qnew, -1
 // otherwise).  The arrays the following kernels start from (touched, flags, the list lengths' end;
 // the chain heads and removal counts of a chain of one) are cleared along the way.
 struct NumberArgs {
@@ -1552,9 +1560,7 @@ struct NumberArgs {
     int dropType;
     const uint8_t* vdead;
     const int32_t* pid;
-    const float *pos, *nrm;
     int32_t *npid, *address, *oldV;
-    float *npos, *nnrm;
     uint8_t* touched;
     uint32_t* vflags;
     int32_t *cnt, *srcHead, *removedAt;
@@ -1622,10 +1628,6 @@ __global__ void __launch_bounds__(kLbBlock) kNumber(NumberArgs a) {
         if (a.removedAt) a.removedAt[e] = 0;
         if (!keep) continue;
         a.oldV[o] = (int32_t)e;
-        for (int k = 0; k < 3; ++k) {
-            a.npos[3 * o + k] = a.pos[3 * e + k];
-            a.nnrm[3 * o + k] = a.nrm[3 * e + k];
-        }
         a.touched[o] = 0;
         a.vflags[o] = 0;
         if (a.pid) a.npid[o] = a.pid[e];
@@ -3478,8 +3480,11 @@ void Pipeline::launchCompaction() {
     const uint32_t* attr = p3333 ? arena.ptr<uint32_t>("fattr") : arena.ptr<uint32_t>("qattr");
     // vertex and quad compaction, each one pass (look-back over tiles), with one read-back of
     // both totals; the outputs are sized for the inputs (at most as many are kept)
-    constexpr int R = 16;  // rounds per tile (tiles of 4096 elements)
-    const int64_t tV = (V + R * kLbBlock - 1) / (R * kLbBlock), tQ = (Q + R * kLbBlock - 1) / (R * kLbBlock);
+    // tiles of 4096 elements, or 1024 where that leaves the chip with fewer than a block per CU
+    // (long look-back chains cost more than they give on large meshes: 0.11 / 0.41 -> 0.18 /
+    // 0.48 ms at 17 M elements; 110 k vertices and quads: 38 -> 12 us)
+    const int R = V + Q < (int64_t)1024 * 16 * kLbBlock ? 4 : 16;
+    const int64_t tile = (int64_t)R * kLbBlock, tV = (V + tile - 1) / tile, tQ = (Q + tile - 1) / tile;
     int32_t* address = arena.get<int32_t>("vaddress", (size_t)std::max<int64_t>(V, 1));  // written for every vertex below
     // the compacted arrays go to the second buffers, which then swap with the primary ones;
     // both are sized for the grid pass's output so that later extractions of the same
@@ -3487,8 +3492,8 @@ void Pipeline::launchCompaction() {
     const size_t capV = (size_t)std::max(V, dmcV), capQ = (size_t)std::max(Q, dmcQ);
     int32_t* npid = pid() ? arena.get<int32_t>("pid2", capV) : nullptr;
     int32_t* oldV = arena.get<int32_t>("oldV", (size_t)std::max<int64_t>(V, 1));
-    float* npos = arena.get<float>("pos2", 3 * capV);
-    float* nnrm = arena.get<float>("nrm2", 3 * capV);
+    arena.get<float>("pos2", 3 * capV);
+    arena.get<float>("nrm2", 3 * capV);
     int4* quads = arena.ptr<int4>("quads");
     int4* nquads = arena.get<int4>("quads2", capQ);
     uint32_t* nattr = arena.get<uint32_t>("qattr2", capQ);
@@ -3517,10 +3522,6 @@ void Pipeline::launchCompaction() {
         na.dropType = dropType;
         na.vdead = chained ? arena.ptr<uint8_t>("vdead") : nullptr;
         na.pid = pid();
-        na.pos = arena.ptr<float>("pos");
-        na.nrm = arena.ptr<float>("nrm");
-        na.npos = npos;
-        na.nnrm = nnrm;
         na.npid = npid;
         na.address = address;
         na.oldV = oldV;
@@ -3543,7 +3544,8 @@ void Pipeline::launchCompaction() {
         na.directOut = lookbackDiag();
         na.step = step;
         na.ctr = counters();
-        if (tV + tQ > 0) kNumber<R><<<(unsigned)(tV + tQ), kLbBlock, 0, stream>>>(na);
+        if (R == 4) kNumber<4><<<(unsigned)(tV + tQ), kLbBlock, 0, stream>>>(na);
+        else kNumber<16><<<(unsigned)(tV + tQ), kLbBlock, 0, stream>>>(na);
     }
     if (Q > 0)
         kCompactQuads<<<gridFor(Q), kBlock, 0, stream>>>(quads, attr, Q, vtarget, address, p3333 ? 1 : 0, nquads, nattr, nfattr, face_he, oldQ, qnew,
@@ -3581,7 +3583,8 @@ void Pipeline::finishChain() {
     if (V > 0) kSources<<<sparseBlocks(V), kBlock, 0, stream>>>(vtype, vtarget, address, V, dropType, touched, srcHead, srcNext, outdeg);
     const int64_t* off = arena.ptr<int64_t>("out_off");
     const int32_t* out = arena.ptr<int32_t>("out_list");
-    if (nV > 0) kOutCount<<<gridFor(nV), kBlock, 0, stream>>>(oldV, nV, off, removedAt, srcHead, srcNext, outdeg, cnt);
+    if (nV > 0) kOutCount<<<gridFor(nV), kBlock, 0, stream>>>(oldV, nV, off, removedAt, srcHead, srcNext, outdeg, cnt, arena.ptr<float>("pos"),
+                                                           arena.ptr<float>("nrm"), arena.ptr<float>("pos2"), arena.ptr<float>("nrm2"));
     int64_t* off2 = arena.get<int64_t>("out_off2", (size_t)std::max<int64_t>(nV, dmcV) + 1);
     scan(cnt, off2, nV + 1);
     int32_t* out2 = arena.get<int32_t>("out_list2", 4 * capQ);
