@@ -170,7 +170,6 @@ class Pipeline {
     int64_t* counters();
     int64_t* nmSlotParts();
     int64_t* nmFoundParts();
-    int64_t scan32(const int32_t* in, int64_t n, const std::string& outName, int64_t** out);
     // exclusive prefix sums in one launch (words of the jobs are set here); total may be null
     void scan(std::initializer_list<ScanJob> jobs, int64_t* stampStart = nullptr, int64_t* stampEnd = nullptr);
     void scan(const int32_t* in, int64_t* out, int64_t n, int64_t* total = nullptr) { scan({ScanJob{in, out, n, total, nullptr}}); }
@@ -193,7 +192,6 @@ class Pipeline {
     void detectSlow(int64_t nSlow, int64_t nSlowOff);
     void launchStats(int guarded);
     const int64_t* waitStats();
-    int64_t touchedV = 0;  // vertices the splitter's touched flags cover
     void zero(void* p, size_t bytes);
     void fillNeg(void* p, size_t bytes);
     void launchFill(void* p, uint8_t byte, size_t bytes);
@@ -211,12 +209,12 @@ class Pipeline {
         FillSet fs;
         unsigned blocks = 0;
     };
-    // the splitter's old -> copy maps: -1 on [0, clean) between steps (each step resets the
+    // the splitter's old -> copy maps and last copies: -1 on [0, clean) between steps (each step resets the
     // entries it set); a map the arena reallocated, or one a failed step left dirty, is filled
     struct WcMap {
         void* ptr = nullptr;
         int64_t clean = 0, cap = 0;
-    } wcMaps[3];
+    } wcMaps[4];
     bool wcMapsDirty = true;
     void gridPass(std::vector<ProblemDev>& problems, int64_t C, int shape, bool surfIter, bool recordAdjoint);
     void slabPass(std::vector<ProblemDev>& problems, int64_t C, int shape, bool surfIter, bool recordAdjoint);
@@ -232,8 +230,7 @@ class Pipeline {
     GridPassArgs fgArgs_{};
     std::vector<int64_t> fgLastEager_;
     std::vector<int64_t> frontBuffers();
-    void buildBuckets(const int32_t* list, int64_t n);
-    void refreshHashTable(const uint8_t* dirtyV, int64_t oldH);
+    void refreshHashTable(size_t Vm, size_t Hm, size_t Fm);
     // a refresh ran whose face-walk check (the invalid-record counter) is not read back yet
     bool refreshUnchecked = false;
     void checkValid(const char* what);
@@ -245,7 +242,6 @@ class Pipeline {
     void launchCompaction();
     void rebuildRegion();
     void finishChain();
-    void buildMergeList(const int2* rec, int64_t R, int count, int32_t* num, int32_t* ex, int32_t* ey, const std::string& tag);
     int32_t* stableSortByKey(const int32_t* key, int64_t n, int B, const std::string& tag);
     void* pinBatch(size_t bytes);
     void* pinBatch_ = nullptr;

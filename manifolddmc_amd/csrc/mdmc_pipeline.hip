@@ -38,7 +38,7 @@ constexpr int kFanGuard = 4096;
 
 // ---------------------------------------------------------------- counters
 enum : int { A_ANOMALY = 0, A_CONFLICT = 1, A_INVALID = 2, A_DIRTY = 3, A_FALLBACK = 4 /* two steps */, A_MERGE_SEQ = 6, A_LB_DIRECT = 7,
-             A_NM = 8, A_NSLOW = 9, A_NSLOW_OFF = 10, A_PIN = 11, A_STAMP = 12, A_STATS = A_STAMP + ST_COUNT, A_TICKET = A_STATS + 9, A_NCOUNTERS };
+             A_NM = 8, A_NSLOW = 9, A_NSLOW_OFF = 10, A_PIN = 11, A_NCOL = 12, A_ADD = 13 /* three */, A_STAMP = 16, A_STATS = A_STAMP + ST_COUNT, A_TICKET = A_STATS + 9, A_NCOUNTERS };
 // the slotted non-manifold halfedges the split's working copy marks (markHalfedgesAsNonManifold,
 // ManifoldSplitter.cu:527-555, reads the four slots of every full vertex-pair bucket): every
 // halfedge of a bucket of 4, and of a larger bucket the ones at ranks 1, 2, 3 and size - 1
@@ -157,12 +157,11 @@ constexpr int kPinSpecial = 3, kPinInvalid = 4, kPinFallback = 5 /* two steps */
 static_assert(kPinFinal + A_NCOUNTERS <= Pipeline::kPinSlots, "pinned words");
 
 // ---------------------------------------------------------------- halfedge construction
-// bucket order after refreshHashTable: (face, position along the face from its first halfedge)
-// and ResetFaceFlags (refreshFaceFlagsGPU) ahead of the NM bits the bucket pass sets again
-// refreshHashTable's per-face part: the face's first halfedge must be a halfedge id, and
+// bucket order after refreshHashTable: (face, position along the face from its first halfedge).
+// refreshHashTable's per-face part, ResetFaceFlags (refreshFaceFlagsGPU) ahead of the NM bits the
+// bucket pass sets again: the face's first halfedge must be a halfedge id, and
 // the pattern / remove / NM bits are cleared (NM is set again from the bucket sizes)
-__global__ void kFaceClear(const int32_t* __restrict__ face_he, int64_t F, int64_t H, uint32_t* __restrict__ fattr, int64_t* ctr) {
-    const int64_t f0 = firstOfFour();
+__device__ void clearFaces(int64_t f0, const int32_t* __restrict__ face_he, int64_t F, int64_t H, uint32_t* __restrict__ fattr, int64_t* ctr) {
     if (f0 >= F) return;
     constexpr uint32_t keep = ~(uint32_t)(QA_PATTERN | QA_REMOVE | QA_NM);
     int bad = 0;
@@ -205,8 +204,16 @@ __device__ __forceinline__ int entryOther(int x) { return x & 0x7FFFFFFF; }
 // come from the keys.
 constexpr int kDirtyPer = 16;
 constexpr int kDirtyBatch = 4;
-__global__ void __launch_bounds__(kBlock) kDirtyRecords(const int4* __restrict__ he, int64_t H, int64_t oldH, int64_t F, int64_t V,
-                                                        const uint8_t* __restrict__ dirtyV, int32_t* __restrict__ dlist, int64_t* ctr) {
+// The blocks from recordBlocks on clear the faces' bits.  The sizes are those before the step plus
+// what it appended, which the host does not know yet (the launch covers the most it can be).
+__global__ void __launch_bounds__(kBlock) kDirtyRecords(const int4* __restrict__ he, int64_t oldH, int64_t oldF, int64_t oldV,
+                                                        const uint8_t* __restrict__ dirtyV, int32_t* __restrict__ dlist, int64_t recordBlocks,
+                                                        const int32_t* __restrict__ face_he, uint32_t* __restrict__ fattr, int64_t* ctr) {
+    const int64_t V = oldV + ctr[A_ADD], H = oldH + ctr[A_ADD + 1], F = oldF + ctr[A_ADD + 2];
+    if ((int64_t)blockIdx.x >= recordBlocks) {
+        clearFaces(4 * (((int64_t)blockIdx.x - recordBlocks) * kBlock + threadIdx.x), face_he, F, H, fattr, ctr);
+        return;
+    }
     __shared__ int s_list[kBlock * kDirtyPer];
     __shared__ int s_n;
     __shared__ long long s_base;
@@ -1886,19 +1893,81 @@ struct WC {
     int32_t *f_c2o, *f_o2c;
     int32_t* pid;  // per vertex its problem (several problems), else nullptr
     // the old vertex and halfedge of each corner slot as kWcCopy took them (4n): the entries
-    // of the old -> copy maps that the step sets, reset to -1 by kWcUndo at the step's end
+    // of the old -> copy maps that the step sets, reset to -1 by kCopyBack at the step's end
     int32_t *v_orig, *h_orig;
+    // per old vertex the last copy of it that survives (-1 between steps, as the maps)
+    int32_t* v_last;
     int n;
 };
+
+// What a split step carries between its launches besides the working copy.  The step was some 50
+// launches with three waits; its passes are independent of each other in groups, so each
+// group is one launch (blocks take ranges of vertices, halfedges and faces), the arrays are
+// grown for the most the step can append (4n vertices, 16n halfedges, 4n faces) before it
+// starts, and the host waits once, for the sizes with the refresh's dirty list: 20 launches.
+// 128^3 lattice (640 faces, one step): 963 us an extraction before, 811 us now; 201x77x131 gyroid
+// (7 k faces) 628 and 493; batch of 16 with few dozen faces 680 and 554.
+struct SplitStep {
+    WC w;
+    int step, vsize, hsize, fsize;
+    // merge marks: vertices and halfedges; records in call order, per target a count, a cursor, its
+    // offset and its records, then the ivec2 the reference keeps
+    int2 *vrec, *hrec;
+    int32_t *cntV, *curV, *idxV, *cntH, *curH, *idxH;
+    int64_t *offV, *offH;
+    int32_t *numV, *exV, *eyV, *numH, *exH, *eyH;
+    int32_t *valid, *firstWriter;  // [hsize], [2 hsize]
+    int32_t *newV, *newH, *newF;   // 1: the copy back appends this element
+    int64_t *addrV, *addrH, *addrF;
+    int64_t V0, H0, F0;
+    int64_t* ctr;
+};
+// block b of a launch over ranges of n0, n1, n2 threads: the range and the thread's index in it
+__device__ __forceinline__ int rangeOf(int n0, int n1, int n2, int& i) {
+    int b = blockIdx.x;
+    const int g0 = (n0 + kBlock - 1) / kBlock, g1 = (n1 + kBlock - 1) / kBlock;
+    int r = 0;
+    if (b >= g0) b -= g0, r = 1;
+    if (r == 1 && b >= g1) b -= g1, r = 2;
+    i = b * kBlock + threadIdx.x;
+    return i < (r == 0 ? n0 : (r == 1 ? n1 : n2)) ? r : 3;
+}
+inline unsigned rangeBlocks(int64_t n0, int64_t n1, int64_t n2) { return gridFor(n0) + gridFor(n1) + gridFor(n2); }
 
 // copyVerticesToWorkingCopy / copyHalfedgesToWorkingCopy / copyFacesToWorkingCopy (ManifoldSplitter.cu:307-457),
 // one thread per face corner: thread 4r + i copies the i-th halfedge of face nm[r] and its
 // origin into slot c = 4r + i, so the copies' stores are consecutive across lanes
+// (flags start at 0: WorkingCopy ignores its initialFlags argument); the threads also start the
+// rest of the step's arrays, 2 vertices, 5 halfedges and up to 2 faces each
 __global__ void kWcCopy(const int32_t* __restrict__ nm, int n, const int4* __restrict__ he, const int32_t* __restrict__ face_he,
                         const uint32_t* __restrict__ fattr, const float* __restrict__ pos, const float* __restrict__ nrm,
-                        const int32_t* __restrict__ pid, WC w) {
+                        const int32_t* __restrict__ pid, SplitStep s) {
+    const WC& w = s.w;
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= 4 * n) return;
+    for (int k = 0; k < 2; ++k) {
+        const int v = c + 4 * n * k;
+        w.vflags[v] = 0;
+        if (k) w.v_c2o[v] = -1;
+        s.cntV[v] = 0;
+        s.curV[v] = 0;
+    }
+    for (int k = 0; k < 5; ++k) {
+        const int h = c + 4 * n * k;
+        w.hflags[h] = 0;
+        if (k) w.h_c2o[h] = -1;
+        s.cntH[h] = 0;
+        s.curH[h] = 0;
+        s.firstWriter[h] = INT32_MAX;  // atomicMin targets
+        s.firstWriter[s.hsize + h] = 0;  // write counts
+    }
+    w.fflags[c] = 0;
+    if (c >= n) w.f_c2o[c] = -1;
+    if (c < n) {
+        w.fflags[4 * n + c] = 0;
+        w.f_c2o[4 * n + c] = -1;
+    }
+    if (c == 0) s.cntV[8 * n] = s.cntH[20 * n] = 0;
     const int r = c >> 2, i = c & 3;
     const int f = nm[r];
     int h = face_he[f];
@@ -1928,45 +1997,29 @@ __global__ void kWcCopy(const int32_t* __restrict__ nm, int n, const int4* __res
     }
 }
 
-// the old -> copy map entries the step set (kWcCopy's, which kSubdivide only re-points) back
-// to -1, so the maps are all -1 again for the next step without a full fill
-__global__ void kWcUndo(const int32_t* __restrict__ nm, WC w) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= 4 * w.n) return;
-    w.v_o2c[w.v_orig[c]] = -1;
-    w.h_o2c[w.h_orig[c]] = -1;
-    if ((c & 3) == 0) w.f_o2c[nm[c >> 2]] = -1;
-}
-
-// updateWorkingCopyHalfedges, ManifoldSplitter.cu:463-505
-__global__ void kWcUpdate(WC w, int count) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= count) return;
-    int4 e = w.he[c];
-    e.x = w.v_o2c[e.x];
-    e.y = w.f_o2c[e.y];
-    e.z = w.h_o2c[e.z];
-    if (e.w >= 0) {
-        const int m = w.h_o2c[e.w];
-        e.w = (m == -1) ? (-e.w - 2) : m;
-    }
-    w.he[c] = e;
-}
-
-// markHalfedgesAsNonManifold, ManifoldSplitter.cu:527-555: the copied halfedges that are
-// slotted non-manifold get the NM flag, as does their origin; their count goes to foundParts
-// (kNMSlotCheck compares it with the count of all of them: the reference would read the copy
-// index of one outside the copy as an invalid id)
-__global__ void __launch_bounds__(kBlock) kWcNMFlags(int n4, const int32_t* __restrict__ bsize, const int32_t* __restrict__ brank, WC w,
-                                                     int64_t* foundParts) {
+// updateWorkingCopyHalfedges, ManifoldSplitter.cu:463-505, and markHalfedgesAsNonManifold,
+// :527-555: the copied halfedges that are slotted non-manifold get the NM flag, as does their
+// origin; their count goes to foundParts (nmSlotCheck compares it with the count of all of
+// them: the reference would read the copy index of one outside the copy as an invalid id)
+__global__ void __launch_bounds__(kBlock) kWcUpdate(int n4, const int32_t* __restrict__ bsize, const int32_t* __restrict__ brank, WC w,
+                                                    int64_t* foundParts) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     int found = 0;
     if (c < n4) {
+        int4 e = w.he[c];
+        e.x = w.v_o2c[e.x];
+        e.y = w.f_o2c[e.y];
+        e.z = w.h_o2c[e.z];
+        if (e.w >= 0) {
+            const int m = w.h_o2c[e.w];
+            e.w = (m == -1) ? (-e.w - 2) : m;
+        }
+        w.he[c] = e;
         const int hh = w.h_orig[c];
         const int n = bsize[hh];
         if (n >= 4 && slottedNM(n, brank[hh])) {
             w.hflags[c] |= VF_NM;
-            atomicOr(&w.vflags[w.he[c].x], (uint32_t)VF_NM);
+            atomicOr(&w.vflags[e.x], (uint32_t)VF_NM);
             found = 1;
         }
     }
@@ -1976,12 +2029,13 @@ __global__ void __launch_bounds__(kBlock) kWcNMFlags(int n4, const int32_t* __re
 // a slotted non-manifold halfedge outside the working copy (its face not marked NM) is an
 // anomaly, one per such halfedge and step, as the reference's working copy would not hold it
 // (one wave: the partial sums of both counts; the found ones are cleared for the next step)
-__global__ void kNMSlotCheck(const int64_t* nmParts, int64_t* foundParts, int64_t* ctr) {
+__device__ __forceinline__ void nmSlotCheck(const int64_t* nmParts, int64_t* foundParts, int64_t* ctr) {
     const int lane = threadIdx.x;
     const int64_t total = sumParts(nmParts, lane), found = sumParts(foundParts, lane);
     foundParts[lane * kPartStride] = 0;
     if (lane == 0 && total > found) ctr[A_ANOMALY] += total - found;
 }
+__global__ void kNMSlotCheck(const int64_t* nmParts, int64_t* foundParts, int64_t* ctr) { nmSlotCheck(nmParts, foundParts, ctr); }
 
 // performSubdivideQuads, ManifoldSplitter.cu:570-731.  Face r appends 4 vertices at 4n+4r,
 // 16 halfedges at 4n+16r and 4 faces at n+4r, which is where the ascending schedule puts them.
@@ -1989,8 +2043,13 @@ __global__ void kNMSlotCheck(const int64_t* nmParts, int64_t* foundParts, int64_
 // halfedge ih[i], the three new halfedges of new face i (with the twins the reference's
 // setTwin calls leave on them) and the outer halfedge that joins that face.  Every lane of
 // the wave has walked the face before any lane rewrites one of its outer halfedges.
-__global__ void kSubdivide(const int32_t* __restrict__ nm, WC w) {
+// (the block after the faces' makes the slot check)
+__global__ void kSubdivide(const int32_t* __restrict__ nm, WC w, const int64_t* nmParts, int64_t* foundParts, int64_t* ctr) {
     const int n = w.n;
+    if (blockIdx.x == gridDim.x - 1) {
+        if (threadIdx.x < 64) nmSlotCheck(nmParts, foundParts, ctr);
+        return;
+    }
     const int c0 = blockIdx.x * blockDim.x + threadIdx.x;
     if (c0 >= 4 * n) return;
     const int r = c0 >> 2, i = c0 & 3;
@@ -2044,25 +2103,13 @@ __global__ void kSubdivide(const int32_t* __restrict__ nm, WC w) {
     if (ao != -1 && bo == -1) w.h_o2c[ao] = b;
 }
 
-// performCollapseNonManifoldHalfedges: which working-copy halfedges collapse
-__global__ void kCollapsePred(const WC w, int count, int32_t* __restrict__ pred, int64_t* ctr) {
-    const int h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= count) return;
-    int p = 0;
-    if (w.hflags[h] & VF_NM) {
-        const int t = heT(w.he, h);
-        if (t < 0) anomaly(ctr);
-        else if (t >= h) p = 1;
-    }
-    pred[h] = p;
-}
-
-// collapseHalfedge, ManifoldSplitter.cu:749-835: remove flags plus the merge marks, recorded in call order
-__global__ void kCollapse(WC w, int count, const int32_t* __restrict__ pred, const int64_t* __restrict__ rank, int2* __restrict__ vrec,
-                          int2* __restrict__ hrec) {
-    const int h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= count || !pred[h]) return;
-    const int64_t k = rank[h];
+// performCollapseNonManifoldHalfedges (only copied halfedges, [0, 4n), carry the NM flag) and
+// collapseHalfedge, ManifoldSplitter.cu:749-835: remove flags plus the merge marks, recorded in
+// call order -- the collapsing halfedges are ranked by a look-back over tiles of 1024 -- and
+// counted per target
+constexpr int kCollapseRounds = 4;
+__device__ void collapseHalfedge(const SplitStep& s, int h, int64_t k) {
+    const WC& w = s.w;
     int cf[2][4];
     int4 cur = w.he[h];
     cf[0][0] = h;
@@ -2078,44 +2125,90 @@ __global__ void kCollapse(WC w, int count, const int32_t* __restrict__ pred, con
         for (int i = 0; i < 4; ++i) atomicOr(&w.hflags[cf[fc][i]], (uint32_t)VF_REMOVE);
         atomicOr(&w.fflags[heF(w.he, cf[fc][0])], (uint32_t)VF_REMOVE);
     }
+    auto mark = [&](int2* rec, int32_t* cnt, int count, int t, int p) {
+        *rec = make_int2(t, p);
+        if (t < 0 || t >= count) anomaly(s.ctr);
+        else atomicAdd(&cnt[t], 1);
+    };
     const int a = heO(w.he, cf[0][2]), b = heO(w.he, cf[1][1]);
     const int c = heO(w.he, cf[0][3]), d = heO(w.he, cf[1][2]);
-    vrec[4 * k + 0] = make_int2(a, b);
-    vrec[4 * k + 1] = make_int2(b, a);
-    vrec[4 * k + 2] = make_int2(c, d);
-    vrec[4 * k + 3] = make_int2(d, c);
+    int2* v = s.vrec + 4 * k;
+    mark(v, s.cntV, s.vsize, a, b);
+    mark(v + 1, s.cntV, s.vsize, b, a);
+    mark(v + 2, s.cntV, s.vsize, c, d);
+    mark(v + 3, s.cntV, s.vsize, d, c);
     for (int i = 1; i < 4; ++i) {
         const int ta = heT(w.he, cf[0][i]), tb = heT(w.he, cf[1][i]);
-        int2* o = hrec + 12 * k + 4 * (i - 1);
-        o[0] = make_int2(cf[0][i], tb);
-        o[1] = make_int2(tb, cf[0][i]);
-        o[2] = make_int2(cf[1][i], ta);
-        o[3] = make_int2(ta, cf[1][i]);
+        int2* o = s.hrec + 12 * k + 4 * (i - 1);
+        mark(o, s.cntH, s.hsize, cf[0][i], tb);
+        mark(o + 1, s.cntH, s.hsize, tb, cf[0][i]);
+        mark(o + 2, s.cntH, s.hsize, cf[1][i], ta);
+        mark(o + 3, s.cntH, s.hsize, ta, cf[1][i]);
     }
 }
-
-__global__ void kRecCount(const int2* __restrict__ rec, int64_t R, int count, int32_t* __restrict__ cnt, int64_t* ctr) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= R) return;
-    const int t = rec[i].x;
-    if (t < 0 || t >= count) { anomaly(ctr); return; }
-    atomicAdd(&cnt[t], 1);
+__global__ void __launch_bounds__(kLbBlock) kCollapse(SplitStep s, unsigned long long* __restrict__ words, uint32_t epoch, int64_t* __restrict__ directOut) {
+    constexpr int R = kCollapseRounds;
+    __shared__ int s_cnt[R * (kLbBlock / 64)], s_pre[R * (kLbBlock / 64) + 1];
+    __shared__ long long s_off;
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int n = 4 * s.w.n;
+    const int64_t t = blockIdx.x, base = t * (int64_t)(R * kLbBlock);
+    // (other tiles only add the REMOVE bit meanwhile, and twins do not change)
+    auto collapses = [&](int64_t e, bool count) {
+        if (e >= n || !(s.w.hflags[e] & VF_NM)) return false;
+        const int tw = heT(s.w.he, (int)e);
+        if (tw < 0 && count) anomaly(s.ctr);
+        return tw >= 0 && tw >= e;
+    };
+    uint64_t m[R];
+    uint32_t kb = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const bool k = collapses(base + r * kLbBlock + threadIdx.x, true);
+        m[r] = __ballot(k);
+        kb |= (k ? 1u : 0u) << r;
+    }
+    const int tileSum = lbBlockRanks<R>(m, s_cnt, s_pre);
+    if (threadIdx.x < 64)
+        lbTileOffset(
+            words, epoch, t, tileSum,
+            [&](int l) {
+                int64_t c = 0;
+                for (int64_t e = l; e < base; e += 64) c += collapses(e, false) ? 1 : 0;
+                return c;
+            },
+            directOut, &s_off);
+    __syncthreads();
+    const uint64_t below = (1ULL << lane) - 1ULL;
+    for (int r = 0; r < R; ++r)
+        if ((kb >> r) & 1u)
+            collapseHalfedge(s, (int)(base + r * kLbBlock + threadIdx.x), s_off + s_pre[r * (kLbBlock / 64) + wid] + __popcll(m[r] & below));
+    if (t == gridDim.x - 1 && threadIdx.x == 0) s.ctr[A_NCOL] = s_off + tileSum;
 }
-__global__ void kRecScatter(const int2* __restrict__ rec, int64_t R, int count, const int64_t* __restrict__ roff, int32_t* __restrict__ cursor,
-                            int32_t* __restrict__ idx) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= R) return;
-    const int t = rec[i].x;
-    if (t < 0 || t >= count) return;
-    idx[roff[t] + atomicAdd(&cursor[t], 1)] = (int32_t)i;
+
+// the records into their targets' lists, and the merge's snapshot of positions and normals
+__global__ void kRecScatter(SplitStep s) {
+    const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+    const int64_t ncol = s.ctr[A_NCOL];
+    for (int64_t i = t0; i < 12 * ncol; i += stride) {
+        const int t = s.hrec[i].x;
+        if (t >= 0 && t < s.hsize) s.idxH[s.offH[t] + atomicAdd(&s.curH[t], 1)] = (int32_t)i;
+    }
+    for (int64_t i = t0; i < 4 * ncol; i += stride) {
+        const int t = s.vrec[i].x;
+        if (t >= 0 && t < s.vsize) s.idxV[s.offV[t] + atomicAdd(&s.curV[t], 1)] = (int32_t)i;
+    }
+    if (s.step >= 3)
+        for (int64_t i = t0; i < 3 * (int64_t)s.vsize; i += stride) {
+            s.w.pos0[i] = s.w.pos[i];
+            s.w.nrm0[i] = s.w.nrm[i];
+        }
 }
 // markVerticesAsMergable / markHalfedgesAsMergeable applied in record order to glm::ivec2
 // storage: the counter always advances; the second mark goes to .y, marks 1, 3, 4, 5 to .x,
 // later marks are dropped (ManifoldSplitter.cu:749-765)
-__global__ void kRecApply(const int2* __restrict__ rec, int count, const int64_t* __restrict__ roff, int32_t* __restrict__ idx,
-                          const int32_t* __restrict__ cnt, int32_t* __restrict__ num, int32_t* __restrict__ ex, int32_t* __restrict__ ey) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= count) return;
+__device__ void applyRecords(int t, const int2* __restrict__ rec, const int64_t* __restrict__ roff, int32_t* __restrict__ idx,
+                             const int32_t* __restrict__ cnt, int32_t* __restrict__ num, int32_t* __restrict__ ex, int32_t* __restrict__ ey) {
     const int m = cnt[t];
     num[t] = 1 + m;
     ex[t] = -1;
@@ -2136,6 +2229,12 @@ __global__ void kRecApply(const int2* __restrict__ rec, int count, const int64_t
         if (j == 1) ey[t] = p;
         else ex[t] = p;
     }
+}
+__global__ void kRecApply(SplitStep s) {
+    int i;
+    const int r = rangeOf(s.vsize, s.hsize, 0, i);
+    if (r == 0) applyRecords(i, s.vrec, s.offV, s.idxV, s.cntV, s.numV, s.exV, s.eyV);
+    else if (r == 1) applyRecords(i, s.hrec, s.offH, s.idxH, s.cntH, s.numH, s.exH, s.eyH);
 }
 
 // DeviceMergeList::getAllPartnersOf, ManifoldSplitter.cu:25-62
@@ -2169,15 +2268,13 @@ __device__ int partnersOf(int v, int size, const int32_t* __restrict__ num, cons
 
 // mergeVertices, ManifoldSplitter.cu:936-990.  A vertex that survives reads partners
 // with larger ids only, which no earlier thread writes, so reading the snapshot is the
-// ascending schedule's result.
-__global__ void kMergeVertices(WC w, int count, const int32_t* __restrict__ num, const int32_t* __restrict__ ex, const int32_t* __restrict__ ey,
-                               int64_t* ctr) {
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= count) return;
+// ascending schedule's result.  True: v does not survive.
+__device__ bool mergeVertex(const WC& w, int v, int count, const int32_t* __restrict__ num, const int32_t* __restrict__ ex,
+                            const int32_t* __restrict__ ey, int64_t* ctr) {
     int P[12];
     const int np = partnersOf(v, count, num, ex, ey, P, ctr);
-    if (np == 1) return;
-    if (np < 1 || np > 12) { anomaly(ctr); return; }
+    if (np == 1) return false;
+    if (np < 1 || np > 12) { anomaly(ctr); return false; }
     int smallest = v;
     f3 p = ld3(w.pos0, v), nn = ld3(w.nrm0, v);
     bool obsolete = false;
@@ -2190,18 +2287,17 @@ __global__ void kMergeVertices(WC w, int count, const int32_t* __restrict__ num,
     }
     if (obsolete) {
         atomicOr(&w.vflags[v], (uint32_t)VF_REMOVE);
-        return;
+        return true;
     }
     p = divs(p, (float)np);
     w.pos[3 * smallest] = p.x; w.pos[3 * smallest + 1] = p.y; w.pos[3 * smallest + 2] = p.z;
     w.nrm[3 * smallest] = p.x; w.nrm[3 * smallest + 1] = p.y; w.nrm[3 * smallest + 2] = p.z;  // position stored as normal, :989
+    return false;
 }
 
 // updateHalfedgeVertexIDs, ManifoldSplitter.cu:992-1019
-__global__ void kUpdateVertexIDs(WC w, int count, int vcount, const int32_t* __restrict__ num, const int32_t* __restrict__ ex,
-                                 const int32_t* __restrict__ ey, int64_t* ctr) {
-    const int h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= count) return;
+__device__ void updateVertexID(const WC& w, int h, int vcount, const int32_t* __restrict__ num, const int32_t* __restrict__ ex,
+                               const int32_t* __restrict__ ey, int64_t* ctr) {
     const int v = heO(w.he, h);
     int P[12];
     const int np = partnersOf(v, vcount, num, ex, ey, P, ctr);
@@ -2214,8 +2310,7 @@ __global__ void kUpdateVertexIDs(WC w, int count, int vcount, const int32_t* __r
 
 // mergeHalfedges, ManifoldSplitter.cu:1021-1067, planned in parallel on the pre-launch twins.
 // valid[h] = new twin or -1.  Flags a conflict when a partner whose twin this launch
-// writes is read, or a halfedge would be written twice; then the ascending-order
-// single-thread kernel below runs instead.
+// writes is read, or a halfedge would be written twice; then mergeSequential runs instead.
 __device__ int planMerge(const WC& w, int h, int count, const int32_t* __restrict__ num, const int32_t* __restrict__ ex, const int32_t* __restrict__ ey,
                          int P[12], int& np, int64_t* ctr) {
     np = partnersOf(h, count, num, ex, ey, P, ctr);
@@ -2229,20 +2324,37 @@ __device__ int planMerge(const WC& w, int h, int count, const int32_t* __restric
     return -1;
 }
 
-__global__ void kMergePlan(WC w, int count, const int32_t* __restrict__ num, const int32_t* __restrict__ ex, const int32_t* __restrict__ ey,
-                           int32_t* __restrict__ valid, int32_t* __restrict__ firstWriter, int64_t* ctr) {
-    const int h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= count) return;
-    valid[h] = -1;
-    if (w.hflags[h] & VF_REMOVE) return;
+__device__ void planHalfedge(const SplitStep& s, int h) {
+    s.valid[h] = -1;
+    if (s.w.hflags[h] & VF_REMOVE) return;
     int P[12], np;
-    const int t = planMerge(w, h, count, num, ex, ey, P, np, ctr);
+    const int t = planMerge(s.w, h, s.hsize, s.numH, s.exH, s.eyH, P, np, s.ctr);
     if (t == -1 || t < h) return;
-    valid[h] = t;
-    atomicMin(&firstWriter[h], h);
-    atomicMin(&firstWriter[t], h);
-    if (atomicAdd(&firstWriter[count + h], 1) > 0) atomicAdd((unsigned long long*)&ctr[A_CONFLICT], 1ULL);
-    if (atomicAdd(&firstWriter[count + t], 1) > 0) atomicAdd((unsigned long long*)&ctr[A_CONFLICT], 1ULL);
+    s.valid[h] = t;
+    atomicMin(&s.firstWriter[h], h);
+    atomicMin(&s.firstWriter[t], h);
+    if (atomicAdd(&s.firstWriter[s.hsize + h], 1) > 0) atomicAdd((unsigned long long*)&s.ctr[A_CONFLICT], 1ULL);
+    if (atomicAdd(&s.firstWriter[s.hsize + t], 1) > 0) atomicAdd((unsigned long long*)&s.ctr[A_CONFLICT], 1ULL);
+}
+
+// the merges' first part, and which elements the copy back appends (copyWorkingCopiesBack,
+// ManifoldSplitter.cu:1176-1295): vertices (step 3) merge; halfedges take their origins' survivors
+// (step 3; a vertex's merge reads no halfedge) and plan their merges (step 4; the plans read
+// twins and flags, which no thread here writes)
+__global__ void kMergePlan(SplitStep s) {
+    int i;
+    const int r = rangeOf(s.vsize, s.hsize, s.fsize, i);
+    const WC& w = s.w;
+    if (r == 0) {
+        const bool gone = s.step >= 3 && mergeVertex(w, i, s.vsize, s.numV, s.exV, s.eyV, s.ctr);
+        s.newV[i] = (!gone && !(w.vflags[i] & VF_REMOVE) && w.v_c2o[i] == -1) ? 1 : 0;
+    } else if (r == 1) {
+        if (s.step >= 3) updateVertexID(w, i, s.vsize, s.numV, s.exV, s.eyV, s.ctr);
+        if (s.step >= 4) planHalfedge(s, i);
+        s.newH[i] = (!(w.hflags[i] & VF_REMOVE) && w.h_c2o[i] == -1) ? 1 : 0;
+    } else if (r == 2) {
+        s.newF[i] = (!(w.fflags[i] & VF_REMOVE) && w.f_c2o[i] == -1) ? 1 : 0;
+    }
 }
 
 __global__ void kMergeCheck(WC w, int count, const int32_t* __restrict__ num, const int32_t* __restrict__ ex, const int32_t* __restrict__ ey,
@@ -2265,42 +2377,21 @@ __global__ void kMergeCheck(WC w, int count, const int32_t* __restrict__ num, co
     }
 }
 
-// firstWriter: [0, count) = INT32_MAX (atomicMin targets), [count, 2 count) = 0 (write counts)
-__global__ void kFillFirstWriter(int32_t* __restrict__ fw, int count) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= 2 * (int64_t)count) return;
-    fw[i] = i < count ? INT32_MAX : 0;
-}
-
-__global__ void kMergeApply(WC w, int count, const int32_t* __restrict__ valid, const int64_t* ctr) {
-    if (ctr[A_CONFLICT] != 0) return;
-    const int h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= count) return;
-    const int t = valid[h];
-    if (t < 0) return;
-    setT(w.he, h, t);
-    setT(w.he, t, h);
-}
-
-__global__ void kMergeSequential(WC w, int count, const int32_t* __restrict__ num, const int32_t* __restrict__ ex, const int32_t* __restrict__ ey,
-                                 int64_t* ctr) {
-    if (ctr[A_CONFLICT] == 0) return;
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    ++ctr[A_MERGE_SEQ];  // the iterations that took this pass (one thread: a plain increment)
-    for (int h = 0; h < count; ++h) {
-        if (w.hflags[h] & VF_REMOVE) continue;
+// the planned merges, or -- with a conflict -- the merges in ascending order by one thread
+__device__ void mergeSequential(const SplitStep& s) {
+    ++s.ctr[A_MERGE_SEQ];  // the iterations that took this pass (one thread: a plain increment)
+    for (int h = 0; h < s.hsize; ++h) {
+        if (s.w.hflags[h] & VF_REMOVE) continue;
         int P[12], np;
-        const int t = planMerge(w, h, count, num, ex, ey, P, np, ctr);
+        const int t = planMerge(s.w, h, s.hsize, s.numH, s.exH, s.eyH, P, np, s.ctr);
         if (t == -1 || t < h) continue;
-        setT(w.he, h, t);
-        setT(w.he, t, h);
+        setT(s.w.he, h, t);
+        setT(s.w.he, t, h);
     }
 }
 
 // performMoveVerticesToSurface, ManifoldSplitter.cu:1130-1160
-__global__ void kMoveToSurface(WC w, int count, const ProblemDev* __restrict__ probs) {
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= count) return;
+__device__ void moveVertexToSurface(const WC& w, int v, const ProblemDev* __restrict__ probs) {
     if (w.vflags[v] & VF_REMOVE) return;
     const ProblemDev& P = probs[w.pid ? w.pid[v] : 0];
     const GridDev g = P.g;
@@ -2327,82 +2418,64 @@ __global__ void kMoveToSurface(WC w, int count, const ProblemDev* __restrict__ p
     w.pos[3 * v + 2] = point.z;
 }
 
-// copyWorkingCopiesBack, ManifoldSplitter.cu:1176-1295
-__global__ void kNewPred(const uint32_t* __restrict__ flags, const int32_t* __restrict__ c2o, int count, int32_t* __restrict__ pred) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    pred[i] = (!(flags[i] & VF_REMOVE) && c2o[i] == -1) ? 1 : 0;
-}
-
-// several working-copy vertices can copy one original; the last one in ascending order writes it
-__global__ void kLastCopy(WC w, int count, int32_t* __restrict__ last) {
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= count) return;
-    if (w.vflags[v] & VF_REMOVE) return;
-    const int o = w.v_c2o[v];
-    if (o >= 0) atomicMax(&last[o], v);
-}
-
-__global__ void kCopyBackVertices(WC w, int count, const int64_t* __restrict__ addr, int64_t V0, float* __restrict__ pos, float* __restrict__ nrm,
-                                  int32_t* __restrict__ pid, const int32_t* __restrict__ last) {
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= count) return;
-    if (w.vflags[v] & VF_REMOVE) return;
-    int64_t o = w.v_c2o[v];
-    if (o == -1) {
-        o = V0 + addr[v];
-        w.v_c2o[v] = (int32_t)o;
-    } else if (last[o] != v) {
-        return;
-    }
-    for (int k = 0; k < 3; ++k) {
-        pos[3 * o + k] = w.pos[3 * v + k];
-        nrm[3 * o + k] = w.nrm[3 * v + k];
-    }
-    if (pid) pid[o] = w.pid[v];
-}
-
-// the ids of the halfedges written back (the records themselves are written by kUpdateBack,
-// from the working copy, once every id is known)
-__global__ void kCopyBackHalfedges(WC w, int count, const int64_t* __restrict__ addr, int64_t H0, uint8_t* __restrict__ canon) {
-    const int h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= count) return;
-    if (w.hflags[h] & VF_REMOVE) return;
-    int64_t o = w.h_c2o[h];
-    if (o == -1) {
-        o = H0 + addr[h];
-        w.h_c2o[h] = (int32_t)o;
-    }
-    canon[o] = 0;  // this record may leave the build's layout
-}
-
-__global__ void kCopyBackFaces(WC w, int count, const int64_t* __restrict__ addr, int64_t F0, int32_t* __restrict__ face_he, uint32_t* __restrict__ fattr) {
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= count) return;
-    if (w.fflags[f] & VF_REMOVE) return;
-    int64_t o = w.f_c2o[f];
-    if (o == -1) {
-        o = F0 + addr[f];
-        w.f_c2o[f] = (int32_t)o;
-    }
-    face_he[o] = w.h_c2o[w.f_first[f]];
-    fattr[o] = w.f_attr[f];
-}
-
-// the vertices a split step touched (its working copy's, by their ids after the copy back)
-__global__ void kMarkWcVertices(WC w, int count, uint8_t* __restrict__ dirtyV, uint8_t* __restrict__ touched) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= count) return;
-    const int o = w.v_c2o[c];
-    if (o >= 0) {
-        dirtyV[o] = 1;
-        touched[o] = 1;
+// the merges' second part (halfedges, step 4) beside the vertices' part of the rest: the last
+// surviving copy of an original in ascending order writes it back, and every surviving
+// vertex moves to the surface (step 5)
+__global__ void kMergeApply(SplitStep s, const ProblemDev* __restrict__ probs) {
+    int i;
+    const int r = rangeOf(s.step >= 4 ? s.hsize : 0, s.vsize, 0, i);
+    const WC& w = s.w;
+    if (r == 0) {
+        if (s.ctr[A_CONFLICT] != 0) {
+            if (i == 0) mergeSequential(s);
+            return;
+        }
+        const int t = s.valid[i];
+        if (t < 0) return;
+        setT(w.he, i, t);
+        setT(w.he, t, i);
+    } else if (r == 1) {
+        const int o = w.v_c2o[i];
+        if (o >= 0 && !(w.vflags[i] & VF_REMOVE)) atomicMax(&w.v_last[o], i);
+        if (s.step >= 5) moveVertexToSurface(w, i, probs);
     }
 }
 
-__global__ void kUpdateBack(WC w, int count, int4* __restrict__ he) {
-    const int h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= count) return;
+// copyWorkingCopiesBack, ManifoldSplitter.cu:1176-1295, in two parts: every element's id, and the
+// vertices; then, with all ids known, the halfedge records and the faces
+__global__ void kCopyBackIds(SplitStep s, float* __restrict__ pos, float* __restrict__ nrm, int32_t* __restrict__ pid, uint8_t* __restrict__ canon) {
+    int i;
+    const int r = rangeOf(s.vsize, s.hsize, s.fsize, i);
+    const WC& w = s.w;
+    if (r == 0) {
+        if (w.vflags[i] & VF_REMOVE) return;
+        int64_t o = w.v_c2o[i];
+        if (o == -1) {
+            o = s.V0 + s.addrV[i];
+            w.v_c2o[i] = (int32_t)o;
+        } else if (w.v_last[o] != i) {
+            return;
+        }
+        for (int k = 0; k < 3; ++k) {
+            pos[3 * o + k] = w.pos[3 * i + k];
+            nrm[3 * o + k] = w.nrm[3 * i + k];
+        }
+        if (pid) pid[o] = w.pid[i];
+    } else if (r == 1) {
+        if (w.hflags[i] & VF_REMOVE) return;
+        int64_t o = w.h_c2o[i];
+        if (o == -1) {
+            o = s.H0 + s.addrH[i];
+            w.h_c2o[i] = (int32_t)o;
+        }
+        canon[o] = 0;  // this record may leave the build's layout
+    } else if (r == 2) {
+        if (w.fflags[i] & VF_REMOVE) return;
+        if (w.f_c2o[i] == -1) w.f_c2o[i] = (int32_t)(s.F0 + s.addrF[i]);
+    }
+}
+
+__device__ void copyBackRecord(const WC& w, int h, int4* __restrict__ he) {
     if (w.hflags[h] & VF_REMOVE) return;
     const int64_t me = w.h_c2o[h];
     int4 e = w.he[h];  // the record copied back to me: no other thread writes he[me]
@@ -2418,6 +2491,38 @@ __global__ void kUpdateBack(WC w, int count, int4* __restrict__ he) {
         e.w = w.h_c2o[t];
     }
     he[me] = e;
+}
+// (the vertices mark what the step touched, by their ids after the copy back, and reset the map
+// entries the step set -- kWcCopy's, which kSubdivide only re-points -- so that the maps are all
+// -1 again for the next step without a full fill; the first block clears the partial sums
+// the refresh counts again)
+__global__ void kCopyBack(SplitStep s, const int32_t* __restrict__ nm, int4* __restrict__ he, int32_t* __restrict__ face_he, uint32_t* __restrict__ fattr,
+                          uint8_t* __restrict__ dirtyV, uint8_t* __restrict__ touched, int64_t* __restrict__ nmParts) {
+    if (blockIdx.x == 0)
+        for (int k = threadIdx.x; k < kPartSlots * kPartStride; k += kBlock) nmParts[k] = 0;
+    int i;
+    const int r = rangeOf(s.vsize, s.hsize, s.fsize, i);
+    const WC& w = s.w;
+    if (r == 0) {
+        const int o = w.v_c2o[i];
+        if (o >= 0) {
+            dirtyV[o] = 1;
+            touched[o] = 1;
+        }
+        if (i < 4 * w.n) {
+            w.v_last[w.v_orig[i]] = -1;
+            w.v_o2c[w.v_orig[i]] = -1;
+            w.h_o2c[w.h_orig[i]] = -1;
+            if ((i & 3) == 0) w.f_o2c[nm[i >> 2]] = -1;
+        }
+    } else if (r == 1) {
+        copyBackRecord(w, i, he);
+    } else if (r == 2) {
+        if (w.fflags[i] & VF_REMOVE) return;
+        const int64_t o = w.f_c2o[i];
+        face_he[o] = w.h_c2o[w.f_first[i]];
+        fattr[o] = w.f_attr[i];
+    }
 }
 
 // ---------------------------------------------------------------- detectNonManifoldVertices
@@ -2782,16 +2887,6 @@ void Pipeline::scan(std::initializer_list<ScanJob> jobs, int64_t* stampStart, in
         words += scanTiles(x.n);
     }
     scanExclusiveI32(j, count, lb.epoch, stream, lookbackDiag(), stampStart, stampEnd);
-}
-
-int64_t Pipeline::scan32(const int32_t* in, int64_t n, const std::string& outName, int64_t** out) {
-    *out = arena.get<int64_t>(outName, (size_t)n + 1);
-    // total straight into pinned host memory
-    int64_t* h = pinHost();
-    int64_t* d = pinDev();
-    scan(in, *out, n, d + 1);
-    MDMC_HIP(hipStreamSynchronize(stream));
-    return h[1];
 }
 
 // lists the faces with the NM bit, ascending (countNonManifoldFaces); their number goes to the
@@ -3250,34 +3345,6 @@ void Pipeline::gridPassBack(std::vector<ProblemDev>& problems, int64_t C, int sh
 
 int32_t* Pipeline::pid() { return nProblems > 1 ? arena.ptr<int32_t>("pid") : nullptr; }
 
-// ---- HalfedgeMesh::initialize / refreshHashTable: CSR of outgoing halfedges and the buckets
-// bucket lists by smaller endpoint (degM holds the counts on entry and is zero on exit),
-// then the per-vertex bucket pass
-// bucket lists by smaller endpoint from the counts in degM and the records of the first
-// list pass, then the per-halfedge bucket pass
-// the split's refresh: lists of the flagged halfedges under their smaller endpoint, with
-// the refresh's keys; sizes and ranks of the flagged halfedges, then the flags from all sizes
-void Pipeline::buildBuckets(const int32_t* list, int64_t n) {
-    int4* he = arena.ptr<int4>("he");
-    int32_t* degM = arena.ptr<int32_t>("degM");
-    int64_t* offM = arena.get<int64_t>("offM", (size_t)V + 1);
-    scan(degM, offM, V + 1);
-    int2* A = arena.get<int2>("listA", (size_t)std::max<int64_t>(H, 1));
-    int32_t* bsize = arena.ptr<int32_t>("bsize");
-    int32_t* brank = arena.ptr<int32_t>("brank");
-    uint32_t* vflags = arena.ptr<uint32_t>("vflags");
-    uint32_t* fattr = arena.ptr<uint32_t>("fattr");
-    zero(vflags, (size_t)V * sizeof(uint32_t));
-    if (n > 0) {
-        const int32_t* lm = arena.ptr<int32_t>("bl_m");
-        const int2* lent = arena.ptr<int2>("bl_entry");
-        kPlaceEntries<<<gridFor(n), kBlock, 0, stream>>>(lm, lent, arena.ptr<int32_t>("bl_rank"), n, offM, A);
-        kBuckets<<<gridFor(n), kBlock, 0, stream>>>(list, lm, lent, n, offM, A, bsize, brank);
-    }
-    zero(nmSlotParts(), kPartSlots * kPartStride * sizeof(int64_t));  // recounted from the new bucket sizes
-    if (H > 0) kFlagsFromBuckets<<<gridFor((H + 3) / 4), kBlock, 0, stream>>>(he, H, bsize, brank, vflags, fattr, nmSlotParts());
-}
-
 // HalfedgeMesh::initialize from the grid pass's output: outgoing lists (lengths and ranks from
 // the vertices' contours), then every halfedge from its bucket
 void Pipeline::halfedgeInitialize() {
@@ -3333,37 +3400,43 @@ void Pipeline::checkValid(const char* what) {
 }
 
 // refreshHashTable (HalfedgeMesh.cu:1063-1100) after a split step: only the halfedges
-// whose bucket can have changed (both endpoints in dirtyV, or appended after oldH), which
+// whose bucket can have changed (both endpoints in dirty_v, or appended), which
 // kDirtyRecords lists, are re-bucketed; the others keep their sizes and ranks (same
-// members, same keys), and the flags are rebuilt from all sizes.
-void Pipeline::refreshHashTable(const uint8_t* dirtyV, int64_t oldH) {
-    int4* he = arena.ptr<int4>("he");
-    int32_t* face_he = arena.ptr<int32_t>("face_he");
-    int32_t* degM = arena.get<int32_t>("degM", (size_t)V + 1);
-    arena.grow<int32_t>("bsize", (size_t)H, (size_t)std::min(oldH, H), stream);
-    arena.grow<int32_t>("brank", (size_t)H, (size_t)std::min(oldH, H), stream);
-    int32_t* dlist = arena.get<int32_t>("dirty_list", (size_t)std::max<int64_t>(H, 1));
-    {
-        FillBatch fb(*this);
-        fb.add(degM, 0x00, ((size_t)V + 1) * sizeof(int32_t));
-        fb.add(counters() + A_DIRTY, 0x00, sizeof(int64_t));
-    }
-    if (F > 0) kFaceClear<<<gridFor((F + 3) / 4), kBlock, 0, stream>>>(face_he, F, H, arena.ptr<uint32_t>("fattr"), counters());
+// members, same keys), and the flags are rebuilt from all sizes.  Vm, Hm, Fm bound the new sizes,
+// which the host learns here; splitStep cleared the arrays that are counted into.
+void Pipeline::refreshHashTable(size_t Vm, size_t Hm, size_t Fm) {
+    const int4* he = arena.ptr<int4>("he");
+    const int32_t* face_he = arena.ptr<int32_t>("face_he");
+    uint32_t* fattr = arena.ptr<uint32_t>("fattr");
+    int32_t* degM = arena.ptr<int32_t>("degM");
+    int32_t* dlist = arena.ptr<int32_t>("dirty_list");
     const int64_t per = (int64_t)kBlock * kDirtyPer;
-    if (H > 0) kDirtyRecords<<<(unsigned)((H + per - 1) / per), kBlock, 0, stream>>>(he, H, oldH, F, V, dirtyV, dlist, counters());
-    // one read-back: the invalid-record count and the dirty-list length
-    int64_t* hp = pinHost();
-    MDMC_HIP(hipMemcpyAsync(hp, counters() + A_INVALID, 2 * sizeof(int64_t), hipMemcpyDeviceToHost, stream));
-    MDMC_HIP(hipStreamSynchronize(stream));
-    if (hp[0]) throw HipError("inconsistent mesh after splitting (" + std::to_string(hp[0]) + " bad ids)", -4);
-    const int64_t nDirty = hp[1];
-    if (nDirty < 0 || nDirty > H) throw HipError("inconsistent mesh after splitting (dirty list of " + std::to_string(nDirty) + ")", -4);
-    if (nDirty > 0) {
-        const size_t nd = (size_t)nDirty;
-        kDirtyKeys<<<gridFor(nDirty), kBlock, 0, stream>>>(he, H, face_he, canonFlags(), dlist, nDirty, degM, arena.get<int32_t>("bl_m", nd), arena.get<int2>("bl_entry", nd),
-                                                          arena.get<int32_t>("bl_rank", nd), counters());
+    const int64_t records = ((int64_t)Hm + per - 1) / per;
+    kDirtyRecords<<<(unsigned)records + gridFor(((int64_t)Fm + 3) / 4), kBlock, 0, stream>>>(he, H, F, V, arena.ptr<uint8_t>("dirty_v"), dlist, records, face_he,
+                                                                                      fattr, counters());
+    const int64_t* c = readCounters();
+    if (c[A_INVALID]) throw HipError("inconsistent mesh after splitting (" + std::to_string(c[A_INVALID]) + " bad ids)", -4);
+    V += c[A_ADD];
+    H += c[A_ADD + 1];
+    F += c[A_ADD + 2];
+    const int64_t n = c[A_DIRTY];
+    if (n < 0 || n > H || V > (int64_t)Vm || H > (int64_t)Hm || F > (int64_t)Fm)
+        throw HipError("inconsistent mesh after splitting (dirty list of " + std::to_string(n) + ")", -4);
+    int32_t* bsize = arena.ptr<int32_t>("bsize");
+    int32_t* brank = arena.ptr<int32_t>("brank");
+    if (n > 0) {
+        int32_t* lm = arena.get<int32_t>("bl_m", (size_t)n);
+        int2* lent = arena.get<int2>("bl_entry", (size_t)n);
+        int32_t* lrank = arena.get<int32_t>("bl_rank", (size_t)n);
+        int64_t* offM = arena.get<int64_t>("offM", (size_t)V + 1);
+        int2* A = arena.get<int2>("listA", (size_t)n);
+        kDirtyKeys<<<gridFor(n), kBlock, 0, stream>>>(he, H, face_he, canonFlags(), dlist, n, degM, lm, lent, lrank, counters());
+        scan(degM, offM, V + 1);
+        kPlaceEntries<<<gridFor(n), kBlock, 0, stream>>>(lm, lent, lrank, n, offM, A);
+        kBuckets<<<gridFor(n), kBlock, 0, stream>>>(dlist, lm, lent, n, offM, A, bsize, brank);
     }
-    buildBuckets(dlist, nDirty);
+    if (H > 0)
+        kFlagsFromBuckets<<<gridFor((H + 3) / 4), kBlock, 0, stream>>>(he, H, bsize, brank, arena.ptr<uint32_t>("vflags"), fattr, nmSlotParts());
     refreshUnchecked = true;  // kDirtyKeys' face-walk check is read back with the next NM-face count
 }
 
@@ -3689,57 +3762,95 @@ void Pipeline::split(int step, int maxIters) {
 void Pipeline::splitStep(int step, int64_t n64, const int32_t* nm) {
     if (20 * n64 >= (int64_t)INT32_MAX / 2) throw HipError("working copy exceeds the int32 id range", -3);
     const int n = (int)n64;
-    const int64_t iterH = H;
-    // every vertex any step touches (for the NM-vertex detection's use of the outgoing lists)
-    if (!splitTouched) {
-        touchedV = V;
-        zero(arena.get<uint8_t>("split_touched", (size_t)std::max<int64_t>(V, 1)), (size_t)V);
-        splitTouched = true;
-    }
-    uint8_t* touched = arena.ptr<uint8_t>("split_touched");
     {
-        WC w;
+        SplitStep st{};
+        WC& w = st.w;
         w.n = n;
         const int nv = 8 * n, nh = 20 * n, nf = 5 * n;
+        st.step = step;
+        st.vsize = step >= 1 ? nv : 4 * n;
+        st.hsize = step >= 1 ? nh : 4 * n;
+        st.fsize = step >= 1 ? nf : n;
+        st.V0 = V;
+        st.H0 = H;
+        st.F0 = F;
+        st.ctr = counters();
         w.pos = arena.get<float>("wc_pos", 3 * (size_t)nv);
         w.nrm = arena.get<float>("wc_nrm", 3 * (size_t)nv);
         w.pos0 = arena.get<float>("wc_pos0", 3 * (size_t)nv);
         w.nrm0 = arena.get<float>("wc_nrm0", 3 * (size_t)nv);
         w.vflags = arena.get<uint32_t>("wc_vflags", (size_t)nv);
         w.v_c2o = arena.get<int32_t>("wc_v_c2o", (size_t)nv);
-        // a map the arena reallocates holds no -1s: its capacity before the get tells
-        wcMaps[0].cap = (int64_t)arena.capacity<int32_t>("wc_v_o2c");
-        wcMaps[1].cap = (int64_t)arena.capacity<int32_t>("wc_h_o2c");
-        wcMaps[2].cap = (int64_t)arena.capacity<int32_t>("wc_f_o2c");
-        w.v_o2c = arena.get<int32_t>("wc_v_o2c", (size_t)(V + nv));
+        // the old -> copy maps and the last copies are all -1 between steps (kCopyBack), so only a
+        // part no step has used yet is filled; a map the arena reallocates holds no -1s: its
+        // capacity before the get tells
+        static const char* mapName[4] = {"wc_v_o2c", "wc_h_o2c", "wc_f_o2c", "wc_v_last"};
+        int32_t* maps[4];
+        const int64_t need[4] = {V + nv, H + nh, F + nf, V + 1};
+        for (int k = 0; k < 4; ++k) {
+            wcMaps[k].cap = (int64_t)arena.capacity<int32_t>(mapName[k]);
+            maps[k] = arena.get<int32_t>(mapName[k], (size_t)need[k]);
+        }
+        w.v_o2c = maps[0];
+        w.h_o2c = maps[1];
+        w.f_o2c = maps[2];
+        w.v_last = maps[3];
         w.he = arena.get<int4>("wc_he", (size_t)nh);
         w.hflags = arena.get<uint32_t>("wc_hflags", (size_t)nh);
         w.h_c2o = arena.get<int32_t>("wc_h_c2o", (size_t)nh);
-        w.h_o2c = arena.get<int32_t>("wc_h_o2c", (size_t)(H + nh));
         w.f_first = arena.get<int32_t>("wc_f_first", (size_t)nf);
         w.f_attr = arena.get<uint32_t>("wc_f_attr", (size_t)nf);
         w.fflags = arena.get<uint32_t>("wc_fflags", (size_t)nf);
         w.f_c2o = arena.get<int32_t>("wc_f_c2o", (size_t)nf);
-        w.f_o2c = arena.get<int32_t>("wc_f_o2c", (size_t)(F + nf));
         w.pid = pid() ? arena.get<int32_t>("wc_pid", (size_t)nv) : nullptr;
         w.v_orig = arena.get<int32_t>("wc_v_orig", 4 * (size_t)n);
         w.h_orig = arena.get<int32_t>("wc_h_orig", 4 * (size_t)n);
-        // positions, normals, halfedge records, first halfedges and face attributes of the
-        // working copy are written in full by kWcCopy ([0, 4n) / [0, n)) and kSubdivide (the
-        // rest) before any read, so only the flags and the id maps are initialised here (one
-        // launch); the old -> copy maps are all -1 between steps (kWcUndo), so only a part no
-        // step has used yet is filled
+        // (only copied halfedges collapse, so at most 4n of them)
+        st.vrec = arena.get<int2>("vrec", 16 * (size_t)n);
+        st.hrec = arena.get<int2>("hrec", 48 * (size_t)n);
+        st.cntV = arena.get<int32_t>("mlv_cnt", (size_t)nv + 1);
+        st.curV = arena.get<int32_t>("mlv_cur", (size_t)nv + 1);
+        st.offV = arena.get<int64_t>("mlv_off", (size_t)nv + 2);
+        st.idxV = arena.get<int32_t>("mlv_idx", 16 * (size_t)n);
+        st.numV = arena.get<int32_t>("mlv_num", (size_t)nv);
+        st.exV = arena.get<int32_t>("mlv_x", (size_t)nv);
+        st.eyV = arena.get<int32_t>("mlv_y", (size_t)nv);
+        st.cntH = arena.get<int32_t>("mlh_cnt", (size_t)nh + 1);
+        st.curH = arena.get<int32_t>("mlh_cur", (size_t)nh + 1);
+        st.offH = arena.get<int64_t>("mlh_off", (size_t)nh + 2);
+        st.idxH = arena.get<int32_t>("mlh_idx", 48 * (size_t)n);
+        st.numH = arena.get<int32_t>("mlh_num", (size_t)nh);
+        st.exH = arena.get<int32_t>("mlh_x", (size_t)nh);
+        st.eyH = arena.get<int32_t>("mlh_y", (size_t)nh);
+        st.valid = arena.get<int32_t>("mvalid", (size_t)nh);
+        st.firstWriter = arena.get<int32_t>("mfirst", 2 * (size_t)nh);
+        st.newV = arena.get<int32_t>("cb_pred_v", (size_t)nv);
+        st.newH = arena.get<int32_t>("cb_pred_h", (size_t)nh);
+        st.newF = arena.get<int32_t>("cb_pred_f", (size_t)nf);
+        st.addrV = arena.get<int64_t>("cb_addr_v", (size_t)nv + 1);
+        st.addrH = arena.get<int64_t>("cb_addr_h", (size_t)nh + 1);
+        st.addrF = arena.get<int64_t>("cb_addr_f", (size_t)nf + 1);
+        // the mesh's arrays for the most the step can append
+        const size_t Vm = (size_t)V + 4 * (size_t)n, Hm = (size_t)H + 16 * (size_t)n, Fm = (size_t)F + 4 * (size_t)n;
+        float* pos = arena.grow<float>("pos", 3 * Vm, 3 * (size_t)V, stream);
+        float* nrm = arena.grow<float>("nrm", 3 * Vm, 3 * (size_t)V, stream);
+        int32_t* vp = pid() ? arena.grow<int32_t>("pid", Vm, (size_t)V, stream) : nullptr;
+        int4* he = arena.grow<int4>("he", Hm, (size_t)H, stream);
+        int32_t* face_he = arena.grow<int32_t>("face_he", Fm, (size_t)F, stream);
+        uint32_t* fattr = arena.grow<uint32_t>("fattr", Fm, (size_t)F, stream);
+        int32_t* bsize = arena.grow<int32_t>("bsize", Hm, (size_t)H, stream);
+        int32_t* brank = arena.grow<int32_t>("brank", Hm, (size_t)H, stream);
+        uint32_t* vflags = arena.grow<uint32_t>("vflags", Vm, 0, stream);  // rebuilt by the refresh
+        uint8_t* dirtyV = arena.get<uint8_t>("dirty_v", Vm);
+        int32_t* degM = arena.get<int32_t>("degM", Vm + 1);
+        int32_t* dlist = arena.get<int32_t>("dirty_list", Hm);
+        // layout flags: all set after the build, cleared for every record written back
+        uint8_t* canon = canonTracked ? arena.grow<uint8_t>("he_canon", Hm, (size_t)H, stream) : arena.get<uint8_t>("he_canon", Hm);
+        // every vertex any step touches (for the NM-vertex detection's use of the outgoing lists)
+        uint8_t* touched = splitTouched ? arena.grow<uint8_t>("split_touched", Vm, (size_t)V, stream) : arena.get<uint8_t>("split_touched", Vm);
         {
             FillBatch fb(*this);
-            fb.add(w.vflags, 0x00, (size_t)nv * sizeof(uint32_t));  // WorkingCopy ignores its initialFlags argument: flags start at 0
-            fb.add(w.v_c2o, 0xFF, (size_t)nv * sizeof(int32_t));
-            fb.add(w.hflags, 0x00, (size_t)nh * sizeof(uint32_t));
-            fb.add(w.h_c2o, 0xFF, (size_t)nh * sizeof(int32_t));
-            fb.add(w.fflags, 0x00, (size_t)nf * sizeof(uint32_t));
-            fb.add(w.f_c2o, 0xFF, (size_t)nf * sizeof(int32_t));
-            const int64_t need[3] = {V + nv, H + nh, F + nf};
-            int32_t* maps[3] = {w.v_o2c, w.h_o2c, w.f_o2c};
-            for (int k = 0; k < 3; ++k) {
+            for (int k = 0; k < 4; ++k) {
                 WcMap& m = wcMaps[k];
                 if (maps[k] != m.ptr || wcMapsDirty || m.cap < need[k]) {
                     fb.add(maps[k], 0xFF, (size_t)need[k] * sizeof(int32_t));
@@ -3750,144 +3861,46 @@ void Pipeline::splitStep(int step, int64_t n64, const int32_t* nm) {
                     m.clean = need[k];
                 }
             }
+            if (splitTouched) fb.add(touched + V, 0x00, Vm - (size_t)V);
+            else fb.add(touched, 0x00, Vm);
+            if (!canonTracked) fb.add(canon, 0x01, (size_t)H);
+            fb.add(canon + H, 0x00, Hm - (size_t)H);
+            fb.add(dirtyV, 0x00, Vm);
+            fb.add(degM, 0x00, (Vm + 1) * sizeof(int32_t));
+            fb.add(vflags, 0x00, Vm * sizeof(uint32_t));
+            for (int k : {(int)A_DIRTY, (int)A_CONFLICT}) fb.add(counters() + k, 0x00, sizeof(int64_t));
         }
-        wcMapsDirty = true;  // until kWcUndo has run
+        splitTouched = canonTracked = true;
+        wcMapsDirty = true;  // until kCopyBack has run
 
-        kWcCopy<<<gridFor(4 * (int64_t)n), kBlock, 0, stream>>>(nm, n, arena.ptr<int4>("he"), arena.ptr<int32_t>("face_he"), arena.ptr<uint32_t>("fattr"),
-                                                   arena.ptr<float>("pos"), arena.ptr<float>("nrm"), pid(), w);
-        int vsize = 4 * n, hsize = 4 * n, fsize = n;
-        kWcUpdate<<<gridFor(hsize), kBlock, 0, stream>>>(w, hsize);
-        kWcNMFlags<<<gridFor(4 * (int64_t)n), kBlock, 0, stream>>>(4 * n, arena.ptr<int32_t>("bsize"), arena.ptr<int32_t>("brank"), w, nmFoundParts());
-        kNMSlotCheck<<<1, 64, 0, stream>>>(nmSlotParts(), nmFoundParts(), counters());
-
-        if (step >= 1) {
-            kSubdivide<<<gridFor(4 * (int64_t)n), kBlock, 0, stream>>>(nm, w);
-            vsize = 8 * n;
-            hsize = 20 * n;
-            fsize = 5 * n;
-        }
+        kWcCopy<<<gridFor(4 * (int64_t)n), kBlock, 0, stream>>>(nm, n, he, face_he, fattr, pos, nrm, pid(), st);
+        kWcUpdate<<<gridFor(4 * (int64_t)n), kBlock, 0, stream>>>(4 * n, bsize, brank, w, nmFoundParts());
+        if (step >= 1) kSubdivide<<<gridFor(4 * (int64_t)n) + 1, kBlock, 0, stream>>>(nm, w, nmSlotParts(), nmFoundParts(), counters());
+        else kNMSlotCheck<<<1, 64, 0, stream>>>(nmSlotParts(), nmFoundParts(), counters());
+        const unsigned all = rangeBlocks(st.vsize, st.hsize, st.fsize);
         if (step >= 2) {
-            int32_t* cpred = arena.get<int32_t>("cpred", (size_t)hsize);
-            kCollapsePred<<<gridFor(hsize), kBlock, 0, stream>>>(w, hsize, cpred, counters());
-            int64_t* crank = nullptr;
-            const int64_t ncol = scan32(cpred, hsize, "crank", &crank);
-            int2* vrec = arena.get<int2>("vrec", 4 * (size_t)ncol);
-            int2* hrec = arena.get<int2>("hrec", 12 * (size_t)ncol);
-            if (ncol > 0) kCollapse<<<gridFor(hsize), kBlock, 0, stream>>>(w, hsize, cpred, crank, vrec, hrec);
-            int32_t* mlvN = arena.get<int32_t>("mlv_num", (size_t)vsize);
-            int32_t* mlvX = arena.get<int32_t>("mlv_x", (size_t)vsize);
-            int32_t* mlvY = arena.get<int32_t>("mlv_y", (size_t)vsize);
-            int32_t* mlhN = arena.get<int32_t>("mlh_num", (size_t)hsize);
-            int32_t* mlhX = arena.get<int32_t>("mlh_x", (size_t)hsize);
-            int32_t* mlhY = arena.get<int32_t>("mlh_y", (size_t)hsize);
-            buildMergeList(vrec, 4 * ncol, vsize, mlvN, mlvX, mlvY, "mlv");
-            buildMergeList(hrec, 12 * ncol, hsize, mlhN, mlhX, mlhY, "mlh");
-            if (step >= 3) {
-                MDMC_HIP(hipMemcpyAsync(w.pos0, w.pos, 3 * (size_t)vsize * sizeof(float), hipMemcpyDeviceToDevice, stream));
-                MDMC_HIP(hipMemcpyAsync(w.nrm0, w.nrm, 3 * (size_t)vsize * sizeof(float), hipMemcpyDeviceToDevice, stream));
-                kMergeVertices<<<gridFor(vsize), kBlock, 0, stream>>>(w, vsize, mlvN, mlvX, mlvY, counters());
-                kUpdateVertexIDs<<<gridFor(hsize), kBlock, 0, stream>>>(w, hsize, vsize, mlvN, mlvX, mlvY, counters());
-            }
-            if (step >= 4) {
-                int32_t* valid = arena.get<int32_t>("mvalid", (size_t)hsize);
-                int32_t* fw = arena.get<int32_t>("mfirst", 2 * (size_t)hsize);
-                kFillFirstWriter<<<gridFor(2 * (int64_t)hsize), kBlock, 0, stream>>>(fw, hsize);
-                zero(counters() + A_CONFLICT, sizeof(int64_t));
-                kMergePlan<<<gridFor(hsize), kBlock, 0, stream>>>(w, hsize, mlhN, mlhX, mlhY, valid, fw, counters());
-                kMergeCheck<<<gridFor(hsize), kBlock, 0, stream>>>(w, hsize, mlhN, mlhX, mlhY, fw, counters());
-                if (sequentialMerges) launchFill(counters() + A_CONFLICT, 0x01, 1);  // as if a conflict was found
-                kMergeApply<<<gridFor(hsize), kBlock, 0, stream>>>(w, hsize, valid, counters());
-                kMergeSequential<<<1, 1, 0, stream>>>(w, hsize, mlhN, mlhX, mlhY, counters());
-            }
+            const int64_t tiles = (4 * (int64_t)n + kCollapseRounds * kLbBlock - 1) / (kCollapseRounds * kLbBlock);
+            const Lookback lb = lookback(tiles);
+            kCollapse<<<(unsigned)tiles, kLbBlock, 0, stream>>>(st, lb.words, lb.epoch, lookbackDiag());
+            scan({ScanJob{st.cntV, st.offV, st.vsize + 1, nullptr, nullptr}, ScanJob{st.cntH, st.offH, st.hsize + 1, nullptr, nullptr}});
+            kRecScatter<<<std::min(gridFor(24 * (int64_t)n), 2048u), kBlock, 0, stream>>>(st);
+            kRecApply<<<rangeBlocks(st.vsize, st.hsize, 0), kBlock, 0, stream>>>(st);
         }
-        if (step >= 5) kMoveToSurface<<<gridFor(vsize), kBlock, 0, stream>>>(w, vsize, probsDev);
-
-        {
-            // the new vertices, halfedges and faces of the working copy: three prefix sums
-            // and one read-back of their totals ([1..3])
-            int32_t* pv = arena.get<int32_t>("cb_pred_v", (size_t)std::max(vsize, 1));
-            int32_t* ph = arena.get<int32_t>("cb_pred_h", (size_t)std::max(hsize, 1));
-            int32_t* pf = arena.get<int32_t>("cb_pred_f", (size_t)std::max(fsize, 1));
-            int64_t* av = arena.get<int64_t>("cb_addr_v", (size_t)vsize + 1);
-            int64_t* ah = arena.get<int64_t>("cb_addr_h", (size_t)hsize + 1);
-            int64_t* af = arena.get<int64_t>("cb_addr_f", (size_t)fsize + 1);
-            kNewPred<<<gridFor(vsize), kBlock, 0, stream>>>(w.vflags, w.v_c2o, vsize, pv);
-            kNewPred<<<gridFor(hsize), kBlock, 0, stream>>>(w.hflags, w.h_c2o, hsize, ph);
-            kNewPred<<<gridFor(fsize), kBlock, 0, stream>>>(w.fflags, w.f_c2o, fsize, pf);
-            int64_t* hp = pinHost();
-            int64_t* dp = pinDev();
-            hp[1] = hp[2] = hp[3] = 0;
-            scan({ScanJob{pv, av, vsize, dp + 1, nullptr}, ScanJob{ph, ah, hsize, dp + 2, nullptr}, ScanJob{pf, af, fsize, dp + 3, nullptr}});
-            MDMC_HIP(hipStreamSynchronize(stream));
-            const int64_t addV = hp[1], addH = hp[2], addF = hp[3];
-            // vertices
-            int64_t* a = av;
-            const int64_t V0 = V;
-            float* pos = arena.grow<float>("pos", 3 * (size_t)(V0 + addV), 3 * (size_t)V0, stream);
-            float* nrm = arena.grow<float>("nrm", 3 * (size_t)(V0 + addV), 3 * (size_t)V0, stream);
-            int32_t* vp = pid() ? arena.grow<int32_t>("pid", (size_t)(V0 + addV), (size_t)V0, stream) : nullptr;
-            int32_t* last = arena.get<int32_t>("cb_last", (size_t)V0 + 1);
-            fillNeg(last, ((size_t)V0 + 1) * sizeof(int32_t));
-            kLastCopy<<<gridFor(vsize), kBlock, 0, stream>>>(w, vsize, last);
-            kCopyBackVertices<<<gridFor(vsize), kBlock, 0, stream>>>(w, vsize, a, V0, pos, nrm, vp, last);
-            // halfedges
-            a = ah;
-            const int64_t H0 = H;
-            int4* he = arena.grow<int4>("he", (size_t)(H0 + addH), (size_t)H0, stream);
-            // layout flags: all set after the build, cleared for every record written back
-            if (!canonTracked) {
-                uint8_t* c0 = arena.get<uint8_t>("he_canon", (size_t)std::max<int64_t>(H0, 1));
-                launchFill(c0, 1, (size_t)H0);
-                canonTracked = true;
-            }
-            uint8_t* canon = arena.grow<uint8_t>("he_canon", (size_t)std::max<int64_t>(H0 + addH, 1), (size_t)H0, stream);
-            zero(canon + H0, (size_t)addH);
-            kCopyBackHalfedges<<<gridFor(hsize), kBlock, 0, stream>>>(w, hsize, a, H0, canon);
-            // faces
-            a = af;
-            const int64_t F0 = F;
-            int32_t* face_he = arena.grow<int32_t>("face_he", (size_t)(F0 + addF), (size_t)F0, stream);
-            uint32_t* fattr = arena.grow<uint32_t>("fattr", (size_t)(F0 + addF), (size_t)F0, stream);
-            kCopyBackFaces<<<gridFor(fsize), kBlock, 0, stream>>>(w, fsize, a, F0, face_he, fattr);
-            kUpdateBack<<<gridFor(hsize), kBlock, 0, stream>>>(w, hsize, he);
-            // the vertex arrays are resized to V + working-copy size (thrust resize: kept
-            // prefix, new slots value-initialised to 0); for the vertex -> halfedge array that
-            // leaves the initialize result on [0, vertHeV) and zeros after it
-            const int64_t Vres = V0 + vsize;
-            arena.grow<uint32_t>("vflags", (size_t)Vres, 0, stream);
-            V = V0 + addV;
-            H = H0 + addH;
-            F = F0 + addF;
+        kMergePlan<<<all, kBlock, 0, stream>>>(st);
+        if (step >= 4) {
+            kMergeCheck<<<gridFor(st.hsize), kBlock, 0, stream>>>(w, st.hsize, st.numH, st.exH, st.eyH, st.firstWriter, counters());
+            if (sequentialMerges) launchFill(counters() + A_CONFLICT, 0x01, 1);  // as if a conflict was found
         }
-        kWcUndo<<<gridFor(4 * (int64_t)n), kBlock, 0, stream>>>(nm, w);
+        kMergeApply<<<rangeBlocks(step >= 4 ? st.hsize : 0, st.vsize, 0), kBlock, 0, stream>>>(st, probsDev);
+        // the new vertices, halfedges and faces of the working copy
+        int64_t* add = counters() + A_ADD;
+        scan({ScanJob{st.newV, st.addrV, st.vsize, add, nullptr}, ScanJob{st.newH, st.addrH, st.hsize, add + 1, nullptr},
+              ScanJob{st.newF, st.addrF, st.fsize, add + 2, nullptr}});
+        kCopyBackIds<<<all, kBlock, 0, stream>>>(st, pos, nrm, vp, canon);
+        kCopyBack<<<all, kBlock, 0, stream>>>(st, nm, he, face_he, fattr, dirtyV, touched, nmSlotParts());
         wcMapsDirty = false;
-        uint8_t* dirtyV = arena.get<uint8_t>("dirty_v", (size_t)std::max<int64_t>(V, 1));
-        {
-            FillBatch fb(*this);
-            fb.add(dirtyV, 0x00, (size_t)std::max<int64_t>(V, 1));
-            if (V > touchedV) {
-                touched = arena.grow<uint8_t>("split_touched", (size_t)V, (size_t)touchedV, stream);
-                fb.add(touched + touchedV, 0x00, (size_t)(V - touchedV));
-                touchedV = V;
-            }
-        }
-        if (vsize > 0) kMarkWcVertices<<<gridFor(vsize), kBlock, 0, stream>>>(w, vsize, dirtyV, touched);
-        refreshHashTable(dirtyV, iterH);
+        refreshHashTable(Vm, Hm, Fm);
     }
-}
-
-void Pipeline::buildMergeList(const int2* rec, int64_t R, int count, int32_t* num, int32_t* ex, int32_t* ey, const std::string& tag) {
-    int32_t* cnt = arena.get<int32_t>(tag + "_cnt", (size_t)count + 1);
-    zero(cnt, ((size_t)count + 1) * sizeof(int32_t));
-    if (R > 0) kRecCount<<<gridFor(R), kBlock, 0, stream>>>(rec, R, count, cnt, counters());
-    // offsets only: the total is not needed on the host
-    int64_t* roff = arena.get<int64_t>(tag + "_off", (size_t)count + 2);
-    scan(cnt, roff, count + 1);
-    int32_t* cursor = arena.get<int32_t>(tag + "_cur", (size_t)count + 1);
-    zero(cursor, ((size_t)count + 1) * sizeof(int32_t));
-    int32_t* idx = arena.get<int32_t>(tag + "_idx", (size_t)R);
-    if (R > 0) kRecScatter<<<gridFor(R), kBlock, 0, stream>>>(rec, R, count, roff, cursor, idx);
-    if (count > 0) kRecApply<<<gridFor(count), kBlock, 0, stream>>>(rec, count, roff, idx, cnt, num, ex, ey);
 }
 
 void Pipeline::launchDetect(int guarded) {
