@@ -66,10 +66,10 @@ class Pipeline {
         int refinement = 0, pad = 0;
     } prep;
     void prepare(const std::vector<ProblemDev>& problems, bool captured);
-    // waits for the front of the grid pass; where the plain copy met values that need the exact
+    // waits for the front of the grid pass (totalsBehind: its totals, else all launched so far); where the plain copy met values that need the exact
     // blend, redoes the padding and calls again() (the front over it)
     template <class Again>
-    void finishPrepare(Again again);
+    void finishPrepare(bool totalsBehind, Again again);
     // the end of an extraction: with the statistics kernel's last block (one problem), or after a
     // batch's regroup, the counters, statistics and stage clocks go to pinned memory in one
     // read-back; the getters below read that copy
@@ -139,7 +139,7 @@ class Pipeline {
 
     int64_t readI64(const int64_t* dev);
     // mapped pinned host words for small read-backs: kernels and copies write them
-    // directly, so a read-back is one stream synchronisation (slots 0..kPinSlots-1)
+    // directly, and the host polls for them (slots 0..kPinSlots-1)
     static constexpr int kPinSlots = 64;
     int64_t* pinHost();
     int64_t* pinDev();
@@ -192,6 +192,10 @@ class Pipeline {
     void detectSlow(int64_t nSlow, int64_t nSlowOff);
     void launchStats(int guarded);
     const int64_t* waitStats();
+    template <class Ready>
+    void await(Ready ready);
+    void expectTotals();
+    bool totalsWritten();
     void zero(void* p, size_t bytes);
     void fillNeg(void* p, size_t bytes);
     void launchFill(void* p, uint8_t byte, size_t bytes);
