@@ -136,12 +136,17 @@ void launchGridEmit(int shape, const GridPassArgs& a, hipStream_t s);
 // vertex work items and the dual vertices
 void launchSlabCount(int shape, const GridPassArgs& a, hipStream_t s);
 void launchSlabEmit(int shape, const GridPassArgs& a, hipStream_t s);
+constexpr int kPairNone = -1, kPairSearch = -2, kPairFace = -3;
 // the halfedge initialize's outgoing lists from the grid pass's quads: entry off[v] + rank (the
-// rank from v's contour) of halfedge 4q + i from corner v = i holds 4q + i (out) and corners
-// i + 1 and i - 1 (ends); also the face -> halfedge array and the face attributes.  Inconsistent
-// quads are counted in *invalid (device) and raise *invalidPin (mapped pinned host memory)
+// rank from v's contour) of halfedge 4q + i from corner v = i holds 4q + i; also the face ->
+// halfedge array and the face attributes.  pairAt[4q + i] says what joins the halfedge's vertices:
+// with it one other, the halfedge before entry pairAt of the lists (>= 0); nothing (kPairNone); up to
+// three others around a face with four crossed edges, from the list that starts at entry kPairFace -
+// pairAt (<= kPairFace): pairFace[4q + i] holds per edge in order around the face its place in that
+// list (4 bits each), which of them join the two vertices (4 bits), and the halfedge's own (2 bits);
+// or what a search of a list finds (kPairSearch).  Inconsistent quads are counted in *invalid (device) and raise *invalidPin (mapped pinned host memory)
 void launchQuadLists(const int4* quads, const uint32_t* qattr, int64_t Q, int64_t V, const int32_t* vcell, const uint16_t* vct, const int32_t* vpid,
-                     const ProblemDev* probs, const int64_t* off, int32_t* out, int2* ends, int32_t* face_he, uint32_t* fattr, int64_t* invalid,
+                     const ProblemDev* probs, const int64_t* off, int32_t* out, int32_t* pairAt, uint32_t* pairFace, int32_t* face_he, uint32_t* fattr, int64_t* invalid,
                      int64_t* invalidPin, hipStream_t s);
 
 }  // namespace mdmc

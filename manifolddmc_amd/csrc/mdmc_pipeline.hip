@@ -473,47 +473,42 @@ __device__ BucketOf bucketFromOut(int h, int a, int b, const int4* __restrict__ 
     return BucketOf{n, rk, bucketTwin(n, rk, partner, mem, dir)};
 }
 
-// bucketFromOut for the initialize, whose lists carry each entry's destination and the origin
-// of the halfedge before it (ends[k], written with the list), so no quad is gathered
-__device__ BucketOf bucketFromOutEnds(int h, int a, int b, int64_t H, const int64_t* __restrict__ off, const int32_t* __restrict__ out,
-                                      const int2* __restrict__ ends, int64_t* ctr) {
-    const int m = min(a, b), o = max(a, b);
-    int mem[4], dir[4];
-    int n = 0, rk = 0, partner = -1;
-    bool self = false;
-    auto add = [&](int id, int d) {
-        if (n < 4) {
+// The same for the initialize, from the place kQuadLists gives (code): a pair's other halfedge ends
+// where the list's entry starts, as do the halfedges of a face's bucket an odd number of edges on.
+// (With a search for the latter, one halfedge in several hundred, kBucketsAll took 690 us at the
+// 512^3 gyroid instead of 505: a wave waits for its longest lane.)
+__device__ __forceinline__ BucketOf bucketFromPair(int h, int code, const uint32_t* pairFace, const int4* __restrict__ quads, int64_t H,
+                                                   const int64_t* __restrict__ off, const int32_t* __restrict__ out, int64_t* ctr) {
+    if (code >= 0) {
+        const int x = out[code];
+        if (x >= 0 && x < H) {
+            const int t = quadNext(x, 3);
+            return BucketOf{2, t < h ? 1 : 0, t};
+        }
+    } else if (code == kPairNone) {
+        return BucketOf{1, 0, -1};
+    } else if (code <= kPairFace) {
+        const uint32_t w = pairFace[h];
+        const int base = kPairFace - code, own = (int)(w >> 20) & 3;
+        int x[4], mem[4], dir[4], n = 0, rk = 0, partner = -1;
+        bool bad = false;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) x[p] = (w >> (16 + p)) & 1u ? out[base + (int)((w >> (4 * p)) & 0xFu)] : -1;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            if (!((w >> (16 + p)) & 1u)) continue;
+            bad = bad || x[p] < 0 || x[p] >= H;
+            const int d = (p ^ own) & 1, id = d ? quadNext(x[p], 3) : x[p];
             mem[n] = id;
             dir[n] = d;
+            ++n;
+            if (id < h) ++rk;
+            if (id != h) partner = id;
         }
-        ++n;
-        if (id < h) ++rk;
-        if (id != h) partner = id;
-        else self = true;
-    };
-    const int64_t k0 = off[m], k1 = min(off[m + 1], H);
-    for (int64_t kb = k0; kb < k1; kb += 4) {
-        int xs[4];
-        int2 es[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            xs[i] = kb + i < k1 ? out[kb + i] : 0;
-            es[i] = kb + i < k1 ? ends[kb + i] : make_int2(0, 0);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            if (kb + i >= k1) continue;
-            const int x = xs[i];
-            if (x < 0 || x >= H) {
-                anomaly(ctr);
-                continue;
-            }
-            if (es[i].x == o) add(x, 0);
-            if (o != m && es[i].y == o) add((x & ~3) | ((x + 3) & 3), 1);
-        }
+        if (!bad) return BucketOf{n, rk, bucketTwin(n, rk, partner, mem, dir)};
     }
-    if (!self) anomaly(ctr);
-    return BucketOf{n, rk, bucketTwin(n, rk, partner, mem, dir)};
+    const int4 q = quads[h >> 2];
+    return bucketFromOut(h, quadCorner(q, h & 3), quadCorner(q, (h + 1) & 3), quads, H, off, out, ctr);
 }
 
 // the members of h's bucket sorted by id (first kMaxBucket), returns the true count
@@ -550,24 +545,27 @@ __device__ int gatherBucketOut(int h, const int4* __restrict__ quads, int64_t H,
     return n;
 }
 
-// the bucket of halfedge h = 4f + i from a to b, and what the bucket pass of an initialize
+// the bucket of halfedge h = 4f + i, and what the bucket pass of an initialize
 // derives from it: vertex flags of the origin, the face's NM bit (fattr and the quad
 // attributes), an incoming boundary halfedge's share of the destination's valence.  Until the
 // simplifications are done a halfedge is its id (origin = corner i of quad f, face f, next
 // 4f + (i + 1) % 4) and its twin; the full records are written once after them
 // (kRemapRebuild, or kBuildHalfedges where none runs).
-__device__ __forceinline__ void storeHalfedge(int h, int a, int b, const BucketOf& bk, int32_t* __restrict__ twin, uint32_t* __restrict__ bpack,
-                                              uint32_t* __restrict__ vflags, uint32_t* __restrict__ fattr,
+__device__ __forceinline__ void storeHalfedge(int h, const int4* __restrict__ quads, const BucketOf& bk, int32_t* __restrict__ twin,
+                                              uint32_t* __restrict__ bpack, uint32_t* __restrict__ vflags, uint32_t* __restrict__ fattr,
                                               uint32_t* __restrict__ qattr, int32_t* __restrict__ valence, int32_t* __restrict__ bdin) {
     const int f = h >> 2;
     twin[h] = bk.twin;
     bpack[h] = packBucket(bk.n, bk.rank);
+    if (bk.n == 2) return;
+    const int4 q = quads[f];
     if (bk.twin == -1) {
+        const int b = quadCorner(q, (h + 1) & 3);
         atomicAdd(&valence[b], 1);
         if (bdin) atomicAdd(&bdin[b], 1);
     }
     const uint32_t vf = bucketVertexFlag(bk.n);
-    if (vf) atomicOr(&vflags[a], vf);
+    if (vf) atomicOr(&vflags[quadCorner(q, h & 3)], vf);
     if (bk.n == 4) {
         atomicOr(&fattr[f], (uint32_t)QA_NM);
         atomicOr(&qattr[f], (uint32_t)QA_NM);
@@ -588,27 +586,28 @@ __device__ __forceinline__ bool storeRecord(int h, int a, const BucketOf& bk, in
     return slottedNM(n, r);
 }
 
-// every halfedge from its bucket
+// Every halfedge from its bucket, found where kQuadLists says (in twin and bpack, which then
+// take the results).
+// Bound by HBM and the gathered list entries: 1.1 GB at least at the 512^3 gyroid's 69 M halfedges
+// (240 us), 505 us; searching the lists for every halfedge took 991 us, one thread per quad 789 us.
 __global__ void kBucketsAll(const int4* __restrict__ quads, int64_t H, const int64_t* __restrict__ off, const int32_t* __restrict__ out,
-                            const int2* __restrict__ ends, int32_t* __restrict__ twin, uint32_t* __restrict__ bpack, uint32_t* __restrict__ vflags,
+                            int32_t* twin, uint32_t* bpack, uint32_t* __restrict__ vflags,
                             uint32_t* __restrict__ fattr, uint32_t* __restrict__ qattr, int32_t* __restrict__ valence, int32_t* __restrict__ bdin,
                             int64_t* ctr) {
     const int64_t hh = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (hh >= H || chainHeld(ctr, 0)) return;
     const int h = (int)hh;
-    const int4 q = quads[h >> 2];
-    const int a = quadCorner(q, h & 3), b = quadCorner(q, (h + 1) & 3);
-    storeHalfedge(h, a, b, bucketFromOutEnds(h, a, b, H, off, out, ends, ctr), twin, bpack, vflags, fattr, qattr, valence, bdin);
+    storeHalfedge(h, quads, bucketFromPair(h, twin[h], bpack, quads, H, off, out, ctr), twin, bpack, vflags, fattr, qattr, valence, bdin);
 }
 
 // The same with the records, sizes and ranks written at once, when no simplification (which
 // reads ids and twins only) follows: one launch and 24 bytes per halfedge less to move than
-// kBucketsAll and a pass that turns its words into records.  Bound by the list gathers, as kBucketsAll is.  The quads are
+// kBucketsAll and a pass that turns its words into records.  The quads are
 // checked (kQuadLists) but the host has not looked yet: if any was inconsistent, every record is
 // a boundary halfedge of vertex 0, which the kernels launched before the host's next wait can
 // follow.
 __global__ void __launch_bounds__(kBlock) kBuildHalfedges(const int4* __restrict__ quads, int64_t H, const int64_t* __restrict__ off,
-                                                          const int32_t* __restrict__ out, const int2* __restrict__ ends, int4* __restrict__ he,
+                                                          const int32_t* __restrict__ out, const int32_t* __restrict__ pairAt, const uint32_t* __restrict__ pairFace, int4* __restrict__ he,
                                                           int32_t* __restrict__ bsize, int32_t* __restrict__ brank, uint32_t* __restrict__ vflags,
                                                           uint32_t* __restrict__ fattr, int64_t* nmParts, int64_t* ctr) {
     const int64_t hh = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -619,9 +618,8 @@ __global__ void __launch_bounds__(kBlock) kBuildHalfedges(const int4* __restrict
         int a = 0;
         BucketOf bk{2, 1, -1};
         if (!bad) {
-            const int4 q = quads[h >> 2];
-            a = quadCorner(q, h & 3);
-            bk = bucketFromOutEnds(h, a, quadCorner(q, (h + 1) & 3), H, off, out, ends, ctr);
+            a = quadCorner(quads[h >> 2], h & 3);
+            bk = bucketFromPair(h, pairAt[h], pairFace, quads, H, off, out, ctr);
         }
         slotted = storeRecord(h, a, bk, he, bsize, brank, vflags, fattr);
     }
@@ -3410,15 +3408,15 @@ void Pipeline::halfedgeInitialize() {
     int64_t* off = arena.get<int64_t>("out_off", (size_t)V + 1);
     scan({ScanJob{cnt, off, V + 1, nullptr, nullptr}}, stamp(ST_INIT));
     int32_t* out = arena.get<int32_t>("out_list", (size_t)std::max<int64_t>(H, 1));
-    int2* ends = arena.get<int2>("out_ends", (size_t)std::max<int64_t>(H, 1));
-    launchQuadLists(quads, qattr, Q, V, arena.ptr<int32_t>("gp_vcell"), arena.ptr<uint16_t>("gp_vct"), pid(), probsDev, off, out, ends, face_he, fattr,
+    int32_t* twin = arena.get<int32_t>("twin", (size_t)std::max<int64_t>(H, 1));
+    uint32_t* bpack = arena.get<uint32_t>("bpack", (size_t)std::max<int64_t>(H, 1));
+    launchQuadLists(quads, qattr, Q, V, arena.ptr<int32_t>("gp_vcell"), arena.ptr<uint16_t>("gp_vct"), pid(), probsDev, off, out, twin, bpack, face_he,
+                    fattr,
                     counters() + A_INVALID, pinDev() + kPinInvalid, stream);
     initUnchecked = true;
     if (!chain.empty()) {
-        int32_t* twin = arena.get<int32_t>("twin", (size_t)std::max<int64_t>(H, 1));
-        uint32_t* bpack = arena.get<uint32_t>("bpack", (size_t)std::max<int64_t>(H, 1));
         if (H > 0)
-            kBucketsAll<<<gridFor(H), kBlock, 0, stream>>>(quads, H, off, out, ends, twin, bpack, vflags, fattr, qattr, arena.ptr<int32_t>("valence"),
+            kBucketsAll<<<gridFor(H), kBlock, 0, stream>>>(quads, H, off, out, twin, bpack, vflags, fattr, qattr, arena.ptr<int32_t>("valence"),
                                                            chain.size() > 1 ? arena.ptr<int32_t>("bdin") : nullptr, counters());
     } else {
         // no simplification reads ids and twins only: the records at once
@@ -3426,7 +3424,7 @@ void Pipeline::halfedgeInitialize() {
         int32_t* bsize = arena.get<int32_t>("bsize", (size_t)std::max<int64_t>(H, 1));
         int32_t* brank = arena.get<int32_t>("brank", (size_t)std::max<int64_t>(H, 1));
         if (H > 0)
-            kBuildHalfedges<<<gridFor(H), kBlock, 0, stream>>>(quads, H, off, out, ends, he, bsize, brank, vflags, fattr, nmSlotParts(), counters());
+            kBuildHalfedges<<<gridFor(H), kBlock, 0, stream>>>(quads, H, off, out, twin, bpack, he, bsize, brank, vflags, fattr, nmSlotParts(), counters());
     }
     listsV = V;
     splitTouched = false;
