@@ -212,31 +212,120 @@ __device__ __forceinline__ int entryOther(int x) { return x & 0x7FFFFFFF; }
 // endpoints were touched.  A bucket changes only through a member that the step wrote back,
 // appended or removed, and every such halfedge joins two touched vertices (the working
 // copy's, before and after the step), so a halfedge with an untouched endpoint keeps its
-// bucket, its members and their keys.  One block checks kDirtyPer * kBlock consecutive halfedges,
+// bucket, its members and their keys.  One block checks kDirtyPer (recordsPerLane) * kBlock consecutive halfedges,
 // gathers its dirty ones in LDS and appends them to the dirty list with one atomic on
 // ctr[A_DIRTY]; the list order is free, since ranks only pick list slots and bucket ranks
 // come from the keys.
-constexpr int kDirtyPer = 16;
 constexpr int kDirtyBatch = 4;
-// The blocks from recordBlocks on clear the faces' bits.  The sizes are those before the step plus
+// records per lane here and in kOutDegreeMoved: 16 where the blocks still fill the chip several times
+// over, else 4 (280 k records of the 201x77x131 gyroid: 9.6 us against 24 in kOutDegreeMoved, 19 either
+// way here)
+inline int recordsPerLane(int64_t H) { return H >= (int64_t)16 * kBlock * 2048 ? 16 : 4; }
+// The blocks before quadBlocks take the records the build wrote, quad by quad: where all four keep its
+// layout (canon), their origins are the quad's corners, 20 bytes per face instead of 64 and no
+// other record's origin to gather; the next recordBlocks take the records appended since, the rest
+// clear the faces' bits.  The sizes are those before the step plus
 // what it appended, which the host does not know yet (the launch covers the most it can be).
-__global__ void __launch_bounds__(kBlock) kDirtyRecords(const int4* __restrict__ he, int64_t oldH, int64_t oldF, int64_t oldV,
-                                                        const uint8_t* __restrict__ dirtyV, int32_t* __restrict__ dlist, int64_t recordBlocks,
-                                                        const int32_t* __restrict__ face_he, uint32_t* __restrict__ fattr, int64_t* ctr) {
-    const int64_t V = oldV + ctr[A_ADD], H = oldH + ctr[A_ADD + 1], F = oldF + ctr[A_ADD + 2];
-    if ((int64_t)blockIdx.x >= recordBlocks) {
-        clearFaces(4 * (((int64_t)blockIdx.x - recordBlocks) * kBlock + threadIdx.x), face_he, F, H, fattr, ctr);
+// 512^3 gyroid, 61 M records: 264 us in the first step, 173 in the second; from the records alone 375 and 265.
+struct DirtyArgs {
+    const int4* he;
+    int64_t oldH, oldF, oldV;
+    const int4* quads;  // the build's Q quads, records [0, 4Q)
+    int64_t Q;
+    const uint8_t *canon, *dirtyV;
+    int32_t* dlist;
+    int64_t quadBlocks, recordBlocks;
+    const int32_t* face_he;
+    uint32_t* fattr;
+    int64_t* ctr;
+};
+template <int kDirtyPer>
+__global__ void __launch_bounds__(kBlock) kDirtyRecords(DirtyArgs a) {
+    int64_t* ctr = a.ctr;
+    const int64_t V = a.oldV + ctr[A_ADD], H = a.oldH + ctr[A_ADD + 1], F = a.oldF + ctr[A_ADD + 2];
+    if ((int64_t)blockIdx.x >= a.quadBlocks + a.recordBlocks) {
+        clearFaces(4 * (((int64_t)blockIdx.x - a.quadBlocks - a.recordBlocks) * kBlock + threadIdx.x), a.face_he, F, H, a.fattr, ctr);
         return;
     }
+    const int4* __restrict__ he = a.he;
+    const uint8_t* __restrict__ dirtyV = a.dirtyV;
+    const int64_t oldH = a.oldH;
     __shared__ int s_list[kBlock * kDirtyPer];
-    __shared__ int s_n;
+    __shared__ int s_face[kBlock * kDirtyPer / 4];
+    __shared__ int s_n, s_nf;
     __shared__ long long s_base;
     const int lane = threadIdx.x & 63;
-    if (threadIdx.x == 0) s_n = 0;
+    if (threadIdx.x == 0) s_n = s_nf = 0;
     __syncthreads();
-    const int64_t b0 = (int64_t)blockIdx.x * (kBlock * kDirtyPer) + threadIdx.x;
     int nbad = 0;
-    for (int k0 = 0; k0 < kDirtyPer; k0 += kDirtyBatch) {
+    auto list = [&](bool hit, int64_t h) {
+        const uint64_t m = __ballot(hit);
+        if (m == 0) return;
+        int at = 0;
+        if (lane == 0) at = atomicAdd(&s_n, __popcll(m));
+        at = __shfl(at, 0, 64);
+        if (hit) s_list[at + __popcll(m & ((1ULL << lane) - 1ULL))] = (int)h;
+    };
+    if ((int64_t)blockIdx.x < a.quadBlocks) {
+        constexpr int kQuads = kDirtyPer / 4;
+        const int64_t f0 = (int64_t)blockIdx.x * (kBlock * kQuads) + threadIdx.x;
+        int4 q[kQuads];
+        uint32_t laid[kQuads];
+#pragma unroll
+        for (int j = 0; j < kQuads; ++j) {
+            const int64_t f = f0 + j * kBlock;
+            q[j] = f < a.Q ? a.quads[f] : make_int4(-1, -1, -1, -1);
+            laid[j] = f < a.Q ? reinterpret_cast<const uint32_t*>(a.canon)[f] : 0u;
+        }
+#pragma unroll
+        for (int j = 0; j < kQuads; ++j) {
+            const int64_t f = f0 + j * kBlock;
+            uint32_t hits = 0;
+            if (laid[j] == 0x01010101u) {
+                const int c[4] = {q[j].x, q[j].y, q[j].z, q[j].w};
+                uint32_t d = 0;
+                bool bad = false;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const bool out = c[i] < 0 || c[i] >= V;
+                    bad = bad || out;
+                    d |= (!out && dirtyV[c[i]] ? 1u : 0u) << i;
+                }
+                nbad += bad ? 1 : 0;
+                hits = d & ((d >> 1) | (d << 3)) & 0xFu;
+            }
+            const uint64_t other = __ballot(f < a.Q && laid[j] != 0x01010101u);
+            if (other) {
+                int at = 0;
+                if (lane == 0) at = atomicAdd(&s_nf, __popcll(other));
+                at = __shfl(at, 0, 64);
+                if ((other >> lane) & 1ULL) s_face[at + __popcll(other & ((1ULL << lane) - 1ULL))] = j * kBlock + threadIdx.x;
+            }
+            if (__ballot(hits != 0) == 0) continue;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) list((hits >> i) & 1u, 4 * f + i);
+        }
+        __syncthreads();
+        // the quads with records written back: those from their records, on full waves
+        const int64_t fb = (int64_t)blockIdx.x * (kBlock * kQuads);
+        const int nf = 4 * s_nf;
+        for (int k0 = 0; k0 < nf; k0 += kBlock) {
+            const int k = k0 + threadIdx.x;
+            const int64_t h = k < nf ? 4 * (fb + s_face[k >> 2]) + (k & 3) : 0;
+            bool hit = false;
+            if (k < nf) {
+                const int4 e = he[h];
+                bool bad = e.x < 0 || e.x >= V || e.y < 0 || e.y >= F || e.z < 0 || e.z >= H || e.w < -1 || e.w >= H;
+                const int b = bad ? 0 : heO(he, e.z);
+                bad = bad || b < 0 || b >= V;
+                nbad += bad ? 1 : 0;
+                hit = !bad && dirtyV[e.x] && dirtyV[b];
+            }
+            list(hit, h);
+        }
+    }
+    const int64_t b0 = 4 * a.Q + ((int64_t)blockIdx.x - a.quadBlocks) * (kBlock * kDirtyPer) + threadIdx.x;
+    for (int k0 = 0; k0 < kDirtyPer && (int64_t)blockIdx.x >= a.quadBlocks; k0 += kDirtyBatch) {
         int4 e[kDirtyBatch];
         int b[kDirtyBatch];
         bool bad[kDirtyBatch], d[kDirtyBatch];
@@ -259,20 +348,14 @@ __global__ void __launch_bounds__(kBlock) kDirtyRecords(const int4* __restrict__
             nbad += bad[j] ? 1 : 0;
         }
 #pragma unroll
-        for (int j = 0; j < kDirtyBatch; ++j) {
-            const uint64_t m = __ballot(d[j]);
-            int at = 0;
-            if (lane == 0 && m) at = atomicAdd(&s_n, __popcll(m));
-            at = __shfl(at, 0, 64);
-            if (d[j]) s_list[at + __popcll(m & ((1ULL << lane) - 1ULL))] = (int)(b0 + (int64_t)(k0 + j) * kBlock);
-        }
+        for (int j = 0; j < kDirtyBatch; ++j) list(d[j], b0 + (int64_t)(k0 + j) * kBlock);
     }
     __syncthreads();
     const int n = s_n;
     if (threadIdx.x == 0 && n > 0) s_base = (long long)atomicAdd((unsigned long long*)&ctr[A_DIRTY], (unsigned long long)n);
     __syncthreads();
     const int64_t base = s_base;
-    for (int i = threadIdx.x; i < n; i += kBlock) dlist[base + i] = s_list[i];
+    for (int i = threadIdx.x; i < n; i += kBlock) a.dlist[base + i] = s_list[i];
     if (nbad) invalid(ctr, nbad);
 }
 
@@ -1265,22 +1348,54 @@ __global__ void __launch_bounds__(kBlock) kOutFromLists(const int64_t* __restric
     }
 }
 
-// the records the splitter wrote back or appended (canon unset), one per lane: each adds to
+// the records the splitter wrote back or appended (canon unset): each adds to
 // its origin's out-degree, and the first one of a vertex with no other outgoing halfedge
-// becomes its walk start
-__global__ void kOutDegreeMoved(const int4* __restrict__ he, int64_t H, int64_t V, int64_t listsV, const uint8_t* __restrict__ touched,
+// becomes its walk start.  A lane looks at the layout flags of PER records at once and the block's
+// unset ones are added on full waves (512^3 gyroid, 61 M records: 127 us; one per lane 209 us, and 51
+// us where the launch is held).
+template <int PER>
+__global__ void __launch_bounds__(kBlock) kOutDegreeMoved(const int4* __restrict__ he, int64_t H, int64_t V, int64_t listsV, const uint8_t* __restrict__ touched,
                                 const uint8_t* __restrict__ canon, int32_t* __restrict__ outdeg, int32_t* __restrict__ rep, int64_t* ctr,
                                 int guarded) {
     if (notYet(ctr, guarded)) return;
-    const int64_t h = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= H || canon[h]) return;
-    const int o = heO(he, (int)h);
-    if (o < 0 || o >= V) {
-        anomaly(ctr);
-        return;
+    __shared__ int s_list[PER * kBlock];
+    __shared__ int s_n;
+    if (threadIdx.x == 0) s_n = 0;
+    __syncthreads();
+    const int64_t h0 = PER * ((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
+    uint32_t moved = 0;  // bit k: record h0 + k
+    if (h0 + PER <= H && (((uintptr_t)canon) & 15) == 0) {
+        uint32_t w[PER / 4];
+        if (PER == 16) {
+            const uint4 c = reinterpret_cast<const uint4*>(canon)[h0 >> 4];
+            w[0] = c.x;
+            w[PER / 4 > 1 ? 1 : 0] = c.y;
+            w[PER / 4 > 2 ? 2 : 0] = c.z;
+            w[PER / 4 > 3 ? 3 : 0] = c.w;
+        } else {
+            w[0] = reinterpret_cast<const uint32_t*>(canon)[h0 >> 2];
+        }
+#pragma unroll
+        for (int k = 0; k < PER; ++k) moved |= ((w[k >> 2] >> (8 * (k & 3))) & 0xFFu ? 0u : 1u) << k;
+    } else {
+        for (int k = 0; k < PER && h0 + k < H; ++k) moved |= (canon[h0 + k] ? 0u : 1u) << k;
     }
-    if (o >= listsV || (touched && touched[o]))
-        if (atomicAdd(&outdeg[o], 1) == 0) rep[o] = (int32_t)h;
+    // (on full waves: a lane has none or many)
+    if (moved) {
+        int at = atomicAdd(&s_n, __popc(moved));
+        for (; moved; moved &= moved - 1) s_list[at++] = (int)(h0 + __ffs(moved) - 1);
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k < s_n; k += kBlock) {
+        const int h = s_list[k];
+        const int o = heO(he, h);
+        if (o < 0 || o >= V) {
+            anomaly(ctr);
+            continue;
+        }
+        if (o >= listsV || (touched && touched[o]))
+            if (atomicAdd(&outdeg[o], 1) == 0) rep[o] = h;
+    }
 }
 
 __global__ void kOutDegreeTouched(const int4* __restrict__ he, int64_t H, int64_t V, int64_t listsV, const uint8_t* __restrict__ touched,
@@ -2162,6 +2277,7 @@ __global__ void __launch_bounds__(kLbBlock) kCollapse(SplitStep s, unsigned long
     constexpr int R = kCollapseRounds;
     __shared__ int s_cnt[R * (kLbBlock / 64)], s_pre[R * (kLbBlock / 64) + 1];
     __shared__ long long s_off;
+    __shared__ int s_list[R * kLbBlock];  // the tile's collapsing halfedges by rank, for full waves
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const int n = 4 * s.w.n;
     const int64_t t = blockIdx.x, base = t * (int64_t)(R * kLbBlock);
@@ -2190,11 +2306,12 @@ __global__ void __launch_bounds__(kLbBlock) kCollapse(SplitStep s, unsigned long
                 return c;
             },
             directOut, &s_off);
-    __syncthreads();
     const uint64_t below = (1ULL << lane) - 1ULL;
+#pragma unroll
     for (int r = 0; r < R; ++r)
-        if ((kb >> r) & 1u)
-            collapseHalfedge(s, (int)(base + r * kLbBlock + threadIdx.x), s_off + s_pre[r * (kLbBlock / 64) + wid] + __popcll(m[r] & below));
+        if ((kb >> r) & 1u) s_list[s_pre[r * (kLbBlock / 64) + wid] + __popcll(m[r] & below)] = (int)(base + r * kLbBlock + threadIdx.x);
+    __syncthreads();
+    for (int j = threadIdx.x; j < tileSum; j += kLbBlock) collapseHalfedge(s, s_list[j], s_off + j);
     if (t == gridDim.x - 1 && threadIdx.x == 0) s.ctr[A_NCOL] = s_off + tileSum;
 }
 
@@ -2249,13 +2366,23 @@ __global__ void kRecApply(SplitStep s) {
     else if (r == 1) applyRecords(i, s.hrec, s.offH, s.idxH, s.cntH, s.numH, s.exH, s.eyH);
 }
 
+// a thread's list of merge partners, in LDS (a private array indexed by a variable would lie in
+// scratch memory: kMergePlan 390 us at the 512^3 gyroid's first step, 269 us now)
+struct Partners {
+    int* p;
+    __device__ __forceinline__ int& operator[](int i) const { return p[i * kBlock]; }
+};
+#define MDMC_PARTNERS(name)              \
+    __shared__ int s_partners[12 * kBlock]; \
+    const Partners name{s_partners + threadIdx.x}
+
 // DeviceMergeList::getAllPartnersOf, ManifoldSplitter.cu:25-62
 __device__ int partnersOf(int v, int size, const int32_t* __restrict__ num, const int32_t* __restrict__ ex, const int32_t* __restrict__ ey,
-                          int out[12], int64_t* ctr) {
-    for (int i = 0; i < 12; ++i) out[i] = -1;
+                          const Partners& out, int64_t* ctr) {
     if (v < 0 || v >= size) { anomaly(ctr); return 1; }
     int n = num[v];
-    if (n <= 1) return n;
+    if (n <= 1) return n;  // (out is not read then)
+    for (int i = 0; i < 12; ++i) out[i] = -1;
     for (int i = 0; i < n - 1; ++i) {
         if (i >= 12) { anomaly(ctr); break; }
         out[i] = (i == 1) ? ey[v] : ex[v];
@@ -2281,9 +2408,8 @@ __device__ int partnersOf(int v, int size, const int32_t* __restrict__ num, cons
 // mergeVertices, ManifoldSplitter.cu:936-990.  A vertex that survives reads partners
 // with larger ids only, which no earlier thread writes, so reading the snapshot is the
 // ascending schedule's result.  True: v does not survive.
-__device__ bool mergeVertex(const WC& w, int v, int count, const int32_t* __restrict__ num, const int32_t* __restrict__ ex,
+__device__ bool mergeVertex(const WC& w, const Partners& P, int v, int count, const int32_t* __restrict__ num, const int32_t* __restrict__ ex,
                             const int32_t* __restrict__ ey, int64_t* ctr) {
-    int P[12];
     const int np = partnersOf(v, count, num, ex, ey, P, ctr);
     if (np == 1) return false;
     if (np < 1 || np > 12) { anomaly(ctr); return false; }
@@ -2308,10 +2434,9 @@ __device__ bool mergeVertex(const WC& w, int v, int count, const int32_t* __rest
 }
 
 // updateHalfedgeVertexIDs, ManifoldSplitter.cu:992-1019
-__device__ void updateVertexID(const WC& w, int h, int vcount, const int32_t* __restrict__ num, const int32_t* __restrict__ ex,
+__device__ void updateVertexID(const WC& w, const Partners& P, int h, int vcount, const int32_t* __restrict__ num, const int32_t* __restrict__ ex,
                                const int32_t* __restrict__ ey, int64_t* ctr) {
     const int v = heO(w.he, h);
-    int P[12];
     const int np = partnersOf(v, vcount, num, ex, ey, P, ctr);
     if (np == 1) return;
     int smallest = v;
@@ -2324,7 +2449,7 @@ __device__ void updateVertexID(const WC& w, int h, int vcount, const int32_t* __
 // valid[h] = new twin or -1.  Flags a conflict when a partner whose twin this launch
 // writes is read, or a halfedge would be written twice; then mergeSequential runs instead.
 __device__ int planMerge(const WC& w, int h, int count, const int32_t* __restrict__ num, const int32_t* __restrict__ ex, const int32_t* __restrict__ ey,
-                         int P[12], int& np, int64_t* ctr) {
+                         const Partners& P, int& np, int64_t* ctr) {
     np = partnersOf(h, count, num, ex, ey, P, ctr);
     if (np == 1) return -1;
     for (int i = 0; i < np - 1; ++i) {
@@ -2336,10 +2461,10 @@ __device__ int planMerge(const WC& w, int h, int count, const int32_t* __restric
     return -1;
 }
 
-__device__ void planHalfedge(const SplitStep& s, int h) {
+__device__ void planHalfedge(const SplitStep& s, const Partners& P, int h) {
     s.valid[h] = -1;
     if (s.w.hflags[h] & VF_REMOVE) return;
-    int P[12], np;
+    int np;
     const int t = planMerge(s.w, h, s.hsize, s.numH, s.exH, s.eyH, P, np, s.ctr);
     if (t == -1 || t < h) return;
     s.valid[h] = t;
@@ -2353,28 +2478,29 @@ __device__ void planHalfedge(const SplitStep& s, int h) {
 // ManifoldSplitter.cu:1176-1295): vertices (step 3) merge; halfedges take their origins' survivors
 // (step 3; a vertex's merge reads no halfedge) and plan their merges (step 4; the plans read
 // twins and flags, which no thread here writes)
-__global__ void kMergePlan(SplitStep s) {
+__global__ void __launch_bounds__(kBlock) kMergePlan(SplitStep s) {
+    MDMC_PARTNERS(P);
     int i;
     const int r = rangeOf(s.vsize, s.hsize, s.fsize, i);
     const WC& w = s.w;
     if (r == 0) {
-        const bool gone = s.step >= 3 && mergeVertex(w, i, s.vsize, s.numV, s.exV, s.eyV, s.ctr);
+        const bool gone = s.step >= 3 && mergeVertex(w, P, i, s.vsize, s.numV, s.exV, s.eyV, s.ctr);
         s.newV[i] = (!gone && !(w.vflags[i] & VF_REMOVE) && w.v_c2o[i] == -1) ? 1 : 0;
     } else if (r == 1) {
-        if (s.step >= 3) updateVertexID(w, i, s.vsize, s.numV, s.exV, s.eyV, s.ctr);
-        if (s.step >= 4) planHalfedge(s, i);
+        if (s.step >= 3) updateVertexID(w, P, i, s.vsize, s.numV, s.exV, s.eyV, s.ctr);
+        if (s.step >= 4) planHalfedge(s, P, i);
         s.newH[i] = (!(w.hflags[i] & VF_REMOVE) && w.h_c2o[i] == -1) ? 1 : 0;
     } else if (r == 2) {
         s.newF[i] = (!(w.fflags[i] & VF_REMOVE) && w.f_c2o[i] == -1) ? 1 : 0;
     }
 }
 
-__global__ void kMergeCheck(WC w, int count, const int32_t* __restrict__ num, const int32_t* __restrict__ ex, const int32_t* __restrict__ ey,
+__global__ void __launch_bounds__(kBlock) kMergeCheck(WC w, int count, const int32_t* __restrict__ num, const int32_t* __restrict__ ex, const int32_t* __restrict__ ey,
                             const int32_t* __restrict__ firstWriter, int64_t* ctr) {
     const int h = blockIdx.x * blockDim.x + threadIdx.x;
     if (h >= count) return;
     if (w.hflags[h] & VF_REMOVE) return;
-    int P[12];
+    MDMC_PARTNERS(P);
     const int np = partnersOf(h, count, num, ex, ey, P, ctr);
     if (np == 1) return;
     for (int i = 0; i < np - 1; ++i) {
@@ -2390,11 +2516,11 @@ __global__ void kMergeCheck(WC w, int count, const int32_t* __restrict__ num, co
 }
 
 // the planned merges, or -- with a conflict -- the merges in ascending order by one thread
-__device__ void mergeSequential(const SplitStep& s) {
+__device__ void mergeSequential(const SplitStep& s, const Partners& P) {
     ++s.ctr[A_MERGE_SEQ];  // the iterations that took this pass (one thread: a plain increment)
     for (int h = 0; h < s.hsize; ++h) {
         if (s.w.hflags[h] & VF_REMOVE) continue;
-        int P[12], np;
+        int np;
         const int t = planMerge(s.w, h, s.hsize, s.numH, s.exH, s.eyH, P, np, s.ctr);
         if (t == -1 || t < h) continue;
         setT(s.w.he, h, t);
@@ -2433,13 +2559,14 @@ __device__ void moveVertexToSurface(const WC& w, int v, const ProblemDev* __rest
 // the merges' second part (halfedges, step 4) beside the vertices' part of the rest: the last
 // surviving copy of an original in ascending order writes it back, and every surviving
 // vertex moves to the surface (step 5)
-__global__ void kMergeApply(SplitStep s, const ProblemDev* __restrict__ probs) {
+__global__ void __launch_bounds__(kBlock) kMergeApply(SplitStep s, const ProblemDev* __restrict__ probs) {
+    MDMC_PARTNERS(P);
     int i;
     const int r = rangeOf(s.step >= 4 ? s.hsize : 0, s.vsize, 0, i);
     const WC& w = s.w;
     if (r == 0) {
         if (s.ctr[A_CONFLICT] != 0) {
-            if (i == 0) mergeSequential(s);
+            if (i == 0) mergeSequential(s, P);
             return;
         }
         const int t = s.valid[i];
@@ -3453,10 +3580,26 @@ void Pipeline::refreshHashTable(size_t Vm, size_t Hm, size_t Fm) {
     uint32_t* fattr = arena.ptr<uint32_t>("fattr");
     int32_t* degM = arena.ptr<int32_t>("degM");
     int32_t* dlist = arena.ptr<int32_t>("dirty_list");
-    const int64_t per = (int64_t)kBlock * kDirtyPer;
-    const int64_t records = ((int64_t)Hm + per - 1) / per;
-    kDirtyRecords<<<(unsigned)records + gridFor(((int64_t)Fm + 3) / 4), kBlock, 0, stream>>>(he, H, F, V, arena.ptr<uint8_t>("dirty_v"), dlist, records, face_he,
-                                                                                      fattr, counters());
+    const int lanePer = recordsPerLane(H);
+    const int64_t per = (int64_t)kBlock * lanePer;
+    DirtyArgs a{};
+    a.he = he;
+    a.oldH = H;
+    a.oldF = F;
+    a.oldV = V;
+    a.quads = arena.ptr<int4>("quads");
+    a.Q = Q;
+    a.canon = canonFlags();
+    a.dirtyV = arena.ptr<uint8_t>("dirty_v");
+    a.dlist = dlist;
+    a.quadBlocks = (4 * Q + per - 1) / per;
+    a.recordBlocks = ((int64_t)Hm - 4 * Q + per - 1) / per;
+    a.face_he = face_he;
+    a.fattr = fattr;
+    a.ctr = counters();
+    const unsigned blocks = (unsigned)(a.quadBlocks + a.recordBlocks) + gridFor(((int64_t)Fm + 3) / 4);
+    if (lanePer == 4) kDirtyRecords<4><<<blocks, kBlock, 0, stream>>>(a);
+    else kDirtyRecords<16><<<blocks, kBlock, 0, stream>>>(a);
     const int64_t* c = readCounters();
     if (c[A_INVALID]) throw HipError("inconsistent mesh after splitting (" + std::to_string(c[A_INVALID]) + " bad ids)", -4);
     V += c[A_ADD];
@@ -3968,7 +4111,10 @@ void Pipeline::launchDetect(int guarded) {
         // (writes every vertex's out-degree)
         kOutFromLists<<<sparseBlocks(V), kBlock, 0, stream>>>(off, out, listsV, touched, canon, V, outdeg, rep, counters(), guarded);
         if (canon) {
-            kOutDegreeMoved<<<gridFor(H), kBlock, 0, stream>>>(he, H, V, listsV, touched, canon, outdeg, rep, counters(), guarded);
+            if (recordsPerLane(H) == 4)
+                kOutDegreeMoved<4><<<gridFor((H + 3) / 4), kBlock, 0, stream>>>(he, H, V, listsV, touched, canon, outdeg, rep, counters(), guarded);
+            else
+                kOutDegreeMoved<16><<<gridFor((H + 15) / 16), kBlock, 0, stream>>>(he, H, V, listsV, touched, canon, outdeg, rep, counters(), guarded);
         } else if (touched || V > listsV) {
             kOutDegreeTouched<<<gridFor(H), kBlock, 0, stream>>>(he, H, V, listsV, touched, outdeg, rep, counters());
         }
