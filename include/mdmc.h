@@ -182,7 +182,8 @@ mdmc_status mdmc_set_graphs(mdmc_ctx* ctx, int32_t enable);
 mdmc_status mdmc_get_graph_replays(const mdmc_ctx* ctx, int64_t* replays);
 /* Local twin update in a chain of simplifications (no reference counterpart).  While another
  * simplification follows, a P3X3Y merge whose neighbourhood is a plain patch rewrites its two
- * new twin pairs directly instead of having its region's buckets rebuilt; the mesh is the same
+ * new twin pairs directly instead of having its region's buckets rebuilt, and a regular P3333
+ * merge's new quad takes over the twins of the removed ones; the mesh is the same
  * either way.  enable = 0 sends every merge through the region rebuild (default on). */
 mdmc_status mdmc_set_local_merges(mdmc_ctx* ctx, int32_t enable);
 /* Verification switch for the splitter's merge phase (no reference counterpart).  The merges

@@ -315,7 +315,7 @@ class DualMarchingCubes:
         self._check(lib().mdmc_set_graphs(self._ctx, 1 if enable else 0))
 
     def set_local_merges(self, enable):
-        """mdmc_set_local_merges: plain-patch P3X3Y merges of a simplification chain update their
+        """mdmc_set_local_merges: plain-patch P3X3Y and regular P3333 merges of a simplification chain update their
         twins directly (False: every merge's region is rebuilt; the mesh is the same)."""
         self._check(lib().mdmc_set_local_merges(self._ctx, 1 if enable else 0))
 

@@ -69,6 +69,14 @@ __device__ __forceinline__ void waveAdd(int64_t* parts, bool c) {
     if (m && (int)(threadIdx.x & 63) == __ffsll((unsigned long long)m) - 1)
         atomicAdd((unsigned long long*)&parts[(blockIdx.x % kPartSlots) * kPartStride], (unsigned long long)__popcll(m));
 }
+// and of counts, called by whole waves
+__device__ __forceinline__ void waveSum(int64_t* parts, int c) {
+    if (__ballot(c != 0) == 0) return;
+    int x = c;
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) x += __shfl_down(x, d, 64);
+    if ((threadIdx.x & 63) == 0) atomicAdd((unsigned long long*)&parts[(blockIdx.x % kPartSlots) * kPartStride], (unsigned long long)x);
+}
 __device__ __forceinline__ int64_t sumParts(const int64_t* parts, int lane) {
     int64_t v = parts[lane * kPartStride];
 #pragma unroll
@@ -719,6 +727,18 @@ __global__ void __launch_bounds__(kBlock) kBuildHalfedges(const int4* __restrict
 // and its halfedges keep size, rank and (renumbered) twin; the others are recomputed from
 // the new outgoing lists.  qnew[f] is the new id of old quad f (-1: removed).
 //
+// Most P3333 merges need no list.  The centre f becomes the quad of the four targets, and its halfedge i
+// takes the place of e_i, the outer halfedge of the removed neighbour across its edge i: same ends,
+// same direction.  A regular centre (kMark3333: each neighbour's twin is mutual and opposite, its outer
+// corners are the targets of the two inner ones) loses
+// no other halfedge between kept vertices.  Its corners' three outgoing halfedges lie in itself and two
+// neighbours, and a neighbour is no centre nor has it a second regular one: either would have
+// a target among its corners, whose valence is not 3.  So every bucket away from the
+// targets of irregular centres keeps its size, and one of one or two halfedges its members, with e_i
+// replaced by 4f + i; from e_i, that is the twin of the halfedge across its quad.  Only the targets of
+// irregular centres are touched then, and larger buckets, whose order may change, are recomputed.
+// (At the 512^3 gyroid a third of the halfedges start or end at a target, 0.8% are recomputed now.)
+//
 // Source chains (by old vertex id): the outgoing halfedges of vertex t are the entries of the
 // lists of t and of every vertex on its chain head[t], next[head[t]], ...  A dropped vertex u
 // joins its target's chain together with its own chain (vertices dropped into u by earlier
@@ -763,7 +783,8 @@ inline unsigned sparseBlocks(int64_t n) { return (unsigned)((n + kSparsePer * kB
 
 __global__ void __launch_bounds__(kBlock) kSources(const int32_t* __restrict__ vtype, const int32_t* __restrict__ vtarget,
                                                    const int32_t* __restrict__ address, int64_t V, int dropType, uint8_t* __restrict__ touched,
-                                                   int32_t* __restrict__ srcHead, int32_t* __restrict__ srcNext, int32_t* __restrict__ outdeg) {
+                                                   int32_t* __restrict__ srcHead, int32_t* __restrict__ srcNext, int32_t* __restrict__ outdeg,
+                                                   bool touch) {
     // the block's dropped vertices gathered in LDS and handled on consecutive lanes
     __shared__ int s_list[kSparsePer * kBlock];
     __shared__ int s_n;
@@ -774,7 +795,7 @@ __global__ void __launch_bounds__(kBlock) kSources(const int32_t* __restrict__ v
         if (t < 0 || t >= V) continue;
         const int tn = address[t];
         if (tn < 0) continue;  // the relabelled quads then hold -1 and fail validation
-        touched[tn] = 1;
+        if (touch) touched[tn] = 1;
         spliceChain(u, t, srcHead, srcNext);
         if (outdeg) {
             atomicAdd(&outdeg[t], outdeg[u]);
@@ -848,61 +869,111 @@ __global__ void kOutFill(const int32_t* __restrict__ oldV, int64_t Vn, const int
     }
 }
 
-// a halfedge with two untouched endpoints takes size, rank and renumbered twin from its old
+constexpr int kRebuilt = INT32_MIN;  // in place of a twin: the halfedge is recomputed
+constexpr int kOldCentre = 1 << 30;  // in oldQ: the old quad is the centre of a P3333 merge (4 Q < 2^31)
+// A halfedge with two untouched endpoints takes size, rank and renumbered twin from its old
 // halfedge; the block's other halfedges are gathered in LDS and recomputed from their
-// buckets by the block's first lanes, so that the long path runs on full waves.  The chain ends
-// here, so the finished records are written: 902 us at the 512^3 gyroid, against 783 us for
-// twins and bucket words and 315 us for a pass that turned them into records.  No barrier
-// follows the second part: waves without recomputed halfedges end early and make room (a
-// block-wide sum or an ordered store behind it: 1215-1264 us).
+// buckets afterwards on full waves.  The chain ends here, so the finished records are written.  A thread
+// takes a quad's four halfedges, so that the loads behind the old quad's id are in flight together, and
+// the records go through LDS, in order across lanes (stored by quad, every line is written
+// back in parts: 2.7 GB instead of 1.4).  Bound by HBM: 2.3 GB moved at the 512^3 gyroid in 653 us; a
+// thread per halfedge 944 us, the records stored by quad 839 us.
 __global__ void __launch_bounds__(kBlock) kRemapRebuild(const int4* __restrict__ quads2, int64_t H2, const uint8_t* __restrict__ touched,
                                                         const int32_t* __restrict__ oldQ, const int32_t* __restrict__ twinOld, int64_t Hold,
                                                         const uint32_t* __restrict__ bpackOld,
                                                         const int32_t* __restrict__ qnew, const int64_t* __restrict__ off2,
                                                         const int32_t* __restrict__ out2, int4* __restrict__ he, int32_t* __restrict__ bsize,
                                                         int32_t* __restrict__ brank, uint32_t* __restrict__ vflags, uint32_t* __restrict__ fattr,
-                                                        int64_t* nmParts, int64_t* ctr) {
-    __shared__ int s_list[kBlock];
-    __shared__ int s_wave[kBlock / 64];
-    const int64_t hh = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    bool later = false, slotted = false;
-    if (hh < H2) {
-        const int h = (int)hh;
-        // the old halfedge's twin and packed bucket are loaded alongside the touched flags
-        // (every new quad has an old one, so ho is in range either way)
-        const int4 q = quads2[h >> 2];
-        const int ho = 4 * oldQ[h >> 2] + (h & 3);
-        const int a = quadCorner(q, h & 3), b = quadCorner(q, (h + 1) & 3);
-        const int tt = twinOld[ho];
-        const uint32_t bo = bpackOld[ho];
-        if (touched[a] | touched[b]) {
-            later = true;
-        } else {
-            int t = -1;
-            if (tt >= Hold) {
-                anomaly(ctr);
-            } else if (tt >= 0) {
-                const int fo = qnew[tt >> 2];
-                if (fo < 0) anomaly(ctr);
-                else t = 4 * fo + (tt & 3);
+                                                        int64_t* nmParts, bool replace, int64_t* ctr) {
+    __shared__ __align__(16) int s_v[4 * kBlock], s_t[4 * kBlock];
+    __shared__ int s_list[4 * kBlock];
+    __shared__ int s_n;
+    if (threadIdx.x == 0) s_n = 0;
+    __syncthreads();
+    const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    int slotted = 0;
+    if (f < H2 / 4) {
+        const int4 q = quads2[f];
+        const int oq = oldQ[f];
+        const int fo = oq & ~kOldCentre;
+        const int4 t4 = reinterpret_cast<const int4*>(twinOld)[fo];
+        const uint4 b4 = reinterpret_cast<const uint4*>(bpackOld)[fo];
+        const int v[4] = {q.x, q.y, q.z, q.w};
+        int tt[4] = {t4.x, t4.y, t4.z, t4.w};
+        uint32_t bo[4] = {b4.x, b4.y, b4.z, b4.w};
+        uint8_t tc[4];
+        bool later[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) tc[i] = touched[v[i]];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) later[i] = (tc[i] | tc[(i + 1) & 3]) != 0;
+        if (replace && (oq & kOldCentre)) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (later[i]) continue;
+                if (tt[i] >= 0 && tt[i] < Hold) {  // (a centre has four neighbours)
+                    const int e = quadNext(tt[i], 2);
+                    tt[i] = twinOld[e];
+                    bo[i] = bpackOld[e];
+                } else {
+                    later[i] = true;
+                }
             }
-            slotted = storeRecord(h, a, BucketOf{(int)(bo & 0xFFFFu), (int)(bo >> 16), t}, he, bsize, brank, vflags, fattr);
         }
+        int fn[4], nb[4], rk[4], tn[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) fn[i] = tt[i] >= 0 && tt[i] < Hold ? qnew[tt[i] >> 2] : 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int h = (int)(4 * f + i);
+            nb[i] = (int)(bo[i] & 0xFFFFu);
+            rk[i] = (int)(bo[i] >> 16);
+            if (replace && nb[i] > 2) later[i] = true;
+            if (later[i]) {
+                s_list[atomicAdd(&s_n, 1)] = h;
+                tn[i] = kRebuilt;
+                continue;
+            }
+            int t = -1;
+            if (tt[i] >= Hold) {
+                anomaly(ctr);
+            } else if (tt[i] >= 0) {
+                int fo2 = fn[i];
+                if (replace && fo2 < 0) {  // an outer halfedge of a removed neighbour
+                    const int opposite = quadNext(tt[i], 2), c = twinOld[opposite];
+                    if (c >= 0 && c < Hold && twinOld[c] == opposite) {
+                        tt[i] = c;
+                        fo2 = qnew[c >> 2];
+                    }
+                }
+                if (fo2 < 0) anomaly(ctr);
+                else t = 4 * fo2 + (tt[i] & 3);
+            }
+            if (replace) rk[i] = t >= 0 && t < h ? 1 : 0;
+            tn[i] = t;
+            const uint32_t vf = bucketVertexFlag(nb[i]);
+            if (vf) atomicOr(&vflags[v[i]], vf);
+            if (nb[i] == 4) atomicOr(&fattr[f], (uint32_t)QA_NM);
+            slotted += slottedNM(nb[i], rk[i]) ? 1 : 0;
+        }
+        reinterpret_cast<int4*>(bsize)[f] = make_int4(nb[0], nb[1], nb[2], nb[3]);
+        reinterpret_cast<int4*>(brank)[f] = make_int4(rk[0], rk[1], rk[2], rk[3]);
+        reinterpret_cast<int4*>(s_v)[threadIdx.x] = q;
+        reinterpret_cast<int4*>(s_t)[threadIdx.x] = make_int4(tn[0], tn[1], tn[2], tn[3]);
     }
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const uint64_t m = __ballot(later);
-    if (lane == 0) s_wave[wid] = __popcll(m);
-    waveAdd(nmParts, slotted);
+    waveSum(nmParts, slotted);
     __syncthreads();
-    int base = 0, total = 0;
-    for (int w = 0; w < kBlock / 64; ++w) {
-        if (w < wid) base += s_wave[w];
-        total += s_wave[w];
+    // the records from LDS, in order across lanes
+    const int64_t h0 = (int64_t)blockIdx.x * (4 * kBlock);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int l = k * kBlock + threadIdx.x;
+        const int h = (int)(h0 + l);
+        if (h0 + l < H2 && s_t[l] != kRebuilt) he[h] = make_int4(s_v[l], h >> 2, quadNext(h, 1), s_t[l]);
     }
-    if (later) s_list[base + __popcll(m & ((1ULL << lane) - 1ULL))] = (int)hh;
-    __syncthreads();
-    if ((int)threadIdx.x < total) {
-        const int h = s_list[threadIdx.x];
+    const int total = s_n;
+    for (int k = threadIdx.x; k < total; k += kBlock) {
+        const int h = s_list[k];
         const int4 q = quads2[h >> 2];
         const int a = quadCorner(q, h & 3), b = quadCorner(q, (h + 1) & 3);
         waveAdd(nmParts, storeRecord(h, a, bucketFromOut(h, a, b, quads2, H2, off2, out2, ctr), he, bsize, brank, vflags, fattr));
@@ -1635,25 +1706,44 @@ __global__ void __launch_bounds__(kBlock) kMerge3x3y(const int4* __restrict__ qu
 // markElementsP3333, HalfedgeMesh.cu:547-628.  Its first half, in which every eligible face clears
 // its pattern bits before any face marks, has nothing to clear here: an initialize and a
 // deferred P3X3Y step leave eligible faces with their colour alone.
-__global__ void kMark3333(const int4* __restrict__ quads, const int32_t* __restrict__ twin, uint32_t* __restrict__ fattr, int64_t F,
-                          const int32_t* __restrict__ valence, int32_t* __restrict__ vtype, int32_t* __restrict__ vtarget, int step, const int64_t* ctr,
-                          int64_t* stamp) {
+// The faces whose four corners have valence 3, one in some thirty, are gathered in LDS and go through
+// their neighbours on full waves: 372 us with every lane going on by itself, 267 us now (512^3 gyroid).
+__global__ void __launch_bounds__(kBlock) kMark3333(const int4* __restrict__ quads, const int32_t* __restrict__ twin, uint32_t* __restrict__ fattr, int64_t F,
+                                                    const int32_t* __restrict__ valence, int32_t* __restrict__ vtype, int32_t* __restrict__ vtarget, int step,
+                                                    const int64_t* ctr, int64_t* stamp) {
     stampClock(stamp);
-    const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= F || chainHeld(ctr, step)) return;
-    const uint32_t a0 = fattr[f];
-    if ((a0 & QA_NM) || (a0 & QA_BOUNDARY) || (a0 & QA_DEAD)) return;
+    __shared__ int s_list[kBlock];
+    __shared__ int s_n;
+    if (threadIdx.x == 0) s_n = 0;
+    __syncthreads();
+    const int64_t ff = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (chainHeld(ctr, step)) return;
+    {
+        const uint32_t a0 = ff < F ? fattr[ff] : (uint32_t)QA_DEAD;
+        bool all3 = !(a0 & (QA_NM | QA_BOUNDARY | QA_DEAD));
+        if (all3) {
+            const int4 q = quads[ff];
+            const int val[4] = {valence[q.x], valence[q.y], valence[q.z], valence[q.w]};
+            for (int i = 0; i < 4; ++i) all3 = all3 && val[i] == 3;
+        }
+        const uint64_t m = __ballot(all3);
+        const int lane = threadIdx.x & 63;
+        int at = 0;
+        if (m && lane == 0) at = atomicAdd(&s_n, __popcll(m));
+        at = __shfl(at, 0, 64);
+        if (all3) s_list[at + __popcll(m & ((1ULL << lane) - 1ULL))] = (int)ff;
+    }
+    __syncthreads();
+    if ((int)threadIdx.x >= s_n) return;
+    const int64_t f = s_list[threadIdx.x];
     const int4 qv = quads[f];
     const int org[4] = {qv.x, qv.y, qv.z, qv.w};
-    // the four valences (and below the four neighbours) loaded side by side before any test
-    const int val[4] = {valence[org[0]], valence[org[1]], valence[org[2]], valence[org[3]]};
-    for (int i = 0; i < 4; ++i)
-        if (val[i] != 3) return;
+    // the four neighbours loaded side by side before any test
     const int4 tw4 = reinterpret_cast<const int4*>(twin)[f];
     const int tw[4] = {tw4.x, tw4.y, tw4.z, tw4.w};
     for (int i = 0; i < 4; ++i)
         if (tw[i] < 0) return;  // no neighbour across a boundary edge
-    int nbf[4], nbv[4], nbval[4];
+    int nbf[4], nbv[4], nbval[4], back[4];
     uint32_t na[4];
     int4 nq[4];
     for (int i = 0; i < 4; ++i) {
@@ -1671,7 +1761,16 @@ __global__ void kMark3333(const int4* __restrict__ quads, const int32_t* __restr
     bool all4 = true;
     for (int i = 0; i < 4; ++i) all4 = all4 && nbval[i] == 4;
     if (all4) return;
-    atomicOr(&fattr[f], (uint32_t)QA_PATTERN);
+    // whether halfedge i simply takes the place of neighbour i's outer one (see kRemapRebuild)
+    bool regular = true;
+    for (int i = 0; i < 4; ++i) back[i] = twin[tw[i]];
+    for (int i = 0; i < 4; ++i) {
+        const int j = (i + 1) & 3;
+        regular = regular && back[i] == (int)(4 * f + i) && nbf[i] != f && nbf[i] != nbf[j] && nbf[i] != nbf[(i + 2) & 3];
+        regular = regular && quadCorner(nq[i], tw[i] & 3) == org[j] && quadCorner(nq[i], (tw[i] + 1) & 3) == org[i];
+        regular = regular && quadCorner(nq[i], (tw[i] + 3) & 3) == nbv[j];
+    }
+    atomicOr(&fattr[f], (uint32_t)(regular ? QA_PATTERN : QA_PATTERN | QA_ODD));
     for (int i = 0; i < 4; ++i) {
         atomicOr(&fattr[nbf[i]], (uint32_t)QA_REMOVE);
         const int v = org[i];
@@ -1773,12 +1872,24 @@ __global__ void __launch_bounds__(kLbBlock) kNumber(NumberArgs a) {
 }
 
 // removeQuadrilateralsP3X3Y (p3333 = 0) / removeQuadsP3333 (p3333 = 1), HalfedgeMesh.cu:513-538, :657-683
+// (touchTargets: the new vertices an irregular or removed P3333 centre's corners move to)
+__device__ __forceinline__ void touchTargets(const int4& q, const int32_t* __restrict__ vtarget, const int32_t* __restrict__ address, int64_t V,
+                                             uint8_t* __restrict__ touched) {
+    for (int i = 0; i < 4; ++i) {
+        const int v = quadCorner(q, i);
+        const int t = v >= 0 && v < V ? vtarget[v] : -1;
+        const int tn = t >= 0 && t < V ? address[t] : -1;
+        if (tn >= 0) touched[tn] = 1;
+    }
+}
 // quad q, kept (new id d) or removed (a quad is removed when it has the remove or the dead bit)
 __device__ __forceinline__ void compactQuad(int64_t q, bool kept, int64_t d, const int4* __restrict__ quads, const uint32_t* __restrict__ attr,
                                             const int32_t* __restrict__ vtarget, const int32_t* __restrict__ address, int p3333,
                                             int4* __restrict__ nquads, uint32_t* __restrict__ nattr, uint32_t* __restrict__ nfattr,
-                                            int32_t* __restrict__ face_he, int32_t* __restrict__ oldQ, int32_t* __restrict__ removedAt, int32_t* __restrict__ outdeg, int64_t V, int64_t* ctr) {
+                                            int32_t* __restrict__ face_he, int32_t* __restrict__ oldQ, int32_t* __restrict__ removedAt, int32_t* __restrict__ outdeg, uint8_t* __restrict__ touched,
+                                            int64_t V, int64_t* ctr) {
     if (!kept) {
+        if (p3333 && (attr[q] & QA_PATTERN)) touchTargets(quads[q], vtarget, address, V, touched);
         // the outgoing halfedges this quad takes from its corners' lists (when the lists are
         // by current corner; a quad dead since an earlier step of the chain takes none)
         if (!(attr[q] & QA_DEAD)) {
@@ -1807,6 +1918,7 @@ __device__ __forceinline__ void compactQuad(int64_t q, bool kept, int64_t d, con
     int o[4];
     bool bad = false;
     const bool pat = p3333 && (a & QA_PATTERN) != 0;
+    if (pat && (a & QA_ODD)) touchTargets(v4, vtarget, address, V, touched);
 #pragma unroll
     for (int i = 0; i < 4; ++i) o[i] = (v[i] >= 0 && v[i] < V && !pat) ? address[v[i]] : -1;
 #pragma unroll
@@ -1826,18 +1938,18 @@ __device__ __forceinline__ void compactQuad(int64_t q, bool kept, int64_t d, con
     nattr[d] = na;
     nfattr[d] = na;
     face_he[d] = (int32_t)(4 * d);
-    oldQ[d] = (int32_t)q;
+    oldQ[d] = (int32_t)q | (pat ? kOldCentre : 0);
 }
 
 // removeQuadrilateralsP3X3Y / removeQuadsP3333 from the numbering, one thread per quad
 __global__ void kCompactQuads(const int4* __restrict__ quads, const uint32_t* __restrict__ attr, int64_t Q, const int32_t* __restrict__ vtarget,
                               const int32_t* __restrict__ address, int p3333, int4* __restrict__ nquads, uint32_t* __restrict__ nattr,
                               uint32_t* __restrict__ nfattr, int32_t* __restrict__ face_he, int32_t* __restrict__ oldQ, const int32_t* __restrict__ qnew, int32_t* __restrict__ removedAt,
-                              int32_t* __restrict__ outdeg, int64_t V, int step, int64_t* ctr) {
+                              int32_t* __restrict__ outdeg, uint8_t* __restrict__ touched, int64_t V, int step, int64_t* ctr) {
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= Q || chainHeld(ctr, step)) return;
     const int32_t d = qnew[q];
-    compactQuad(q, d >= 0, d, quads, attr, vtarget, address, p3333, nquads, nattr, nfattr, face_he, oldQ, removedAt, outdeg, V, ctr);
+    compactQuad(q, d >= 0, d, quads, attr, vtarget, address, p3333, nquads, nattr, nfattr, face_he, oldQ, removedAt, outdeg, touched, V, ctr);
 }
 
 // ---------------------------------------------------------------- fixManifoldTwins
@@ -3810,7 +3922,7 @@ void Pipeline::launchCompaction() {
     }
     if (Q > 0)
         kCompactQuads<<<gridFor(Q), kBlock, 0, stream>>>(quads, attr, Q, vtarget, address, p3333 ? 1 : 0, nquads, nattr, nfattr, face_he, oldQ, qnew,
-                                                         removedAt, outdeg, V, step, counters());
+                                                         removedAt, outdeg, touched, V, step, counters());
 }
 
 // the compacted mesh's lists and records, once its sizes are known
@@ -3841,7 +3953,8 @@ void Pipeline::finishChain() {
     // outgoing lists are the old ones of each new vertex's own and relabelled vertices,
     // renumbered; halfedges with untouched endpoints keep their bucket results
     const int64_t nH = 4 * nQ;
-    if (V > 0) kSources<<<sparseBlocks(V), kBlock, 0, stream>>>(vtype, vtarget, address, V, dropType, touched, srcHead, srcNext, outdeg);
+    if (V > 0) kSources<<<sparseBlocks(V), kBlock, 0, stream>>>(vtype, vtarget, address, V, dropType, touched, srcHead, srcNext, outdeg,
+                                                              !(p3333 && localMerges));  // else kCompactQuads touched what there is to touch
     const int64_t* off = arena.ptr<int64_t>("out_off");
     const int32_t* out = arena.ptr<int32_t>("out_list");
     if (nV > 0) kOutCount<<<gridFor(nV), kBlock, 0, stream>>>(oldV, nV, off, removedAt, srcHead, srcNext, outdeg, cnt, arena.ptr<float>("pos"),
@@ -3857,8 +3970,8 @@ void Pipeline::finishChain() {
     int32_t* brank = arena.get<int32_t>("brank", (size_t)std::max<int64_t>(nH, 1));
     // (the partial sums of slotted halfedges are clear since the extraction's start)
     if (nH > 0)
-        kRemapRebuild<<<gridFor(nH), kBlock, 0, stream>>>(nquads, nH, touched, oldQ, arena.ptr<int32_t>("twin"), H, arena.ptr<uint32_t>("bpack"),
-                                                         qnew, off2, out2, he, bsize, brank, vflags, nfattr, nmSlotParts(), counters());
+        kRemapRebuild<<<gridFor(nQ), kBlock, 0, stream>>>(nquads, nH, touched, oldQ, arena.ptr<int32_t>("twin"), H, arena.ptr<uint32_t>("bpack"),
+                                                         qnew, off2, out2, he, bsize, brank, vflags, nfattr, nmSlotParts(), p3333 && localMerges, counters());
     arena.swap("pos", "pos2");
     arena.swap("nrm", "nrm2");
     arena.swap("quads", "quads2");
