@@ -367,6 +367,13 @@ __device__ __forceinline__ void scanCounts(const uint32_t* s_rec, int NA, uint16
     QT = tot >> 16;
 }
 
+// A value that is the same in every lane but came from vector memory, into scalar registers
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ int64_t uniform(int64_t v) {
+    return (int64_t)(((uint64_t)(uint32_t)uniform((int)((uint64_t)v >> 32)) << 32) | (uint32_t)uniform((int)(uint32_t)v));
+}
+__device__ __forceinline__ float uniform(float v) { return __int_as_float(uniform(__float_as_int(v))); }
+
 struct TileCtx {
     int64_t t;
     int prob;
@@ -379,14 +386,15 @@ template <int TILE>
 __device__ __forceinline__ TileCtx tileCtxOf(const GridPassArgs& a, int64_t t) {
     TileCtx c;
     c.t = t;
-    c.prob = problemOfTile(a.probs, a.nProblems, c.t);
+    c.prob = a.nProblems > 1 ? uniform(problemOfTile(a.probs, a.nProblems, c.t)) : 0;
     const ProblemDev& P = a.probs[c.prob];
-    c.c0 = (c.t - P.tileBase) * TILE;
-    c.gc0 = P.cellBase + c.c0;
-    const int64_t r0 = c.c0 / P.CX;
-    c.tb.x0 = (int)(c.c0 - r0 * P.CX);
-    c.tb.y0 = (int)(r0 % P.CY);
-    c.tb.z0 = (int)(r0 / P.CY);
+    c.c0 = (c.t - uniform(P.tileBase)) * TILE;
+    c.gc0 = uniform(P.cellBase) + c.c0;
+    // (a grid has fewer than 2^31 cells: 32-bit divisions, ahead of everything else in a tile)
+    const unsigned CX = (unsigned)uniform(P.CX), CY = (unsigned)uniform(P.CY), c0 = (unsigned)c.c0, r0 = c0 / CX, z0 = r0 / CY;
+    c.tb.x0 = uniform((int)(c0 - r0 * CX));
+    c.tb.y0 = uniform((int)(r0 - z0 * CY));
+    c.tb.z0 = uniform((int)z0);
     return c;
 }
 
@@ -400,7 +408,7 @@ __device__ __forceinline__ int64_t nextTile(const GridPassArgs& a, int slot, int
     if (!QUEUE) return iter == 0 ? tileOfBlock(blockIdx.x, a.numTiles, chunked != 0) : -1;
     if (threadIdx.x == 0) *s_t = atomicAdd((unsigned long long*)&a.queue[slot], 1ULL);
     __syncthreads();
-    const int64_t t = *s_t;
+    const int64_t t = uniform(*s_t);
     return t < a.numTiles ? t : -1;
 }
 
@@ -421,108 +429,223 @@ __device__ __forceinline__ void stampClassify(const GridPassArgs& a) {
     for (int i = threadIdx.x; i < (int)a.lbWords; i += blockDim.x) a.lb[i] = 0;
 }
 
-// ---- classify: active cells of one tile, their records, counts and map entries
+// The MC cases of a tile's cells.  A wave's 64 consecutive cells (a run) compare their four x corners, and
+// the x + 1 corners are the ballots shifted by a lane, except in lane 63 and at a row's end.  Where a row
+// has 64 cells or more that is at most one more lane, and one load by eight lanes covers the eight corners;
+// the run then starts in one row and ends in it or the next, and its place is kept in scalar
+// registers.  In shorter rows, and in the grid's last tile, every lane finds its own cell, and those at
+// an end read their own corners.  Whether a cell is active is bit arithmetic on the ballots, in scalar
+// registers, and only waves with active cells build cases.  Returns whether the wave has an active cell.
+typedef const __attribute__((address_space(1))) char GlobalBytes;
+template <int CPT>
+__device__ __forceinline__ bool classifyRuns(const GridDev& g, float iso, int CX, int CY, const TileBase& tb, int64_t c0, int64_t C,
+                                             unsigned long long* s_mask, unsigned long long* s_edgy, uint8_t* s_mc) {
+    const int tid = threadIdx.x, lane = tid & 63, wid = uniform(tid >> 6);
+    const int64_t nx4 = 4 * (int64_t)g.nx, nxy4 = nx4 * g.ny;
+    constexpr int kAhead = CPT < 8 ? CPT : 8;  // runs whose loads are in flight together
+    auto at = [](GlobalBytes* q, unsigned bytes) { return *(GlobalFloat*)(q + bytes); };
+    uint64_t some = 0;
+    // run k's masks, collected in lane k and stored together
+    int maskLo = 0, maskHi = 0, edgyLo = 0, edgyHi = 0;
+    auto keep = [&](int k, uint64_t m, uint64_t edgy) {
+        const bool me = lane == k;
+        maskLo = me ? (int)m : maskLo;
+        maskHi = me ? (int)(m >> 32) : maskHi;
+        edgyLo = me ? (int)edgy : edgyLo;
+        edgyHi = me ? (int)(edgy >> 32) : edgyHi;
+    };
+    // bits 0, 2, 4, 6 of a case from four corners
+    auto bits = [&](const float c[4]) {
+        return (c[0] >= iso ? 1 : 0) | (c[1] >= iso ? 4 : 0) | (c[2] >= iso ? 16 : 0) | (c[3] >= iso ? 64 : 0);
+    };
+    auto spread = [](unsigned n) {
+        n = (n | (n << 2)) & 0x33u;
+        return (int)((n | (n << 1)) & 0x55u);
+    };
+    if (CX >= 64 && c0 + CPT * GP_THREADS <= C) {
+        // the run's first cell
+        int x = tb.x0 + wid * 64, y = tb.y0;
+        GlobalBytes* q = (GlobalBytes*)fieldOf(g) + (tb.z0 * nxy4 + tb.y0 * nx4 + 4 * (int64_t)(tb.x0 + wid * 64));
+        const int64_t corner = 4 + ((lane & 1) ? nx4 : 0) + ((lane & 2) ? nxy4 : 0);
+        auto settle = [&]() {  // past a row's end: a row has one point more than cells, a slice one row
+            while (x >= CX) {
+                x -= CX;
+                q += 4;
+                if (++y == CY) {
+                    y = 0;
+                    q += nx4;
+                }
+            }
+        };
+#pragma unroll 1
+        for (int k0 = 0; k0 < CPT; k0 += kAhead) {
+            float c[kAhead][4], ce[kAhead];
+            int turn[kAhead];
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) {
+                settle();
+                // lanes from `turn` on lie in the next row
+                turn[k] = CX - x;
+                const int skip = y + 1 == CY ? 4 + (int)nx4 : 4;
+                const unsigned o = 4u * lane + (lane >= turn[k] ? (unsigned)skip : 0u);
+                GlobalBytes* qz = q + nxy4;
+                const unsigned oy = o + (unsigned)nx4;
+                c[k][0] = at(q, o);
+                c[k][1] = at(q, oy);
+                c[k][2] = at(qz, o);
+                c[k][3] = at(qz, oy);
+                const unsigned oEnd = 4u * (unsigned)(min(turn[k], 64) - 1), oLast = 4u * 63u + (turn[k] < 64 ? (unsigned)skip : 0u);
+                ce[k] = -INFINITY;
+                if (lane < 8) ce[k] = *(GlobalFloat*)(q + corner + ((lane & 4) ? oLast : oEnd));
+                x += GP_THREADS;
+                q += 4 * GP_THREADS;
+            }
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) {
+                const uint64_t b0 = __ballot(c[k][0] >= iso), b1 = __ballot(c[k][1] >= iso), b2 = __ballot(c[k][2] >= iso), b3 = __ballot(c[k][3] >= iso);
+                const uint32_t e = (uint32_t)__ballot(ce[k] >= iso) & 0xFFu;  // (an iso-value of -infinity: lanes 8 to 63 count)
+                const uint64_t any4 = b0 | b1 | b2 | b3, all4 = b0 & b1 & b2 & b3;
+                if ((any4 == 0 && e == 0) || (all4 == ~0ULL && e == 0xFFu)) continue;  // all outside or all inside
+                const int end = min(turn[k], 64) - 1;
+                const uint64_t mEnd = 1ULL << end, mLast = 1ULL << 63;
+                uint64_t any = any4 | ((any4 >> 1) & ~mEnd), all = (all4 >> 1) & ~mEnd;
+                any |= (e & 15u) ? mEnd : 0ULL;
+                any |= e > 15u ? mLast : 0ULL;
+                all |= (e & 15u) == 15u ? mEnd : 0ULL;
+                all |= e >= 0xF0u ? mLast : 0ULL;
+                const uint64_t m = any & ~(all4 & all);
+                if (m == 0) continue;
+                some |= m;
+                keep(k0 + k, m, __ballot(c[k][0] < iso));
+                const int own = bits(c[k]);
+                int next = __builtin_amdgcn_mov_dpp(own, 0x130, 0xF, 0xF, true);  // wave_shl: 1: the next lane's
+                next = lane == 63 ? spread(e >> 4) : next;
+                next = lane == end ? spread(e & 15u) : next;
+                if ((m >> lane) & 1ULL) s_mc[(k0 + k) * GP_THREADS + tid] = (uint8_t)(own | (next << 1));
+            }
+        }
+    } else {
+        const SmallDiv dX = smallDiv((unsigned)CX), dY = smallDiv((unsigned)CY);
+        GlobalBytes* q = (GlobalBytes*)fieldOf(g) + (tb.z0 * nxy4 + tb.y0 * nx4 + 4 * (int64_t)tb.x0);
+        constexpr int N = 4;
+#pragma unroll 1
+        for (int k0 = 0; k0 < CPT; k0 += N) {
+            float c[N][4], ce[N][4];
+            uint64_t ends[N];
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+                const int l = (k0 + k) * GP_THREADS + tid;
+                int x, y, z;
+                tileCellXYZ(tb, l, dX, dY, x, y, z);
+                // (cells past the grid's end read the tile's first cell and are dropped)
+                const int64_t o = c0 + l < C ? (z - tb.z0) * nxy4 + (y - tb.y0) * nx4 + 4 * (int64_t)(x - tb.x0) : 0;
+                c[k][0] = *(GlobalFloat*)(q + o);
+                c[k][1] = *(GlobalFloat*)(q + o + nx4);
+                c[k][2] = *(GlobalFloat*)(q + o + nxy4);
+                c[k][3] = *(GlobalFloat*)(q + o + nxy4 + nx4);
+                const bool end = x == CX - 1 || lane == 63;
+                ends[k] = __ballot(end);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) ce[k][j] = 0.f;
+                if (end) {
+                    ce[k][0] = *(GlobalFloat*)(q + o + 4);
+                    ce[k][1] = *(GlobalFloat*)(q + o + nx4 + 4);
+                    ce[k][2] = *(GlobalFloat*)(q + o + nxy4 + 4);
+                    ce[k][3] = *(GlobalFloat*)(q + o + nxy4 + nx4 + 4);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+                const int l = (k0 + k) * GP_THREADS + tid;
+                const int own = bits(c[k]), extra = bits(ce[k]);
+                int next = __builtin_amdgcn_mov_dpp(own, 0x130, 0xF, 0xF, true);
+                if ((ends[k] >> lane) & 1ULL) next = extra;
+                const int mc = own | (next << 1);
+                const uint64_t m = __ballot(mc != 0 && mc != 255 && c0 + l < C);
+                if (m == 0) continue;
+                some |= m;
+                keep(k0 + k, m, __ballot(c[k][0] < iso));
+                s_mc[l] = (uint8_t)mc;
+            }
+        }
+    }
+    if (lane < CPT) {
+        s_mask[lane * GP_WAVES + wid] = ((uint64_t)(uint32_t)maskHi << 32) | (uint32_t)maskLo;
+        s_edgy[lane * GP_WAVES + wid] = ((uint64_t)(uint32_t)edgyHi << 32) | (uint32_t)edgyLo;
+    }
+    return some != 0;
+}
+
+// ---- classify: active cells of one tile, their records, counts and map entries.  Bound by
+// instruction issue, vector and scalar (one per CU and cycle each): some 440 vector instructions per
+// wave of an empty 2048-cell tile, 780 with eight corner loads and compares per cell.  Tiles
+// without an active cell end at the first barrier.  Padded 512^3 gyroid (12% of the cells active)
+// 555 us, 256^3 blobs (1%) 49 us; eight corners per cell and a case for every cell 612 and 58
+// us; the x + 1 corners' bits inserted one corner at a time, 150 scalar instructions a run, 754 and 82 us.
+// Bounds: 80 registers, six waves per SIMD; 64 spill (665 us), 102 as the compiler likes 640 us.
 template <int CPT, bool QUEUE>
-__global__ void __launch_bounds__(GP_THREADS) kClassify(GridPassArgs a, int chunked) {
+__global__ void __launch_bounds__(GP_THREADS, 6) kClassify(GridPassArgs a, int chunked) {
     constexpr int TILE = GP_THREADS * CPT, RUNS = TILE / 64;
     __shared__ uint32_t s_rec[TILE];
     __shared__ uint32_t s_base[256];          // c_polyBase
     __shared__ uint32_t s_tab[kPolyTabSize];  // c_polyCmap
-    __shared__ uint16_t s_cell[TILE];
-    __shared__ uint16_t s_vpre[TILE];
-    __shared__ uint16_t s_mc[TILE];  // MC case of each tile cell | edgy << 8
-    __shared__ unsigned long long s_mask[RUNS];
-    __shared__ int s_mpre[RUNS + 1];
+    __shared__ uint16_t s_idx[TILE];          // the active cells, then the records' first vertices
+    __shared__ uint8_t s_mc[TILE];            // MC case of each active cell
+    __shared__ unsigned long long s_mask[RUNS], s_edgy[RUNS];
     __shared__ int s_wave[GP_WAVES];
 
     __shared__ int64_t s_t;
+    uint16_t *s_cell = s_idx, *s_vpre = s_idx;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wid = tid >> 6;
     stampClassify(a);
-    // the two small tables in LDS (read after the first barrier below)
-    s_base[tid] = c_polyBase[tid];
-    for (int i = tid; i < kPolyTabSize; i += GP_THREADS) s_tab[i] = c_polyCmap[i];
     for (int iter = 0;; ++iter) {
     const int64_t tile = nextTile<QUEUE>(a, 0, chunked, iter, &s_t);
     if (tile < 0) break;
     const TileCtx tc = tileCtxOf<TILE>(a, tile);
     const ProblemDev& P = a.probs[tc.prob];
-    const GridDev g = P.g;
-    const float iso = P.iso;
-    const int CX = P.CX, CY = P.CY;
-    const int64_t C = P.cells;
-
-    // MC case of every cell; a ballot per run of 64 cells marks the active ones.  This thread's
-    // cells are GP_THREADS apart: their coordinates advance from the first one's, with no
-    // division per cell.  Cells past the grid's end (last tile only) read cell 0 and are
-    // dropped, so that every corner load is issued before the first compare.
-    const SmallDiv dX = smallDiv((unsigned)CX), dY = smallDiv((unsigned)CY);
-    int cx[CPT], cy[CPT], cz[CPT];
-    tileCellXYZ(tc.tb, tid, dX, dY, cx[0], cy[0], cz[0]);
-#pragma unroll
-    for (int k = 1; k < CPT; ++k) {
-        cx[k] = cx[k - 1];
-        cy[k] = cy[k - 1];
-        cz[k] = cz[k - 1];
-        if (CX >= GP_THREADS) {  // at most one row boundary per step
-            cx[k] += GP_THREADS;
-            if (cx[k] >= CX) {
-                cx[k] -= CX;
-                if (++cy[k] == CY) {
-                    cy[k] = 0;
-                    ++cz[k];
-                }
-            }
-        } else {
-            tileCellXYZ(tc.tb, k * GP_THREADS + tid, dX, dY, cx[k], cy[k], cz[k]);
+    GridDev g;
+    g.v = (const float*)(intptr_t)uniform((int64_t)(intptr_t)P.g.v);
+    g.nx = uniform(P.g.nx);
+    g.ny = uniform(P.g.ny);
+    const float iso = uniform(P.iso);
+    const int CX = uniform(P.CX), CY = uniform(P.CY);
+    const bool active = classifyRuns<CPT>(g, iso, CX, CY, tc.tb, tc.c0, uniform(P.cells), s_mask, s_edgy, s_mc);
+    if (!__syncthreads_or(active ? 1 : 0)) {
+        if (tid == 0) {
+            a.tileV[tc.t] = a.tileQ[tc.t] = a.tileNA[tc.t] = 0;
+            if (tc.t == a.numTiles - 1) a.tileV[a.numTiles] = a.tileQ[a.numTiles] = 0;
         }
+        continue;
     }
-    float cs[CPT][8];
+    // the two small tables in LDS (read after the next barrier)
+    s_base[tid] = c_polyBase[tid];
+    for (int i = tid; i < kPolyTabSize; i += GP_THREADS) s_tab[i] = c_polyCmap[i];
+    // every wave scans the runs' counts
+    const int rc = lane < RUNS ? __popcll(s_mask[lane]) : 0;
+    int rx = rc;
 #pragma unroll
-    for (int k = 0; k < CPT; ++k) {
-        const bool in = tc.c0 + k * GP_THREADS + tid < C;
-        loadCorners(g, in ? cx[k] : 0, in ? cy[k] : 0, in ? cz[k] : 0, cs[k]);
+    for (int d = 1; d < RUNS; d <<= 1) {
+        const int v = __shfl_up(rx, d, 64);
+        if (lane >= d) rx += v;
     }
-#pragma unroll
-    for (int k = 0; k < CPT; ++k) {
-        const int l = k * GP_THREADS + tid;
-        int mc = 0, edgy = 0;
-        if (tc.c0 + l < C) {
-#pragma unroll
-            for (int q = 0; q < 8; ++q) mc |= (cs[k][q] >= iso ? 1 : 0) << q;
-            edgy = cs[k][0] < iso ? 1 : 0;
-        }
-        const uint64_t m = __ballot(mc != 0 && mc != 255);
-        if (lane == 0) s_mask[k * GP_WAVES + wid] = m;
-        s_mc[l] = (uint16_t)(mc | (edgy << 8));
-    }
-    __syncthreads();
-    if (tid < 64) {
-        const int v = tid < RUNS ? __popcll(s_mask[tid]) : 0;
-        int x = v;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int y = __shfl_up(x, d, 64);
-            if (tid >= d) x += y;
-        }
-        if (tid < RUNS) s_mpre[tid] = x - v;
-        if (tid == RUNS - 1) s_mpre[RUNS] = x;
-    }
-    __syncthreads();
-    const int NA = s_mpre[RUNS];
+    const int NA = __shfl(rx, RUNS - 1, 64);
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
         const int run = k * GP_WAVES + wid;
         const uint64_t m = s_mask[run];
-        if ((m >> lane) & 1ULL) s_cell[s_mpre[run] + __popcll(m & ((1ULL << lane) - 1ULL))] = (uint16_t)(k * GP_THREADS + tid);
+        const int first = __shfl(rx - rc, run, 64);
+        if ((m >> lane) & 1ULL) s_cell[first + __popcll(m & ((1ULL << lane) - 1ULL))] = (uint16_t)(k * GP_THREADS + tid);
     }
     __syncthreads();
 
     // records of the active cells, every lane busy: the corners are loaded again only for the
     // cases with an ambiguous face (the decider reads them); owned edges come from the case
+    const SmallDiv dX = smallDiv((unsigned)CX), dY = smallDiv((unsigned)CY);
+#pragma unroll 1
     for (int ai = tid; ai < NA; ai += GP_THREADS) {
         const int l = s_cell[ai];
-        const int mce = s_mc[l], mc = mce & 0xFF;
+        const int mc = s_mc[l], edgy = (int)(s_edgy[l >> 6] >> (l & 63)) & 1;
         int x, y, z;
         tileCellXYZ(tc.tb, l, dX, dY, x, y, z);
         const uint32_t b = s_base[mc];
@@ -532,7 +655,7 @@ __global__ void __launch_bounds__(GP_THREADS) kClassify(GridPassArgs a, int chun
             loadCorners(g, x, y, z, s);
             idx = deciderIndex(b, s, iso);
         }
-        const int own = ownedBitsCase(mc, mce >> 8, x, y, z);
+        const int own = ownedBitsCase(mc, edgy, x, y, z);
         s_rec[ai] = (uint32_t)idx | ((uint32_t)l << 10) | ((uint32_t)own << 22) | ((s_tab[idx] >> 24) << 26);
     }
     __syncthreads();
@@ -541,6 +664,7 @@ __global__ void __launch_bounds__(GP_THREADS) kClassify(GridPassArgs a, int chun
     __syncthreads();
 
     const int64_t rb = tc.t * TILE;
+#pragma unroll 1
     for (int ai = tid; ai < NA; ai += GP_THREADS) {
         const uint32_t r = s_rec[ai];
         a.rec[rb + ai] = r;
@@ -555,7 +679,7 @@ __global__ void __launch_bounds__(GP_THREADS) kClassify(GridPassArgs a, int chun
             a.tileQ[a.numTiles] = 0;
         }
     }
-    __syncthreads();  // the next tile reuses the block's LDS
+    if (QUEUE) __syncthreads();  // the next tile reuses the block's LDS
     }
 }
 
@@ -573,16 +697,20 @@ __global__ void __launch_bounds__(GP_THREADS) kEmit(GridPassArgs a, int chunked)
     __shared__ int64_t s_t;
     stampClock(a.stampEmit);
     const int tid = threadIdx.x;
-    for (int i = tid; i < kPolyTabSize; i += GP_THREADS) s_tab[i] = c_polyCmap[i];
     for (int iter = 0;; ++iter) {
     const int64_t tile = nextTile<QUEUE>(a, 1, chunked, iter, &s_t);
     if (tile < 0) break;
+    const int NA = a.tileNA[tile];
+    if (NA == 0 && !a.adjMap) {
+        if (QUEUE) __syncthreads();
+        continue;
+    }
+    for (int i = tid; i < kPolyTabSize; i += GP_THREADS) s_tab[i] = c_polyCmap[i];
     const TileCtx tc = tileCtxOf<TILE>(a, tile);
     const ProblemDev& P = a.probs[tc.prob];
     const int CX = P.CX, CY = P.CY;
     const int64_t C = P.cells;
     const int64_t c0 = tc.c0;
-    const int NA = a.tileNA[tc.t];
     const int64_t rb = tc.t * TILE;
     if (a.adjMap) {
         for (int l = tid; l < TILE; l += GP_THREADS) s_aidx[l] = 0xFFFF;
