@@ -277,13 +277,13 @@ struct MoveArgs {
     RegroupArgs r;
     const float *pos, *nrm;
     const uint32_t *vflags, *fattr;
-    const int32_t *bsize, *brank;
+    const int32_t* bsize;
     const uint8_t* canon;
     const int64_t* listOff;  // the outgoing lists of the last initialize's vertices (the prefix)
     const int32_t* list;
     float *npos, *nnrm;
     uint32_t *nvflags, *nfattr;
-    int32_t *npid, *nbsize, *nbrank, *nface_he, *vh;
+    int32_t *npid, *nface_he, *vh;
     int4* nhe;
     unsigned long long* out;
     int* bad;
@@ -314,18 +314,16 @@ __global__ void __launch_bounds__(kBlock) kRegroup(MoveArgs a, int64_t chunk) {
         const int p = !live ? 0 : (one ? pbase : problemOf(i));
         const int64_t d = !live ? 0 : (MOVE ? newId(r, KIND, p, (int)i) : i);
         if (KIND == RG_H) {
-            int nb = 0, rk = 1;
+            int w = 0;
             if (live) {
-                nb = a.bsize[i];
-                rk = a.brank[i];
+                w = a.bsize[i];
                 if (MOVE) {
                     const int4 e = r.he[i];
                     a.nhe[d] = make_int4(newId(r, RG_V, p, e.x), newId(r, RG_F, p, e.y), newId(r, RG_H, p, e.z), e.w >= 0 ? newId(r, RG_H, p, e.w) : e.w);
-                    a.nbsize[d] = nb;
-                    a.nbrank[d] = rk;
                 }
             }
-            const bool count = live && rk == 0;
+            const bool count = live && bucketFirst(w);
+            const int nb = bucketSize(w);
             statAdd(acc, a.out, count, p, pbase, 0, 0, nb == 4);
             statAdd(acc, a.out, count, p, pbase, 1, 1, nb == 3);
             statAdd(acc, a.out, count, p, pbase, 2, 2, nb > 0);
@@ -337,11 +335,11 @@ __global__ void __launch_bounds__(kBlock) kRegroup(MoveArgs a, int64_t chunk) {
                 const int q4 = h0 & ~3;
                 if (q4 + 3 < r.n[RG_H] && (!a.canon || *reinterpret_cast<const uint32_t*>(a.canon + q4) == 0x01010101u)) {
                     const int4 s = reinterpret_cast<const int4*>(a.bsize)[q4 >> 2];
-                    k = (s.x > 2) + (s.y > 2) + (s.z > 2) + (s.w > 2);
+                    k = (bucketSize(s.x) > 2) + (bucketSize(s.y) > 2) + (bucketSize(s.z) > 2) + (bucketSize(s.w) > 2);
                 } else {
                     int h = h0;
                     for (int j = 0; j < 4; ++j) {
-                        if (a.bsize[h] > 2) ++k;
+                        if (bucketSize(a.bsize[h]) > 2) ++k;
                         h = ((const int*)r.he)[4 * (int64_t)h + 2];
                     }
                 }
@@ -496,7 +494,6 @@ void Pipeline::regroupBatch(int B) {
     m.vflags = arena.ptr<uint32_t>("vflags");
     m.fattr = arena.ptr<uint32_t>("fattr");
     m.bsize = arena.ptr<int32_t>("bsize");
-    m.brank = arena.ptr<int32_t>("brank");
     m.canon = canonFlags();
     m.listOff = arena.ptr<int64_t>("out_off");
     m.list = arena.ptr<int32_t>("out_list");
@@ -511,14 +508,12 @@ void Pipeline::regroupBatch(int B) {
         m.nvflags = arena.get<uint32_t>("vflags2", nv);
         m.npid = arena.get<int32_t>("pid2", nv);
         m.nhe = arena.get<int4>("he2", nh);
-        m.nbsize = arena.get<int32_t>("bsize2", nh);
-        m.nbrank = arena.get<int32_t>("brank2", nh);
         m.nface_he = arena.get<int32_t>("face_he2", nf);
         m.nfattr = arena.get<uint32_t>("fattr2", nf);
         if (H > 0) kRegroup<RG_H, true><<<chunks(H), kBlock, 0, stream>>>(m, statChunk(H));
         if (F > 0) kRegroup<RG_F, true><<<chunks(F), kBlock, 0, stream>>>(m, statChunk(F));
         if (V > 0) kRegroup<RG_V, true><<<chunks(V), kBlock, 0, stream>>>(m, statChunk(V));
-        for (const char* name : {"pos", "nrm", "vflags", "pid", "he", "bsize", "brank", "face_he", "fattr"}) arena.swap(name, std::string(name) + "2");
+        for (const char* name : {"pos", "nrm", "vflags", "pid", "he", "face_he", "fattr"}) arena.swap(name, std::string(name) + "2");
     } else {
         if (H > 0) kRegroup<RG_H, false><<<chunks(H), kBlock, 0, stream>>>(m, statChunk(H));
         if (F > 0) kRegroup<RG_F, false><<<chunks(F), kBlock, 0, stream>>>(m, statChunk(F));

@@ -270,6 +270,14 @@ __device__ __forceinline__ void movePointToSurface(const float* s, float iso, f3
 // QuadrilateralAttribute bits (DeviceVectors.h:334-450) and vertex Flags bits (Halfedge.h:14-111).
 // QA_DEAD has no reference counterpart: a quad removed by an earlier simplification of a chain
 // whose compaction is deferred to the chain's last step (never in an output array).
+// A halfedge's bucket word: the bucket's size and whether the halfedge is its first member (rank 0).
+// The rank itself lies in an array of its own and is written, and read, for buckets of four and
+// more only: nothing else asks for it (4 bytes per halfedge less to write and to read back).
+constexpr int kFirstOfBucket = (int)0x80000000u;
+__device__ __forceinline__ int bucketWord(int n, int rank) { return rank == 0 ? n | kFirstOfBucket : n; }
+__device__ __forceinline__ int bucketSize(int word) { return word & ~kFirstOfBucket; }
+__device__ __forceinline__ bool bucketFirst(int word) { return word < 0; }
+
 enum : uint32_t { QA_COLOR = 0x1F, QA_NM = 0x20, QA_PATTERN = 0x40, QA_REMOVE = 0x80, QA_BOUNDARY = 0x100, QA_DEAD = 0x200,
                   QA_ODD = 0x400 /* a P3333 centre whose twins are not replaced by the rule (within that step) */ };
 enum : uint32_t { VF_NM = 1, VF_BOUNDARY = 2, VF_WEIRD = 4, VF_FANS = 8, VF_REMOVE = 16 };

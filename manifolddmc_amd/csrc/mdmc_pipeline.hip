@@ -436,8 +436,8 @@ __global__ void kBuckets(const int32_t* __restrict__ dlist, const int32_t* __res
         if (f.y < key) ++rk;
     }
     const int h = dlist[t];
-    bsize[h] = n;
-    brank[h] = rk;
+    bsize[h] = bucketWord(n, rk);
+    if (n >= 4) brank[h] = rk;
 }
 
 // vertex flags and face NM bits from the bucket sizes of all halfedges (vflags and the
@@ -446,12 +446,12 @@ __global__ void kBuckets(const int32_t* __restrict__ dlist, const int32_t* __res
 __device__ __forceinline__ void sizes4(const int32_t* __restrict__ bsize, int64_t H, int64_t h0, int n[4]) {
     if (h0 + 3 < H) {
         const int4 v = reinterpret_cast<const int4*>(bsize)[h0 >> 2];
-        n[0] = v.x;
-        n[1] = v.y;
-        n[2] = v.z;
-        n[3] = v.w;
+        n[0] = bucketSize(v.x);
+        n[1] = bucketSize(v.y);
+        n[2] = bucketSize(v.z);
+        n[3] = bucketSize(v.w);
     } else {
-        for (int j = 0; j < 4; ++j) n[j] = h0 + j < H ? bsize[h0 + j] : 2;
+        for (int j = 0; j < 4; ++j) n[j] = h0 + j < H ? bucketSize(bsize[h0 + j]) : 2;
     }
 }
 __global__ void __launch_bounds__(kBlock) kFlagsFromBuckets(const int4* __restrict__ he, int64_t H, const int32_t* __restrict__ bsize,
@@ -669,8 +669,8 @@ __device__ __forceinline__ bool storeRecord(int h, int a, const BucketOf& bk, in
                                            int32_t* __restrict__ brank, uint32_t* __restrict__ vflags, uint32_t* __restrict__ fattr) {
     const int n = min(bk.n, 0xFFFF), r = min(bk.rank, 0xFFFF);
     he[h] = make_int4(a, h >> 2, quadNext(h, 1), bk.twin);
-    bsize[h] = n;
-    brank[h] = r;
+    bsize[h] = bucketWord(n, r);
+    if (n >= 4) brank[h] = r;
     const uint32_t vf = bucketVertexFlag(n);
     if (vf) atomicOr(&vflags[a], vf);
     if (n == 4) atomicOr(&fattr[h >> 2], (uint32_t)QA_NM);
@@ -955,9 +955,10 @@ __global__ void __launch_bounds__(kBlock) kRemapRebuild(const int4* __restrict__
             if (vf) atomicOr(&vflags[v[i]], vf);
             if (nb[i] == 4) atomicOr(&fattr[f], (uint32_t)QA_NM);
             slotted += slottedNM(nb[i], rk[i]) ? 1 : 0;
+            if (nb[i] >= 4) brank[h] = rk[i];
         }
-        reinterpret_cast<int4*>(bsize)[f] = make_int4(nb[0], nb[1], nb[2], nb[3]);
-        reinterpret_cast<int4*>(brank)[f] = make_int4(rk[0], rk[1], rk[2], rk[3]);
+        reinterpret_cast<int4*>(bsize)[f] =
+            make_int4(bucketWord(nb[0], rk[0]), bucketWord(nb[1], rk[1]), bucketWord(nb[2], rk[2]), bucketWord(nb[3], rk[3]));
         reinterpret_cast<int4*>(s_v)[threadIdx.x] = q;
         reinterpret_cast<int4*>(s_t)[threadIdx.x] = make_int4(tn[0], tn[1], tn[2], tn[3]);
     }
@@ -2255,7 +2256,7 @@ __global__ void __launch_bounds__(kBlock) kWcUpdate(int n4, const int32_t* __res
         }
         w.he[c] = e;
         const int hh = w.h_orig[c];
-        const int n = bsize[hh];
+        const int n = bucketSize(bsize[hh]);
         if (n >= 4 && slottedNM(n, brank[hh])) {
             w.hflags[c] |= VF_NM;
             atomicOr(&w.vflags[e.x], (uint32_t)VF_NM);
@@ -2881,8 +2882,7 @@ __global__ void __launch_bounds__(kBlock) kDetectFans(const int4* __restrict__ h
 // ---------------------------------------------------------------- statistics
 // counts over the vertex-pair buckets (HalfedgeMesh.cu:1164-1239, ManifoldCreator.cu:545-549)
 __global__ void __launch_bounds__(kBlock) kStats(const int4* __restrict__ he, int64_t H, const int32_t* __restrict__ face_he, int64_t F,
-                                                 const int32_t* __restrict__ bsize, const int32_t* __restrict__ brank, const uint32_t* __restrict__ vflags,
-                                                 int64_t V, const uint8_t* __restrict__ canon, int64_t* ctr, int64_t* pin, int guarded) {
+                                                 const int32_t* __restrict__ bsize, const uint32_t* __restrict__ vflags, int64_t V, const uint8_t* __restrict__ canon, int64_t* ctr, int64_t* pin, int guarded) {
     if (notYet(ctr, guarded)) {
         if (blockIdx.x == 0 && threadIdx.x < 64) handOver(ctr, pin);
         return;
@@ -2894,46 +2894,54 @@ __global__ void __launch_bounds__(kBlock) kStats(const int4* __restrict__ he, in
     __syncthreads();
     unsigned int loc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
-    auto bucket = [&](int r, int n) {
-        if (r != 0) return;
+    auto bucket = [&](int w) {
+        if (!bucketFirst(w)) return;
+        const int n = bucketSize(w);
         loc[0] += (n == 4);
         loc[1] += (n == 3);
         loc[2] += (n > 0);
     };
-    // buckets: four halfedges per 16-byte load, then the tail
-    const int64_t H4 = H >> 2;
-#pragma unroll 4
-    for (int64_t i = t0; i < H4; i += stride) {
-        const int4 r = reinterpret_cast<const int4*>(brank)[i];
-        const int4 n = reinterpret_cast<const int4*>(bsize)[i];
-        bucket(r.x, n.x);
-        bucket(r.y, n.y);
-        bucket(r.z, n.z);
-        bucket(r.w, n.w);
-    }
-    for (int64_t i = 4 * H4 + t0; i < H; i += stride) bucket(brank[i], bsize[i]);
-    // faces: a face whose four records all keep the build's layout is the four halfedges of
-    // one quad slot (next = quadNext from any of them), read with one load; others are walked
-    for (int64_t f = t0; f < F; f += stride) {
-        int h = face_he[f];
-        const int q4 = h & ~3;
-        int k = 0;
-        if (q4 + 3 < H && (!canon || *reinterpret_cast<const uint32_t*>(canon + q4) == 0x01010101u)) {
-            const int4 n = reinterpret_cast<const int4*>(bsize)[q4 >> 2];
-            k = (n.x > 2) + (n.y > 2) + (n.z > 2) + (n.w > 2);
-        } else {
-            for (int j = 0; j < 4; ++j) {
-                if (bsize[h] > 2) ++k;
-                h = nextOf(he, canon, h);
-            }
-        }
-        // (constant indices only: a computed index would put loc in scratch memory)
+    // the number of a face's edges in buckets of three and more
+    // (constant indices only: a computed index would put loc in scratch memory)
+    auto face = [&](int k) {
         loc[3] += k == 0;
         loc[4] += k == 1;
         loc[5] += k == 2;
         loc[6] += k == 3;
         loc[7] += k == 4;
+    };
+    auto wide = [&](const int4& w) { return (bucketSize(w.x) > 2) + (bucketSize(w.y) > 2) + (bucketSize(w.z) > 2) + (bucketSize(w.w) > 2); };
+    // four halfedges per 16-byte load, then the tail; a face whose four records, the ones of its own
+    // id, all keep the build's layout is those four halfedges, counted from the same load (read
+    // again by face they cost 245 MB of the 512^3 gyroid's 675)
+    const int64_t H4 = H >> 2, n4 = H4 > F ? H4 : F;
+#pragma unroll 4
+    for (int64_t i = t0; i < n4; i += stride) {
+        int4 w = make_int4(0, 0, 0, 0);
+        if (i < H4) {
+            w = reinterpret_cast<const int4*>(bsize)[i];
+            bucket(w.x);
+            bucket(w.y);
+            bucket(w.z);
+            bucket(w.w);
+        }
+        if (i < F) {
+            int h = face_he[i];
+            const int64_t q = h >> 2;
+            if (4 * q + 3 < H && (!canon || reinterpret_cast<const uint32_t*>(canon)[q] == 0x01010101u)) {
+                if (q != i) w = reinterpret_cast<const int4*>(bsize)[q];
+                face(wide(w));
+            } else {
+                int k = 0;
+                for (int j = 0; j < 4; ++j) {
+                    if (bucketSize(bsize[h]) > 2) ++k;
+                    h = nextOf(he, canon, h);
+                }
+                face(k);
+            }
+        }
     }
+    for (int64_t i = 4 * H4 + t0; i < H; i += stride) bucket(bsize[i]);
     for (int64_t v = t0; v < V; v += stride) loc[8] += (vflags[v] & VF_FANS) ? 1u : 0u;
     for (int k = 0; k < 9; ++k) {
         unsigned int v = loc[k];
@@ -4277,7 +4285,7 @@ void Pipeline::launchStats(int guarded) {
     pinHost()[kPinDone] = 0;
     const int64_t blocks = std::min<int64_t>(gridFor(n, 4 * kBlock), std::max<int64_t>(256, std::min<int64_t>(n / (16 * kBlock), 2048)));
     kStats<<<(unsigned)blocks, kBlock, 0, stream>>>(
-        arena.ptr<int4>("he"), H, arena.ptr<int32_t>("face_he"), F, arena.ptr<int32_t>("bsize"), arena.ptr<int32_t>("brank"),
+        arena.ptr<int4>("he"), H, arena.ptr<int32_t>("face_he"), F, arena.ptr<int32_t>("bsize"),
         arena.ptr<uint32_t>("vflags"), V, canonFlags(), counters(), pinDev() + kPinFinal, guarded);
     MDMC_HIP(hipGetLastError());
 }
