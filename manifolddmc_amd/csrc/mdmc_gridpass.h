@@ -64,11 +64,12 @@ void launchPrepareGrids(const PrepareDesc& one, const PrepareDesc* descDev, int 
 // the exact blend of every grid, after a plain copy that raised *special (no refinement)
 void launchPrepareExact(const PrepareDesc& one, const PrepareDesc* descDev, int G, int64_t rows, int pad, hipStream_t s);
 
-// What a chain of simplifications starts from, per vertex: no type and target, the valence (the
+// What a chain of simplifications starts from, per vertex: no type (a target is read only behind a type, which is set with it), the valence (the
 // out-degree until the bucket pass adds boundary halfedges); count (pattern counts of the old
 // P3X3Y rule) and, when more than one step follows, the deferred steps' arrays; null: not needed
 struct ChainInit {
-    int32_t *vtype, *vtarget, *valence, *count;
+    uint8_t* vtype;
+    int32_t *valence, *count;
     int32_t *head, *outdeg, *bdin;
     uint8_t *vdead, *touched;
 };

@@ -1134,7 +1134,6 @@ __global__ void __launch_bounds__(GP_THREADS) kVertices(GridPassArgs a, int chun
         a.outdeg[v] = deg;
         if (a.chain.vtype) {
             a.chain.vtype[v] = 0;
-            a.chain.vtarget[v] = -1;
             a.chain.valence[v] = deg;
             if (a.chain.count) a.chain.count[v] = 0;
             if (a.chain.head) {

@@ -781,7 +781,7 @@ __device__ __forceinline__ int gatherSparse(int64_t n, Pred pred, int* s_list, i
 }
 inline unsigned sparseBlocks(int64_t n) { return (unsigned)((n + kSparsePer * kBlock - 1) / (kSparsePer * kBlock)); }
 
-__global__ void __launch_bounds__(kBlock) kSources(const int32_t* __restrict__ vtype, const int32_t* __restrict__ vtarget,
+__global__ void __launch_bounds__(kBlock) kSources(const uint8_t* __restrict__ vtype, const int32_t* __restrict__ vtarget,
                                                    const int32_t* __restrict__ address, int64_t V, int dropType, uint8_t* __restrict__ touched,
                                                    int32_t* __restrict__ srcHead, int32_t* __restrict__ srcNext, int32_t* __restrict__ outdeg,
                                                    bool touch) {
@@ -1015,7 +1015,7 @@ __device__ __forceinline__ bool pattern2(const int v[4]) { return v[0] >= 5 && v
 // -1 and marks it dead.  For a local merge the two corners holding z in N_A and N_Z are
 // recorded (zslot) for kDropVertices; a fallback merge's target relabels through z's lists.
 __global__ void __launch_bounds__(kBlock) kLocalMerge(int4* __restrict__ quads, uint32_t* qattr, uint32_t* fattr, int64_t Q,
-                                                      const int32_t* __restrict__ valence, const int32_t* __restrict__ vtype,
+                                                      const int32_t* __restrict__ valence, const uint8_t* __restrict__ vtype,
                                                       const int32_t* __restrict__ vtarget, int32_t* __restrict__ twin, uint32_t* __restrict__ bpack,
                                                       int32_t* __restrict__ outdeg, int2* __restrict__ zslot, int64_t V, uint8_t* __restrict__ touched,
                                                       int allowLocal, int step, int64_t* ctr) {
@@ -1108,15 +1108,14 @@ __global__ void __launch_bounds__(kBlock) kLocalMerge(int4* __restrict__ quads, 
 }
 
 // the end of a deferred step: valence = out-degree + incoming boundary halfedges, and the next
-// step's start (types, targets, touched flags, the old rule's counts when that is next)
+// step's start (types, touched flags, the old rule's counts when that is next)
 __global__ void kStepEnd(const int32_t* __restrict__ outdeg, const int32_t* __restrict__ bdin, int64_t V, int32_t* __restrict__ valence,
-                         int32_t* __restrict__ vtype, int32_t* __restrict__ vtarget, uint8_t* __restrict__ touched, int32_t* __restrict__ count, int step,
+                         uint8_t* __restrict__ vtype, uint8_t* __restrict__ touched, int32_t* __restrict__ count, int step,
                          const int64_t* ctr) {
     const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= V || chainHeld(ctr, step + 1)) return;
     valence[v] = outdeg[v] + bdin[v];
     vtype[v] = 0;
-    vtarget[v] = -1;
     touched[v] = 0;
     if (count) count[v] = 0;
 }
@@ -1129,7 +1128,7 @@ __global__ void kStepEnd(const int32_t* __restrict__ outdeg, const int32_t* __re
 // compacting path.
 // (the dropped vertices of a block are gathered in LDS and handled on consecutive lanes: each
 // one's work is a chain of dependent loads, which sparse lanes would spread over every wave)
-__device__ __forceinline__ void dropVertex(int u, const int32_t* __restrict__ vtype, const int32_t* __restrict__ vtarget, int64_t V, int dropType,
+__device__ __forceinline__ void dropVertex(int u, const uint8_t* __restrict__ vtype, const int32_t* __restrict__ vtarget, int64_t V, int dropType,
                                            int4* __restrict__ quads, int64_t H, const int64_t* __restrict__ off, const int32_t* __restrict__ out,
                                            uint8_t* __restrict__ vdead, int32_t* __restrict__ head, int32_t* __restrict__ next,
                                            int32_t* __restrict__ outdeg, const int2* __restrict__ zslot, int64_t* ctr) {
@@ -1162,7 +1161,7 @@ __device__ __forceinline__ void dropVertex(int u, const int32_t* __restrict__ vt
     outdeg[u] = 0;
 }
 
-__global__ void __launch_bounds__(kBlock) kDropVertices(const int32_t* __restrict__ vtype, const int32_t* __restrict__ vtarget, int64_t V,
+__global__ void __launch_bounds__(kBlock) kDropVertices(const uint8_t* __restrict__ vtype, const int32_t* __restrict__ vtarget, int64_t V,
                                                         int dropType, int4* __restrict__ quads, int64_t H, const int64_t* __restrict__ off,
                                                         const int32_t* __restrict__ out, uint8_t* __restrict__ vdead, int32_t* __restrict__ head,
                                                         int32_t* __restrict__ next, int32_t* __restrict__ outdeg, const int2* __restrict__ zslot,
@@ -1616,7 +1615,7 @@ __global__ void kCount3x3yOld(const int4* __restrict__ quads, uint32_t* __restri
 // HalfedgeMesh.cu:368-388 (markTarget: the target gets vtype kTargetType, for the deferred steps'
 // local twin update)
 constexpr int kTargetType = 4;
-__device__ __forceinline__ void handleMerge(float* pos, float* nrm, int32_t* vtype, int32_t* vtarget, int x, int y, int z, int w,
+__device__ __forceinline__ void handleMerge(float* pos, float* nrm, uint8_t* vtype, int32_t* vtarget, int x, int y, int z, int w,
                                             int markTarget) {
     const int64_t sx = x, sy = y, sw = w;
     f3 p = mk3(pos[3 * sy], pos[3 * sy + 1], pos[3 * sy + 2]);
@@ -1654,7 +1653,7 @@ __device__ __forceinline__ bool neighborFaces(const int32_t* __restrict__ twin, 
 // mergeVerticesP3X3YColor (colour = 1) and mergeVerticesP3X3Y (colour = 0), HalfedgeMesh.cu:391-498
 __global__ void __launch_bounds__(kBlock) kMerge3x3y(const int4* __restrict__ quads, uint32_t* __restrict__ qattr, int64_t Q, const int32_t* __restrict__ twin,
                            const int32_t* __restrict__ valence, const int32_t* __restrict__ count,
-                           float* __restrict__ pos, float* __restrict__ nrm, int32_t* __restrict__ vtype, int32_t* __restrict__ vtarget, int colour,
+                           float* __restrict__ pos, float* __restrict__ nrm, uint8_t* __restrict__ vtype, int32_t* __restrict__ vtarget, int colour,
                            int markTarget, int step, const int64_t* ctr) {
     if (chainHeld(ctr, step)) return;
     // the block's pattern quads gathered in LDS and handled on consecutive lanes (each is a
@@ -1710,7 +1709,7 @@ __global__ void __launch_bounds__(kBlock) kMerge3x3y(const int4* __restrict__ qu
 // The faces whose four corners have valence 3, one in some thirty, are gathered in LDS and go through
 // their neighbours on full waves: 372 us with every lane going on by itself, 267 us now (512^3 gyroid).
 __global__ void __launch_bounds__(kBlock) kMark3333(const int4* __restrict__ quads, const int32_t* __restrict__ twin, uint32_t* __restrict__ fattr, int64_t F,
-                                                    const int32_t* __restrict__ valence, int32_t* __restrict__ vtype, int32_t* __restrict__ vtarget, int step,
+                                                    const int32_t* __restrict__ valence, uint8_t* __restrict__ vtype, int32_t* __restrict__ vtarget, int step,
                                                     const int64_t* ctr, int64_t* stamp) {
     stampClock(stamp);
     __shared__ int s_list[kBlock];
@@ -1789,7 +1788,7 @@ __global__ void __launch_bounds__(kBlock) kMark3333(const int4* __restrict__ qua
 // otherwise).  The arrays the following kernels start from (touched, flags, the list lengths' end;
 // the chain heads and removal counts of a chain of one) are cleared along the way.
 struct NumberArgs {
-    const int32_t* vtype;
+    const uint8_t* vtype;
     int64_t V;
     int dropType;
     const uint8_t* vdead;
@@ -1888,7 +1887,7 @@ __device__ __forceinline__ void compactQuad(int64_t q, bool kept, int64_t d, con
                                             const int32_t* __restrict__ vtarget, const int32_t* __restrict__ address, int p3333,
                                             int4* __restrict__ nquads, uint32_t* __restrict__ nattr, uint32_t* __restrict__ nfattr,
                                             int32_t* __restrict__ face_he, int32_t* __restrict__ oldQ, int32_t* __restrict__ removedAt, int32_t* __restrict__ outdeg, uint8_t* __restrict__ touched,
-                                            int64_t V, int64_t* ctr) {
+                                            const uint8_t* __restrict__ vdead, int64_t V, int64_t* ctr) {
     if (!kept) {
         if (p3333 && (attr[q] & QA_PATTERN)) touchTargets(quads[q], vtarget, address, V, touched);
         // the outgoing halfedges this quad takes from its corners' lists (when the lists are
@@ -1926,7 +1925,8 @@ __device__ __forceinline__ void compactQuad(int64_t q, bool kept, int64_t d, con
     for (int i = 0; i < 4; ++i) {
         const bool in = v[i] >= 0 && v[i] < V;
         if (in && (pat || (!p3333 && o[i] < 0))) {
-            const int src = vtarget[v[i]];
+            // (a vertex that died in an earlier step has no target)
+            const int src = !pat && vdead && vdead[v[i]] ? -1 : vtarget[v[i]];
             o[i] = (src >= 0 && src < V) ? address[src] : -1;
         }
         bad = bad || o[i] < 0;  // a dropped vertex or a missing target: the quad is invalid
@@ -1946,11 +1946,12 @@ __device__ __forceinline__ void compactQuad(int64_t q, bool kept, int64_t d, con
 __global__ void kCompactQuads(const int4* __restrict__ quads, const uint32_t* __restrict__ attr, int64_t Q, const int32_t* __restrict__ vtarget,
                               const int32_t* __restrict__ address, int p3333, int4* __restrict__ nquads, uint32_t* __restrict__ nattr,
                               uint32_t* __restrict__ nfattr, int32_t* __restrict__ face_he, int32_t* __restrict__ oldQ, const int32_t* __restrict__ qnew, int32_t* __restrict__ removedAt,
-                              int32_t* __restrict__ outdeg, uint8_t* __restrict__ touched, int64_t V, int step, int64_t* ctr) {
+                              int32_t* __restrict__ outdeg, uint8_t* __restrict__ touched, const uint8_t* __restrict__ vdead, int64_t V, int step,
+                              int64_t* ctr) {
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= Q || chainHeld(ctr, step)) return;
     const int32_t d = qnew[q];
-    compactQuad(q, d >= 0, d, quads, attr, vtarget, address, p3333, nquads, nattr, nfattr, face_he, oldQ, removedAt, outdeg, touched, V, ctr);
+    compactQuad(q, d >= 0, d, quads, attr, vtarget, address, p3333, nquads, nattr, nfattr, face_he, oldQ, removedAt, outdeg, touched, vdead, V, ctr);
 }
 
 // ---------------------------------------------------------------- fixManifoldTwins
@@ -3322,8 +3323,8 @@ void Pipeline::emitArgs(GridPassArgs& a, int64_t C, bool recordAdjoint) {
     a.vflags = arena.get<uint32_t>("vflags", (size_t)std::max<int64_t>(V, 1));
     if (!chain.empty()) {
         const size_t nv = (size_t)std::max<int64_t>(V, 1);
-        a.chain.vtype = arena.get<int32_t>("vtype", nv);
-        a.chain.vtarget = arena.get<int32_t>("vtarget", nv);
+        a.chain.vtype = arena.get<uint8_t>("vtype", nv);
+        arena.get<int32_t>("vtarget", nv);
         a.chain.valence = arena.get<int32_t>("valence", nv);
         if (std::count(chain.begin(), chain.end(), (int)S_OLD)) a.chain.count = arena.get<int32_t>("vcount", nv);
         if (chain.size() > 1) {
@@ -3793,7 +3794,7 @@ void Pipeline::launchChain(int from, bool ended) {
     int32_t* twin = arena.ptr<int32_t>("twin");
     int32_t* valence = arena.ptr<int32_t>("valence");
     int32_t* count = arena.ptr<int32_t>("vcount");
-    int32_t* vtype = arena.ptr<int32_t>("vtype");
+    uint8_t* vtype = arena.ptr<uint8_t>("vtype");
     int32_t* vtarget = arena.ptr<int32_t>("vtarget");
     const size_t nv = (size_t)V;
     for (int k = from; k < (int)chain.size(); ++k) {
@@ -3821,7 +3822,7 @@ void Pipeline::launchChain(int from, bool ended) {
             }
         }
         if (!last)
-            kStepEnd<<<gridFor(V), kBlock, 0, stream>>>(arena.ptr<int32_t>("outdeg"), arena.ptr<int32_t>("bdin"), V, valence, vtype, vtarget,
+            kStepEnd<<<gridFor(V), kBlock, 0, stream>>>(arena.ptr<int32_t>("outdeg"), arena.ptr<int32_t>("bdin"), V, valence, vtype,
                                                         arena.ptr<uint8_t>("touched"), chain[k + 1] == S_OLD ? count : nullptr, k, counters());
     }
     launchCompaction();
@@ -3856,7 +3857,7 @@ void Pipeline::launchCompaction() {
     const bool p3333 = chain[step] == S_3333, chained = step > 0;
     const int dropType = p3333 ? 1 : 3;
     // the chain's last step: this step's removals and the dead elements of the earlier ones
-    int32_t* vtype = arena.ptr<int32_t>("vtype");
+    uint8_t* vtype = arena.ptr<uint8_t>("vtype");
     int32_t* vtarget = arena.ptr<int32_t>("vtarget");
     const uint32_t* attr = p3333 ? arena.ptr<uint32_t>("fattr") : arena.ptr<uint32_t>("qattr");
     // vertex and quad compaction, each one pass (look-back over tiles), with one read-back of
@@ -3930,7 +3931,7 @@ void Pipeline::launchCompaction() {
     }
     if (Q > 0)
         kCompactQuads<<<gridFor(Q), kBlock, 0, stream>>>(quads, attr, Q, vtarget, address, p3333 ? 1 : 0, nquads, nattr, nfattr, face_he, oldQ, qnew,
-                                                         removedAt, outdeg, touched, V, step, counters());
+                                                         removedAt, outdeg, touched, chained ? arena.ptr<uint8_t>("vdead") : nullptr, V, step, counters());
 }
 
 // the compacted mesh's lists and records, once its sizes are known
@@ -3942,7 +3943,7 @@ void Pipeline::finishChain() {
     const int64_t nV = h[1], nQ = h[2];
     if (nV < 0 || nV > V || nQ < 0 || nQ > Q) throw HipError("inconsistent compaction counts", -4);
     const size_t capQ = (size_t)std::max(Q, dmcQ);
-    const int32_t* vtype = arena.ptr<int32_t>("vtype");
+    const uint8_t* vtype = arena.ptr<uint8_t>("vtype");
     const int32_t* vtarget = arena.ptr<int32_t>("vtarget");
     const int32_t* address = arena.ptr<int32_t>("vaddress");
     const int32_t* oldV = arena.ptr<int32_t>("oldV");
