@@ -683,15 +683,22 @@ __global__ void __launch_bounds__(GP_THREADS, 6) kClassify(GridPassArgs a, int c
     }
 }
 
-// ---- emit: the tile's dual vertices and the quads its cells own, one active cell per thread
+// ---- emit: the tile's dual vertices, one active cell per thread, and the quads its cells own, one
+// quad per thread (a cell owns none to three; walked by their cell's thread, a wave took three
+// rounds of look-ups for one or two).  Bound by the latency of those look-ups: what is the same for
+// all lanes is kept in scalar registers, and 67 vector registers leave six waves per SIMD.
+// Padded 512^3 gyroid 445 us, 256^3 blobs 25; a cell per thread 617 and 31; a quad per thread with 64-bit
+// cell numbers in 85 registers 562 and 31.
+constexpr int kEmitQuads = 1024;
 template <int CPT, bool QUEUE>
-__global__ void __launch_bounds__(GP_THREADS) kEmit(GridPassArgs a, int chunked) {
+__global__ void __launch_bounds__(GP_THREADS, 6) kEmit(GridPassArgs a, int chunked) {
     constexpr int TILE = GP_THREADS * CPT;
     __shared__ uint32_t s_rec[TILE];
     __shared__ uint32_t s_tab[kPolyTabSize];  // c_polyCmap: per table entry the contour of each crossed edge
     __shared__ uint16_t s_vpre[TILE];
     __shared__ uint16_t s_qpre[TILE];
     __shared__ uint16_t s_aidx[TILE];  // per tile cell: its active index (0xFFFF: inactive, adjoint map only)
+    __shared__ uint16_t s_quad[kEmitQuads];  // per quad of the current round: its cell's active index | axis << 12
     __shared__ int s_wave[GP_WAVES];
 
     __shared__ int64_t s_t;
@@ -708,9 +715,11 @@ __global__ void __launch_bounds__(GP_THREADS) kEmit(GridPassArgs a, int chunked)
     for (int i = tid; i < kPolyTabSize; i += GP_THREADS) s_tab[i] = c_polyCmap[i];
     const TileCtx tc = tileCtxOf<TILE>(a, tile);
     const ProblemDev& P = a.probs[tc.prob];
-    const int CX = P.CX, CY = P.CY;
-    const int64_t C = P.cells;
+    const int CX = uniform(P.CX), CY = uniform(P.CY);
+    const int64_t C = uniform(P.cells);
     const int64_t c0 = tc.c0;
+    const uint32_t* __restrict__ cellMap = a.cellMap + uniform(P.cellBase);
+    const int64_t* __restrict__ tileVOff = a.tileVOff + uniform(P.tileBase);
     const int64_t rb = tc.t * TILE;
     if (a.adjMap) {
         for (int l = tid; l < TILE; l += GP_THREADS) s_aidx[l] = 0xFFFF;
@@ -725,7 +734,7 @@ __global__ void __launch_bounds__(GP_THREADS) kEmit(GridPassArgs a, int chunked)
     int VT, QT;
     scanCounts<CPT>(s_rec, NA, s_vpre, s_qpre, s_wave, VT, QT);
     __syncthreads();
-    const int64_t voff = a.tileVOff[tc.t], qoff = a.tileQOff[tc.t];
+    const int64_t voff = uniform(a.tileVOff[tc.t]), qoff = uniform(a.tileQOff[tc.t]);
 
     // for the adjoint: cell -> (first vertex << 2 | contours - 1), -1 for empty cells
     if (a.adjMap) {
@@ -738,66 +747,81 @@ __global__ void __launch_bounds__(GP_THREADS) kEmit(GridPassArgs a, int chunked)
         }
     }
 
+    // per vertex: its cell, table entry and contour; kVertices computes position and normal.  The
+    // quads a cell owns go to the list, a round of them at a time (one, but for very dense tiles).
     const SmallDiv dX = smallDiv((unsigned)CX), dY = smallDiv((unsigned)CY);
+    for (int q0 = 0; q0 < QT || q0 == 0; q0 += kEmitQuads) {
+    if (q0 > 0) __syncthreads();
     for (int ai = tid; ai < NA; ai += GP_THREADS) {
         const uint32_t r = s_rec[ai];
-        const int l = recCell(r);
-        const uint32_t cmap = s_tab[recIndex(r)];
-        // per vertex: its cell, table entry and contour; kVertices computes position and normal
-        const int nv = recVerts(r);
-        const int64_t v0 = voff + s_vpre[ai];
-        for (int t = 0; t < nv; ++t) {
-            a.vcell[v0 + t] = (int)(c0 + l);
-            a.vct[v0 + t] = (uint16_t)(recIndex(r) | (t << 10));
-            if (a.vpid) a.vpid[v0 + t] = tc.prob;
+        if (q0 == 0) {
+            const int nv = recVerts(r);
+            const int64_t v0 = voff + s_vpre[ai];
+            for (int t = 0; t < nv; ++t) {
+                a.vcell[v0 + t] = (int)(c0 + recCell(r));
+                a.vct[v0 + t] = (uint16_t)(recIndex(r) | (t << 10));
+                if (a.vpid) a.vpid[v0 + t] = tc.prob;
+            }
         }
-        // quads whose edge starts at this cell.  Their other cells lie 1, CX, CX+1, CX*CY,
-        // CX*CY+1 or CX*CY+CX cells back: in this tile (LDS) or an earlier one (map).
         const int own = recOwn(r);
-        if ((own & 7) == 0) continue;
-        int x, y, z;
-        tileCellXYZ(tc.tb, l, dX, dY, x, y, z);
-        const int edgy = (own >> 3) & 1;
-        int64_t q = qoff + s_qpre[ai];
+        int q = s_qpre[ai] - q0;
+#pragma unroll
         for (int axis = 0; axis < 3; ++axis) {
             if (!((own >> axis) & 1)) continue;
-            // own edge, then (dx, dy, dz, edge) of the three other cells around it, packed
-            // 4 bits each (dx | dy<<1 | dz<<2, edge) per cell: x: (y-1: e2) (z-1: e4) (y-1,z-1: e6);
-            // y: (x-1: e1) (z-1: e7) (x-1,z-1: e5); z: (x-1: e9) (y-1: e11) (x-1,y-1: e10)
-            const int ownE = axis == 0 ? 0 : (axis == 1 ? 3 : 8);
-            const uint32_t nbTable = axis == 0 ? 0x664422u : (axis == 1 ? 0x557411u : 0xA3B291u);
-            int s0 = -1, s1 = -1, s2 = -1, s3 = -1;
-            {
-                const int sl = edgeSlot(ownE, edgy);
-                const int vid = (int)(v0 + (int)((cmap >> (2 * ownE)) & 3u));
-                s0 = sl == 0 ? vid : s0;
-                s1 = sl == 1 ? vid : s1;
-                s2 = sl == 2 ? vid : s2;
-                s3 = sl == 3 ? vid : s3;
-            }
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const uint32_t ent = (nbTable >> (8 * k)) & 0xFFu;
-                const int d = (int)(ent & 0xF), e = (int)(ent >> 4);
-                const int64_t n = (int64_t)(z - ((d >> 2) & 1)) * CX * CY + (int64_t)(y - ((d >> 1) & 1)) * CX + (x - (d & 1));
-                int vid;
-                if (n >= c0) {
-                    const int an = s_aidx[n - c0];
-                    vid = (int)(voff + s_vpre[an] + (int)((s_tab[recIndex(s_rec[an])] >> (2 * e)) & 3u));
-                } else {
-                    const uint32_t m = a.cellMap[P.cellBase + n];
-                    vid = (int)(a.tileVOff[P.tileBase + n / TILE] + (int64_t)(m & 0x3FFFu) + mapContour(m, e));
-                }
-                const int sl = edgeSlot(e, edgy);
-                s0 = sl == 0 ? vid : s0;
-                s1 = sl == 1 ? vid : s1;
-                s2 = sl == 2 ? vid : s2;
-                s3 = sl == 3 ? vid : s3;
-            }
-            a.quads[q] = make_int4(s0, s1, s2, s3);
-            a.qattr[q] = (uint32_t)(3 * ((x & 1) | ((y & 1) << 1) | ((z & 1) << 2)) + axis);
+            if (q >= 0 && q < kEmitQuads) s_quad[q] = (uint16_t)(ai | (axis << 12));
             ++q;
         }
+    }
+    __syncthreads();
+    // quads whose edge starts at an own cell, one per thread.  Their other cells lie 1, CX, CX+1, CX*CY,
+    // CX*CY+1 or CX*CY+CX cells back: in this tile (LDS) or an earlier one (map).
+    const int round = QT - q0 < kEmitQuads ? QT - q0 : kEmitQuads;
+    for (int qi = tid; qi < round; qi += GP_THREADS) {
+        const int ai = s_quad[qi] & 0xFFF, axis = s_quad[qi] >> 12;
+        const uint32_t r = s_rec[ai];
+        const uint32_t cmap = s_tab[recIndex(r)];
+        const int v0 = (int)voff + s_vpre[ai];
+        int x, y, z;
+        tileCellXYZ(tc.tb, recCell(r), dX, dY, x, y, z);
+        const int edgy = (recOwn(r) >> 3) & 1;
+        // own edge, then (dx, dy, dz, edge) of the three other cells around it, packed
+        // 4 bits each (dx | dy<<1 | dz<<2, edge) per cell: x: (y-1: e2) (z-1: e4) (y-1,z-1: e6);
+        // y: (x-1: e1) (z-1: e7) (x-1,z-1: e5); z: (x-1: e9) (y-1: e11) (x-1,y-1: e10)
+        const int ownE = axis == 0 ? 0 : (axis == 1 ? 3 : 8);
+        const uint32_t nbTable = axis == 0 ? 0x664422u : (axis == 1 ? 0x557411u : 0xA3B291u);
+        int s0 = -1, s1 = -1, s2 = -1, s3 = -1;
+        {
+            const int sl = edgeSlot(ownE, edgy);
+            const int vid = v0 + (int)((cmap >> (2 * ownE)) & 3u);
+            s0 = sl == 0 ? vid : s0;
+            s1 = sl == 1 ? vid : s1;
+            s2 = sl == 2 ? vid : s2;
+            s3 = sl == 3 ? vid : s3;
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const uint32_t ent = (nbTable >> (8 * k)) & 0xFFu;
+            const int d = (int)(ent & 0xF), e = (int)(ent >> 4);
+            // (fewer than 2^31 cells in a grid)
+            const int n = ((z - ((d >> 2) & 1)) * CY + (y - ((d >> 1) & 1))) * CX + (x - (d & 1));
+            int vid;
+            if (n >= (int)c0) {
+                const int an = s_aidx[n - (int)c0];
+                vid = (int)voff + s_vpre[an] + (int)((s_tab[recIndex(s_rec[an])] >> (2 * e)) & 3u);
+            } else {
+                const uint32_t m = cellMap[(unsigned)n];
+                vid = (int)tileVOff[(unsigned)n / TILE] + (int)(m & 0x3FFFu) + mapContour(m, e);
+            }
+            const int sl = edgeSlot(e, edgy);
+            s0 = sl == 0 ? vid : s0;
+            s1 = sl == 1 ? vid : s1;
+            s2 = sl == 2 ? vid : s2;
+            s3 = sl == 3 ? vid : s3;
+        }
+        const int64_t q = qoff + q0 + qi;
+        a.quads[q] = make_int4(s0, s1, s2, s3);
+        a.qattr[q] = (uint32_t)(3 * ((x & 1) | ((y & 1) << 1) | ((z & 1) << 2)) + axis);
+    }
     }
     __syncthreads();  // the next tile reuses the block's LDS
     }
