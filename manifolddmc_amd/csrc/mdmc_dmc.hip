@@ -37,10 +37,11 @@ __device__ __forceinline__ bool plainValue(float v) {
     return (b & 0x7FFFFFFFu) < 0x7E800000u && b != 0x80000000u;
 }
 
-// one output row; its points x = lane, lane + width, ... (a block, or one wave in MODE 0)
+// one output row by one wave
 template <int MODE>
 __device__ __forceinline__ void prepareRow(const PrepareDesc& one, const PrepareDesc* __restrict__ d, int G, int refinement, int pad, int64_t row,
-                                           const PrepareSetup& setup, int lane, int width) {
+                                           const PrepareSetup& setup, int lane) {
+    constexpr int width = 64;
     int lo = 0, hi = d ? G : 1;  // d[lo].base <= row
     while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
@@ -102,9 +103,10 @@ __device__ __forceinline__ void prepareRow(const PrepareDesc& one, const Prepare
     }
 }
 
-// MODE 0 copies one row per wave (kBlock / 64 rows per block); the blending modes take a
-// block per row
-constexpr int kPlainRowsPerBlock = kBlock / 64;
+// One row per wave, so that what a row costs by itself (its place, two divisions) is paid once per 64
+// points and most lanes have one: a block per row left 44% of the lanes of a 145-point row without
+// work (48^3 refined by two cuts to 145^3, padded: 24.4 us, 13.6 us now; issue bound).
+constexpr int kRowsPerBlock = kBlock / 64;
 template <int MODE>
 __global__ void __launch_bounds__(kBlock) kPrepareGrids(PrepareDesc one, const PrepareDesc* __restrict__ d, int G, int refinement, int pad, int64_t rows,
                                                         PrepareSetup setup) {
@@ -116,12 +118,8 @@ __global__ void __launch_bounds__(kBlock) kPrepareGrids(PrepareDesc one, const P
         stampClock(setup.stamp);  // one of the counters cleared above
         if (setup.pin && threadIdx.x == 0) setup.ctr[setup.pinAt] = (int64_t)(intptr_t)setup.pin;
     }
-    if (MODE == 0) {
-        const int64_t row = (int64_t)blockIdx.x * kPlainRowsPerBlock + (threadIdx.x >> 6);
-        if (row < rows) prepareRow<0>(one, d, G, refinement, pad, row, setup, threadIdx.x & 63, 64);
-        return;
-    }
-    prepareRow<MODE>(one, d, G, refinement, pad, blockIdx.x, setup, threadIdx.x, kBlock);
+    const int64_t row = (int64_t)blockIdx.x * kRowsPerBlock + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (row < rows) prepareRow<MODE>(one, d, G, refinement, pad, row, setup, threadIdx.x & 63);
 }
 
 __global__ void kTriangles(const int4* __restrict__ he, const int32_t* __restrict__ face_he, int64_t F, uint32_t* __restrict__ idx) {
@@ -224,13 +222,13 @@ int64_t prepareBlocks(const int od[3]) { return (int64_t)od[1] * od[2]; }
 void launchPrepareGrids(const PrepareDesc& one, const PrepareDesc* descDev, int G, int64_t rows, int refinement, int pad, const PrepareSetup& setup,
                         hipStream_t s) {
     if (rows <= 0) return;
-    if (refinement > 0) kPrepareGrids<2><<<(unsigned)rows, kBlock, 0, s>>>(one, descDev, G, refinement, pad, rows, setup);
-    else kPrepareGrids<0><<<(unsigned)((rows + kPlainRowsPerBlock - 1) / kPlainRowsPerBlock), kBlock, 0, s>>>(one, descDev, G, refinement, pad, rows, setup);
+    if (refinement > 0) kPrepareGrids<2><<<(unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock), kBlock, 0, s>>>(one, descDev, G, refinement, pad, rows, setup);
+    else kPrepareGrids<0><<<(unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock), kBlock, 0, s>>>(one, descDev, G, refinement, pad, rows, setup);
 }
 
 void launchPrepareExact(const PrepareDesc& one, const PrepareDesc* descDev, int G, int64_t rows, int pad, hipStream_t s) {
     PrepareSetup none{};
-    if (rows > 0) kPrepareGrids<1><<<(unsigned)rows, kBlock, 0, s>>>(one, descDev, G, 0, pad, rows, none);
+    if (rows > 0) kPrepareGrids<1><<<(unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock), kBlock, 0, s>>>(one, descDev, G, 0, pad, rows, none);
 }
 
 void launchDmcTrianglesFromFaces(const int4* he, const int32_t* face_he, int64_t F, uint32_t* idx, hipStream_t s) {
