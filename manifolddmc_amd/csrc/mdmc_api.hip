@@ -307,7 +307,7 @@ mdmc_status runExtraction(mdmc_ctx* ctx, const mdmc_grid* grids, int G, const fl
         if (p.V > 0) {
             p.halfedgeInitialize();
             p.simplify();
-            p.fixManifoldTwins();
+            p.fixManifoldTwins((flags & MDMC_SPLIT_NM) != 0);
             const int maxIters = opt->max_split_iters > 0 ? opt->max_split_iters : 64;
             if (B == 1) {
                 p.finishSingle((flags & MDMC_SPLIT_NM) != 0, opt->split_step, maxIters, (flags & MDMC_DETECT_NM_VERTS) != 0, st9);

@@ -113,4 +113,77 @@ __device__ __forceinline__ int lbBlockRanks(const uint64_t m[R], int* s_cnt, int
     return s_pre[N];
 }
 
+// Stream compaction in the same single pass as the prefix sum (mdmc_scan.hip): the indices i < n with
+// (attr[i] & mask) != 0, in increasing order, into idx[0 .. total).  Each tile counts its selected
+// elements (16 per thread), scans the counts in the block, gets the tile's first output slot by the
+// same look-back (and the same exact fallback: a direct count of the selected elements before the
+// tile) and writes its indices; nothing is written per unselected element.  A block of kLbBlock threads
+// takes tile t of kListTile elements (tiles in block order).
+constexpr int kListItems = 16, kListTile = kLbBlock * kListItems;
+struct FlagList {
+    const uint32_t* attr;
+    int64_t n;
+    uint32_t mask;
+    int32_t* idx;
+    unsigned long long* words;
+    uint32_t epoch;
+    int64_t *total, *directOut;
+};
+__device__ __forceinline__ void compactFlaggedTile(const FlagList& a, int64_t t) {
+    __shared__ int s_wave[kLbBlock / 64];
+    __shared__ long long s_off;
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int64_t n = a.n, numTiles = n > 0 ? (n + kListTile - 1) / kListTile : 1;
+    if (t >= numTiles) return;
+    const int64_t base = t * kListTile;
+    const int64_t first = base + (int64_t)tid * kListItems;  // this thread's 16 consecutive elements
+
+    uint32_t bits = 0;
+    if (first + kListItems <= n && (((uintptr_t)a.attr) & 15) == 0) {
+        const uint4* p = reinterpret_cast<const uint4*>(a.attr + first);
+#pragma unroll
+        for (int k = 0; k < kListItems / 4; ++k) {
+            const uint4 q = p[k];
+            bits |= ((q.x & a.mask) ? 1u : 0u) << (4 * k);
+            bits |= ((q.y & a.mask) ? 1u : 0u) << (4 * k + 1);
+            bits |= ((q.z & a.mask) ? 1u : 0u) << (4 * k + 2);
+            bits |= ((q.w & a.mask) ? 1u : 0u) << (4 * k + 3);
+        }
+    } else {
+        for (int k = 0; k < kListItems; ++k)
+            if (first + k < n && (a.attr[first + k] & a.mask)) bits |= 1u << k;
+    }
+    const int cnt = __popc(bits);
+    int x = cnt;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int y = __shfl_up(x, d, 64);
+        if (lane >= d) x += y;
+    }
+    if (lane == 63) s_wave[wid] = x;
+    __syncthreads();
+    int add = 0, tileSum = 0;
+#pragma unroll
+    for (int w = 0; w < kLbBlock / 64; ++w) {
+        const int sw = s_wave[w];
+        if (w < wid) add += sw;
+        tileSum += sw;
+    }
+    const int run = x - cnt + add;  // exclusive prefix of this thread inside the tile
+
+    if (tid < 64)
+        lbTileOffset(
+            a.words, a.epoch, t, tileSum,
+            [&](int l) {
+                int64_t sum = 0;
+                for (int64_t k = l; k < base; k += 64) sum += (a.attr[k] & a.mask) ? 1 : 0;
+                return sum;
+            },
+            a.directOut, &s_off);
+    __syncthreads();
+    int64_t o = s_off + run;
+    for (uint32_t b = bits; b; b &= b - 1) a.idx[o++] = (int32_t)(first + __ffs(b) - 1);
+    if (t == numTiles - 1 && tid == 0) *a.total = s_off + tileSum;
+}
+
 }  // namespace mdmc

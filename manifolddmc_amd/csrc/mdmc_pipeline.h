@@ -126,7 +126,9 @@ class Pipeline {
     bool batchVertHe = false;
     void halfedgeInitialize();
     void simplify();
-    void fixManifoldTwins();
+    // list: the list of the non-manifold faces with it (the split's first)
+    void fixManifoldTwins(bool list);
+    bool listed = false;
     void split(int step, int maxIters);
     void detectNonManifoldVertices();
 

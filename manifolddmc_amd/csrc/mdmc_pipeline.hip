@@ -2084,13 +2084,18 @@ __device__ void fixBucket(int h, int4* __restrict__ he, int64_t H, const int4* _
 // a long dependent chain.  A block takes kFixPer * kBlock consecutive halfedges, reads their
 // bucket sizes four at a time (16-byte loads) and the rank only where the size is four or
 // more, gathers the rank-0 members in LDS and repairs them on consecutive lanes, so that the
-// chains run on full waves.
+// chains run on full waves.  The blocks from fixBlocks on list the non-manifold faces meanwhile
+// (the bits do not change here), which by itself is a launch of 5 us on any small mesh.
 constexpr int kFixPer = 16;
 __global__ void __launch_bounds__(kBlock) kFixTwins(int4* __restrict__ he, int64_t H, const int4* __restrict__ quads, const int64_t* __restrict__ off,
                                                     const int32_t* __restrict__ out, const int32_t* __restrict__ bsize, const int32_t* __restrict__ brank,
                                                     const float* __restrict__ pos, const ProblemDev* __restrict__ probs, const int32_t* __restrict__ pid,
-                                                    int64_t* ctr, int64_t* stamp) {
+                                                    FlagList list, unsigned fixBlocks, int64_t* ctr, int64_t* stamp) {
     stampClock(stamp);
+    if (blockIdx.x >= fixBlocks) {
+        compactFlaggedTile(list, blockIdx.x - fixBlocks);
+        return;
+    }
     __shared__ int s_list[kFixPer * kBlock];
     __shared__ int s_n;
     const int lane = threadIdx.x & 63;
@@ -3182,6 +3187,7 @@ void Pipeline::scan(std::initializer_list<ScanJob> jobs, int64_t* stampStart, in
 // counter A_NM
 int32_t* Pipeline::listNM(bool first) {
     int32_t* nm = arena.get<int32_t>("nmlist", (size_t)std::max<int64_t>(F, 1));
+    if (first && listed) return nm;  // by the twin repair
     const Lookback lb = lookback(scanTiles(F));
     compactFlagged(arena.ptr<uint32_t>("fattr"), F, (uint32_t)QA_NM, nm, counters() + A_NM, lb.words, lb.epoch, stream, lookbackDiag(),
                    first ? stamp(ST_SPLIT) : nullptr);
@@ -4000,11 +4006,19 @@ void Pipeline::finishChain() {
     canonTracked = false;
 }
 
-void Pipeline::fixManifoldTwins() {
+void Pipeline::fixManifoldTwins(bool list) {
+    listed = false;
     if (H == 0) return;
-    kFixTwins<<<(unsigned)((H + kFixPer * kBlock - 1) / (kFixPer * kBlock)), kBlock, 0, stream>>>(arena.ptr<int4>("he"), H, arena.ptr<int4>("quads"), arena.ptr<int64_t>("out_off"), arena.ptr<int32_t>("out_list"),
-                                                 arena.ptr<int32_t>("bsize"), arena.ptr<int32_t>("brank"), arena.ptr<float>("pos"), probsDev, pid(),
-                                                 counters(), stamp(ST_TWINS));
+    FlagList fl{};
+    if (list && F > 0) {
+        const Lookback lb = lookback(scanTiles(F));
+        fl = FlagList{arena.ptr<uint32_t>("fattr"), F, (uint32_t)QA_NM, arena.get<int32_t>("nmlist", (size_t)F), lb.words, lb.epoch, counters() + A_NM, lookbackDiag()};
+        listed = true;
+    }
+    const unsigned fixBlocks = (unsigned)((H + kFixPer * kBlock - 1) / (kFixPer * kBlock));
+    kFixTwins<<<fixBlocks + (listed ? (unsigned)scanTiles(F) : 0u), kBlock, 0, stream>>>(
+        arena.ptr<int4>("he"), H, arena.ptr<int4>("quads"), arena.ptr<int64_t>("out_off"), arena.ptr<int32_t>("out_list"), arena.ptr<int32_t>("bsize"),
+        arena.ptr<int32_t>("brank"), arena.ptr<float>("pos"), probsDev, pid(), fl, fixBlocks, counters(), stamp(ST_TWINS));
 }
 
 // ---- ManifoldSplitter::run, one problem and all that follows: the last stages are launched
@@ -4160,6 +4174,7 @@ void Pipeline::splitStep(int step, int64_t n64, const int32_t* nm) {
         uint8_t* touched = splitTouched ? arena.grow<uint8_t>("split_touched", Vm, (size_t)V, stream) : arena.get<uint8_t>("split_touched", Vm);
         {
             FillBatch fb(*this);
+            if (splitIterations == 0 && listed) fb.stampAt(stamp(ST_SPLIT));
             for (int k = 0; k < 4; ++k) {
                 WcMap& m = wcMaps[k];
                 if (maps[k] != m.ptr || wcMapsDirty || m.cap < need[k]) {

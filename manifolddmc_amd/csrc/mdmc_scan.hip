@@ -25,7 +25,7 @@ constexpr int kScanBlock = 256;
 constexpr int kScanItems = 16;
 constexpr int kTile = kScanBlock * kScanItems;
 static_assert(kTile == kScanTile, "tile size");
-static_assert(kScanBlock == kLbBlock, "block size of the look-back");
+static_assert(kScanBlock == kLbBlock && kListTile == kScanTile, "block size of the look-back, words of a list");
 
 // One launch scans up to kScanJobs arrays: blockIdx.y picks the job, blockIdx.x its tile (a job
 // with fewer tiles than the widest leaves the rest of its row idle).
@@ -132,69 +132,11 @@ __global__ void __launch_bounds__(kScanBlock) kScan(ScanJobs jobs, uint32_t epoc
         if (jobs.stampEnd && blockIdx.y == 0) *jobs.stampEnd = wall_clock64();
     }
 }
-// Stream compaction in the same single pass: the indices i < n with (attr[i] & mask) != 0, in
-// increasing order, into idx[0 .. total).  Each tile counts its selected elements (16 per
-// thread), scans the counts in the block, gets the tile's first output slot by the same
-// look-back as kScan (and the same exact fallback: a direct count of the selected elements
-// before the tile) and writes its indices; nothing is written per unselected element.
 __global__ void __launch_bounds__(kScanBlock) kCompactFlagged(const uint32_t* __restrict__ attr, int64_t n, uint32_t mask, int32_t* __restrict__ idx,
                                                               unsigned long long* __restrict__ words, uint32_t epoch,
                                                               int64_t* __restrict__ total, int64_t* __restrict__ directOut, int64_t* stamp) {
     stampClock(stamp);
-    __shared__ int s_wave[kScanBlock / 64];
-    __shared__ long long s_off;
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const int64_t t = blockIdx.x, numTiles = scanTiles(n);
-    if (t >= numTiles) return;
-    const int64_t base = t * kTile;
-    const int64_t first = base + (int64_t)tid * kScanItems;  // this thread's 16 consecutive elements
-
-    uint32_t bits = 0;
-    if (first + kScanItems <= n && (((uintptr_t)attr) & 15) == 0) {
-        const uint4* p = reinterpret_cast<const uint4*>(attr + first);
-#pragma unroll
-        for (int k = 0; k < kScanItems / 4; ++k) {
-            const uint4 q = p[k];
-            bits |= ((q.x & mask) ? 1u : 0u) << (4 * k);
-            bits |= ((q.y & mask) ? 1u : 0u) << (4 * k + 1);
-            bits |= ((q.z & mask) ? 1u : 0u) << (4 * k + 2);
-            bits |= ((q.w & mask) ? 1u : 0u) << (4 * k + 3);
-        }
-    } else {
-        for (int k = 0; k < kScanItems; ++k)
-            if (first + k < n && (attr[first + k] & mask)) bits |= 1u << k;
-    }
-    const int cnt = __popc(bits);
-    int x = cnt;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int y = __shfl_up(x, d, 64);
-        if (lane >= d) x += y;
-    }
-    if (lane == 63) s_wave[wid] = x;
-    __syncthreads();
-    int add = 0, tileSum = 0;
-#pragma unroll
-    for (int w = 0; w < kScanBlock / 64; ++w) {
-        const int sw = s_wave[w];
-        if (w < wid) add += sw;
-        tileSum += sw;
-    }
-    const int run = x - cnt + add;  // exclusive prefix of this thread inside the tile
-
-    if (tid < 64)
-        lbTileOffset(
-            words, epoch, t, tileSum,
-            [&](int l) {
-                int64_t sum = 0;
-                for (int64_t k = l; k < base; k += 64) sum += (attr[k] & mask) ? 1 : 0;
-                return sum;
-            },
-            directOut, &s_off);
-    __syncthreads();
-    int64_t o = s_off + run;
-    for (uint32_t b = bits; b; b &= b - 1) idx[o++] = (int32_t)(first + __ffs(b) - 1);
-    if (t == numTiles - 1 && tid == 0) *total = s_off + tileSum;
+    compactFlaggedTile(FlagList{attr, n, mask, idx, words, epoch, total, directOut}, blockIdx.x);
 }
 }  // namespace
 
