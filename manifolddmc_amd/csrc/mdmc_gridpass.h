@@ -88,6 +88,10 @@ struct GridPassArgs {
     int32_t* tileV;   // [numTiles + 1], last entry 0 (scanned in place of a total)
     int32_t* tileQ;   // [numTiles + 1]
     int32_t* tileNA;  // [numTiles]
+    // few tiles (kTotalsTiles): the last block of classify to finish (ticket, zero before and after)
+    // makes their offsets, the totals and the time stamp itself; null: a scan follows
+    unsigned long long* ticket;
+    int64_t *sumV, *sumQ, *totalV, *totalQ, *stampTotals;
     // per active cell (concatenated cell index): vertex index inside its tile (14 bits) and the
     // contour of each edge a later cell's quads read (2 bits each for edges 1,2,4,5,6,7,9,10,11)
     uint32_t* cellMap;
@@ -137,6 +141,7 @@ void launchGridEmit(int shape, const GridPassArgs& a, hipStream_t s);
 // vertex work items and the dual vertices
 void launchSlabCount(int shape, const GridPassArgs& a, hipStream_t s);
 void launchSlabEmit(int shape, const GridPassArgs& a, hipStream_t s);
+constexpr int kTotalsTiles = 512;
 constexpr int kPairNone = -1, kPairSearch = -2, kPairFace = -3;
 // the halfedge initialize's outgoing lists from the grid pass's quads: entry off[v] + rank (the
 // rank from v's contour) of halfedge 4q + i from corner v = i holds 4q + i; also the face ->

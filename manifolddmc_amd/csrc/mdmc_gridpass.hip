@@ -576,6 +576,56 @@ __device__ __forceinline__ bool classifyRuns(const GridDev& g, float iso, int CX
     return some != 0;
 }
 
+// The offsets of few tiles by the last block that wrote counts: 2 counts per thread.  The counts were
+// stored and are loaded past the L1 and the XCDs' L2s (device scope), so no block needs a fence.
+__device__ __forceinline__ void storeCount(int32_t* p, int v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ void finishTotals(const GridPassArgs& a, int* s_wave) {
+    __shared__ bool s_last;
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    if (tid == 0) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread stored the tile's counts
+        s_last = atomicAdd(a.ticket, 1ULL) == (unsigned long long)(a.numTiles - 1);
+    }
+    __syncthreads();
+    if (!s_last) return;
+    const int n = (int)a.numTiles, i0 = 2 * tid;
+    static_assert(kTotalsTiles == 2 * GP_THREADS && GP_WAVES <= 4, "two tiles per thread");
+    int v[2], q[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        v[j] = i0 + j < n ? __hip_atomic_load(&a.tileV[i0 + j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+        q[j] = i0 + j < n ? __hip_atomic_load(&a.tileQ[i0 + j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    }
+    int xv = v[0] + v[1], xq = q[0] + q[1];
+    const int cv = xv, cq = xq;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int yv = __shfl_up(xv, d, 64), yq = __shfl_up(xq, d, 64);
+        if (lane >= d) xv += yv, xq += yq;
+    }
+    __shared__ int s_q[GP_WAVES];
+    if (lane == 63) s_wave[wid] = xv, s_q[wid] = xq;
+    __syncthreads();
+    int bv = 0, bq = 0, tv = 0, tq = 0;
+#pragma unroll
+    for (int w = 0; w < GP_WAVES; ++w) {
+        if (w < wid) bv += s_wave[w], bq += s_q[w];
+        tv += s_wave[w];
+        tq += s_q[w];
+    }
+    bv += xv - cv;
+    bq += xq - cq;
+    if (i0 <= n) a.sumV[i0] = bv, a.sumQ[i0] = bq;
+    if (i0 + 1 <= n) a.sumV[i0 + 1] = bv + v[0], a.sumQ[i0 + 1] = bq + q[0];
+    if (tid == GP_THREADS - 1 && n == kTotalsTiles) a.sumV[n] = tv, a.sumQ[n] = tq;
+    if (tid == 0) {
+        *a.ticket = 0;
+        *(volatile int64_t*)a.totalV = tv;
+        *(volatile int64_t*)a.totalQ = tq;
+        if (a.stampTotals) *a.stampTotals = wall_clock64();
+    }
+}
+
 // ---- classify: active cells of one tile, their records, counts and map entries.  Bound by
 // instruction issue, vector and scalar (one per CU and cycle each): some 440 vector instructions per
 // wave of an empty 2048-cell tile, 780 with eight corner loads and compares per cell.  Tiles
@@ -583,7 +633,9 @@ __device__ __forceinline__ bool classifyRuns(const GridDev& g, float iso, int CX
 // 555 us, 256^3 blobs (1%) 49 us; eight corners per cell and a case for every cell 612 and 58
 // us; the x + 1 corners' bits inserted one corner at a time, 150 scalar instructions a run, 754 and 82 us.
 // Bounds: 80 registers, six waves per SIMD; 64 spill (665 us), 102 as the compiler likes 640 us.
-template <int CPT, bool QUEUE>
+// TOTALS: few tiles, whose totals the last block makes (a variant of its own: its registers would
+// spill the others')
+template <int CPT, bool QUEUE, bool TOTALS>
 __global__ void __launch_bounds__(GP_THREADS, 6) kClassify(GridPassArgs a, int chunked) {
     constexpr int TILE = GP_THREADS * CPT, RUNS = TILE / 64;
     __shared__ uint32_t s_rec[TILE];
@@ -613,9 +665,12 @@ __global__ void __launch_bounds__(GP_THREADS, 6) kClassify(GridPassArgs a, int c
     const bool active = classifyRuns<CPT>(g, iso, CX, CY, tc.tb, tc.c0, uniform(P.cells), s_mask, s_edgy, s_mc);
     if (!__syncthreads_or(active ? 1 : 0)) {
         if (tid == 0) {
-            a.tileV[tc.t] = a.tileQ[tc.t] = a.tileNA[tc.t] = 0;
+            storeCount(a.tileV + tc.t, 0);
+            storeCount(a.tileQ + tc.t, 0);
+            a.tileNA[tc.t] = 0;
             if (tc.t == a.numTiles - 1) a.tileV[a.numTiles] = a.tileQ[a.numTiles] = 0;
         }
+        if (TOTALS) finishTotals(a, s_wave);
         continue;
     }
     // the two small tables in LDS (read after the next barrier)
@@ -671,14 +726,15 @@ __global__ void __launch_bounds__(GP_THREADS, 6) kClassify(GridPassArgs a, int c
         a.cellMap[tc.gc0 + recCell(r)] = mapEntry(s_vpre[ai], s_tab[recIndex(r)]);
     }
     if (tid == 0) {
-        a.tileV[tc.t] = VT;
-        a.tileQ[tc.t] = QT;
+        storeCount(a.tileV + tc.t, VT);
+        storeCount(a.tileQ + tc.t, QT);
         a.tileNA[tc.t] = NA;
         if (tc.t == a.numTiles - 1) {
             a.tileV[a.numTiles] = 0;
             a.tileQ[a.numTiles] = 0;
         }
     }
+    if (TOTALS) finishTotals(a, s_wave);
     if (QUEUE) __syncthreads();  // the next tile reuses the block's LDS
     }
 }
@@ -1460,13 +1516,14 @@ void launchGridClassify(int shape, const GridPassArgs& a, hipStream_t s) {
     const unsigned nb = (unsigned)a.numTiles;
     if (gridPassIsQueue(shape)) {
         kResetQueue<<<1, 64, 0, s>>>(reinterpret_cast<unsigned long long*>(a.queue));
-        kClassify<8, true><<<queueBlocks(kClassify<8, true>, a.numTiles), GP_THREADS, 0, s>>>(a, 0);
+        kClassify<8, true, false><<<queueBlocks(kClassify<8, true, false>, a.numTiles), GP_THREADS, 0, s>>>(a, 0);
         return;
     }
+    auto launch = [&](auto kernel) { kernel<<<nb, GP_THREADS, 0, s>>>(a, chunked); };
     switch (gridPassTile(shape)) {
-        case 1024: kClassify<4, false><<<nb, GP_THREADS, 0, s>>>(a, chunked); break;
-        case 2048: kClassify<8, false><<<nb, GP_THREADS, 0, s>>>(a, chunked); break;
-        default: kClassify<16, false><<<nb, GP_THREADS, 0, s>>>(a, chunked); break;
+        case 1024: a.ticket ? launch(kClassify<4, false, true>) : launch(kClassify<4, false, false>); break;
+        case 2048: a.ticket ? launch(kClassify<8, false, true>) : launch(kClassify<8, false, false>); break;
+        default: a.ticket ? launch(kClassify<16, false, true>) : launch(kClassify<16, false, false>); break;
     }
 }
 
