@@ -113,7 +113,8 @@ mdmc_status mdmc_create(mdmc_ctx** out, int32_t device);
 void mdmc_destroy(mdmc_ctx* ctx);
 const char* mdmc_last_error(const mdmc_ctx* ctx);
 
-/* Run all following work on this stream (hipStream_t passed as void*); NULL = own stream. */
+/* Run all following work on this stream (hipStream_t passed as void*); NULL = own stream (which does
+ * not wait for the device's default stream, nor that for it), hipStreamLegacy = the default stream. */
 mdmc_status mdmc_set_stream(mdmc_ctx* ctx, void* hip_stream);
 
 /* Shape of the grid pass (no reference counterpart; the reference launches one thread
@@ -221,7 +222,8 @@ mdmc_status mdmc_backward_noalloc(mdmc_ctx* ctx, const float* dL_dpos, float* dL
 
 /* The surface as an autograd graph holds it (no reference counterpart): positions float[3*nV] and
  * the faces' vertex ids int64[4*nF] in walk order (Mesh.cu:446-506), device buffers; either may be
- * NULL.  Asynchronous on the context's stream, like mdmc_backward. */
+ * NULL.  Asynchronous on the context's stream, like mdmc_backward; a following mdmc_extract on another
+ * stream waits for it. */
 mdmc_status mdmc_mesh_quads(const mdmc_ctx* ctx, float* positions, int64_t* quads);
 
 /* Triangle index buffer, two triangles per face (x,y,z),(z,w,x): HalfedgeMesh.cu:690-714.

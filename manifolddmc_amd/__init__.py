@@ -24,6 +24,7 @@ P3333 = 0x10
 SPLIT_NM = 0x20
 DETECT_NM_VERTS = 0x40
 RECORD_ADJOINT = 0x80  # keep the DMC topology for backward() (no reference counterpart)
+DEFAULT_STREAM = 1  # hipStreamLegacy, for set_stream
 DEFAULT_FLAGS = PAD1 | SURF_ITER | SPLIT_NM | DETECT_NM_VERTS
 ALL_POST = P3X3Y_COLOR | P3X3Y_OLD | P3333 | SPLIT_NM | DETECT_NM_VERTS
 
@@ -330,6 +331,8 @@ class DualMarchingCubes:
         return n.value
 
     def set_stream(self, stream_ptr):
+        """mdmc_set_stream: a hipStream_t as an integer, 0 for the context's own stream, DEFAULT_STREAM for the
+        device's default stream (torch's, whose handle is 0, unless a program chose another)."""
         st = lib().mdmc_set_stream(self._ctx, ctypes.c_void_p(stream_ptr))
         self._check(st)
 

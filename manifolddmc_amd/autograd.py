@@ -7,7 +7,7 @@ with the topology of the forward frozen.  Both run on torch's current stream.
 """
 import torch
 
-from . import PAD1, RECORD_ADJOINT, DualMarchingCubes, MdmcError
+from . import DEFAULT_STREAM, PAD1, RECORD_ADJOINT, DualMarchingCubes, MdmcError
 
 _default = {}
 
@@ -19,13 +19,18 @@ def _context(device_index):
     return d
 
 
+def _use_current_stream(dmc, device):
+    # torch's default stream has handle 0, which for a context means its own stream, unordered with torch's
+    dmc.set_stream(torch.cuda.current_stream(device).cuda_stream or DEFAULT_STREAM)
+
+
 class DMCFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, field, iso, origin, delta, pad, refinement, dmc):
         if field.dtype != torch.float32 or not field.is_cuda or field.dim() != 3:
             raise ValueError("field must be a 3-D float32 tensor on a GPU")
         field = field.contiguous()
-        dmc.set_stream(torch.cuda.current_stream(field.device).cuda_stream)
+        _use_current_stream(dmc, field.device)
         nz, ny, nx = field.shape
         flags = RECORD_ADJOINT | (PAD1 if pad else 0)
         dmc.extract_raw(field.data_ptr(), (nx, ny, nz), origin, delta, float(iso), flags, refinement, True)
@@ -48,7 +53,7 @@ class DMCFunction(torch.autograd.Function):
             raise MdmcError(6, "the DMC context ran another extraction after this forward; backward needs the latest one")
         dfield = torch.empty(ctx.shape, dtype=torch.float32, device=ctx.device)
         g = gpos.contiguous() if gpos is not None else torch.zeros((0, 3), dtype=torch.float32, device=ctx.device)
-        dmc.set_stream(torch.cuda.current_stream(ctx.device).cuda_stream)
+        _use_current_stream(dmc, ctx.device)
         dmc.backward(g.data_ptr() if g.numel() else 0, dfield.data_ptr(), False)
         return dfield, None, None, None, None, None, None
 

@@ -33,6 +33,9 @@ struct mdmc_ctx {
     mdmc::Pipeline p;
     std::string err;
     bool hasResult = false;
+    // the last mdmc_mesh_quads reads the mesh on quadsStream until this event
+    hipEvent_t quadsRead = nullptr;
+    hipStream_t quadsStream = nullptr;
     AdjointState adj;
     int nProblems = 0;  // problems of the resident result
     int flags = 0;
@@ -141,8 +144,9 @@ void mdmc_destroy(mdmc_ctx* ctx) {
     if (!ctx) return;
     {
         DeviceGuard g(ctx->device);
-        if (ctx->p.stream) (void)hipStreamSynchronize(ctx->p.stream);
+        (void)hipStreamSynchronize(ctx->p.stream);
         ctx->p.arena.release();
+        if (ctx->quadsRead) (void)hipEventDestroy(ctx->quadsRead);
         if (ctx->own) (void)hipStreamDestroy(ctx->own);
     }
     delete ctx;
@@ -152,7 +156,7 @@ const char* mdmc_last_error(const mdmc_ctx* ctx) { return ctx ? ctx->err.c_str()
 
 mdmc_status mdmc_set_stream(mdmc_ctx* ctx, void* s) {
     if (!ctx) return MDMC_ERR_INVALID_ARG;
-    ctx->p.stream = s ? (hipStream_t)s : ctx->own;
+    ctx->p.stream = !s ? ctx->own : (hipStream_t)s == hipStreamLegacy ? nullptr : (hipStream_t)s;
     return MDMC_OK;
 }
 
@@ -227,6 +231,7 @@ mdmc_status runExtraction(mdmc_ctx* ctx, const mdmc_grid* grids, int G, const fl
     const int B = G * I;
     try {
         hipStream_t s = p.stream;
+        if (ctx->quadsRead && ctx->quadsStream != s) MDMC_HIP(hipStreamWaitEvent(s, ctx->quadsRead, 0));
         p.splitIterations = 0;
         p.extraAnomalies = 0;
         p.setChain((flags & MDMC_P3X3Y_COLOR) != 0, (flags & MDMC_P3X3Y_OLD) != 0, (flags & MDMC_P3333) != 0);
@@ -523,8 +528,11 @@ mdmc_status mdmc_mesh_quads(const mdmc_ctx* cctx, float* positions, int64_t* qua
     DeviceGuard dg(ctx->device);
     try {
         mdmc::Pipeline& p = ctx->p;
+        if (!ctx->quadsRead) MDMC_HIP(hipEventCreateWithFlags(&ctx->quadsRead, hipEventDisableTiming));
         mdmc::launchQuadIds(p.arena.ptr<int4>("he"), p.arena.ptr<int32_t>("face_he"), p.F, p.arena.ptr<float>("pos"), p.V, positions, quads, p.stream);
         MDMC_HIP(hipGetLastError());
+        ctx->quadsStream = p.stream;
+        MDMC_HIP(hipEventRecord(ctx->quadsRead, p.stream));
         return MDMC_OK;
     } catch (const std::exception& e) {
         return fromException(ctx, e);

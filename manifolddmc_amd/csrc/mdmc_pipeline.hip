@@ -3494,6 +3494,7 @@ void Pipeline::releaseGraphs() {
 }
 
 bool Pipeline::runFrontGraph(const std::vector<int64_t>& shapeSig, std::vector<ProblemDev>& problems, int64_t C, int shape, bool surfIter) {
+    if (!stream) return false;  // the default stream cannot be captured
     const size_t prepBytes = prep.desc.size() * sizeof(PrepareDesc);
     std::vector<int64_t> sig = shapeSig;
     const std::vector<int64_t> bufs = frontBuffers();
