@@ -240,9 +240,13 @@ __device__ __forceinline__ int problemOfQuad(const int64_t* __restrict__ startQ,
 // bucket's first member), 1: faces (slots 3-7: quads with k NM edges), 2: vertices (slot 8:
 // non-manifold vertices).  out[9 * problem + slot].
 constexpr int kStatRows = 32;
-// elements per block: up to 4096 (fewer global additions), down to one per thread while that
-// gives fewer than 1024 blocks (110 k vertices: 56 us in 27 blocks, 6 us in 432)
-inline int64_t statChunk(int64_t n) { return std::min<int64_t>(4096, std::max<int64_t>(kBlock, n / 1024 / kBlock * kBlock)); }
+// elements per block: enough that what a block does once (its problem's search, the global additions)
+// does not count, few enough that the chip stays full to the end; down to one per thread while that
+// gives fewer than 1024 blocks (110 k vertices: 56 us in 27 blocks, 6 us in 432).  5.4 M vertices 350 us with
+// 4096, 246 with 1024, 225 with 512, 222 with 256; as many faces 180, 116, 119 with 4096, 1024, 512; 21.6 M
+// halfedges 242 with 2048, 243 with 1024, 292 with 512.
+template <int KIND>
+inline int64_t statChunk(int64_t n) { return std::min<int64_t>(KIND == RG_V ? 512 : 1024, std::max<int64_t>(kBlock, n / 1024 / kBlock * kBlock)); }
 
 __device__ __forceinline__ void statAdd(unsigned* acc, unsigned long long* out, bool live, int p, int pbase, int slot, int accSlot, bool v) {
     // one LDS atomic per wave when all its live lanes share the problem
@@ -272,7 +276,7 @@ __device__ __forceinline__ void statAdd(unsigned* acc, unsigned long long* out, 
 //
 // Bound by HBM: the permutations, their inverses and a copy back of every array, keys for every
 // element and an atomicMax per halfedge came to 3.1 ms of the 64-grid batch's 9.4 ms (5.4 M
-// vertices); 1.0 ms now.
+// vertices); 0.58 ms now (0.93 with 4096 elements a block and every id's shift loaded by itself).
 struct MoveArgs {
     RegroupArgs r;
     const float *pos, *nrm;
@@ -306,20 +310,24 @@ __global__ void __launch_bounds__(kBlock) kRegroup(MoveArgs a, int64_t chunk) {
     const int pbase = problemOf(c0);
     // most blocks lie in one problem's prefix: no search per element
     const bool one = KIND != RG_V && c1 <= n0 && problemOf(c1 - 1) == pbase;
+    // and most elements in the first one's problem, whose shifts are read once
+    int64_t shift[3];
+    for (int k = 0; k < 3; ++k) shift[k] = MOVE ? r.shift[(int64_t)k * r.B + pbase] : 0;
+    auto idOf = [&](int arr, int p, int x) -> int { return p == pbase && x < r.n0[arr] ? (int)(x + shift[arr]) : newId(r, arr, p, x); };
     __syncthreads();
     // uniform trip count so that every lane takes part in the wave reductions
     for (int64_t i0 = c0; i0 < c1; i0 += kBlock) {
         const int64_t i = i0 + threadIdx.x;
         const bool live = i < c1;
         const int p = !live ? 0 : (one ? pbase : problemOf(i));
-        const int64_t d = !live ? 0 : (MOVE ? newId(r, KIND, p, (int)i) : i);
+        const int64_t d = !live ? 0 : (MOVE ? idOf(KIND, p, (int)i) : i);
         if (KIND == RG_H) {
             int w = 0;
             if (live) {
                 w = a.bsize[i];
                 if (MOVE) {
                     const int4 e = r.he[i];
-                    a.nhe[d] = make_int4(newId(r, RG_V, p, e.x), newId(r, RG_F, p, e.y), newId(r, RG_H, p, e.z), e.w >= 0 ? newId(r, RG_H, p, e.w) : e.w);
+                    a.nhe[d] = make_int4(idOf(RG_V, p, e.x), idOf(RG_F, p, e.y), idOf(RG_H, p, e.z), e.w >= 0 ? idOf(RG_H, p, e.w) : e.w);
                 }
             }
             const bool count = live && bucketFirst(w);
@@ -344,7 +352,7 @@ __global__ void __launch_bounds__(kBlock) kRegroup(MoveArgs a, int64_t chunk) {
                     }
                 }
                 if (MOVE) {
-                    a.nface_he[d] = newId(r, RG_H, p, h0);
+                    a.nface_he[d] = idOf(RG_H, p, h0);
                     a.nfattr[d] = a.fattr[i];
                 }
             }
@@ -358,7 +366,12 @@ __global__ void __launch_bounds__(kBlock) kRegroup(MoveArgs a, int64_t chunk) {
                     if (p < 0 || p >= r.B || i < r.startV[p] || i >= r.startV[p + 1]) atomicOr(a.bad, 1);
                     best = -1;
                     const int64_t e = a.listOff[i + 1];
-                    for (int64_t q = a.listOff[i]; q < e; ++q) best = max(best, a.list[q]);
+                    for (int64_t q = a.listOff[i]; q < e; q += 4) {
+                        int h[4];
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) h[k] = a.list[q + k < e ? q + k : e - 1];
+                        best = max(max(best, max(h[0], h[1])), max(h[2], h[3]));
+                    }
                     if (best >= 0) best -= (int)(4 * r.startQ[p]);
                 }
                 a.vh[d] = best;
@@ -380,6 +393,12 @@ __global__ void __launch_bounds__(kBlock) kRegroup(MoveArgs a, int64_t chunk) {
         const unsigned v = acc[row * 5 + sl];
         if (v) atomicAdd(&a.out[(int64_t)(pbase + row) * 9 + base + sl], (unsigned long long)v);
     }
+}
+
+template <int KIND, bool MOVE>
+void launchRegroup(const MoveArgs& m, int64_t n, hipStream_t s) {
+    const int64_t chunk = statChunk<KIND>(n);
+    if (n > 0) kRegroup<KIND, MOVE><<<(unsigned)((n + chunk - 1) / chunk), kBlock, 0, s>>>(m, chunk);
 }
 
 }  // namespace
@@ -501,7 +520,6 @@ void Pipeline::regroupBatch(int B) {
     m.bad = bad;
     const size_t nv = (size_t)std::max<int64_t>(V, 1), nh = (size_t)std::max<int64_t>(H, 1), nf = (size_t)std::max<int64_t>(F, 1);
     m.vh = arena.get<int32_t>("batch_vert_he", nv);
-    auto chunks = [](int64_t n) { return (unsigned)((n + statChunk(n) - 1) / statChunk(n)); };
     if (tail > 0) {
         m.npos = arena.get<float>("pos2", 3 * nv);
         m.nnrm = arena.get<float>("nrm2", 3 * nv);
@@ -510,14 +528,14 @@ void Pipeline::regroupBatch(int B) {
         m.nhe = arena.get<int4>("he2", nh);
         m.nface_he = arena.get<int32_t>("face_he2", nf);
         m.nfattr = arena.get<uint32_t>("fattr2", nf);
-        if (H > 0) kRegroup<RG_H, true><<<chunks(H), kBlock, 0, stream>>>(m, statChunk(H));
-        if (F > 0) kRegroup<RG_F, true><<<chunks(F), kBlock, 0, stream>>>(m, statChunk(F));
-        if (V > 0) kRegroup<RG_V, true><<<chunks(V), kBlock, 0, stream>>>(m, statChunk(V));
+        launchRegroup<RG_H, true>(m, H, stream);
+        launchRegroup<RG_F, true>(m, F, stream);
+        launchRegroup<RG_V, true>(m, V, stream);
         for (const char* name : {"pos", "nrm", "vflags", "pid", "he", "face_he", "fattr"}) arena.swap(name, std::string(name) + "2");
     } else {
-        if (H > 0) kRegroup<RG_H, false><<<chunks(H), kBlock, 0, stream>>>(m, statChunk(H));
-        if (F > 0) kRegroup<RG_F, false><<<chunks(F), kBlock, 0, stream>>>(m, statChunk(F));
-        if (V > 0) kRegroup<RG_V, false><<<chunks(V), kBlock, 0, stream>>>(m, statChunk(V));
+        launchRegroup<RG_H, false>(m, H, stream);
+        launchRegroup<RG_F, false>(m, F, stream);
+        launchRegroup<RG_V, false>(m, V, stream);
     }
     batchVertHe = true;
     kStamp<<<1, 1, 0, stream>>>(stamp(ST_END));
