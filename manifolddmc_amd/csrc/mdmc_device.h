@@ -282,4 +282,20 @@ enum : uint32_t { QA_COLOR = 0x1F, QA_NM = 0x20, QA_PATTERN = 0x40, QA_REMOVE = 
                   QA_ODD = 0x400 /* a P3333 centre whose twins are not replaced by the rule (within that step) */ };
 enum : uint32_t { VF_NM = 1, VF_BOUNDARY = 2, VF_WEIRD = 4, VF_FANS = 8, VF_REMOVE = 16 };
 
+// Accesses to arrays that are not used again soon, past the caches' usual order of replacement.
+template <class T>
+__device__ __forceinline__ void storeStreaming(T* p, T v) { __builtin_nontemporal_store(v, p); }
+__device__ __forceinline__ void storeStreaming(uint4* p, uint4 v) {
+    typedef uint32_t Words __attribute__((ext_vector_type(4)));
+    __builtin_nontemporal_store(Words{v.x, v.y, v.z, v.w}, reinterpret_cast<Words*>(p));
+}
+__device__ __forceinline__ uint4 loadStreaming(const uint4* p) {
+    typedef uint32_t Words __attribute__((ext_vector_type(4)));
+    const Words w = __builtin_nontemporal_load(reinterpret_cast<const Words*>(p));
+    return make_uint4(w.x, w.y, w.z, w.w);
+}
+__device__ __forceinline__ void storeStreaming(int4* p, int4 v) {
+    storeStreaming(reinterpret_cast<uint4*>(p), make_uint4((uint32_t)v.x, (uint32_t)v.y, (uint32_t)v.z, (uint32_t)v.w));
+}
+
 }  // namespace mdmc

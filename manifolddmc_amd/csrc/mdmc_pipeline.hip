@@ -876,7 +876,8 @@ constexpr int kOldCentre = 1 << 30;  // in oldQ: the old quad is the centre of a
 // buckets afterwards on full waves.  The chain ends here, so the finished records are written.  A thread
 // takes a quad's four halfedges, so that the loads behind the old quad's id are in flight together, and
 // the records go through LDS, in order across lanes (stored by quad, every line is written
-// back in parts: 2.7 GB instead of 1.4).  Bound by HBM: 2.3 GB moved at the 512^3 gyroid in 653 us; a
+// back in parts: 2.7 GB instead of 1.4).  Bound by HBM: 2.3 GB moved at the 512^3 gyroid in 579 us
+// (616 with the records stored through the caches, and the twin repair behind it 214 instead of 203); a
 // thread per halfedge 944 us, the records stored by quad 839 us.
 __global__ void __launch_bounds__(kBlock) kRemapRebuild(const int4* __restrict__ quads2, int64_t H2, const uint8_t* __restrict__ touched,
                                                         const int32_t* __restrict__ oldQ, const int32_t* __restrict__ twinOld, int64_t Hold,
@@ -970,7 +971,7 @@ __global__ void __launch_bounds__(kBlock) kRemapRebuild(const int4* __restrict__
     for (int k = 0; k < 4; ++k) {
         const int l = k * kBlock + threadIdx.x;
         const int h = (int)(h0 + l);
-        if (h0 + l < H2 && s_t[l] != kRebuilt) he[h] = make_int4(s_v[l], h >> 2, quadNext(h, 1), s_t[l]);
+        if (h0 + l < H2 && s_t[l] != kRebuilt) storeStreaming(he + h, make_int4(s_v[l], h >> 2, quadNext(h, 1), s_t[l]));
     }
     const int total = s_n;
     for (int k = threadIdx.x; k < total; k += kBlock) {
@@ -2980,9 +2981,10 @@ __global__ void __launch_bounds__(kBlock) kStats(const int4* __restrict__ he, in
 // thread order): the maximum of the vertex's outgoing list, whose entries are consecutive;
 // -1 where the list is empty, 0 in the slots a split's resizes added.
 //
-// Bound by HBM: 2.5 GB moved at the 512^3 gyroid in 684 us (3.7 TB/s).  The eleven launches this replaces
-// took 1.43 ms there (700 us of it one atomicMax per halfedge) and 100 us of launch time on a
-// mesh of any size.
+// Bound by HBM: 2.5 GB moved at the 512^3 gyroid in 587 us (4.3 TB/s).  Nothing here is read twice, so loads
+// and stores pass the caches by: 651 us there through them, and 20 us instead of 10 at the 256^3 blobs, whose
+// 13 MB of stores waited for older lines to be written back.  The eleven launches this replaces
+// took 1.43 ms (700 us of it one atomicMax per halfedge) and 100 us of launch time on a mesh of any size.
 constexpr int kCopyPer = 4;
 enum : int { CM_POS, CM_NRM, CM_HE, CM_FACE, CM_VHE_COPY, CM_FATTR, CM_VFLAGS, CM_VHE, CM_COUNT };
 struct CopyMesh {
@@ -3007,12 +3009,12 @@ __global__ void __launch_bounds__(kBlock) kCopyMesh(CopyMesh c) {
 #pragma unroll
         for (int k = 0; k < kCopyPer; ++k) {
             const int64_t i = i0 + (int64_t)k * kBlock;
-            if (vec && 4 * i + 3 < n) w[k] = reinterpret_cast<const uint4*>(src)[i];
+            if (vec && 4 * i + 3 < n) w[k] = loadStreaming(reinterpret_cast<const uint4*>(src) + i);
         }
 #pragma unroll
         for (int k = 0; k < kCopyPer; ++k) {
             const int64_t i = i0 + (int64_t)k * kBlock;
-            if (vec && 4 * i + 3 < n) reinterpret_cast<uint4*>(dst)[i] = w[k];
+            if (vec && 4 * i + 3 < n) storeStreaming(reinterpret_cast<uint4*>(dst) + i, w[k]);
             else
                 for (int64_t t = 4 * i; t < 4 * i + 4 && t < n; ++t) dst[t] = src[t];
         }
@@ -3027,16 +3029,21 @@ __global__ void __launch_bounds__(kBlock) kCopyMesh(CopyMesh c) {
             if (i < c.listsV) {
                 best = -1;
                 const int64_t e = c.off[i + 1];
-                for (int64_t q = c.off[i]; q < e; ++q) best = max(best, list[q]);
+                for (int64_t q = c.off[i]; q < e; q += 4) {
+                    int h[4];
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) h[t] = list[q + t < e ? q + t : e - 1];
+                    best = max(max(best, max(h[0], h[1])), max(h[2], h[3]));
+                }
             }
-            ((int32_t*)c.dst[j])[i] = best;
+            storeStreaming((int32_t*)c.dst[j] + i, best);
             continue;
         }
         const uint32_t* src = (const uint32_t*)c.src[j];
         if (vec && 4 * i + 3 < n) {
             const uint4 w = reinterpret_cast<const uint4*>(src)[i];
-            if (j == CM_FATTR) reinterpret_cast<ushort4*>(c.dst[j])[i] = make_ushort4((uint16_t)w.x, (uint16_t)w.y, (uint16_t)w.z, (uint16_t)w.w);
-            else reinterpret_cast<uchar4*>(c.dst[j])[i] = make_uchar4((uint8_t)w.x, (uint8_t)w.y, (uint8_t)w.z, (uint8_t)w.w);
+            if (j == CM_FATTR) storeStreaming((uint64_t*)c.dst[j] + i, (uint64_t)((w.x & 0xFFFFu) | (w.y << 16)) | (uint64_t)((w.z & 0xFFFFu) | (w.w << 16)) << 32);
+            else storeStreaming((uint32_t*)c.dst[j] + i, (w.x & 0xFFu) | ((w.y & 0xFFu) << 8) | ((w.z & 0xFFu) << 16) | (w.w << 24));
         } else {
             for (int64_t t = 4 * i; t < 4 * i + 4 && t < n; ++t) {
                 if (j == CM_FATTR) ((uint16_t*)c.dst[j])[t] = (uint16_t)src[t];
