@@ -529,8 +529,8 @@ mdmc_status mdmc_mesh_quads(const mdmc_ctx* cctx, float* positions, int64_t* qua
     try {
         mdmc::Pipeline& p = ctx->p;
         if (!ctx->quadsRead) MDMC_HIP(hipEventCreateWithFlags(&ctx->quadsRead, hipEventDisableTiming));
-        mdmc::launchQuadIds(p.arena.ptr<int4>("he"), p.arena.ptr<int32_t>("face_he"), p.F, p.arena.ptr<float>("pos"), p.V, positions, quads, p.stream);
-        MDMC_HIP(hipGetLastError());
+        MDMC_HIP(mdmc::launchQuadIds(p.arena.ptr<int4>("he"), p.arena.ptr<int32_t>("face_he"), p.F, p.arena.ptr<float>("pos"), p.V, positions, quads,
+                                     p.stream));
         ctx->quadsStream = p.stream;
         MDMC_HIP(hipEventRecord(ctx->quadsRead, p.stream));
         return MDMC_OK;

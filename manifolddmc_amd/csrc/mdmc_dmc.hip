@@ -235,9 +235,11 @@ void launchDmcTrianglesFromFaces(const int4* he, const int32_t* face_he, int64_t
     if (F > 0) kTriangles<<<gridFor(F), kBlock, 0, s>>>(he, face_he, F, idx);
 }
 
-void launchQuadIds(const int4* he, const int32_t* face_he, int64_t F, const float* src, int64_t V, float* positions, int64_t* quads, hipStream_t s) {
-    const int64_t qb = quads ? (F + kBlock - 1) / kBlock : 0, pb = positions ? (3 * V + kBlock - 1) / kBlock : 0;
-    if (qb + pb > 0) kQuadIds<<<(unsigned)(qb + pb), kBlock, 0, s>>>(he, face_he, F, src, 3 * V, positions, quads, qb);
+hipError_t launchQuadIds(const int4* he, const int32_t* face_he, int64_t F, const float* src, int64_t V, float* positions, int64_t* quads, hipStream_t s) {
+    int64_t qb = quads ? (F + kBlock - 1) / kBlock : 0, pb = positions ? (3 * V + kBlock - 1) / kBlock : 0, n3 = 3 * V;
+    if (qb + pb == 0) return hipSuccess;
+    void* args[] = {&he, &face_he, &F, &src, &n3, &positions, &quads, &qb};
+    return hipLaunchKernel((const void*)kQuadIds, dim3((unsigned)(qb + pb)), dim3(kBlock), args, 0, s);
 }
 
 void launchRenderVertices(const int4* he, int64_t H, const float* pos, const float* nrm, const uint32_t* vflags, float* out, hipStream_t s) {

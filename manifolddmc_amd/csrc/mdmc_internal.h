@@ -80,8 +80,8 @@ struct PrepareDesc {
 int64_t prepareBlocks(const int od[3]);
 void launchDmcTrianglesFromFaces(const int4* he, const int32_t* face_he, int64_t F, uint32_t* idx, hipStream_t s);
 // positions copied from src to positions[3V] and the faces' vertex ids to quads[4F], in one launch
-// (either output may be null)
-void launchQuadIds(const int4* he, const int32_t* face_he, int64_t F, const float* src, int64_t V, float* positions, int64_t* quads, hipStream_t s);
+// (either output may be null); the launch's own status
+hipError_t launchQuadIds(const int4* he, const int32_t* face_he, int64_t F, const float* src, int64_t V, float* positions, int64_t* quads, hipStream_t s);
 // render vertices {position, normal, rgba by vertex flags} of every vertex with an outgoing
 // halfedge into out[10 * V] (the caller zero-fills out first)
 void launchRenderVertices(const int4* he, int64_t H, const float* pos, const float* nrm, const uint32_t* vflags, float* out, hipStream_t s);

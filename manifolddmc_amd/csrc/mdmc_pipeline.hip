@@ -4327,13 +4327,15 @@ void Pipeline::launchStats(int guarded) {
     kStats<<<(unsigned)blocks, kBlock, 0, stream>>>(
         arena.ptr<int4>("he"), H, arena.ptr<int32_t>("face_he"), F, arena.ptr<int32_t>("bsize"),
         arena.ptr<uint32_t>("vflags"), V, canonFlags(), counters(), pinDev() + kPinFinal, guarded);
-    MDMC_HIP(hipGetLastError());
 }
 
-// waits for the statistics; the counters they handed over
+// waits for the statistics; the counters they handed over.  A launch that failed leaves the word
+// behind them unset.  (hipGetLastError behind the launch would also report an error that another call of this
+// thread left long before, one that has nothing to do with the extraction.)
 const int64_t* Pipeline::waitStats() {
     const volatile int64_t* done = pinHost() + kPinDone;
     await([&] { return *done != 0; });
+    if (*done == 0) throw HipError("the extraction's last kernel did not run", (int)hipErrorLaunchFailure);
     return pinHost() + kPinFinal;
 }
 
@@ -4381,8 +4383,8 @@ void Pipeline::copyOut(float* positions, float* normals, int32_t* halfedges, int
     c.start[CM_COUNT] = blocks;
     c.off = arena.ptr<int64_t>("out_off");
     c.listsV = std::min(vertHeV, V);
-    if (blocks > 0) kCopyMesh<<<blocks, kBlock, 0, stream>>>(c);
-    MDMC_HIP(hipGetLastError());
+    void* args[] = {&c};
+    if (blocks > 0) MDMC_HIP(hipLaunchKernel((const void*)kCopyMesh, dim3(blocks), dim3(kBlock), args, 0, stream));
     if (!dstDevice) {
         auto down = [&](void* dst, const void* src, size_t bytes) {
             if (dst && bytes) MDMC_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream));
