@@ -4344,39 +4344,56 @@ void Pipeline::finishEmpty() {
     waitStats();
 }
 
+// Whether the mesh copy's kernel may store there: memory of the current device.  Another GPU's may not be
+// mapped here, and host memory is the copy engine's anyway.
+static bool ownMemory(const void* p) {
+    hipPointerAttribute_t a{};
+    int dev = 0;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();  // memory that HIP does not know
+        return false;
+    }
+    return a.type == hipMemoryTypeDevice && hipGetDevice(&dev) == hipSuccess && a.device == dev;
+}
+
 void Pipeline::copyOut(float* positions, float* normals, int32_t* halfedges, int32_t* face_halfedge, uint16_t* face_attr, uint8_t* vertex_flags,
                        int32_t* vertex_halfedge, bool dstDevice) {
-    // one launch into device buffers; for host ones it makes the three derived arrays in device
-    // memory and copies follow
-    int32_t* vhe = vertex_halfedge;
-    uint16_t* fa = face_attr;
-    uint8_t* vf = vertex_flags;
-    if (!dstDevice) {
-        if (vhe && V) vhe = batchVertHe ? arena.ptr<int32_t>("batch_vert_he") : arena.get<int32_t>("vert_he", (size_t)V);
-        if (fa && F) fa = arena.get<uint16_t>("out_fattr", (size_t)F);
-        if (vf && V) vf = arena.get<uint8_t>("out_vflags", (size_t)V);
-    }
+    // one launch into buffers of this device; for others it makes the three derived arrays in
+    // device memory and copies follow
+    struct Array {
+        int kind;
+        const char* name;
+        void* dst;
+        int64_t n;
+        size_t bytes;
+        const char* made;  // where a derived array is made for a copy
+    };
+    const Array arrays[] = {
+        {CM_POS, "pos", positions, 3 * V, 3 * (size_t)V * sizeof(float), nullptr},
+        {CM_NRM, "nrm", normals, 3 * V, 3 * (size_t)V * sizeof(float), nullptr},
+        {CM_HE, "he", halfedges, 4 * H, (size_t)H * sizeof(int4), nullptr},
+        {CM_FACE, "face_he", face_halfedge, F, (size_t)F * sizeof(int32_t), nullptr},
+        {batchVertHe ? CM_VHE_COPY : CM_VHE, batchVertHe ? "batch_vert_he" : "out_list", vertex_halfedge, V, (size_t)V * sizeof(int32_t),
+         batchVertHe ? nullptr : "vert_he"},
+        {CM_FATTR, "fattr", face_attr, F, (size_t)F * sizeof(uint16_t), "out_fattr"},
+        {CM_VFLAGS, "vflags", vertex_flags, V, (size_t)V, "out_vflags"},
+    };
     CopyMesh c{};
+    const void* from[CM_COUNT] = {};  // what the copies read
+    for (const Array& x : arrays) {
+        if (!x.dst || x.n == 0) continue;
+        void* dst = x.dst;
+        if (!dstDevice || !ownMemory(x.dst)) {
+            dst = x.made ? arena.get<char>(x.made, x.bytes) : nullptr;
+            from[x.kind] = x.made ? dst : arena.ptr<char>(x.name);
+        }
+        c.src[x.kind] = arena.ptr<char>(x.name);
+        c.dst[x.kind] = dst;
+        c.n[x.kind] = dst ? x.n : 0;
+    }
     unsigned blocks = 0;
     for (int j = 0; j < CM_COUNT; ++j) {
-        const void* src = nullptr;
-        void* dst = nullptr;
-        int64_t n = 0;
-        auto set = [&](const void* from, void* to, int64_t count) { src = from, dst = to, n = to ? count : 0; };
-        switch (j) {
-            case CM_POS: set(arena.ptr<float>("pos"), dstDevice ? positions : nullptr, 3 * V); break;
-            case CM_NRM: set(arena.ptr<float>("nrm"), dstDevice ? normals : nullptr, 3 * V); break;
-            case CM_HE: set(arena.ptr<int4>("he"), dstDevice ? halfedges : nullptr, 4 * H); break;
-            case CM_FACE: set(arena.ptr<int32_t>("face_he"), dstDevice ? face_halfedge : nullptr, F); break;
-            case CM_VHE_COPY: set(arena.ptr<int32_t>("batch_vert_he"), dstDevice && batchVertHe ? vhe : nullptr, V); break;
-            case CM_FATTR: set(arena.ptr<uint32_t>("fattr"), fa, F); break;
-            case CM_VFLAGS: set(arena.ptr<uint32_t>("vflags"), vf, V); break;
-            case CM_VHE: set(arena.ptr<int32_t>("out_list"), batchVertHe ? nullptr : vhe, V); break;
-        }
-        const int64_t items = j == CM_VHE ? n : (n + 3) / 4;
-        c.src[j] = src;
-        c.dst[j] = dst;
-        c.n[j] = n;
+        const int64_t items = j == CM_VHE ? c.n[j] : (c.n[j] + 3) / 4;
         c.start[j] = blocks;
         blocks += (unsigned)((items + kCopyPer * kBlock - 1) / (kCopyPer * kBlock));
     }
@@ -4385,18 +4402,8 @@ void Pipeline::copyOut(float* positions, float* normals, int32_t* halfedges, int
     c.listsV = std::min(vertHeV, V);
     void* args[] = {&c};
     if (blocks > 0) MDMC_HIP(hipLaunchKernel((const void*)kCopyMesh, dim3(blocks), dim3(kBlock), args, 0, stream));
-    if (!dstDevice) {
-        auto down = [&](void* dst, const void* src, size_t bytes) {
-            if (dst && bytes) MDMC_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream));
-        };
-        down(positions, arena.ptr<float>("pos"), 3 * (size_t)V * sizeof(float));
-        down(normals, arena.ptr<float>("nrm"), 3 * (size_t)V * sizeof(float));
-        down(halfedges, arena.ptr<int4>("he"), (size_t)H * sizeof(int4));
-        down(face_halfedge, arena.ptr<int32_t>("face_he"), (size_t)F * sizeof(int32_t));
-        down(vertex_halfedge, vhe, (size_t)V * sizeof(int32_t));
-        down(face_attr, fa, (size_t)F * sizeof(uint16_t));
-        down(vertex_flags, vf, (size_t)V);
-    }
+    for (const Array& x : arrays)
+        if (from[x.kind]) MDMC_HIP(hipMemcpyAsync(x.dst, from[x.kind], x.bytes, dstDevice ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, stream));
     MDMC_HIP(hipStreamSynchronize(stream));
 }
 
