@@ -193,6 +193,10 @@ mdmc_status mdmc_set_local_merges(mdmc_ctx* ctx, int32_t enable);
  * makes every iteration take that pass, so tests can compare it with the parallel one and
  * with the reference's results (default 0).  The mesh is the same either way. */
 mdmc_status mdmc_set_sequential_merges(mdmc_ctx* ctx, int32_t enable);
+/* Verification switch for the checks of a chain of simplifications (no reference counterpart).
+ * enable = 1 has its compaction count one inconsistent quad, as a vertex id out of range would be:
+ * an extraction with any of the P3X3Y / P3333 flags then ends with MDMC_ERR_INTERNAL (default off). */
+mdmc_status mdmc_set_fail_compaction(mdmc_ctx* ctx, int32_t enable);
 
 /* Per-problem offsets of the resident result (host arrays of n_problems + 1; any may be NULL).
  * After mdmc_extract (one problem) they are {0, n}. */

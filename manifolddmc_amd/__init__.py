@@ -107,7 +107,7 @@ EXPORTS = ["mdmc_create", "mdmc_destroy", "mdmc_last_error", "mdmc_set_stream", 
            "mdmc_extract_batch", "mdmc_batch_offsets", "mdmc_batch_stats", "mdmc_set_tile_shape", "mdmc_get_tile_shape",
            "mdmc_generate_surface", "mdmc_generate_edge_case", "mdmc_mesh_face_colors", "mdmc_mesh_triangulate_maxmin",
            "mdmc_backward_noalloc", "mdmc_set_graphs", "mdmc_get_graph_replays", "mdmc_processed_grid",
-           "mdmc_set_local_merges", "mdmc_set_sequential_merges", "mdmc_mesh_quads"]
+           "mdmc_set_local_merges", "mdmc_set_sequential_merges", "mdmc_set_fail_compaction", "mdmc_mesh_quads"]
 
 
 def lib():
@@ -166,6 +166,8 @@ def lib():
         L.mdmc_set_local_merges.restype = i32
         L.mdmc_set_sequential_merges.argtypes = [vp, i32]
         L.mdmc_set_sequential_merges.restype = i32
+        L.mdmc_set_fail_compaction.argtypes = [vp, i32]
+        L.mdmc_set_fail_compaction.restype = i32
         L.mdmc_get_graph_replays.argtypes = [vp, ctypes.POINTER(i64)]
         L.mdmc_get_graph_replays.restype = i32
         L.mdmc_backward_noalloc.restype = i32
@@ -324,6 +326,11 @@ class DualMarchingCubes:
         """mdmc_set_sequential_merges: the splitter's merge phase always takes the one-thread
         ascending pass it otherwise takes only on schedule conflicts (the mesh is the same)."""
         self._check(lib().mdmc_set_sequential_merges(self._ctx, 1 if enable else 0))
+
+    def set_fail_compaction(self, enable):
+        """mdmc_set_fail_compaction: a chain's compaction counts one quad as inconsistent (a verification
+        switch: the extraction raises)."""
+        self._check(lib().mdmc_set_fail_compaction(self._ctx, 1 if enable else 0))
 
     def graph_replays(self):
         n = ctypes.c_int64()

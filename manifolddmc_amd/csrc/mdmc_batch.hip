@@ -542,7 +542,7 @@ void Pipeline::regroupBatch(int B) {
     const int64_t* h = (const int64_t*)pinBatch(words * sizeof(int64_t));
     MDMC_HIP(hipMemcpyAsync((void*)h, res, words * sizeof(int64_t), hipMemcpyDeviceToHost, stream));
     const int64_t* ctr = readCounters();
-    if (initUnchecked || refreshUnchecked) checkNM(ctr);
+    checkNM(ctr);
     if (*(const int*)(h + 5 * (nb + 1) + 9 * nb)) throw HipError("batched form: elements out of problem order", -4);
     batchDmc.resize(2 * nb);
     for (size_t b = 0; b < nb; ++b) {

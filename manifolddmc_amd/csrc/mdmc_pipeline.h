@@ -110,6 +110,8 @@ class Pipeline {
     bool localMerges = true;
     // the splitter's merge phase always in the one-thread ascending pass (a verification switch)
     bool sequentialMerges = false;
+    // a chain's compaction counts one quad as inconsistent (a verification switch)
+    bool failCompaction = false;
     int64_t graphReplays = 0;
     int nProblems = 1;
     ProblemDev* probsDev = nullptr;
@@ -240,9 +242,6 @@ class Pipeline {
     // a refresh ran whose face-walk check (the invalid-record counter) is not read back yet
     bool refreshUnchecked = false;
     void checkValid(const char* what);
-    // after a wait: whether the initialize's quads were consistent (its count raises a pinned word)
-    void checkInit();
-    bool initUnchecked = false;
     void emitArgs(GridPassArgs& a, int64_t C, bool recordAdjoint);
     void launchChain(int from, bool ended);
     void launchCompaction();

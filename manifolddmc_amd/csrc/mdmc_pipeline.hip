@@ -87,10 +87,12 @@ __device__ __forceinline__ int64_t sumParts(const int64_t* parts, int lane) {
 // The kernels that end an extraction are launched behind the list of the non-manifold faces
 // without waiting for its length (kAwaitSplit): they return at once where faces are left to
 // split, or a check failed, and the host then splits and launches them again.  The statistics
-// also wait (kAwaitFans) where the fan detection left vertices to its slow pass.
-enum : int { kAwaitSplit = 1, kAwaitFans = 2 };
+// also wait (kAwaitFans) where the fan detection left vertices to its slow pass.  A batch's fan
+// detection, which follows its split, waits for the checks alone (kAwaitValid).
+enum : int { kAwaitSplit = 1, kAwaitFans = 2, kAwaitValid = 4 };
 __device__ __forceinline__ bool notYet(const int64_t* ctr, int guarded) {
-    return ((guarded & kAwaitSplit) && (ctr[A_NM] != 0 || ctr[A_INVALID] != 0)) || ((guarded & kAwaitFans) && ctr[A_NSLOW] != 0);
+    return ((guarded & (kAwaitSplit | kAwaitValid)) && ctr[A_INVALID] != 0) || ((guarded & kAwaitSplit) && ctr[A_NM] != 0) ||
+           ((guarded & kAwaitFans) && ctr[A_NSLOW] != 0);
 }
 
 // a failed check: counted, and reported through the pinned word whose address the counters hold,
@@ -879,6 +881,9 @@ constexpr int kOldCentre = 1 << 30;  // in oldQ: the old quad is the centre of a
 // back in parts: 2.7 GB instead of 1.4).  Bound by HBM: 2.3 GB moved at the 512^3 gyroid in 579 us
 // (616 with the records stored through the caches, and the twin repair behind it 214 instead of 203); a
 // thread per halfedge 944 us, the records stored by quad 839 us.
+// The compaction checks the quads' new corners, but the host may go on before it has looked (it waits for
+// the numbering's totals only): with a bad one, every record is a boundary halfedge of vertex 0, as in
+// kBuildHalfedges, no corner is followed, and the next read-back reports it.
 __global__ void __launch_bounds__(kBlock) kRemapRebuild(const int4* __restrict__ quads2, int64_t H2, const uint8_t* __restrict__ touched,
                                                         const int32_t* __restrict__ oldQ, const int32_t* __restrict__ twinOld, int64_t Hold,
                                                         const uint32_t* __restrict__ bpackOld,
@@ -889,9 +894,13 @@ __global__ void __launch_bounds__(kBlock) kRemapRebuild(const int4* __restrict__
     __shared__ __align__(16) int s_v[4 * kBlock], s_t[4 * kBlock];
     __shared__ int s_list[4 * kBlock];
     __shared__ int s_n;
+    const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (ctr[A_INVALID] != 0) {
+        for (int i = 0; i < 4 && f < H2 / 4; ++i) storeRecord((int)(4 * f + i), 0, BucketOf{2, 1, -1}, he, bsize, brank, vflags, fattr);
+        return;
+    }
     if (threadIdx.x == 0) s_n = 0;
     __syncthreads();
-    const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     int slotted = 0;
     if (f < H2 / 4) {
         const int4 q = quads2[f];
@@ -3206,7 +3215,7 @@ int64_t Pipeline::checkNM(const int64_t* h) {
     if (h[A_INVALID])
         throw HipError(std::string("inconsistent mesh after ") + (refreshUnchecked ? "splitting" : "quad vertex ids") + " (" +
                            std::to_string(h[A_INVALID]) + " bad ids)", -4);
-    initUnchecked = refreshUnchecked = false;
+    refreshUnchecked = false;
     const int64_t n = h[A_NM];
     if (n < 0 || n > F) throw HipError("inconsistent NM-face count (" + std::to_string(n) + ")", -4);
     return n;
@@ -3274,7 +3283,6 @@ void Pipeline::prepare(const std::vector<ProblemDev>& problems, bool captured) {
     su.token = captured ? 0 : ++prepToken_;
     pinHost()[kPinSpecial] = 0;
     pinHost()[kPinInvalid] = 0;
-    initUnchecked = false;
     launchPrepareGrids(prep.desc[0], prep.dev, (int)prep.desc.size(), prep.rows, prep.refinement, prep.pad, su, stream);
 }
 
@@ -3515,7 +3523,6 @@ bool Pipeline::runFrontGraph(const std::vector<int64_t>& shapeSig, std::vector<P
         std::memcpy((char*)fg_.stage + probOff, problems.data(), pbytes);
         probsDev = arena.ptr<ProblemDev>("gp_probs");
         refreshUnchecked = false;
-        initUnchecked = false;
         pinHost()[kPinSpecial] = 0;
         pinHost()[kPinInvalid] = 0;
         expectTotals();
@@ -3691,7 +3698,6 @@ void Pipeline::halfedgeInitialize() {
     launchQuadLists(quads, qattr, Q, V, arena.ptr<int32_t>("gp_vcell"), arena.ptr<uint16_t>("gp_vct"), pid(), probsDev, off, out, twin, bpack, face_he,
                     fattr,
                     counters() + A_INVALID, pinDev() + kPinInvalid, stream);
-    initUnchecked = true;
     if (!chain.empty()) {
         if (H > 0)
             kBucketsAll<<<gridFor(H), kBlock, 0, stream>>>(quads, H, off, out, twin, bpack, vflags, fattr, qattr, arena.ptr<int32_t>("valence"),
@@ -3707,12 +3713,6 @@ void Pipeline::halfedgeInitialize() {
     listsV = V;
     splitTouched = false;
     canonTracked = false;
-}
-
-void Pipeline::checkInit() {
-    if (!initUnchecked) return;
-    initUnchecked = false;
-    if (pinHost()[kPinInvalid]) checkValid("quad vertex ids");
 }
 
 void Pipeline::checkValid(const char* what) {
@@ -3800,7 +3800,6 @@ void Pipeline::simplify() {
         launchChain(from, ended);
         const volatile int64_t* hv = h;  // where the totals are written, no kernel before them was held
         await([&] { return totalsWritten() || hv[kPinInvalid] || hv[kPinFallback] || hv[kPinFallback + 1]; });
-        initUnchecked = false;
         if (!totalsWritten()) MDMC_HIP(hipStreamSynchronize(stream));
         if (h[kPinInvalid]) checkValid("quad vertex ids");
         int s = 0;
@@ -3962,6 +3961,7 @@ void Pipeline::launchCompaction() {
     if (Q > 0)
         kCompactQuads<<<gridFor(Q), kBlock, 0, stream>>>(quads, attr, Q, vtarget, address, p3333 ? 1 : 0, nquads, nattr, nfattr, face_he, oldQ, qnew,
                                                          removedAt, outdeg, touched, chained ? arena.ptr<uint8_t>("vdead") : nullptr, V, step, counters());
+    if (failCompaction) launchFill(counters() + A_INVALID, 0x01, 1);  // as if a corner was out of range
 }
 
 // the compacted mesh's lists and records, once its sizes are known
@@ -4288,12 +4288,9 @@ void Pipeline::launchDetect(int guarded) {
 }
 
 void Pipeline::detectNonManifoldVertices() {
-    if (initUnchecked) {  // the walks follow the lists
-        MDMC_HIP(hipStreamSynchronize(stream));
-        checkInit();
-    }
-    launchDetect(0);
+    launchDetect(kAwaitValid);  // the walks follow the lists
     const int64_t* h = readCounters();
+    if (h[A_INVALID]) checkNM(h);
     if (h[A_NSLOW]) detectSlow(h[A_NSLOW], h[A_NSLOW_OFF]);
 }
 
