@@ -1176,7 +1176,8 @@ __global__ void __launch_bounds__(kBlock) kDropVertices(const uint8_t* __restric
                                                         const int32_t* __restrict__ out, uint8_t* __restrict__ vdead, int32_t* __restrict__ head,
                                                         int32_t* __restrict__ next, int32_t* __restrict__ outdeg, const int2* __restrict__ zslot,
                                                         int step, int64_t* ctr) {
-    if (chainHeld(ctr, step)) return;
+    // (as one block: another may count an invalid target between two waves' looks)
+    if (__syncthreads_or(chainHeld(ctr, step) ? 1 : 0)) return;
     __shared__ int s_list[kSparsePer * kBlock];
     __shared__ int s_n;
     const int total = gatherSparse(V, [&](int64_t i) { return vtype[i] == dropType; }, s_list, &s_n);
