@@ -211,7 +211,8 @@ mdmc_status mdmc_batch_stats(const mdmc_ctx* ctx, mdmc_stats* per_problem);
  * to dL_dfield (device float[dims[0]*dims[1]*dims[2]] of the grid passed to mdmc_extract),
  * through the dual-vertex formula of CellIntersection::sliceP (CellIntersection.inl:368-439)
  * and the padding / refinement of refineGrid (UniformGrid.inl:279-319).  accumulate = 1 adds
- * to dL_dfield instead of overwriting it.  Asynchronous on the context's stream; deterministic. */
+ * to dL_dfield instead of overwriting it.  Asynchronous on the context's stream; deterministic.
+ * A following call on another stream waits for it (but not for one that a caller's graph replays). */
 mdmc_status mdmc_backward(mdmc_ctx* ctx, const float* dL_dpos, float* dL_dfield, int32_t accumulate);
 
 /* No reference counterpart: mdmc_backward for callers that cannot allocate device memory
@@ -226,8 +227,7 @@ mdmc_status mdmc_backward_noalloc(mdmc_ctx* ctx, const float* dL_dpos, float* dL
 
 /* The surface as an autograd graph holds it (no reference counterpart): positions float[3*nV] and
  * the faces' vertex ids int64[4*nF] in walk order (Mesh.cu:446-506), device buffers; either may be
- * NULL.  Asynchronous on the context's stream, like mdmc_backward; a following mdmc_extract on another
- * stream waits for it. */
+ * NULL.  Asynchronous on the context's stream, like mdmc_backward. */
 mdmc_status mdmc_mesh_quads(const mdmc_ctx* ctx, float* positions, int64_t* quads);
 
 /* Triangle index buffer, two triangles per face (x,y,z),(z,w,x): HalfedgeMesh.cu:690-714.

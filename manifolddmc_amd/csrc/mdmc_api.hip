@@ -33,9 +33,11 @@ struct mdmc_ctx {
     mdmc::Pipeline p;
     std::string err;
     bool hasResult = false;
-    // the last mdmc_mesh_quads reads the mesh on quadsStream until this event
-    hipEvent_t quadsRead = nullptr;
-    hipStream_t quadsStream = nullptr;
+    // the last asynchronous call (mdmc_mesh_quads, the backwards) uses the result on readStream until
+    // this event, and so did those before it
+    hipEvent_t lastRead = nullptr;
+    hipStream_t readStream = nullptr;
+    bool hasReader = false;
     AdjointState adj;
     int nProblems = 0;  // problems of the resident result
     int flags = 0;
@@ -81,6 +83,28 @@ void launchAdjoint(const AdjointState& a, const int32_t* map, const int32_t* cel
         mdmc::launchAdjointPoints(a.outDims, a.outDims, 0, map, cell, a.V, contrib, dproc, 0, s);
         mdmc::launchPrepareAdjoint(a.inDims, a.outDims, a.refinement, a.pad, dproc, dL_dfield, accumulate, s);
     }
+}
+
+// The context's buffers are free for stream s once the asynchronous calls on another one are done.
+// Inside a capture there is no such order to be had: the caller's graph has to be placed by its caller.
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+void awaitReaders(mdmc_ctx* ctx, hipStream_t s) {
+    if (!ctx->hasReader || (!s && !ctx->readStream)) return;
+    // (an equal handle can be a newer stream's; a wait on the event's own stream queues nothing)
+    if (!capturing(s)) MDMC_HIP(hipStreamWaitEvent(s, ctx->lastRead, 0));
+}
+// The event is recorded at once (309 us a step of the 65^3 spheres without one behind the backward, 316 with):
+// by the time the context is given another stream, this one may be gone.
+void noteReader(mdmc_ctx* ctx, hipStream_t s) {
+    if (capturing(s)) return;
+    MDMC_HIP(hipEventRecord(ctx->lastRead, s));
+    ctx->readStream = s;
+    ctx->hasReader = true;
 }
 
 struct DeviceGuard {
@@ -131,7 +155,9 @@ mdmc_status mdmc_create(mdmc_ctx** out, int32_t device) {
     mdmc_ctx* ctx = new (std::nothrow) mdmc_ctx();
     if (!ctx) return MDMC_ERR_OOM;
     ctx->device = dev;
-    if (hipStreamCreateWithFlags(&ctx->own, hipStreamNonBlocking) != hipSuccess) {
+    if (hipStreamCreateWithFlags(&ctx->own, hipStreamNonBlocking) != hipSuccess ||
+        hipEventCreateWithFlags(&ctx->lastRead, hipEventDisableTiming) != hipSuccess) {
+        if (ctx->own) (void)hipStreamDestroy(ctx->own);
         delete ctx;
         return MDMC_ERR_HIP;
     }
@@ -146,7 +172,7 @@ void mdmc_destroy(mdmc_ctx* ctx) {
         DeviceGuard g(ctx->device);
         (void)hipStreamSynchronize(ctx->p.stream);
         ctx->p.arena.release();
-        if (ctx->quadsRead) (void)hipEventDestroy(ctx->quadsRead);
+        if (ctx->lastRead) (void)hipEventDestroy(ctx->lastRead);
         if (ctx->own) (void)hipStreamDestroy(ctx->own);
     }
     delete ctx;
@@ -231,7 +257,8 @@ mdmc_status runExtraction(mdmc_ctx* ctx, const mdmc_grid* grids, int G, const fl
     const int B = G * I;
     try {
         hipStream_t s = p.stream;
-        if (ctx->quadsRead && ctx->quadsStream != s) MDMC_HIP(hipStreamWaitEvent(s, ctx->quadsRead, 0));
+        awaitReaders(ctx, s);
+        ctx->hasReader = false;
         p.splitIterations = 0;
         p.extraAnomalies = 0;
         p.setChain((flags & MDMC_P3X3Y_COLOR) != 0, (flags & MDMC_P3X3Y_OLD) != 0, (flags & MDMC_P3333) != 0);
@@ -468,8 +495,14 @@ mdmc_status mdmc_backward_noalloc(mdmc_ctx* ctx, const float* dL_dpos, float* dL
     const int32_t* cell = p.arena.ptr<int32_t>("gp_vcell");
     // contributions at the start of the scratch, the processed-grid gradient after them (both
     // written in full by their kernels, so nothing from an earlier call needs clearing)
-    launchAdjoint(a, map, cell, dL_dpos, base, base + 8 * a.V, dL_dfield, accumulate ? 1 : 0, s);
-    if (hipGetLastError() != hipSuccess) return fail(ctx, MDMC_ERR_HIP, "mdmc_backward_noalloc: kernel launch failed");
+    try {
+        awaitReaders(ctx, s);
+        launchAdjoint(a, map, cell, dL_dpos, base, base + 8 * a.V, dL_dfield, accumulate ? 1 : 0, s);
+        if (hipGetLastError() != hipSuccess) return fail(ctx, MDMC_ERR_HIP, "mdmc_backward_noalloc: kernel launch failed");
+        noteReader(ctx, s);
+    } catch (const std::exception& e) {
+        return fromException(ctx, e);
+    }
     return MDMC_OK;
 }
 
@@ -484,6 +517,7 @@ mdmc_status mdmc_backward(mdmc_ctx* ctx, const float* dL_dpos, float* dL_dfield,
     mdmc::Pipeline& p = ctx->p;
     try {
         hipStream_t s = p.stream;
+        awaitReaders(ctx, s);  // (they share the scratch, too)
         const int32_t* map = p.arena.ptr<int32_t>("adj_map");
         const int32_t* cell = p.arena.ptr<int32_t>("gp_vcell");
         float* contrib = p.arena.get<float>("adj_contrib", 8 * (size_t)std::max<int64_t>(a.V, 1));
@@ -491,6 +525,7 @@ mdmc_status mdmc_backward(mdmc_ctx* ctx, const float* dL_dpos, float* dL_dfield,
         float* dproc = a.refinement ? p.arena.get<float>("adj_dproc", P) : nullptr;
         launchAdjoint(a, map, cell, dL_dpos, contrib, dproc, dL_dfield, accumulate ? 1 : 0, s);
         MDMC_HIP(hipGetLastError());
+        noteReader(ctx, s);
         return MDMC_OK;
     } catch (const std::exception& e) {
         (void)hipStreamSynchronize(p.stream);
@@ -528,11 +563,10 @@ mdmc_status mdmc_mesh_quads(const mdmc_ctx* cctx, float* positions, int64_t* qua
     DeviceGuard dg(ctx->device);
     try {
         mdmc::Pipeline& p = ctx->p;
-        if (!ctx->quadsRead) MDMC_HIP(hipEventCreateWithFlags(&ctx->quadsRead, hipEventDisableTiming));
+        awaitReaders(ctx, p.stream);
         MDMC_HIP(mdmc::launchQuadIds(p.arena.ptr<int4>("he"), p.arena.ptr<int32_t>("face_he"), p.F, p.arena.ptr<float>("pos"), p.V, positions, quads,
                                      p.stream));
-        ctx->quadsStream = p.stream;
-        MDMC_HIP(hipEventRecord(ctx->quadsRead, p.stream));
+        noteReader(ctx, p.stream);
         return MDMC_OK;
     } catch (const std::exception& e) {
         return fromException(ctx, e);
