@@ -86,7 +86,8 @@ typedef struct {
                           read, fan walks past 4096 steps, buckets past 16 halfedges); 0 normally */
     int64_t cells;     /* cells of the processed grid */
     /* stage times (ms, the GPU's clock at the start of each stage's first kernel): whole call,
-     * pad/refine, DMC grid pass, halfedge build, simplifications, twin repair, split, detection */
+     * upload of host fields and pad/refine, DMC grid pass, halfedge build, simplifications, twin
+     * repair, split, detection */
     double ms_total, ms_grid, ms_dmc, ms_halfedge, ms_simplify, ms_fix_twins, ms_split, ms_detect;
     /* the grid-pass kernel alone (classification, dual vertices, quads) */
     double ms_grid_pass_kernel;

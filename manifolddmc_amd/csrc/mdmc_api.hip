@@ -265,6 +265,7 @@ mdmc_status runExtraction(mdmc_ctx* ctx, const mdmc_grid* grids, int G, const fl
         // ---- grids: upload if needed, then pad / refine (refineGrid)
         float* gp = p.arena.get<float>("grid", (size_t)Ptot);
         float* up = PinTot ? p.arena.get<float>("input", (size_t)PinTot) : nullptr;
+        p.stampUpload(PinTot > 0);
         std::vector<mdmc::ProblemDev> problems;
         problems.reserve((size_t)B);
         std::vector<mdmc::PrepareDesc>& prep = p.prep.desc;

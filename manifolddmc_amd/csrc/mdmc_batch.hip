@@ -31,9 +31,6 @@ namespace {
 
 __device__ __forceinline__ int heO(const int4* he, int h) { return ((const int*)he)[4 * (int64_t)h]; }
 
-// the clock alone, where no kernel begins or ends a stage
-__global__ void kStamp(int64_t* stamp) { *stamp = wall_clock64(); }
-
 __global__ void kIota(int32_t* __restrict__ p, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = (int32_t)i;
@@ -538,7 +535,7 @@ void Pipeline::regroupBatch(int B) {
         launchRegroup<RG_V, false>(m, V, stream);
     }
     batchVertHe = true;
-    kStamp<<<1, 1, 0, stream>>>(stamp(ST_END));
+    launchStamp(stamp(ST_END));
     const int64_t* h = (const int64_t*)pinBatch(words * sizeof(int64_t));
     MDMC_HIP(hipMemcpyAsync((void*)h, res, words * sizeof(int64_t), hipMemcpyDeviceToHost, stream));
     const int64_t* ctr = readCounters();

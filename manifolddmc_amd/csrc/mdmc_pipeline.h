@@ -80,6 +80,9 @@ class Pipeline {
     // seven stages of mdmc_stats in order, then the grid pass alone
     void stageTimes(double ms[9]);
     int64_t* stamp(int slot);
+    void launchStamp(int64_t* at);
+    // before any upload of a field: where the first stage's time then begins
+    void stampUpload(bool uploads);
     // device word the single-pass scans and compactions count their direct-sum tiles in
     int64_t* lookbackDiag();
 

@@ -164,8 +164,9 @@ __device__ __forceinline__ bool vec4(int64_t i0, int64_t n, const void* a, const
 }
 
 // pinned words: the padding pass's "needs the exact blend", the initialize's "inconsistent
-// quads", a deferred simplification's "region rebuild needed", the copy of the counters at the end
-constexpr int kPinSpecial = 3, kPinInvalid = 4, kPinFallback = 5 /* two steps */, kPinFinal = 16;
+// quads", a deferred simplification's "region rebuild needed", the clock ahead of the uploads, the
+// copy of the counters at the end
+constexpr int kPinSpecial = 3, kPinInvalid = 4, kPinFallback = 5 /* two steps */, kPinUpload = 7, kPinFinal = 16;
 // and behind that copy the word that says that it is whole
 constexpr int kPinDone = kPinFinal + A_NCOUNTERS;
 static_assert(kPinDone < Pipeline::kPinSlots && A_NCOUNTERS < 64, "pinned words, handed over by one wave");
@@ -178,6 +179,8 @@ __device__ __forceinline__ void handOver(const int64_t* ctr, int64_t* pin) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (k == 0) p[A_NCOUNTERS] = 1;
 }
+// the clock alone, where no kernel begins or ends a stage
+__global__ void kStamp(int64_t* stamp) { *stamp = wall_clock64(); }
 __global__ void kReadBack(const int64_t* __restrict__ ctr, int64_t* pin) { handOver(ctr, pin); }
 
 // ---------------------------------------------------------------- halfedge construction
@@ -3302,6 +3305,12 @@ void Pipeline::finishPrepare(bool totalsBehind, Again again) {
 int64_t* Pipeline::lookbackDiag() { return counters() + A_LB_DIRECT; }
 
 int64_t* Pipeline::stamp(int slot) { return counters() + A_STAMP + slot; }
+void Pipeline::launchStamp(int64_t* at) { kStamp<<<1, 1, 0, stream>>>(at); }
+// the counters are cleared behind the uploads, so this stamp goes to the pinned words
+void Pipeline::stampUpload(bool uploads) {
+    pinHost()[kPinUpload] = 0;
+    if (uploads) launchStamp(pinDev() + kPinUpload);
+}
 
 void Pipeline::counterTotals(int64_t* anomalyCount, int64_t* mergeSeq, int64_t* lookbackDirect) {
     const int64_t* h = pinHost() + kPinFinal;
@@ -3322,6 +3331,7 @@ void Pipeline::stageTimes(double ms[9]) {
     std::memcpy(t, pinHost() + kPinFinal + A_STAMP, sizeof t);
     for (int i = ST_END - 1; i >= 0; --i)
         if (t[i] == 0) t[i] = t[i + 1];
+    if (pinHost()[kPinUpload]) t[ST_PAD] = pinHost()[kPinUpload];
     const double k = 1.0 / clockKHz_;
     ms[0] = (double)(t[ST_END] - t[ST_PAD]) * k;
     for (int i = 0; i < 7; ++i) ms[1 + i] = (double)(t[i + 1] - t[i]) * k;
