@@ -204,7 +204,6 @@ class Pipeline {
     void expectTotals();
     bool totalsWritten();
     void zero(void* p, size_t bytes);
-    void fillNeg(void* p, size_t bytes);
     void launchFill(void* p, uint8_t byte, size_t bytes);
     // fills collected and launched together (at flush or at the end of the scope)
     class FillBatch {

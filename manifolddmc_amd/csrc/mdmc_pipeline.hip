@@ -20,7 +20,6 @@
 #include <algorithm>
 #include <atomic>
 #include <chrono>
-#include <chrono>
 #include <cstring>
 #include <vector>
 
@@ -1344,7 +1343,7 @@ __global__ void __launch_bounds__(kBlock) kAffectedFlags(const uint8_t* __restri
 }
 
 // list lengths of the fan detection's slow vertices: their out-degree (the halfedges
-// kOutDegree / the outgoing lists counted per origin), 0 for the others
+// kOutFromLists and kOutDegreeMoved counted per origin), 0 for the others
 // (outdeg null: the build's list lengths)
 __global__ void kSlowDegree(const uint8_t* __restrict__ slow, const int32_t* __restrict__ outdeg, const int64_t* __restrict__ listOff, int64_t V,
                             int32_t* __restrict__ deg) {
@@ -1376,27 +1375,13 @@ __global__ void kFillLists(const int4* __restrict__ he, int64_t H, int64_t V, co
     if (slot >= 0) list[off[o] + slot] = (int32_t)h;
 }
 
-// out-degree of every vertex and one of its outgoing halfedges
-__global__ void kOutDegree(const int4* __restrict__ he, int64_t H, int64_t V, int32_t* __restrict__ outdeg, int32_t* __restrict__ rep,
-                           int64_t* ctr) {
-    const int64_t h = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= H) return;
-    const int o = heO(he, (int)h);
-    if (o < 0 || o >= V) {
-        anomaly(ctr);
-        return;
-    }
-    if (atomicAdd(&outdeg[o], 1) == 0) rep[o] = (int32_t)h;
-}
-
 // out-degree and one outgoing halfedge from the outgoing lists of the last build, for the
 // vertices they still describe: those below listsV that no split step touched (a split
 // step rewrites only halfedges whose origin is in its working copy, before and after).
-// With the layout flags (canon), a touched vertex counts the entries of its list whose
+// By the layout flags (canon), a touched vertex counts the entries of its list whose
 // records keep the build's layout (never written back, so still starting at it; the
 // block's touched vertices are gathered in LDS, their list walks run on full waves) and
-// kOutDegreeMoved adds the records the splitter wrote; without them kOutDegreeTouched
-// counts every touched vertex from all records.  Vertices from listsV on are counted there.
+// kOutDegreeMoved adds the records the splitter wrote, those of the vertices from listsV on among them.
 __global__ void __launch_bounds__(kBlock) kOutFromLists(const int64_t* __restrict__ off, const int32_t* __restrict__ out, int64_t listsV,
                                                         const uint8_t* __restrict__ touched, const uint8_t* __restrict__ canon, int64_t V,
                                                         int32_t* __restrict__ outdeg, int32_t* __restrict__ rep, int64_t* ctr, int guarded) {
@@ -1415,7 +1400,7 @@ __global__ void __launch_bounds__(kBlock) kOutFromLists(const int64_t* __restric
                 return false;
             }
             outdeg[v] = 0;
-            return v < listsV && canon != nullptr;
+            return v < listsV;
         },
         s_list, &s_n);
     for (int j = threadIdx.x; j < total; j += kBlock) {
@@ -1481,19 +1466,6 @@ __global__ void __launch_bounds__(kBlock) kOutDegreeMoved(const int4* __restrict
         if (o >= listsV || (touched && touched[o]))
             if (atomicAdd(&outdeg[o], 1) == 0) rep[o] = h;
     }
-}
-
-__global__ void kOutDegreeTouched(const int4* __restrict__ he, int64_t H, int64_t V, int64_t listsV, const uint8_t* __restrict__ touched,
-                                  int32_t* __restrict__ outdeg, int32_t* __restrict__ rep, int64_t* ctr) {
-    const int64_t h = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= H) return;
-    const int o = heO(he, (int)h);
-    if (o < 0 || o >= V) {
-        anomaly(ctr);
-        return;
-    }
-    if (o >= listsV || (touched && touched[o]))
-        if (atomicAdd(&outdeg[o], 1) == 0) rep[o] = (int32_t)h;
 }
 
 // A vertex whose outgoing halfedges form one closed clockwise cycle (next(twin(h)) from
@@ -3233,7 +3205,6 @@ const int64_t* Pipeline::readCounters() {
 
 // fills with one launch (the runtime's memset launches a body and a tail kernel)
 void Pipeline::zero(void* p, size_t bytes) { launchFill(p, 0x00, bytes); }
-void Pipeline::fillNeg(void* p, size_t bytes) { launchFill(p, 0xFF, bytes); }
 void Pipeline::launchFill(void* p, uint8_t byte, size_t bytes) {
     if (bytes == 0) return;
     const size_t head = std::min<size_t>((16 - ((uintptr_t)p & 15)) & 15, bytes);
@@ -4270,32 +4241,19 @@ void Pipeline::launchDetect(int guarded) {
     uint8_t* slow = arena.get<uint8_t>("fan_slow", (size_t)V);
     const int64_t *off = arena.ptr<int64_t>("out_off");
     const int32_t* out = arena.ptr<int32_t>("out_list");
-    const bool fromLists = listsV >= 0 && listsV <= V;
-    const uint8_t* touched = (fromLists && splitTouched) ? arena.ptr<uint8_t>("split_touched") : nullptr;
-    const uint8_t* canon = canonFlags();  // kept since the splitter's first write-back
-    if (fromLists && listsV == V && !touched && !canon) {
+    const uint8_t* canon = canonFlags();  // kept since the splitter's first write-back, as its touched flags
+    if (!canon) {
         kFanFast<true><<<gridFor(V), kBlock, 0, stream>>>(he, H, V, off, out, nullptr, nullptr, vflags, slow, nullptr, V, nullptr, counters(), guarded);
         return;
     }
+    const uint8_t* touched = arena.ptr<uint8_t>("split_touched");
     int32_t* outdeg = arena.get<int32_t>("outdeg", (size_t)V);
     int32_t* rep = arena.get<int32_t>("outrep", (size_t)V);
-    if (fromLists) {
-        // (writes every vertex's out-degree)
-        kOutFromLists<<<sparseBlocks(V), kBlock, 0, stream>>>(off, out, listsV, touched, canon, V, outdeg, rep, counters(), guarded);
-        if (canon) {
-            if (recordsPerLane(H) == 4)
-                kOutDegreeMoved<4><<<gridFor((H + 3) / 4), kBlock, 0, stream>>>(he, H, V, listsV, touched, canon, outdeg, rep, counters(), guarded);
-            else
-                kOutDegreeMoved<16><<<gridFor((H + 15) / 16), kBlock, 0, stream>>>(he, H, V, listsV, touched, canon, outdeg, rep, counters(), guarded);
-        } else if (touched || V > listsV) {
-            kOutDegreeTouched<<<gridFor(H), kBlock, 0, stream>>>(he, H, V, listsV, touched, outdeg, rep, counters());
-        }
-    } else {
-        zero(outdeg, (size_t)V * sizeof(int32_t));
-        kOutDegree<<<gridFor(H), kBlock, 0, stream>>>(he, H, V, outdeg, rep, counters());
-    }
-    kFanFast<false><<<gridFor(V), kBlock, 0, stream>>>(he, H, V, off, out, outdeg, rep, vflags, slow, touched, fromLists ? listsV : 0, canon, counters(),
-                                                       guarded);
+    // (writes every vertex's out-degree)
+    kOutFromLists<<<sparseBlocks(V), kBlock, 0, stream>>>(off, out, listsV, touched, canon, V, outdeg, rep, counters(), guarded);
+    if (recordsPerLane(H) == 4) kOutDegreeMoved<4><<<gridFor((H + 3) / 4), kBlock, 0, stream>>>(he, H, V, listsV, touched, canon, outdeg, rep, counters(), guarded);
+    else kOutDegreeMoved<16><<<gridFor((H + 15) / 16), kBlock, 0, stream>>>(he, H, V, listsV, touched, canon, outdeg, rep, counters(), guarded);
+    kFanFast<false><<<gridFor(V), kBlock, 0, stream>>>(he, H, V, off, out, outdeg, rep, vflags, slow, touched, listsV, canon, counters(), guarded);
 }
 
 void Pipeline::detectNonManifoldVertices() {
