@@ -14,8 +14,9 @@ def sphere(r):
     return (np.sqrt(t[:, None, None] ** 2 + t[None, :, None] ** 2 + t[None, None, :] ** 2) - r).astype(np.float32)
 
 
+@pytest.mark.parametrize("first", ["stream", "default", "own"])
 @pytest.mark.parametrize("call", ["backward", "backward_noalloc", "two backwards", "quads"])
-def test_extraction_on_another_stream_waits(call):
+def test_extraction_on_another_stream_waits(call, first):
     import torch
 
     import manifolddmc_amd as mdmc
@@ -29,8 +30,11 @@ def test_extraction_on_another_stream_waits(call):
         d.extract_raw(f.data_ptr(), SHAPE, (-1, -1, -1), (2 / (N - 1),) * 3, 0.0, flags, 0, True)
         return d.info()
 
+    handle = {"stream": a.cuda_stream, "default": mdmc.DEFAULT_STREAM, "own": 0}[first]
+    queue = {"stream": a, "default": torch.cuda.default_stream(), "own": None}[first]
+
     def read(stream, dpos, out, use):
-        d.set_stream(stream.cuda_stream)
+        d.set_stream(handle if stream is a else stream.cuda_stream)
         if use == "quads":
             d.copy_quads(out[0].data_ptr(), out[1].data_ptr())
         elif use == "backward_noalloc":
@@ -40,7 +44,7 @@ def test_extraction_on_another_stream_waits(call):
 
     try:
         torch.cuda.synchronize()
-        d.set_stream(a.cuda_stream)
+        d.set_stream(handle)
         V, _, F = extract(big)
         dpos = torch.randn((V, 3), device="cuda", generator=torch.Generator(device="cuda").manual_seed(5))
         make = lambda: (torch.zeros((V, 3), device="cuda"), torch.zeros((F, 4), dtype=torch.int64, device="cuda")) if call == "quads" else (torch.zeros(SHAPE, device="cuda"),)
@@ -49,13 +53,14 @@ def test_extraction_on_another_stream_waits(call):
         read(a, dpos, want, call)
         torch.cuda.synchronize()
         for rep in range(3):
-            print("reader streams", call, rep, flush=True)
-            d.set_stream(a.cuda_stream)
+            print("reader streams", call, first, rep, flush=True)
+            d.set_stream(handle)
             assert extract(big) == (V, 4 * F, F)
-            with torch.cuda.stream(a):  # some ms of work that the reader stands behind
-                h = busy
-                for _ in range(12):
-                    h = h @ busy
+            if queue is not None:
+                with torch.cuda.stream(queue):  # some ms of work that the reader stands behind
+                    h = busy
+                    for _ in range(12):
+                        h = h @ busy
             read(a, dpos, got, call)
             if call == "two backwards":
                 read(c, dpos, more, call)
