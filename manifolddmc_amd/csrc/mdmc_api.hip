@@ -487,6 +487,7 @@ mdmc_status mdmc_backward_noalloc(mdmc_ctx* ctx, const float* dL_dpos, float* dL
     if (!dL_dfield) return fail(ctx, MDMC_ERR_INVALID_ARG, "null dL_dfield");
     float* base = g_noallocScratch[ctx->device];
     if (!base) return fail(ctx, MDMC_ERR_INTERNAL, "no-allocation scratch not set up for this device");
+    // (with padding alone no launch uses the points' share; the limit counts it all the same)
     const bool direct = a.pad == 0 && a.refinement == 0;
     const int64_t P = (int64_t)a.outDims[0] * a.outDims[1] * a.outDims[2];
     const int64_t need = 8 * a.V + (direct ? 0 : P);
@@ -498,8 +499,8 @@ mdmc_status mdmc_backward_noalloc(mdmc_ctx* ctx, const float* dL_dpos, float* dL
     hipStream_t s = p.stream;
     const int32_t* map = p.arena.ptr<int32_t>("adj_map");
     const int32_t* cell = p.arena.ptr<int32_t>("gp_vcell");
-    // contributions at the start of the scratch, the processed-grid gradient after them (both
-    // written in full by their kernels, so nothing from an earlier call needs clearing)
+    // contributions at the start of the scratch, written in full; with refinement the processed-grid
+    // gradient after them, which the first launch clears: nothing from an earlier call is read
     try {
         awaitReaders(ctx, s);
         launchAdjoint(a, map, cell, dL_dpos, base, base + 8 * a.V, dL_dfield, accumulate ? 1 : 0, s);
